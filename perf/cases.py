@@ -270,9 +270,7 @@ _PREPARE = dict(layer=_prepare_layer, head=_prepare_head, projection=_prepare_pr
 
 
 def prepare(case, seed):
-    generator = torch.Generator(device="cuda")
-    generator.manual_seed(int(seed))
-    state = _PREPARE[case["kind"]](case, generator)
+    state = _PREPARE[case["kind"]](case, _generator(seed))
     state["kind"] = case["kind"]
     if "calls" in state:
         state["calls"] = engine.make_calls(state["calls"])
@@ -298,6 +296,111 @@ def run(state):
         return dict(q=q, scales=scales, y=state["y"])
     ctx.q4_sequence(state["calls"])
     return state["out"]
+
+
+# ---- the same in 64 bits, from the codes a state was made of -----------------------------------
+
+
+def _generator(seed):
+    generator = torch.Generator(device="cuda")
+    generator.manual_seed(int(seed))
+    return generator
+
+
+def _product64(x, N, K, values):
+    """x [M][K] times the transpose of a weight whose rows low .. high values(low, high) gives."""
+    y = torch.empty((x.shape[0], N), dtype=torch.float64, device="cuda")
+    for low, high in _row_blocks(N, K):
+        y[:, low:high] = x.double() @ values(low, high).t()
+    return y
+
+
+def _affine64(generator, N, K, meta, bits=4):
+    """A function of x: the product with the weight that _affine_planes draws here."""
+    codes, a, b = _affine_planes(generator, N, K, meta, bits)
+
+    def values(low, high):
+        q = codes[low:high]
+        q = q if bits == 8 else torch.stack((q & 15, q >> 4), dim=2)
+        scale, bias = (a[low:high, :, 0], a[low:high, :, 1]) if b is None else (a[low:high], b[low:high])
+        q = q.reshape(high - low, K // 64, 64).double()
+        return q.mul_(scale.double().unsqueeze(2)).add_(bias.double().unsqueeze(2)).view(high - low, K)
+
+    return lambda x: _product64(x, N, K, values)
+
+
+def _sym64(generator, N, K):
+    records = _sym128_records(generator, N, K)
+
+    def values(low, high):
+        scale = records[low:high, :, :2].contiguous().view(torch.bfloat16).double()
+        q = records[low:high, :, 2:]
+        q = torch.stack((q & 15, q >> 4), dim=3).view(high - low, K // 128, 128).double()
+        return torch.where(q < 8, q, q - 16).mul_(scale).view(high - low, K)
+
+    return lambda x: _product64(x, N, K, values)
+
+
+def _exact_layer(c, g):
+    M, H, I = c["rows"], c["hidden"], c["inter"]
+    shapes = dict(q=(c["q"], H), k=(c["kv"], H), v=(c["kv"], H), o=(H, c["q"]), gate=(I, H), up=(I, H), down=(H, I))
+    w = {name: _affine64(g, N, K, c["meta"]) for name, (N, K) in shapes.items()}
+    x, attended, x_mlp = _normal(g, (M, H)), _normal(g, (M, c["q"])), _normal(g, (M, H))
+    stream = _normal(g, (M, H), engine.F32).double()
+    y = {name: w[name](x) for name in ("q", "k", "v")}
+    y["o"] = w["o"](attended) + stream
+    gate, up = w["gate"](x_mlp), w["up"](x_mlp)
+    if M <= 16:
+        y["h"] = torch.nn.functional.silu(gate) * up
+        between = y["h"].half()  # an fp16 buffer between the two calls
+    else:
+        y["gate"], y["up"] = gate, up
+        between = _normal(g, (M, I))
+    y["down"] = w["down"](between) + stream
+    return y
+
+
+def _exact_encoder(c, g):
+    M, H, I = c["rows"], c["hidden"], c["inter"]
+    shapes = dict(q=(H, H), k=(H, H), v=(H, H), o=(H, H), fc1=(I, H), fc2=(H, I))
+    w = {name: _sym64(g, N, K) for name, (N, K) in shapes.items()}
+    b = {name: _normal(g, (N,), engine.F32, 0.1) for name, (N, K) in shapes.items()}
+    x = {name: _normal(g, (M, K), engine.F32) for name, K in (("qkv", H), ("o", H), ("fc1", H), ("fc2", I))}
+    return {name: w[name](x["qkv" if name in "qkv" else name]) + b[name].double() for name in shapes}
+
+
+def _exact_w8a8(c, g):
+    M, N, K = c["rows"], c["N"], c["K"]
+    weights = []
+    for _ in range(3):
+        w = torch.randn((N, K), device="cuda", generator=g).mul_(0.02)
+        scale = w.abs().amax(dim=1, keepdim=True) / 127
+        weights.append(((w / scale).round_().clamp_(-127, 127).double(), scale.double()))
+    x = _normal(g, (M, K), engine.F32)
+    bias = [_normal(g, (N,), engine.F32, 0.1) for _ in weights]
+    scales = x.abs().amax(dim=1) / 127
+    q = (x * (1 / scales).unsqueeze(1)).round_().double()
+    y = [(q @ w.t()) * scale.t() * scales.double().unsqueeze(1) + b.double() for (w, scale), b in zip(weights, bias)]
+    return dict(q=None, scales=x.abs().amax(dim=1).double() / 127, y=y)
+
+
+def exact(case, seed):
+    """What run() returns for these inputs, in 64 bits and with the weights' exact values."""
+    c, g = case, _generator(seed)
+    if c["kind"] == "layer":
+        return _exact_layer(c, g)
+    if c["kind"] == "encoder":
+        return _exact_encoder(c, g)
+    if c["kind"] == "w8a8":
+        return _exact_w8a8(c, g)
+    if c["kind"] == "hook":
+        weight = _sym64(g, c["N"], c["K"])
+        x, bias = _normal(g, (c["rows"], c["K"]), engine.F32), _normal(g, (c["N"],), engine.F32, 0.1)
+        return weight(x) + bias.double()
+    if c["kind"] == "head":
+        return _affine64(g, c["vocab"], c["hidden"], c["meta"])(_normal(g, (c["rows"], c["hidden"])))
+    weight = _affine64(g, c["N"], c["K"], c["meta"], 8 if c["kind"] == "q8" else 4)
+    return weight(_normal(g, (c["rows"], c["K"]), engine.BF16 if c.get("x") == "bf16" else engine.F16))
 
 
 # ---- what a pass cannot do without ----------------------------------------------------------
