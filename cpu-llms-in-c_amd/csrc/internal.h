@@ -53,7 +53,7 @@ struct Q4Device {
 }  // namespace mi355q
 
 namespace mi355q {
-constexpr int kStageSlots = 7;
+constexpr int kStageSlots = 6;
 }
 struct mi355q_context {
     int device;
@@ -67,8 +67,7 @@ struct mi355q_context {
     std::vector<hipEvent_t> *profile_events;
     size_t profile_used;
     // staging: 0 host x, 1 host y, 2 host residual, 3 activations converted to fp16,
-    // 4 fp32 partial sums of a K-split GEMM, 5 the high-nibble half of an affine-Q8 linear,
-    // 6 the fp32 outputs of a GEMM on converted activations, before their rows are finished
+    // 4 fp32 partial sums of a K-split GEMM, 5 the high-nibble half of an affine-Q8 linear
     void *stage[mi355q::kStageSlots];
     size_t stage_bytes[mi355q::kStageSlots];
     // bumped whenever a staging buffer is reallocated: recorded graphs hold the old
@@ -241,7 +240,8 @@ int chain_after_wait(mi355q_context *ctx, char *error, size_t error_capacity);
 int q4_linear_multi_repeated(mi355q_context *ctx, const mi355q_q4_target *targets, uint32_t count, const void *x,
                              int x_dtype, uint32_t M, int y_dtype, int residual_dtype, uint32_t flags,
                              uint32_t x_columns, char *error, size_t error_capacity);
-// q4_gemm.hip (one target at a time: `target` selects it)
+// q4_gemm.hip (one target at a time: `target` selects it; target 0 first, whose call converts
+// activations that are not fp16 for all of them)
 int q4_gemm_linear(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, char *error,
                    size_t error_capacity);
 

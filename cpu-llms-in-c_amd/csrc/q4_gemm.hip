@@ -46,67 +46,67 @@ extern template __global__ void q4_gemm_pipe_kernel<128, 3, true, false, true>(c
 // Adds the K splits in split order (a fixed order) and applies the epilogue.  WIDE: a thread
 // takes four adjacent outputs of one row (N a multiple of 4, y 16-byte aligned): 16-byte loads
 // of each split's partial sums and one store; the additions are the same, in the same order.
-template <bool WIDE>
-__global__ void __launch_bounds__(256) q4_gemm_reduce_kernel(const GemmParams p)
-{
-    const size_t total = (size_t)p.M * p.N;
-    constexpr size_t PER = WIDE ? 4 : 1;
-    const size_t at = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * PER;
-    if (at >= total) return;
-    if constexpr (WIDE) {
-        floatx4 value = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (uint32_t s = 0; s < p.splits; ++s) {
-            const floatx4 more = *(const floatx4 *)(p.partials + (size_t)s * total + at);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) value[j] += more[j];
-        }
-        if (p.residual) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                value[j] += load_as_float(p.residual, p.residual_dtype, p.residual_is_bias ? (at + j) % p.N : at + j);
-        }
-        if (p.y_dtype == MI355Q_F32) {
-            *(floatx4 *)((float *)p.y + at) = value;
-        } else if (p.y_dtype == MI355Q_F16) {
-            typedef _Float16 half4v __attribute__((ext_vector_type(4)));
-            const half4v packed = {(_Float16)value[0], (_Float16)value[1], (_Float16)value[2], (_Float16)value[3]};
-            *(half4v *)((_Float16 *)p.y + at) = packed;
-        } else {
-            *(uint2 *)((uint16_t *)p.y + at) = make_uint2(bf16_bits(value[0]) | (bf16_bits(value[1]) << 16),
-                                                          bf16_bits(value[2]) | (bf16_bits(value[3]) << 16));
-        }
-        return;
-    }
-    float value = 0.0f;
-    for (uint32_t s = 0; s < p.splits; ++s) value += p.partials[(size_t)s * total + at];
-    if (p.residual)
-        value += load_as_float(p.residual, p.residual_dtype, p.residual_is_bias ? at % p.N : at);
-    store_from_float(p.y, p.y_dtype, at, value);
-}
-
+//
 // Activations that are not fp16 get the streaming kernel's treatment (q4_convert_x_launch): every
 // row scaled by a power of two into fp16's range, bf16 rows as one fp16 row, fp32 rows as two
-// (value, rounding remainder).  The matrix kernels then multiply those M or 2 M rows into an fp32
-// staging matrix, and this kernel finishes the outputs: the two rows of a pair added, the row's
-// scale taken out again, then residual and output type as in the matrix kernels' own epilogue.
-// (The reference's grouped linear keeps fp32 activations at any row count,
-// whisper_turbo_encoder.c:128-176; cpu_q4_dot_float, qwen38_m3_layer.m:375-393.)
-__global__ void __launch_bounds__(256)
-q4_gemm_finish_kernel(const float *__restrict__ staged, const float *__restrict__ row_scale, int pair,
-                      void *__restrict__ y, int y_dtype, const void *__restrict__ residual, int residual_dtype,
-                      int residual_is_bias, uint32_t M, uint32_t N)
+// (value, rounding remainder).  The matrix kernels multiply those M or 2 M rows; whoever holds the
+// finished sums - their epilogue, or this kernel behind a K split - adds the two rows of a pair,
+// takes the row's scale out again, adds the residual and converts.  (The reference's grouped
+// linear keeps fp32 activations at any row count, whisper_turbo_encoder.c:128-176;
+// cpu_q4_dot_float, qwen38_m3_layer.m:375-393.)
+// A workgroup takes 256 (1024) adjacent columns of one output row: no index is ever divided (a
+// division per thread cost the 27B prefill step's reductions about a microsecond each).
+constexpr uint32_t kReduceThreads = 256;
+template <bool WIDE>
+__global__ void __launch_bounds__(kReduceThreads) q4_gemm_reduce_kernel(const GemmParams p)
 {
-    const size_t total = (size_t)M * N;
-    for (size_t at = (size_t)blockIdx.x * blockDim.x + threadIdx.x; at < total; at += (size_t)gridDim.x * blockDim.x) {
-        const uint32_t m = (uint32_t)(at / N), n = (uint32_t)(at % N);
-        float value;
-        if (pair)
-            value = staged[(size_t)(2u * m) * N + n] + staged[(size_t)(2u * m + 1u) * N + n];
-        else
-            value = staged[at];
-        value *= row_scale[m];
-        if (residual) value += load_as_float(residual, residual_dtype, residual_is_bias ? n : at);
-        store_from_float(y, y_dtype, at, value);
+    constexpr int PER = WIDE ? 4 : 1;
+    const uint32_t n = (blockIdx.x * kReduceThreads + threadIdx.x) * PER;
+    if (n >= p.N) return;
+    const size_t stride = (size_t)p.M * p.N;
+    auto add_splits = [&](size_t from, float (&value)[PER]) {
+#pragma unroll
+        for (int j = 0; j < PER; ++j) value[j] = 0.0f;
+        // eight splits' loads are on their way before the first is added: one trip to memory
+        // instead of one per split
+        typedef std::conditional_t<WIDE, floatx4, float> Piece;
+        for (uint32_t first = 0; first < p.splits; first += 8u) {
+            Piece piece[8];
+#pragma unroll
+            for (uint32_t s = 0; s < 8u; ++s)
+                if (first + s < p.splits) piece[s] = *(const Piece *)(p.partials + (first + s) * stride + from);
+#pragma unroll
+            for (uint32_t s = 0; s < 8u; ++s) {
+                if (first + s >= p.splits) continue;
+                if constexpr (WIDE) {
+#pragma unroll
+                    for (int j = 0; j < PER; ++j) value[j] += piece[s][j];
+                } else {
+                    value[0] += piece[s];
+                }
+            }
+        }
+    };
+    const uint32_t rows = p.pair ? p.M / 2u : p.M;
+    for (uint32_t m = blockIdx.y; m < rows; m += gridDim.y) {
+        float value[PER];
+        if (p.pair) {
+            float remainder[PER];
+            add_splits((size_t)(2u * m) * p.N + n, value);
+            add_splits((size_t)(2u * m + 1u) * p.N + n, remainder);
+#pragma unroll
+            for (int j = 0; j < PER; ++j) value[j] += remainder[j];
+        } else {
+            add_splits((size_t)m * p.N + n, value);
+        }
+        if constexpr (WIDE) {
+            finish_four(p, false, 0, m, n, floatx4{value[0], value[1], value[2], value[3]});
+        } else {
+            const size_t at = (size_t)m * p.N + n;
+            if (p.row_scale) value[0] *= p.row_scale[m];
+            if (p.residual) value[0] += load_as_float(p.residual, p.residual_dtype, p.residual_is_bias ? n : at);
+            store_from_float(p.y, p.y_dtype, at, value[0]);
+        }
     }
 }
 
@@ -175,21 +175,21 @@ int q4_gemm_linear(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, 
     // rows the matrix kernels see: M, or 2 M when fp32 activations go in as (value, remainder) pairs
     const bool converted_x = a.x_dtype != MI355Q_F16, pair = a.x_dtype == MI355Q_F32;
     const uint32_t rows = pair ? 2u * a.M : a.M;
-    const float *row_scale = nullptr;
     if (converted_x) {
-        // [ the rows' inverse scales, padded to 256 bytes | rows * K fp16 ], then the fp32 staging matrix
+        // [ the rows' inverse scales, padded to 256 bytes | rows * K fp16 ]
         const size_t scale_bytes = ((size_t)a.M * sizeof(float) + 255u) & ~(size_t)255u;
         int status = ensure_stage(ctx, 3, scale_bytes + (size_t)rows * x_columns * sizeof(_Float16), error, error_capacity);
-        if (status == MI355Q_OK)
-            status = ensure_stage(ctx, 6, (size_t)rows * w.N * sizeof(float), error, error_capacity);
         if (status != MI355Q_OK) return status;
         float *const scales = (float *)ctx->stage[3];
         _Float16 *const fp16_rows = (_Float16 *)((char *)ctx->stage[3] + scale_bytes);
-        hipError_t converted = q4_convert_x_launch(ctx, a.x, a.x_dtype, fp16_rows, scales, a.M, x_columns);
-        if (converted != hipSuccess)
-            return fail_hip(converted, "activation conversion launch", error, error_capacity);
+        if (target == 0) {  // the targets of one call share their activations: converted once
+            hipError_t converted = q4_convert_x_launch(ctx, a.x, a.x_dtype, fp16_rows, scales, a.M, x_columns);
+            if (converted != hipSuccess)
+                return fail_hip(converted, "activation conversion launch", error, error_capacity);
+        }
         p.x = fp16_rows;
-        row_scale = scales;
+        p.row_scale = scales;
+        p.pair = pair;
     }
     // The doubled form of an 8-bit weight whose activation row the kernels would read twice: the
     // kernel for 8-bit codes reads the bytes themselves instead, one pass over the row, half the
@@ -201,15 +201,15 @@ int q4_gemm_linear(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, 
         p.codes = w.codes8;
         p.meta = w.meta8;
     }
-    p.y = converted_x ? ctx->stage[6] : a.targets[target].y;
-    p.residual = converted_x ? nullptr : a.targets[target].residual;
+    p.y = a.targets[target].y;
+    p.residual = a.targets[target].residual;
     p.M = rows;
     p.N = w.N;
     p.K = x_columns;
     p.wrap_steps = a.x_columns && !bytes_native ? a.x_columns / kStepColumns : 0xffffffffu;
     p.NT = w.NT;
     p.T = T;
-    p.y_dtype = converted_x ? MI355Q_F32 : a.y_dtype;
+    p.y_dtype = a.y_dtype;
     p.residual_dtype = a.residual_dtype;
     p.residual_is_bias = a.residual_is_bias;
     p.wide_stores = w.N % 4u == 0u && (uintptr_t)p.y % 16u == 0u;
@@ -344,23 +344,12 @@ int q4_gemm_linear(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, 
     if (launched != hipSuccess)
         return fail_hip(launched, "q4 gemm kernel launch", error, error_capacity);
     if (p.splits > 1u) {
-        const size_t total = (size_t)rows * w.N;
-        if (p.wide_stores)
-            launched = launch(ctx, q4_gemm_reduce_kernel<true>, dim3((uint32_t)((total / 4u + 255u) / 256u)),
-                              dim3(256), 0, p);
-        else
-            launched = launch(ctx, q4_gemm_reduce_kernel<false>, dim3((uint32_t)((total + 255u) / 256u)),
-                              dim3(256), 0, p);
+        const uint32_t columns = kReduceThreads * (p.wide_stores ? 4u : 1u);
+        const dim3 reduce_grid((w.N + columns - 1u) / columns, a.M < 65535u ? a.M : 65535u);
+        launched = p.wide_stores ? launch(ctx, q4_gemm_reduce_kernel<true>, reduce_grid, dim3(kReduceThreads), 0, p)
+                                 : launch(ctx, q4_gemm_reduce_kernel<false>, reduce_grid, dim3(kReduceThreads), 0, p);
         if (launched != hipSuccess)
             return fail_hip(launched, "q4 gemm reduce launch", error, error_capacity);
-    }
-    if (converted_x) {
-        const size_t total = (size_t)a.M * w.N;
-        const uint32_t blocks = (uint32_t)((total + 255u) / 256u < 65536u ? (total + 255u) / 256u : 65536u);
-        launched = launch(ctx, q4_gemm_finish_kernel, dim3(blocks), dim3(256), 0, (const float *)ctx->stage[6], row_scale,
-                          pair ? 1 : 0, a.targets[target].y, a.y_dtype, a.targets[target].residual, a.residual_dtype,
-                          a.residual_is_bias ? 1 : 0, a.M, w.N);
-        if (launched != hipSuccess) return fail_hip(launched, "q4 gemm finish launch", error, error_capacity);
     }
     return MI355Q_OK;
 }

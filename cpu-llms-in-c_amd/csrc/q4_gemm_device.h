@@ -28,6 +28,11 @@ struct GemmParams {
     int y_dtype, residual_dtype;
     int residual_is_bias;  // residual is one row [N], added to every activation row
     int wide_stores;       // N % 4 == 0 and y 16-byte aligned: four adjacent outputs go out as one store
+    // Converted activations (x was not fp16): M counts the fp16 rows the kernels multiply.  The
+    // finished sums of caller's row m are multiplied by row_scale[m]; with pair that row is the sum
+    // of rows 2m (value) and 2m + 1 (rounding remainder).  Null: fp16 activations as given.
+    const float *row_scale;
+    int pair;
     int xcd_order;         // pipelined kernel: blocks that share weights are placed on one XCD (see there)
 };
 
@@ -61,7 +66,8 @@ __device__ __forceinline__ void static_for(F &&f)
 
 // Output of one accumulator fragment: lane (r, kq) holds rows row0 + 4*kq + j (j = 0..3) of
 // column n.  MODE 0..2: plain store as fp16 / fp32 / bf16 (no residual, no K split: the common
-// case, with nothing to decide per element); MODE 3: everything else.
+// case, with nothing to decide per element); MODE 4: converted activations without a K split;
+// MODE 3: everything else.
 template <int MODE>
 __device__ __forceinline__ void store_fragment(const GemmParams &p, uint32_t split, uint32_t row0,
                                                uint32_t kq, uint32_t n, const floatx4 &values)
@@ -70,6 +76,17 @@ __device__ __forceinline__ void store_fragment(const GemmParams &p, uint32_t spl
     for (int j = 0; j < 4; ++j) {
         const uint32_t m = row0 + 4u * kq + j;
         if (m >= p.M) continue;
+        if (MODE == 4) {  // row0 is even and so is M with pairs: a pair is j and j + 1 of one lane
+            if (p.pair && (j & 1)) continue;
+            const float sum = p.pair ? values[j] + values[(j + 1) & 3] : values[j];
+            const uint32_t row = p.pair ? m >> 1 : m;
+            const size_t at = (size_t)row * p.N + n;
+            float value = sum * p.row_scale[row];
+            if (p.residual)
+                value += load_as_float(p.residual, p.residual_dtype, p.residual_is_bias ? n : at);
+            store_from_float(p.y, p.y_dtype, at, value);
+            continue;
+        }
         const size_t at = (size_t)m * p.N + n;
         if (MODE == 0) {
             ((_Float16 *)p.y)[at] = (_Float16)values[j];
@@ -94,57 +111,46 @@ __device__ __forceinline__ uint32_t bf16_bits(float v)  // round to nearest even
     return (bits + 0x7fffu + ((bits >> 16) & 1u)) >> 16;
 }
 
-// The pipelined kernel multiplies with the weight tile as the first operand, which transposes the
-// result: lane (r, kq) holds row `m` = 16*i + r and the four adjacent columns n0 .. n0 + 3,
-// n0 = 16*tile + 4*kq.  They leave as one 8- or 16-byte store (a quarter of the store
-// instructions of the column-per-lane layout, whose 2-byte stores took 5 us per workgroup).
-template <int MODE>
-__device__ __forceinline__ void store_columns(const GemmParams &p, uint32_t split, uint32_t m, uint32_t n0,
-                                              const floatx4 &values)
+// Four adjacent columns n .. n + 3 of output row m: row scale, residual, conversion, store; or, when
+// partial, of row m of a K split's partial sums.  Columns from N on are not stored.
+__device__ __forceinline__ void finish_four(const GemmParams &p, bool partial, uint32_t split, uint32_t m, uint32_t n,
+                                            floatx4 values)
 {
-    if (m >= p.M || n0 >= p.N) return;
-    const size_t at = (size_t)m * p.N + n0;
-    if (p.wide_stores) {  // then n0 + 3 < N as well
-        if (MODE == 0) {
-            typedef _Float16 half4v __attribute__((ext_vector_type(4)));
-            const half4v packed = {(_Float16)values[0], (_Float16)values[1], (_Float16)values[2],
-                                   (_Float16)values[3]};
-            *(half4v *)((_Float16 *)p.y + at) = packed;
-            return;
+    const size_t at = (size_t)m * p.N + n;
+    if (!partial) {
+        if (p.row_scale) {
+            const float scale = p.row_scale[m];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) values[j] *= scale;
         }
-        if (MODE == 1) {
-            *(floatx4 *)((float *)p.y + at) = values;
-            return;
-        }
-        if (MODE == 2) {
-            const uint32_t b0 = bf16_bits(values[0]), b1 = bf16_bits(values[1]);
-            const uint32_t b2 = bf16_bits(values[2]), b3 = bf16_bits(values[3]);
-            *(uint2 *)((uint16_t *)p.y + at) = make_uint2(b0 | (b1 << 16), b2 | (b3 << 16));
-            return;
-        }
-        if (p.splits > 1u) {
-            *(floatx4 *)(p.partials + (size_t)split * p.M * p.N + at) = values;
-            return;
+        if (p.residual) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (n + j < p.N) values[j] += load_as_float(p.residual, p.residual_dtype, p.residual_is_bias ? n + j : at + j);
         }
     }
+    float *const out32 = partial ? p.partials + (size_t)split * p.M * p.N : (float *)p.y;
+    if (!p.wide_stores) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const uint32_t n = n0 + j;
-        if (n >= p.N) break;
-        if (p.splits > 1u) {
-            p.partials[(size_t)split * p.M * p.N + at + j] = values[j];
-            continue;
-        }
-        float value = values[j];
-        if (p.residual)
-            value += load_as_float(p.residual, p.residual_dtype, p.residual_is_bias ? n : at + j);
-        store_from_float(p.y, p.y_dtype, at + j, value);
+        for (int j = 0; j < 4; ++j)
+            if (n + j < p.N) store_from_float(out32, partial ? MI355Q_F32 : p.y_dtype, at + j, values[j]);
+    } else if (partial || p.y_dtype == MI355Q_F32) {
+        *(floatx4 *)(out32 + at) = values;
+    } else if (p.y_dtype == MI355Q_F16) {
+        typedef _Float16 half4v __attribute__((ext_vector_type(4)));
+        const half4v packed = {(_Float16)values[0], (_Float16)values[1], (_Float16)values[2], (_Float16)values[3]};
+        *(half4v *)((_Float16 *)p.y + at) = packed;
+    } else {
+        *(uint2 *)((uint16_t *)p.y + at) = make_uint2(bf16_bits(values[0]) | (bf16_bits(values[1]) << 16),
+                                                      bf16_bits(values[2]) | (bf16_bits(values[3]) << 16));
     }
 }
 
 __device__ __forceinline__ int store_mode(const GemmParams &p)
 {
-    if (p.splits > 1u || p.residual != nullptr) return 3;
+    if (p.splits > 1u) return 3;
+    if (p.row_scale != nullptr) return 4;
+    if (p.residual != nullptr) return 3;
     return p.y_dtype == MI355Q_F16 ? 0 : p.y_dtype == MI355Q_F32 ? 1 : 2;
 }
 
@@ -319,6 +325,7 @@ __global__ void __launch_bounds__(256, 2) q4_gemm_kernel(const GemmParams p)
     case 0: store_all(std::integral_constant<int, 0>()); break;
     case 1: store_all(std::integral_constant<int, 1>()); break;
     case 2: store_all(std::integral_constant<int, 2>()); break;
+    case 4: store_all(std::integral_constant<int, 4>()); break;
     default: store_all(std::integral_constant<int, 3>()); break;
     }
 }
@@ -821,45 +828,27 @@ __global__ void __launch_bounds__(256, 1) q4_gemm_pipe_kernel(const GemmParams p
     for (int set = 0; set < 3; ++set) landed(b_codes[set], b_meta[set]);
     __builtin_amdgcn_sched_barrier(0);
 
-    // ---- lane (r, kq) holds row 16*i + r, columns tile*16 + 4*kq .. + 3
-    auto store_all = [&](auto mode) {
-#pragma unroll
-        for (int t = 0; t < NTW; ++t) {
-            const uint32_t tile = tile0 + t;
-            if (tile >= p.NT) continue;
-#pragma unroll
-            for (int i = 0; i < MI; ++i)
-                store_columns<decltype(mode)::value>(p, split, m0 + 16u * i + r, tile * kTileRows + 4u * kq,
-                                                     acc[i][t]);
-        }
-        if (XT) {
-            if (shared_tile < p.NT) {
-#pragma unroll
-                for (int i = 0; i < XI; ++i)
-                    store_columns<decltype(mode)::value>(p, split, m0 + 16u * (XI * wave + i) + r,
-                                                         shared_tile * kTileRows + 4u * kq, acc_shared[i]);
-            }
-        }
-    };
-    // 16-bit outputs of whole, aligned blocks leave through LDS, row by row: the accumulators hold
-    // 4 adjacent columns of 16 rows per store instruction (16 pieces of 8 bytes, 34 KB apart),
-    // which the memory system takes at 2.4 TB/s; whole rows of the block (544 contiguous bytes,
-    // 16 per lane) go out at 3.8 TB/s (17.8 MB from 256 workgroups at once: 4.6 against 7.5 us).
+    // ---- The kernel multiplies with the weight tile as the first operand, which transposes the
+    // result: lane (r, kq) holds row 16*i + r, columns tile*16 + 4*kq .. + 3.
+    // 16-bit outputs leave through LDS, row by row: the accumulators hold 4 adjacent columns of 16
+    // rows per store instruction (16 pieces of 8 bytes, 34 KB apart), which the memory system
+    // takes at 2.4 TB/s; whole rows of the block (544 contiguous bytes, 16 per lane) go out at
+    // 3.8 TB/s (17.8 MB from 256 workgroups at once: 4.6 against 7.5 us).
     // The activation stage is free by now: every wave has waited for its last loads into it, and
     // the barrier below says every wave has read its last fragments.
-    const int mode = store_mode(p);
     constexpr uint32_t WIDTH = TPB * kTileRows;                   // columns of the block
     constexpr uint32_t PITCH = (WIDTH * 2u + 16u + 15u) / 16u * 16u + ((WIDTH * 2u + 16u) / 16u % 2u ? 0u : 16u);
     static_assert(PITCH % 16u == 0u && (PITCH / 16u) % 2u == 1u, "rows start 16-byte aligned, an odd number of 16-byte units apart");
     static_assert((size_t)BM * PITCH <= pipe_lds_bytes(BM), "the block fits the activation stage");
     const uint32_t n_first = block_first_tile * kTileRows;
-    const bool through_lds = (mode == 0 || mode == 2) && p.wide_stores && p.N % 8u == 0u &&
-                             n_first + WIDTH <= p.N && m0 + BM <= p.M;
+    char *const stage = (char *)a_lds_raw;
+    const bool through_lds = p.splits <= 1u && p.residual == nullptr && !p.pair && p.y_dtype != MI355Q_F32 &&
+                             p.wide_stores && p.N % 8u == 0u;
+    const bool whole = n_first + WIDTH <= p.N && m0 + BM <= p.M;
     if (through_lds) {
-        char *const stage = (char *)a_lds_raw;
         auto put = [&](uint32_t row, uint32_t column, const floatx4 &values) {
             uint2 packed;
-            if (mode == 0) {
+            if (p.y_dtype == MI355Q_F16) {
                 typedef _Float16 half4v __attribute__((ext_vector_type(4)));
                 const half4v h = {(_Float16)values[0], (_Float16)values[1], (_Float16)values[2], (_Float16)values[3]};
                 packed = __builtin_bit_cast(uint2, h);
@@ -869,66 +858,98 @@ __global__ void __launch_bounds__(256, 1) q4_gemm_pipe_kernel(const GemmParams p
             }
             *(uint2 *)(stage + row * PITCH + column * 2u) = packed;
         };
-        __syncthreads();
-#pragma unroll
-        for (int t = 0; t < NTW; ++t)
-#pragma unroll
-            for (int i = 0; i < MI; ++i) put(16u * i + r, (wave * NTW + t) * kTileRows + 4u * kq, acc[i][t]);
-        if (XT) {
-#pragma unroll
-            for (int i = 0; i < XI; ++i) put(16u * (XI * wave + i) + r, 4u * NTW * kTileRows + 4u * kq, acc_shared[i]);
-        }
-        __syncthreads();
-        constexpr uint32_t PIECES = WIDTH / 8u;  // 16-byte pieces per row
-        uint16_t *const y = (uint16_t *)p.y;
-        for (uint32_t piece = threadIdx.x; piece < BM * PIECES; piece += 256u) {
-            const uint32_t row = piece / PIECES, column = piece % PIECES * 8u;
-            *(uint4 *)(y + (size_t)(m0 + row) * p.N + n_first + column) = *(const uint4 *)(stage + row * PITCH + column * 2u);
-        }
-        return;
-    }
-    // The fp32 partial sums of a K split leave the same way, in two halves of 64 rows (a whole
-    // block of them is a few KB more than the stage): 16 bytes per lane, a row of the block
-    // contiguous, instead of 16-byte pieces of 16 rows 4 N bytes apart.
-    constexpr uint32_t PITCH32 = WIDTH * 4u + 16u;
-    static_assert(PITCH32 % 16u == 0u && (PITCH32 / 16u) % 2u == 1u, "rows start 16-byte aligned, an odd number of 16-byte units apart");
-    static_assert((size_t)(BM / 2) * PITCH32 <= pipe_lds_bytes(BM), "half a block fits the activation stage");
-    const bool partials_through_lds = mode == 3 && p.splits > 1u && p.wide_stores && n_first + WIDTH <= p.N && m0 + BM <= p.M;
-    if (partials_through_lds) {
-        char *const stage = (char *)a_lds_raw;
-        float *const out = p.partials + ((size_t)split * p.M + m0) * p.N + n_first;
-        constexpr uint32_t PIECES = WIDTH / 4u;  // 16-byte pieces per row
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            __syncthreads();  // the stage is free: the main loop's reads, or the first half's
+        // (two copies: with a test of row_scale for every fragment of fp16 activations the 27B
+        // gate at 512 rows took 2 us more)
+        auto put_scaled = [&](uint32_t row, uint32_t column, const floatx4 &sums) {
+            const uint32_t m = m0 + row;
+            const float scale = p.row_scale[m < p.M ? m : p.M - 1u];
+            put(row, column, floatx4{sums[0] * scale, sums[1] * scale, sums[2] * scale, sums[3] * scale});
+        };
+        auto put_all = [&](auto &&put_one) {
 #pragma unroll
             for (int t = 0; t < NTW; ++t)
 #pragma unroll
-                for (int i = 0; i < MI / 2; ++i)
-                    *(floatx4 *)(stage + (16u * i + r) * PITCH32 + ((wave * NTW + t) * kTileRows + 4u * kq) * 4u) =
-                        acc[half * (MI / 2) + i][t];
+                for (int i = 0; i < MI; ++i) put_one(16u * i + r, (wave * NTW + t) * kTileRows + 4u * kq, acc[i][t]);
             if (XT) {
-                if (wave / 2u == (uint32_t)half) {  // this wave's row groups of the shared tile lie in this half
 #pragma unroll
-                    for (int i = 0; i < XI; ++i)
-                        *(floatx4 *)(stage + (16u * (XI * (wave % 2u) + i) + r) * PITCH32 +
-                                     (4u * NTW * kTileRows + 4u * kq) * 4u) = acc_shared[i];
-                }
+                for (int i = 0; i < XI; ++i)
+                    put_one(16u * (XI * wave + i) + r, 4u * NTW * kTileRows + 4u * kq, acc_shared[i]);
             }
-            __syncthreads();
-            for (uint32_t piece = threadIdx.x; piece < BM / 2u * PIECES; piece += 256u) {
-                const uint32_t row = piece / PIECES, column = piece % PIECES * 4u;
-                *(floatx4 *)(out + (size_t)(half * (BM / 2) + row) * p.N + column) =
-                    *(const floatx4 *)(stage + row * PITCH32 + column * 4u);
+        };
+        __syncthreads();
+        if (p.row_scale)
+            put_all(put_scaled);
+        else
+            put_all(put);
+        __syncthreads();
+        constexpr uint32_t PIECES = WIDTH / 8u;  // 16-byte pieces per row
+        uint16_t *const y = (uint16_t *)p.y;
+        if (whole) {
+            for (uint32_t piece = threadIdx.x; piece < BM * PIECES; piece += 256u) {
+                const uint32_t row = piece / PIECES, column = piece % PIECES * 8u;
+                *(uint4 *)(y + (size_t)(m0 + row) * p.N + n_first + column) = *(const uint4 *)(stage + row * PITCH + column * 2u);
+            }
+        } else {
+            for (uint32_t piece = threadIdx.x; piece < BM * PIECES; piece += 256u) {
+                const uint32_t row = piece / PIECES, column = piece % PIECES * 8u;
+                if (m0 + row < p.M && n_first + column < p.N)
+                    *(uint4 *)(y + (size_t)(m0 + row) * p.N + n_first + column) =
+                        *(const uint4 *)(stage + row * PITCH + column * 2u);
             }
         }
         return;
     }
-    switch (mode) {
-    case 0: store_all(std::integral_constant<int, 0>()); break;
-    case 1: store_all(std::integral_constant<int, 1>()); break;
-    case 2: store_all(std::integral_constant<int, 2>()); break;
-    default: store_all(std::integral_constant<int, 3>()); break;
+    // Everything else - the fp32 partial sums of a K split, fp32 outputs, residuals, the pairs of
+    // fp32 activations - leaves the same way as fp32, in two halves of 64 rows (a whole block of
+    // them is a few KB more than the stage): a thread takes four adjacent columns of a row of the
+    // block, 16 bytes per lane and the row contiguous, instead of 16-byte pieces of 16 rows 4 N
+    // bytes apart.  The two rows of a pair meet here, so that converted activations need no
+    // staging matrix and no second kernel.
+    constexpr uint32_t PITCH32 = WIDTH * 4u + 16u;
+    static_assert(PITCH32 % 16u == 0u && (PITCH32 / 16u) % 2u == 1u, "rows start 16-byte aligned, an odd number of 16-byte units apart");
+    static_assert((size_t)(BM / 2) * PITCH32 <= pipe_lds_bytes(BM), "half a block fits the activation stage");
+    const bool pairs = p.splits <= 1u && p.pair;  // (the kernel that adds K splits adds pairs itself)
+    const uint32_t rows_out = pairs ? BM / 4u : BM / 2u;
+    constexpr uint32_t FOURS = WIDTH / 4u;  // groups of four columns per row
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        __syncthreads();  // the stage is free: the main loop's reads, or the first half's
+#pragma unroll
+        for (int t = 0; t < NTW; ++t)
+#pragma unroll
+            for (int i = 0; i < MI / 2; ++i)
+                *(floatx4 *)(stage + (16u * i + r) * PITCH32 + ((wave * NTW + t) * kTileRows + 4u * kq) * 4u) =
+                    acc[half * (MI / 2) + i][t];
+        if (XT) {
+            if (wave / 2u == (uint32_t)half) {  // this wave's row groups of the shared tile lie in this half
+#pragma unroll
+                for (int i = 0; i < XI; ++i)
+                    *(floatx4 *)(stage + (16u * (XI * (wave % 2u) + i) + r) * PITCH32 +
+                                 (4u * NTW * kTileRows + 4u * kq) * 4u) = acc_shared[i];
+            }
+        }
+        __syncthreads();
+        if (p.splits > 1u && p.wide_stores && whole) {  // whole blocks of partial sums: a plain copy
+            float *const out = p.partials + ((size_t)split * p.M + m0 + half * (BM / 2)) * p.N + n_first;
+            for (uint32_t piece = threadIdx.x; piece < BM / 2u * FOURS; piece += 256u) {
+                const uint32_t row = piece / FOURS, column = piece % FOURS * 4u;
+                *(floatx4 *)(out + (size_t)row * p.N + column) = *(const floatx4 *)(stage + row * PITCH32 + column * 4u);
+            }
+            continue;
+        }
+        for (uint32_t piece = threadIdx.x; piece < rows_out * FOURS; piece += 256u) {
+            const uint32_t row = piece / FOURS, column = piece % FOURS * 4u, n = n_first + column;
+            const uint32_t local = pairs ? 2u * row : row;
+            if (m0 + half * (BM / 2) + local >= p.M || n >= p.N) continue;
+            const char *const from = stage + local * PITCH32 + column * 4u;
+            floatx4 values = *(const floatx4 *)from;
+            if (pairs) {
+                const floatx4 remainder = *(const floatx4 *)(from + PITCH32);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) values[j] += remainder[j];
+            }
+            finish_four(p, p.splits > 1u, split, (pairs ? m0 / 2u : m0) + half * rows_out + row, n, values);
+        }
     }
 }
 

@@ -124,18 +124,49 @@ __global__ void __launch_bounds__(256) q4_stream_reduce_kernel(const StreamParam
 // row's maximum); fp32 -> two rows: the value rounded to fp16 and the rounding remainder,
 // whose results the kernel adds (about 22 significant bits relative to the row's maximum).
 // Infinities saturate at the largest fp16 value, NaN stays NaN.
-constexpr uint32_t kConvertThreads = 1024;
+//
+// Bound by memory (each row is read once from HBM and once more from the compute unit's vector
+// cache).  A thread takes eight adjacent columns at a time, 16- and 32-byte loads and 16-byte
+// stores: with one element per thread and access the 4646 x 5376 bf16 rows of a video clip took
+// 74 us (1.4 TB/s), now NEW_US (rows are whole 64-column groups and the entry points take
+// 16-byte aligned activations only).
+constexpr uint32_t kConvertThreads = 256;
+template <bool BF16>
 __global__ void __launch_bounds__(kConvertThreads)
-q4_convert_x_kernel(const void *__restrict__ x, int x_dtype, _Float16 *__restrict__ out,
-                    float *__restrict__ row_scale, uint32_t M, uint32_t K)
+q4_convert_x_kernel(const void *__restrict__ x, _Float16 *__restrict__ out, float *__restrict__ row_scale,
+                    uint32_t K)
 {
     __shared__ float wave_max[kConvertThreads / 64u];
-    const uint32_t m = blockIdx.x;
+    const uint32_t m = blockIdx.x, pieces = K / 8u;
     const size_t row_at = (size_t)m * K;
+    auto load = [&](uint32_t piece, float (&v)[8]) {
+        if constexpr (BF16) {
+            const u32x4 bits = *(const u32x4 *)((const uint16_t *)x + row_at + 8u * piece);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                v[2 * j] = __builtin_bit_cast(float, bits[j] << 16);
+                v[2 * j + 1] = __builtin_bit_cast(float, bits[j] & 0xffff0000u);
+            }
+        } else {
+            const floatx4 *from = (const floatx4 *)((const float *)x + row_at + 8u * piece);
+            const floatx4 low = from[0], high = from[1];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                v[j] = low[j];
+                v[j + 4] = high[j];
+            }
+        }
+    };
     float biggest = 0.0f;
-    for (uint32_t k = threadIdx.x; k < K; k += kConvertThreads) {
-        const float magnitude = __builtin_fabsf(load_as_float(x, x_dtype, row_at + k));
-        if (magnitude > biggest && magnitude <= 3.4028234e38f) biggest = magnitude;  // finite values only
+#pragma unroll 4
+    for (uint32_t piece = threadIdx.x; piece < pieces; piece += kConvertThreads) {
+        float v[8];
+        load(piece, v);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float magnitude = __builtin_fabsf(v[j]);
+            if (magnitude > biggest && magnitude <= 3.4028234e38f) biggest = magnitude;  // finite values only
+        }
     }
 #pragma unroll
     for (int offset = 32; offset > 0; offset >>= 1) {
@@ -154,15 +185,24 @@ q4_convert_x_kernel(const void *__restrict__ x, int x_dtype, _Float16 *__restric
     const float forward = __builtin_ldexpf(1.0f, shift), back = __builtin_ldexpf(1.0f, -shift);
     if (threadIdx.x == 0) row_scale[m] = back;
     const float limit = 65504.0f;
-    for (uint32_t k = threadIdx.x; k < K; k += kConvertThreads) {
-        const float value = load_as_float(x, x_dtype, row_at + k) * forward;
-        const _Float16 head = (_Float16)(value > limit ? limit : value < -limit ? -limit : value);
-        if (x_dtype == MI355Q_BF16) {
-            out[row_at + k] = head;
-        } else {
+#pragma unroll 2
+    for (uint32_t piece = threadIdx.x; piece < pieces; piece += kConvertThreads) {
+        float v[8];
+        load(piece, v);
+        half8 heads, rests;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float value = v[j] * forward;
+            const _Float16 head = (_Float16)(value > limit ? limit : value < -limit ? -limit : value);
             const float rest = value - (float)head;
-            out[(size_t)(2u * m) * K + k] = head;
-            out[(size_t)(2u * m + 1u) * K + k] = (_Float16)(rest > limit ? limit : rest < -limit ? -limit : rest);
+            heads[j] = head;
+            rests[j] = (_Float16)(rest > limit ? limit : rest < -limit ? -limit : rest);
+        }
+        if constexpr (BF16) {
+            *(half8 *)(out + row_at + 8u * piece) = heads;
+        } else {
+            *(half8 *)(out + 2u * row_at + 8u * piece) = heads;
+            *(half8 *)(out + 2u * row_at + K + 8u * piece) = rests;
         }
     }
 }
@@ -376,7 +416,9 @@ StreamShape choose_shape(const mi355q_context *ctx, uint32_t NT_total, uint32_t 
 hipError_t q4_convert_x_launch(mi355q_context *ctx, const void *x, int x_dtype, _Float16 *out, float *row_scale,
                                uint32_t M, uint32_t K)
 {
-    return launch(ctx, q4_convert_x_kernel, dim3(M), dim3(kConvertThreads), 0, x, x_dtype, out, row_scale, M, K);
+    if (x_dtype == MI355Q_BF16)
+        return launch(ctx, q4_convert_x_kernel<true>, dim3(M), dim3(kConvertThreads), 0, x, out, row_scale, K);
+    return launch(ctx, q4_convert_x_kernel<false>, dim3(M), dim3(kConvertThreads), 0, x, out, row_scale, K);
 }
 
 hipError_t zero_words_launch(mi355q_context *ctx, uint32_t *words, uint32_t count)

@@ -256,3 +256,66 @@ def test_block_order_does_not_change_the_bits(engine, gpu, force, N, K, M, force
         weight.destroy()
     assert np.array_equal(in_launch_order.view(np.uint32), renumbered.view(np.uint32))
     assert np.any(renumbered != 0)
+
+
+@pytest.mark.parametrize("forced", ["1,1", "2,2", "4,1", "5,1", "6,1", "6,2", "7,1", "7,2", "8,1"])
+@pytest.mark.parametrize("x_dtype,y_dtype,N", [("F32", "F32", 1104), ("F32", "F32", 1102), ("F32", "BF16", 1100),
+                                               ("BF16", "BF16", 1104), ("BF16", "F16", 1100), ("BF16", "F32", 1101)])
+def test_converted_activations_finish_in_the_kernel(engine, oracle, gpu, force, forced, x_dtype, y_dtype, N):
+    """Activations that are not fp16: the matrix kernel's own epilogue (or the kernel that adds K
+    splits) adds the two rows of a pair, undoes the row scale, adds the residual and converts.
+    Ragged last tiles, widths that are and are not multiples of 4 and 8, a last block of rows that
+    is partly filled, with and without a residual."""
+    force("q4_gemm", forced)
+    kind, K, M = engine.META_BF16_PLANES, 256, 75
+    quants, meta_a, meta_b = engine.synth_q4_affine(77, 0.02, N, K, kind)
+    x32 = make_x(engine, 78, M, K)
+    x = x32 if x_dtype == "F32" else bf16_bits(x32).reshape(M, K)
+    res = engine.synth_normal_f32(79, 1.0, M * N).reshape(M, N)
+    product = oracle.q4_linear(quants, meta_a, meta_b, kind, N, K, x, oracle.X_F32 if x_dtype == "F32" else oracle.X_BF16,
+                               M, weight_rounding=oracle.W_ROUND_F16)
+    weight = gpu.q4_prepare(quants, meta_a, meta_b, N, K, kind)
+    try:
+        for residual in (None, res):
+            print(f"gemm epilogue N={N} x={x_dtype} y={y_dtype} forced={forced} residual={residual is not None}", flush=True)
+            y = gpu.q4_linear(weight, x, getattr(engine, x_dtype), getattr(engine, y_dtype), residual, engine.F32)
+            y = (y.astype(np.uint32) << 16).view(np.float32) if y_dtype == "BF16" else y
+            # a bf16 output is rounded by at most half a unit of its eight bits: 2^-8 of its value
+            error = q4_relative_error(y, product if residual is None else product + res)
+            assert error <= (2.0 ** -8 if y_dtype == "BF16" else 1e-3)
+    finally:
+        weight.destroy()
+
+
+@pytest.mark.parametrize("x_dtype", ["F32", "BF16"])
+@pytest.mark.parametrize("M", [9, 40, 150])
+def test_targets_share_converted_activations(engine, gpu, x_dtype, M):
+    """Weights of one call multiply activations that were converted once: the same bits as one
+    call per weight."""
+    K, widths = 384, (272, 1000, 100)
+    x32 = make_x(engine, 81, M, K)
+    x = x32 if x_dtype == "F32" else bf16_bits(x32).reshape(M, K)
+    kind, x_dtype = engine.META_BF16_PLANES, getattr(engine, x_dtype)
+    weights = [gpu.q4_prepare(*engine.synth_q4_affine(82 + i, 0.02, N, K, kind), N, K, kind) for i, N in enumerate(widths)]
+    biases = [gpu.to_device(engine.synth_normal_f32(90 + i, 1.0, N)) for i, N in enumerate(widths)]
+    x_ptr = gpu.to_device(x)
+    outputs = [gpu.alloc(M * N * 4) for N in widths]
+    try:
+        results = []
+        targets = list(zip(weights, outputs, biases))
+        for groups in ([targets], [[t] for t in targets]):
+            print(f"gemm targets M={M} x={x_dtype} calls={len(groups)}", flush=True)
+            calls = engine.make_calls([(g, x_ptr, x_dtype, M, engine.F32, engine.F32, engine.RESIDUAL_IS_BIAS)
+                                       for g in groups])
+            gpu.q4_sequence(calls)
+            gpu.sync()
+            results.append([gpu.download(p, (M, N), np.uint32) for p, N in zip(outputs, widths)])
+        for together, alone in zip(*results):
+            assert np.any(alone != 0)
+            close = np.abs(together.view(np.float32) - alone.view(np.float32))
+            assert np.max(close) <= 2e-6 * np.max(np.abs(alone.view(np.float32)))
+    finally:
+        for pointer in [x_ptr] + outputs + biases:
+            gpu.free(pointer)
+        for weight in weights:
+            weight.destroy()
