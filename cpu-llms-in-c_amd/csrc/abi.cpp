@@ -854,9 +854,7 @@ int q4_linear_multi_repeated(mi355q_context *ctx, const mi355q_q4_target *target
     if (stream_rows <= 16u) {
         status = q4_stream_linear(ctx, args, error, error_capacity);
     } else {
-        status = MI355Q_OK;
-        for (uint32_t t = 0; t < count && status == MI355Q_OK; ++t)
-            status = q4_gemm_linear(ctx, args, t, error, error_capacity);
+        status = q4_gemm_linears(ctx, args, error, error_capacity);
     }
     if (status != MI355Q_OK) return status;
 

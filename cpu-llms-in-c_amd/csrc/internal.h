@@ -95,6 +95,7 @@ struct mi355q_context {
     bool gemm_plain_loads;  // option "gemm_loads" = "plain": the 17-tile GEMM shape with compiler-managed weight loads
     int w8a8_tiles;       // option "w8a8" = "1" .. "4": tiles per W8A8 workgroup (0: chosen by the launch)
     bool lds_raised[16];  // q4_gemm_pipe_kernel instantiations whose dynamic LDS limit has been raised
+    bool rows_lds_raised[9][5];  // the same for q4_rows_kernel<fragments, tiles per wave>
     // device address of the library's fixed scratch array on this context's device (for the
     // entry point that allocates nothing); every context on the device sees the same array
     unsigned char *fixed_scratch;
@@ -240,9 +241,7 @@ int chain_after_wait(mi355q_context *ctx, char *error, size_t error_capacity);
 int q4_linear_multi_repeated(mi355q_context *ctx, const mi355q_q4_target *targets, uint32_t count, const void *x,
                              int x_dtype, uint32_t M, int y_dtype, int residual_dtype, uint32_t flags,
                              uint32_t x_columns, char *error, size_t error_capacity);
-// q4_gemm.hip (one target at a time: `target` selects it; target 0 first, whose call converts
-// activations that are not fp16 for all of them)
-int q4_gemm_linear(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, char *error,
-                   size_t error_capacity);
+// q4_gemm.hip: more than 16 rows of x (8 of fp32)
+int q4_gemm_linears(mi355q_context *ctx, const Q4LinearArgs &a, char *error, size_t error_capacity);
 
 }  // namespace mi355q

@@ -15,13 +15,16 @@
 // each lane exactly the eight consecutive columns the instruction wants), so
 // each weight is dequantized once per workgroup and never passes through LDS.
 // The metadata is read as fp16 {scale, bias} pairs (converted at prepare for
-// bf16 images).  Two kernels:
+// bf16 images).  Three kernels:
 //   q4_gemm_kernel: two workgroups per compute unit overlap each other's
 //     dequantization and matrix instructions (six tile shapes);
 //   q4_gemm_pipe_kernel: one workgroup per compute unit, software pipelined by
-//     hand (128 rows x 16 or 17 tiles).
+//     hand (128 rows x 16 or 17 tiles);
+//   q4_rows_kernel (q4_rows_device.h): up to 128 rows, all weights of a call as
+//     one launch.
 // The host picks shape and K split by a time estimate fitted on this GPU, e.g.
 // 17 tiles for the 17408-row matrices: 64 x 4 = 256 workgroups at M = 512.
+#include <algorithm>
 #include <cstdio>
 #include "device_util.h"
 #include "internal.h"
@@ -31,7 +34,7 @@
 #include <type_traits>
 #include <utility>
 
-#include "q4_gemm_device.h"
+#include "q4_rows_device.h"
 
 namespace mi355q {
 
@@ -57,55 +60,63 @@ extern template __global__ void q4_gemm_pipe_kernel<128, 3, true, false, true>(c
 // A workgroup takes 256 (1024) adjacent columns of one output row: no index is ever divided (a
 // division per thread cost the 27B prefill step's reductions about a microsecond each).
 constexpr uint32_t kReduceThreads = 256;
-template <bool WIDE>
-__global__ void __launch_bounds__(kReduceThreads) q4_gemm_reduce_kernel(const GemmParams p)
+// SPLITS: their number when the host knows it and it is small - the loads of all of them are then
+// on their way before the first is added (the 27B q projection at 512 rows with its four: 50.0 us,
+// with a test of the count in front of every load 50.9); 0: a loop, and the workgroups that share a
+// column's block of q4_rows_kernel counted here.
+template <bool WIDE, int SPLITS>
+__global__ void __launch_bounds__(kReduceThreads) q4_gemm_reduce_kernel(const GemmGroup group)
 {
     constexpr int PER = WIDE ? 4 : 1;
-    const uint32_t n = (blockIdx.x * kReduceThreads + threadIdx.x) * PER;
+    typedef std::conditional_t<WIDE, floatx4, float> Piece;
+    uint32_t block = blockIdx.x;
+    const GemmParams p = SPLITS ? only_target(group) : select_target<true>(group, block);
+    const uint32_t n = (block * kReduceThreads + threadIdx.x) * PER;
     if (n >= p.N) return;
     const size_t stride = (size_t)p.M * p.N;
-    auto add_splits = [&](size_t from, float (&value)[PER]) {
+    uint32_t splits = p.splits;
+    if (!SPLITS && p.units) {  // one workgroup alone has stored the outputs
+        const uint32_t begin = (p.first_block + n / p.block_columns) * p.T;
+        splits = (begin + p.T - 1u) / p.units - begin / p.units + 1u;
+        if (splits == 1u) return;
+    }
+    auto add = [](Piece &sum, const Piece &more) {
+        if constexpr (WIDE) {
 #pragma unroll
-        for (int j = 0; j < PER; ++j) value[j] = 0.0f;
-        // eight splits' loads are on their way before the first is added: one trip to memory
-        // instead of one per split
-        typedef std::conditional_t<WIDE, floatx4, float> Piece;
-        for (uint32_t first = 0; first < p.splits; first += 8u) {
-            Piece piece[8];
-#pragma unroll
-            for (uint32_t s = 0; s < 8u; ++s)
-                if (first + s < p.splits) piece[s] = *(const Piece *)(p.partials + (first + s) * stride + from);
-#pragma unroll
-            for (uint32_t s = 0; s < 8u; ++s) {
-                if (first + s >= p.splits) continue;
-                if constexpr (WIDE) {
-#pragma unroll
-                    for (int j = 0; j < PER; ++j) value[j] += piece[s][j];
-                } else {
-                    value[0] += piece[s];
-                }
-            }
+            for (int j = 0; j < 4; ++j) sum[j] += more[j];
+        } else {
+            sum += more;
         }
+    };
+    auto add_splits = [&](size_t from) {
+        Piece sum = {};
+        if constexpr (SPLITS > 0) {
+            Piece piece[SPLITS];
+#pragma unroll
+            for (int s = 0; s < SPLITS; ++s) piece[s] = *(const Piece *)(p.partials + s * stride + from);
+#pragma unroll
+            for (int s = 0; s < SPLITS; ++s) add(sum, piece[s]);
+        } else {
+            for (uint32_t s = 0; s < splits; ++s) add(sum, *(const Piece *)(p.partials + s * stride + from));
+        }
+        return sum;
     };
     const uint32_t rows = p.pair ? p.M / 2u : p.M;
     for (uint32_t m = blockIdx.y; m < rows; m += gridDim.y) {
-        float value[PER];
+        Piece value;
         if (p.pair) {
-            float remainder[PER];
-            add_splits((size_t)(2u * m) * p.N + n, value);
-            add_splits((size_t)(2u * m + 1u) * p.N + n, remainder);
-#pragma unroll
-            for (int j = 0; j < PER; ++j) value[j] += remainder[j];
+            value = add_splits((size_t)(2u * m) * p.N + n);
+            add(value, add_splits((size_t)(2u * m + 1u) * p.N + n));
         } else {
-            add_splits((size_t)m * p.N + n, value);
+            value = add_splits((size_t)m * p.N + n);
         }
         if constexpr (WIDE) {
-            finish_four(p, false, 0, m, n, floatx4{value[0], value[1], value[2], value[3]});
+            finish_four(p, false, 0, m, n, value);
         } else {
             const size_t at = (size_t)m * p.N + n;
-            if (p.row_scale) value[0] *= p.row_scale[m];
-            if (p.residual) value[0] += load_as_float(p.residual, p.residual_dtype, p.residual_is_bias ? n : at);
-            store_from_float(p.y, p.y_dtype, at, value[0]);
+            if (p.row_scale) value *= p.row_scale[m];
+            if (p.residual) value += load_as_float(p.residual, p.residual_dtype, p.residual_is_bias ? n : at);
+            store_from_float(p.y, p.y_dtype, at, value);
         }
     }
 }
@@ -158,62 +169,94 @@ static hipError_t launch_pipe_plain(mi355q_context *ctx, dim3 grid, const GemmPa
     return launch(ctx, q4_gemm_pipe_kernel<128, 4, true, true>, grid, dim3(256), bytes, p);
 }
 
-int q4_gemm_linear(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, char *error,
-                   size_t error_capacity)
+// Adds the K splits of a launch's targets.
+static hipError_t launch_reduce(mi355q_context *ctx, GemmGroup &group)
 {
-    const Q4Device &w = *a.targets[target].w;
-    GemmParams p;
-    memset(&p, 0, sizeof p);
-    p.codes = w.codes;
-    p.meta = w.meta16;  // fp16 {scale, bias}: the weight is evaluated in fp16 here
-    p.x = (const _Float16 *)a.x;
-    if (a.x_columns != 0 && (a.x_columns * 2u != w.K || a.x_columns % kStepColumns != 0)) {
-        set_error(error, error_capacity, "q4 gemm: a repeated activation row is half the weight's columns, whole 128-column steps");
-        return MI355Q_ERROR_INVALID;
+    bool wide = true;
+    for (uint32_t t = 0; t < group.targets; ++t) wide = wide && group.target[t].wide_stores;
+    const uint32_t columns = kReduceThreads * (wide ? 4u : 1u);
+    uint32_t blocks = 0;
+    for (uint32_t t = 0; t < group.targets; ++t) {
+        group.target[t].first_reduce = blocks;
+        blocks += (group.target[t].N + columns - 1u) / columns;
     }
-    const uint32_t x_columns = a.x_columns ? a.x_columns : w.K;
-    // rows the matrix kernels see: M, or 2 M when fp32 activations go in as (value, remainder) pairs
-    const bool converted_x = a.x_dtype != MI355Q_F16, pair = a.x_dtype == MI355Q_F32;
-    const uint32_t rows = pair ? 2u * a.M : a.M;
-    if (converted_x) {
-        // [ the rows' inverse scales, padded to 256 bytes | rows * K fp16 ]
-        const size_t scale_bytes = ((size_t)a.M * sizeof(float) + 255u) & ~(size_t)255u;
-        int status = ensure_stage(ctx, 3, scale_bytes + (size_t)rows * x_columns * sizeof(_Float16), error, error_capacity);
-        if (status != MI355Q_OK) return status;
-        float *const scales = (float *)ctx->stage[3];
-        _Float16 *const fp16_rows = (_Float16 *)((char *)ctx->stage[3] + scale_bytes);
-        if (target == 0) {  // the targets of one call share their activations: converted once
-            hipError_t converted = q4_convert_x_launch(ctx, a.x, a.x_dtype, fp16_rows, scales, a.M, x_columns);
-            if (converted != hipSuccess)
-                return fail_hip(converted, "activation conversion launch", error, error_capacity);
-        }
-        p.x = fp16_rows;
-        p.row_scale = scales;
-        p.pair = pair;
+    const uint32_t rows = group.shared.pair ? group.shared.M / 2u : group.shared.M;
+    const dim3 grid(blocks, rows < 65535u ? rows : 65535u);
+    if (!wide) return launch(ctx, q4_gemm_reduce_kernel<false, 0>, grid, dim3(kReduceThreads), 0, group);
+    switch (group.targets == 1u && group.shared.units == 0u ? group.shared.splits : 0u) {
+    case 2: return launch(ctx, q4_gemm_reduce_kernel<true, 2>, grid, dim3(kReduceThreads), 0, group);
+    case 3: return launch(ctx, q4_gemm_reduce_kernel<true, 3>, grid, dim3(kReduceThreads), 0, group);
+    case 4: return launch(ctx, q4_gemm_reduce_kernel<true, 4>, grid, dim3(kReduceThreads), 0, group);
+    case 5: return launch(ctx, q4_gemm_reduce_kernel<true, 5>, grid, dim3(kReduceThreads), 0, group);
+    case 6: return launch(ctx, q4_gemm_reduce_kernel<true, 6>, grid, dim3(kReduceThreads), 0, group);
+    default: return launch(ctx, q4_gemm_reduce_kernel<true, 0>, grid, dim3(kReduceThreads), 0, group);
     }
-    // The doubled form of an 8-bit weight whose activation row the kernels would read twice: the
-    // kernel for 8-bit codes reads the bytes themselves instead, one pass over the row, half the
-    // matrix instructions.  It is the pipelined kernel, with that kernel's conditions.
-    const bool bytes_native = w.codes8 != nullptr && a.x_columns != 0 && !ctx->q8_gemm_doubled &&
-                              (uint64_t)rows * x_columns * sizeof(_Float16) + 16384u < (1ull << 32);
-    const uint32_t T = bytes_native ? w.T / 2u : w.T;
-    if (bytes_native) {
-        p.codes = w.codes8;
-        p.meta = w.meta8;
-    }
-    p.y = a.targets[target].y;
-    p.residual = a.targets[target].residual;
-    p.M = rows;
-    p.N = w.N;
-    p.K = x_columns;
-    p.wrap_steps = a.x_columns && !bytes_native ? a.x_columns / kStepColumns : 0xffffffffu;
-    p.NT = w.NT;
-    p.T = T;
-    p.y_dtype = a.y_dtype;
-    p.residual_dtype = a.residual_dtype;
-    p.residual_is_bias = a.residual_is_bias;
-    p.wide_stores = w.N % 4u == 0u && (uintptr_t)p.y % 16u == 0u;
+}
 
+// Rows, row scales and pairs of the activations the matrix kernels see: x itself when it is fp16,
+// else its conversion in the context's staging buffer (made here when `convert`: the targets of
+// one call share it): M rows, or 2 M when fp32 activations go in as (value, remainder) pairs.
+static int gemm_activations(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t x_columns, bool convert, GemmParams &p,
+                            char *error, size_t error_capacity)
+{
+    p.pair = a.x_dtype == MI355Q_F32;
+    p.M = p.pair ? 2u * a.M : a.M;
+    p.x = (const _Float16 *)a.x;
+    if (a.x_dtype == MI355Q_F16) return MI355Q_OK;
+    // [ the rows' inverse scales, padded to 256 bytes | rows * K fp16 ]
+    const size_t scale_bytes = ((size_t)a.M * sizeof(float) + 255u) & ~(size_t)255u;
+    int status = ensure_stage(ctx, 3, scale_bytes + (size_t)p.M * x_columns * sizeof(_Float16), error, error_capacity);
+    if (status != MI355Q_OK) return status;
+    float *const scales = (float *)ctx->stage[3];
+    _Float16 *const fp16_rows = (_Float16 *)((char *)ctx->stage[3] + scale_bytes);
+    if (convert) {
+        hipError_t converted = q4_convert_x_launch(ctx, a.x, a.x_dtype, fp16_rows, scales, a.M, x_columns);
+        if (converted != hipSuccess) return fail_hip(converted, "activation conversion launch", error, error_capacity);
+    }
+    p.x = fp16_rows;
+    p.row_scale = scales;
+    return MI355Q_OK;
+}
+
+// One target's parameters as the launches take them.
+static GemmTarget gemm_target(const GemmParams &p)
+{
+    GemmTarget t;
+    memset(&t, 0, sizeof t);
+    t.codes = p.codes;
+    t.meta = p.meta;
+    t.y = p.y;
+    t.residual = p.residual;
+    t.partials = p.partials;
+    t.N = p.N;
+    t.NT = p.NT;
+    t.wide_stores = p.wide_stores;
+    return t;
+}
+
+struct Variant {
+    int bm, ntw, extra;
+    int resident;          // workgroups that fit one compute unit (registers, LDS)
+    double alone, shared;  // fraction of matrix-instruction peak, one / several per CU
+    double step_us;        // pipelined kernel: measured time of one 128-column step, chip full
+};
+static const Variant variants[] = {
+    {128, 4, 0, 2, 0.399, 0.491, 0.0}, {128, 2, 0, 2, 0.327, 0.434, 0.0}, {64, 4, 0, 3, 0.333, 0.460, 0.0},
+    {64, 4, 1, 2, 0.347, 0.444, 0.0},  {64, 2, 0, 4, 0.288, 0.422, 0.0},  {64, 2, 1, 2, 0.308, 0.443, 0.0},
+    {128, 4, 0, 1, 0.0, 0.0, 1.493}, {128, 4, 1, 1, 0.0, 0.0, 1.675}, {128, 5, 0, 1, 0.0, 0.0, 1.849},
+    {128, 4, 0, 1, 0.0, 0.0, 1.60}, {128, 3, 1, 1, 0.0, 0.0, 1.40}};  // 9, 10: 16 and 13 tiles on 8-bit codes, and only for them
+constexpr int kBytesVariant = 9;  // the first of them
+
+// the pipelined kernel addresses x with 32-bit byte offsets and whole 128-column steps
+static bool gemm_pipe_ok(const Q4Device &w, uint32_t rows, uint32_t x_columns)
+{
+    return w.K % kStepColumns == 0 && (uint64_t)rows * x_columns * sizeof(_Float16) + 16384u < (1ull << 32);
+}
+
+// The shape and K split with the smallest estimated time for one target, and that time in us.
+static double gemm_decompose(mi355q_context *ctx, uint32_t NT, uint32_t N, uint32_t T, uint32_t rows, bool bytes_native,
+                             bool pipe_ok, int &best, uint32_t &best_splits)
+{
     // Decomposition: BM rows x (4*NTW + EXTRA) tiles per workgroup, K split in `splits`.
     // The choice minimises a microsecond estimate fitted to sweeps over every variant
     // and split on this GPU.  Kernels 0-5: a workgroup that has a compute unit to itself
@@ -223,18 +266,6 @@ int q4_gemm_linear(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, 
     // runs in rounds of `step_us` per 128-column step; a round that does not fill the chip is
     // shorter (partial_round).  A K split pays for writing its fp32
     // partials and for the kernel that adds them.
-    struct Variant {
-        int bm, ntw, extra;
-        int resident;          // workgroups that fit one compute unit (registers, LDS)
-        double alone, shared;  // fraction of matrix-instruction peak, one / several per CU
-        double step_us;        // pipelined kernel: measured time of one 128-column step, chip full
-    };
-    static const Variant variants[] = {
-        {128, 4, 0, 2, 0.399, 0.491, 0.0}, {128, 2, 0, 2, 0.327, 0.434, 0.0}, {64, 4, 0, 3, 0.333, 0.460, 0.0},
-        {64, 4, 1, 2, 0.347, 0.444, 0.0},  {64, 2, 0, 4, 0.288, 0.422, 0.0},  {64, 2, 1, 2, 0.308, 0.443, 0.0},
-        {128, 4, 0, 1, 0.0, 0.0, 1.493}, {128, 4, 1, 1, 0.0, 0.0, 1.675}, {128, 5, 0, 1, 0.0, 0.0, 1.849},
-        {128, 4, 0, 1, 0.0, 0.0, 1.60}, {128, 3, 1, 1, 0.0, 0.0, 1.40}};  // 9, 10: 16 and 13 tiles on 8-bit codes, and only for them
-    constexpr int kBytesVariant = 9;  // the first of them
     // A round of the pipelined kernel that fills only the fraction r of the compute units runs
     // faster than a full one: the chip is power limited, and up to about half of it the clock
     // stays near its maximum, from there it falls to the sustained clock of a full chip
@@ -245,11 +276,7 @@ int q4_gemm_linear(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, 
         return r <= 0.562 ? 0.771 - 0.081 * r / 0.562 : 1.0 - 0.31 * over * over;
     };
     const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
-    int best = 0;
-    uint32_t best_splits = 1;
     double best_cost = 1e30;
-    // the pipelined kernel addresses x with 32-bit byte offsets and whole 128-column steps
-    const bool pipe_ok = w.K % kStepColumns == 0 && (uint64_t)rows * x_columns * sizeof(_Float16) + 16384u < (1ull << 32);
     for (int v = 0; v < (int)(sizeof variants / sizeof variants[0]); ++v) {
         if (v >= 6 && !pipe_ok) continue;
         if ((v >= kBytesVariant) != bytes_native) continue;
@@ -257,7 +284,7 @@ int q4_gemm_linear(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, 
         const uint32_t tpb = 4u * c.ntw + c.extra;
         const uint32_t slots = cus * (uint32_t)c.resident;
         const uint32_t m_blocks = (rows + c.bm - 1) / c.bm;
-        const uint32_t n_blocks = (w.NT + tpb - 1) / tpb;
+        const uint32_t n_blocks = (NT + tpb - 1) / tpb;
         for (uint32_t want = 1; want <= 8u && want * 8u <= T + 7u; ++want) {
             const uint32_t steps = (T + want - 1) / want;
             const uint32_t splits = (T + steps - 1) / steps;
@@ -286,7 +313,7 @@ int q4_gemm_linear(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, 
             else
                 cost = ((double)groups / slots + (groups % slots ? 0.31 : 0.0)) * c.resident * peak_us / c.shared;
             if (splits > 1)  // fp32 partials at 4.6 TB/s and the kernel that adds them
-                cost += (double)splits * rows * (double)w.N * 4.0 / 4.63e6 + (v >= 6 ? 2.0 : 6.3);
+                cost += (double)splits * rows * (double)N * 4.0 / 4.63e6 + (v >= 6 ? 2.0 : 6.3);
             if (cost < best_cost) {
                 best_cost = cost;
                 best = v;
@@ -294,6 +321,51 @@ int q4_gemm_linear(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, 
             }
         }
     }
+    return best_cost;
+}
+
+static int gemm_one_target(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, char *error,
+                           size_t error_capacity)
+{
+    const Q4Device &w = *a.targets[target].w;
+    GemmParams p;
+    memset(&p, 0, sizeof p);
+    p.codes = w.codes;
+    p.meta = w.meta16;  // fp16 {scale, bias}: the weight is evaluated in fp16 here
+    if (a.x_columns != 0 && (a.x_columns * 2u != w.K || a.x_columns % kStepColumns != 0)) {
+        set_error(error, error_capacity, "q4 gemm: a repeated activation row is half the weight's columns, whole 128-column steps");
+        return MI355Q_ERROR_INVALID;
+    }
+    const uint32_t x_columns = a.x_columns ? a.x_columns : w.K;
+    int status = gemm_activations(ctx, a, x_columns, target == 0, p, error, error_capacity);
+    if (status != MI355Q_OK) return status;
+    const uint32_t rows = p.M;
+    // The doubled form of an 8-bit weight whose activation row the kernels would read twice: the
+    // kernel for 8-bit codes reads the bytes themselves instead, one pass over the row, half the
+    // matrix instructions.  It is the pipelined kernel, with that kernel's conditions.
+    const bool bytes_native = w.codes8 != nullptr && a.x_columns != 0 && !ctx->q8_gemm_doubled &&
+                              (uint64_t)rows * x_columns * sizeof(_Float16) + 16384u < (1ull << 32);
+    const uint32_t T = bytes_native ? w.T / 2u : w.T;
+    if (bytes_native) {
+        p.codes = w.codes8;
+        p.meta = w.meta8;
+    }
+    p.y = a.targets[target].y;
+    p.residual = a.targets[target].residual;
+    p.N = w.N;
+    p.K = x_columns;
+    p.wrap_steps = a.x_columns && !bytes_native ? a.x_columns / kStepColumns : 0xffffffffu;
+    p.NT = w.NT;
+    p.T = T;
+    p.y_dtype = a.y_dtype;
+    p.residual_dtype = a.residual_dtype;
+    p.residual_is_bias = a.residual_is_bias;
+    p.wide_stores = w.N % 4u == 0u && (uintptr_t)p.y % 16u == 0u;
+
+    const bool pipe_ok = gemm_pipe_ok(w, rows, x_columns);
+    int best = 0;
+    uint32_t best_splits = 1;
+    (void)gemm_decompose(ctx, w.NT, w.N, T, rows, bytes_native, pipe_ok, best, best_splits);
     // option "q4_gemm" = "VARIANT,SPLITS" for experiments
     if (ctx->force_gemm[1] >= 1 && ctx->force_gemm[0] < (int)(sizeof variants / sizeof variants[0]) &&
         (ctx->force_gemm[0] < 6 || pipe_ok) && (ctx->force_gemm[0] >= kBytesVariant) == bytes_native) {
@@ -313,7 +385,7 @@ int q4_gemm_linear(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, 
     p.splits = (T + p.steps_per_split - 1) / p.steps_per_split;
     if (p.splits > 1u) {
         const size_t bytes = (size_t)p.splits * rows * w.N * sizeof(float);
-        int status = ensure_stage(ctx, 4, bytes, error, error_capacity);
+        status = ensure_stage(ctx, 4, bytes, error, error_capacity);
         if (status != MI355Q_OK) return status;
         p.partials = (float *)ctx->stage[4];
     }
@@ -344,14 +416,233 @@ int q4_gemm_linear(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, 
     if (launched != hipSuccess)
         return fail_hip(launched, "q4 gemm kernel launch", error, error_capacity);
     if (p.splits > 1u) {
-        const uint32_t columns = kReduceThreads * (p.wide_stores ? 4u : 1u);
-        const dim3 reduce_grid((w.N + columns - 1u) / columns, a.M < 65535u ? a.M : 65535u);
-        launched = p.wide_stores ? launch(ctx, q4_gemm_reduce_kernel<true>, reduce_grid, dim3(kReduceThreads), 0, p)
-                                 : launch(ctx, q4_gemm_reduce_kernel<false>, reduce_grid, dim3(kReduceThreads), 0, p);
+        GemmGroup group;
+        group.shared = p;
+        group.targets = 1;
+        group.target[0] = gemm_target(p);
+        launched = launch_reduce(ctx, group);
         if (launched != hipSuccess)
             return fail_hip(launched, "q4 gemm reduce launch", error, error_capacity);
     }
     return MI355Q_OK;
+}
+
+// ---- 17..128 rows: q4_rows_kernel (q4_rows_device.h) ---------------------------------------
+
+struct RowsPlan {
+    int mf, ntw, waves;            // 16-row fragments, tiles per wave, waves
+    uint32_t blocks, units;        // blocks in all, units per workgroup
+};
+
+// The launch of q4_rows_kernel for a call's targets together; false: not the kernel for it.
+// Shape and workgroups minimise a microsecond estimate fitted to 1430 timings on this GPU (three
+// layer shapes, 17 to 128 rows, every block width, whole blocks and 128 to 768 workgroups; 8 % rms,
+// the choice within 8 % of the best timed one in 82 of 84 calls): 4.4 us, then per unit the longer
+// of one workgroup's own chain (0.22 + 0.12 us per 16 rows) and its share of the compute unit,
+// then, where workgroups share blocks, 3.7 us and the partial sums at 2.1 TB/s.  Chosen where that
+// is at most 1 us per target more than the other kernels' estimate, which leaves out the launches
+// behind a K split: at 27B shapes gate|up up to 128 rows (49 -> 33 us at 32, 82 -> 49 at 80, 77 ->
+// 65 at 128) and q|k|v (40 -> 14, 49 -> 23, 52 -> 30); o and down up to 48 and from 65 to 96 rows
+// (27 -> 23 us at 32, 37 -> 34 at 80; the other kernels' 27 against 30 at 64, 38 against 44 at 128).
+static bool rows_plan(mi355q_context *ctx, const Q4LinearArgs &a, RowsPlan &plan)
+{
+    const uint32_t rows = a.x_dtype == MI355Q_F32 ? 2u * a.M : a.M;
+    const Q4Device &first = *a.targets[0].w;
+    const uint32_t T = first.T;
+    if (rows > 128u) return false;
+    // 8-bit weights with byte tiles have a kernel that reads those
+    if (a.x_columns != 0 && first.codes8 != nullptr && !ctx->q8_gemm_doubled) return false;
+    plan.mf = (int)((rows + 15u) / 16u);
+    if (plan.mf < 2) plan.mf = 2;
+    if (plan.mf == 7) plan.mf = 8;
+    auto shape = [&](int which) {
+        plan.waves = which == 0 ? 4 : 8;
+        plan.ntw = which == 2 ? 2 : 1;
+        plan.blocks = 0;
+        for (uint32_t t = 0; t < a.count; ++t)
+            plan.blocks += (a.targets[t].w->NT + plan.waves * plan.ntw - 1u) / (plan.waves * plan.ntw);
+        return (uint64_t)plan.blocks * T < (1ull << 31);
+    };
+    if (ctx->force_gemm[1] >= 1) {
+        // option "q4_gemm": 11, 12, 13 = 4, 8, 16 tiles a block; 1 = whole blocks, s = 64 (s - 1) workgroups
+        if (ctx->force_gemm[0] < 11 || ctx->force_gemm[0] > 13 || !shape(ctx->force_gemm[0] - 11)) return false;
+        const uint32_t groups = ctx->force_gemm[1] == 1 ? plan.blocks : 64u * (uint32_t)(ctx->force_gemm[1] - 1);
+        plan.units = (plan.blocks * T + groups - 1u) / groups;
+        return true;
+    }
+    const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
+    double outputs = 0.0, best_cost = 1e30;
+    for (uint32_t t = 0; t < a.count; ++t) outputs += (double)rows * a.targets[t].w->N;
+    RowsPlan best = plan;
+    for (int which = 0; which < 3; ++which) {
+        if (!shape(which)) return false;
+        const uint32_t total = plan.blocks * T;
+        const uint32_t lds = rows_stages(plan.mf, plan.ntw, plan.waves) * rows_stage_bytes(plan.mf, plan.ntw, plan.waves);
+        const uint32_t places = std::min(160u * 1024u / lds, 2048u / (64u * plan.waves));  // on a compute unit
+        for (const uint32_t want : {plan.blocks, cus / 2u, cus, cus + cus / 2u, 2u * cus}) {
+            plan.units = (total + want - 1u) / want;
+            const uint32_t groups = (total + plan.units - 1u) / plan.units;
+            const uint32_t together = std::min(places, (groups + cus - 1u) / cus);
+            const uint32_t rounds = (groups + cus * together - 1u) / (cus * together);
+            const double tiles = plan.waves * plan.ntw, mf = plan.mf;
+            const double alone = 0.222 + 0.119 * mf, sharing = together * (tiles * (0.0344 + 0.0075 * mf) + 0.0282 * mf);
+            double cost = 4.4 + (double)rounds * plan.units * (alone > sharing ? alone : sharing);
+            if (plan.units % T != 0u && plan.units < total)
+                cost += 3.7 + 0.466e-6 * 4.0 * outputs * (T + plan.units - 1.0) / plan.units;
+            if (cost < best_cost) {
+                best_cost = cost;
+                best = plan;
+            }
+        }
+    }
+    plan = best;
+    double others = 0.0;
+    for (uint32_t t = 0; t < a.count; ++t) {
+        const Q4Device &w = *a.targets[t].w;
+        int variant;
+        uint32_t splits;
+        others += gemm_decompose(ctx, w.NT, w.N, T, rows, false, gemm_pipe_ok(w, rows, a.x_columns ? a.x_columns : w.K),
+                                 variant, splits);
+    }
+    return best_cost <= others + 1.0 * a.count;
+}
+
+template <int MF, int NTW, int W>
+static hipError_t launch_rows(mi355q_context *ctx, uint32_t groups, const GemmGroup &group)
+{
+    constexpr uint32_t bytes = rows_lds_bytes(MF, NTW, W);
+    bool &raised = ctx->rows_lds_raised[MF][W == 4 ? 0 : NTW];
+    if (!raised) {  // per context, as in launch_pipe
+        hipError_t status = hipFuncSetAttribute((const void *)q4_rows_kernel<MF, NTW, W>,
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        if (status != hipSuccess) return status;
+        raised = true;
+    }
+    return launch(ctx, q4_rows_kernel<MF, NTW, W>, dim3(groups), dim3(64u * W), bytes, group);
+}
+
+template <int NTW, int W>
+static hipError_t launch_rows_of(mi355q_context *ctx, int mf, uint32_t groups, const GemmGroup &group)
+{
+    switch (mf) {
+    case 2: return launch_rows<2, NTW, W>(ctx, groups, group);
+    case 3: return launch_rows<3, NTW, W>(ctx, groups, group);
+    case 4: return launch_rows<4, NTW, W>(ctx, groups, group);
+    case 5: return launch_rows<5, NTW, W>(ctx, groups, group);
+    case 6: return launch_rows<6, NTW, W>(ctx, groups, group);
+    default: return launch_rows<8, NTW, W>(ctx, groups, group);
+    }
+}
+
+static int q4_rows_linears(mi355q_context *ctx, const Q4LinearArgs &a, const RowsPlan &plan, char *error,
+                           size_t error_capacity)
+{
+    const Q4Device &first = *a.targets[0].w;
+    if (a.x_columns != 0 && (a.x_columns * 2u != first.K || a.x_columns % kStepColumns != 0)) {
+        set_error(error, error_capacity, "q4 gemm: a repeated activation row is half the weight's columns, whole 128-column steps");
+        return MI355Q_ERROR_INVALID;
+    }
+    const uint32_t x_columns = a.x_columns ? a.x_columns : first.K;
+    GemmGroup group;
+    memset(&group, 0, sizeof group);
+    GemmParams &p = group.shared;
+    int status = gemm_activations(ctx, a, x_columns, true, p, error, error_capacity);
+    if (status != MI355Q_OK) return status;
+    p.K = x_columns;
+    p.T = first.T;
+    p.wrap_steps = a.x_columns ? a.x_columns / kStepColumns : 0xffffffffu;
+    p.y_dtype = a.y_dtype;
+    p.residual_dtype = a.residual_dtype;
+    p.residual_is_bias = a.residual_is_bias;
+    p.splits = 1;
+    p.units = plan.units;
+    p.total_units = plan.blocks * p.T;
+    p.block_columns = (uint32_t)(plan.waves * plan.ntw) * kTileRows;
+    group.targets = a.count;
+    // blocks are shared unless every workgroup takes whole ones; a block meets at most this many
+    const bool sharing = p.units % p.T != 0u && p.units < p.total_units;
+    const uint32_t sharers = (p.T - 1u) / p.units + 2u;
+    if (sharing) {
+        size_t columns = 0;
+        for (uint32_t t = 0; t < a.count; ++t) columns += a.targets[t].w->N;
+        status = ensure_stage(ctx, 4, ((size_t)sharers * p.M * columns + 4u * a.count) * sizeof(float), error, error_capacity);
+        if (status != MI355Q_OK) return status;
+    }
+    float *partials = (float *)ctx->stage[4];
+    uint32_t blocks = 0;
+    for (uint32_t t = 0; t < a.count; ++t) {
+        const Q4Device &w = *a.targets[t].w;
+        GemmTarget &target = group.target[t];
+        target.codes = w.codes;
+        target.meta = w.meta16;
+        target.y = a.targets[t].y;
+        target.residual = a.targets[t].residual;
+        target.N = w.N;
+        target.NT = w.NT;
+        target.wide_stores = w.N % 4u == 0u && (uintptr_t)target.y % 16u == 0u;
+        target.first_block = blocks;
+        blocks += (w.NT + plan.waves * plan.ntw - 1u) / (plan.waves * plan.ntw);
+        if (sharing) {
+            target.partials = partials;
+            partials += ((size_t)sharers * p.M * w.N + 3u) / 4u * 4u;  // 16-byte aligned
+        }
+    }
+    const uint32_t groups = (p.total_units + p.units - 1u) / p.units;
+    if (ctx->trace)
+        fprintf(stderr, "mi355q: q4 rows M=%u K=%u -> %d rows x %u columns, %u workgroups of %d waves, %u steps each\n", p.M,
+                p.K, 16 * plan.mf, p.block_columns, groups, plan.waves, p.units);
+    hipError_t launched = plan.waves == 4 ? launch_rows_of<1, 4>(ctx, plan.mf, groups, group)
+                          : plan.ntw == 1 ? launch_rows_of<1, 8>(ctx, plan.mf, groups, group)
+                                          : launch_rows_of<2, 8>(ctx, plan.mf, groups, group);
+    if (launched != hipSuccess) return fail_hip(launched, "q4 rows kernel launch", error, error_capacity);
+    if (sharing) {
+        launched = launch_reduce(ctx, group);
+        if (launched != hipSuccess) return fail_hip(launched, "q4 gemm reduce launch", error, error_capacity);
+    }
+    return MI355Q_OK;
+}
+
+// Whether no target of the call writes what another one reads or writes, nor the activations:
+// only then may they run at the same time (and share converted activations).
+static bool targets_independent(const Q4LinearArgs &a)
+{
+    auto overlap = [](const void *p, size_t p_bytes, const void *q, size_t q_bytes) {
+        return (uintptr_t)p < (uintptr_t)q + q_bytes && (uintptr_t)q < (uintptr_t)p + p_bytes;
+    };
+    const size_t x_bytes = (size_t)a.M * (a.x_columns ? a.x_columns : a.targets[0].w->K) * dtype_bytes(a.x_dtype);
+    for (uint32_t t = 0; t < a.count; ++t) {
+        const size_t y_bytes = (size_t)a.M * a.targets[t].w->N * dtype_bytes(a.y_dtype);
+        if (overlap(a.targets[t].y, y_bytes, a.x, x_bytes)) return false;
+        for (uint32_t u = 0; u < a.count; ++u) {
+            if (u == t) continue;
+            const size_t cells = (a.residual_is_bias ? 1u : (size_t)a.M) * a.targets[u].w->N;
+            if (overlap(a.targets[t].y, y_bytes, a.targets[u].y, (size_t)a.M * a.targets[u].w->N * dtype_bytes(a.y_dtype)))
+                return false;
+            if (a.targets[u].residual != nullptr &&
+                overlap(a.targets[t].y, y_bytes, a.targets[u].residual, cells * dtype_bytes(a.residual_dtype)))
+                return false;
+        }
+    }
+    return true;
+}
+
+int q4_gemm_linears(mi355q_context *ctx, const Q4LinearArgs &a, char *error, size_t error_capacity)
+{
+    int status = MI355Q_OK;
+    if (a.count > 1u && !targets_independent(a)) {  // one after the other, in the caller's order
+        for (uint32_t t = 0; t < a.count && status == MI355Q_OK; ++t) {
+            Q4LinearArgs one = a;
+            one.count = 1;
+            one.targets[0] = a.targets[t];
+            status = q4_gemm_linears(ctx, one, error, error_capacity);
+        }
+        return status;
+    }
+    RowsPlan plan;
+    if (rows_plan(ctx, a, plan)) return q4_rows_linears(ctx, a, plan, error, error_capacity);
+    for (uint32_t t = 0; t < a.count && status == MI355Q_OK; ++t)
+        status = gemm_one_target(ctx, a, t, error, error_capacity);
+    return status;
 }
 
 }  // namespace mi355q

@@ -33,8 +33,58 @@ struct GemmParams {
     // of rows 2m (value) and 2m + 1 (rounding remainder).  Null: fp16 activations as given.
     const float *row_scale;
     int pair;
+    // q4_rows_kernel: units (128-column steps of a block) per workgroup and in all, columns of a
+    // block, and the target's first block (set by select_target); units 0: K splits as above
+    uint32_t units, total_units, block_columns, first_block;
     int xcd_order;         // pipelined kernel: blocks that share weights are placed on one XCD (see there)
 };
+
+// Up to kMaxTargets weights that share their activations go out as one launch: workgroups
+// [first_block, the next target's first_block) of the grid's x work on a target.
+struct GemmTarget {
+    const uint4 *codes;
+    const uint2 *meta;
+    void *y;
+    const void *residual;
+    float *partials;
+    uint32_t N, NT, first_block;
+    uint32_t first_reduce;  // the same for the kernel that adds K splits
+    int wide_stores;
+};
+struct GemmGroup {
+    GemmParams shared;  // everything else; its per-target fields are not read
+    GemmTarget target[kMaxTargets];
+    uint32_t targets;
+};
+
+// The parameters of one target.
+__device__ __forceinline__ GemmParams target_params(const GemmGroup &group, const GemmTarget &target)
+{
+    GemmParams p = group.shared;
+    p.codes = target.codes;
+    p.meta = target.meta;
+    p.y = target.y;
+    p.residual = target.residual;
+    p.partials = target.partials;
+    p.N = target.N;
+    p.NT = target.NT;
+    p.wide_stores = target.wide_stores;
+    p.first_block = target.first_block;
+    return p;
+}
+__device__ __forceinline__ GemmParams only_target(const GemmGroup &group) { return target_params(group, group.target[0]); }
+// Those of the target that workgroup `block` works on; `block` becomes its number there.
+template <bool REDUCE = false>
+__device__ __forceinline__ GemmParams select_target(const GemmGroup &group, uint32_t &block)
+{
+    uint32_t t = 0;
+#pragma unroll
+    for (uint32_t i = 1; i < kMaxTargets; ++i)
+        if (i < group.targets && block >= (REDUCE ? group.target[i].first_reduce : group.target[i].first_block)) t = i;
+    const GemmTarget &target = group.target[t];
+    block -= REDUCE ? target.first_reduce : target.first_block;
+    return target_params(group, target);
+}
 
 __device__ __forceinline__ half8 dequant8(uint32_t word, const NibbleMasks &masks, half8 scale,
                                           half8 bias)
@@ -903,8 +953,10 @@ __global__ void __launch_bounds__(256, 1) q4_gemm_pipe_kernel(const GemmParams p
     // fp32 activations - leaves the same way as fp32, in two halves of 64 rows (a whole block of
     // them is a few KB more than the stage): a thread takes four adjacent columns of a row of the
     // block, 16 bytes per lane and the row contiguous, instead of 16-byte pieces of 16 rows 4 N
-    // bytes apart.  The two rows of a pair meet here, so that converted activations need no
-    // staging matrix and no second kernel.
+    // bytes apart.  The two rows of a pair meet here, so that converted activations need no fp32
+    // staging matrix and no second kernel over it: 4646 rows of 5376 bf16 columns by 14336 took
+    // 821 us with them (150 in that kernel) and take 623 without, the six linears of a 1280-wide
+    // encoder layer over 1500 fp32 rows 315 and 257.
     constexpr uint32_t PITCH32 = WIDTH * 4u + 16u;
     static_assert(PITCH32 % 16u == 0u && (PITCH32 / 16u) % 2u == 1u, "rows start 16-byte aligned, an odd number of 16-byte units apart");
     static_assert((size_t)(BM / 2) * PITCH32 <= pipe_lds_bytes(BM), "half a block fits the activation stage");

@@ -128,7 +128,7 @@ __global__ void __launch_bounds__(256) q4_stream_reduce_kernel(const StreamParam
 // Bound by memory (each row is read once from HBM and once more from the compute unit's vector
 // cache).  A thread takes eight adjacent columns at a time, 16- and 32-byte loads and 16-byte
 // stores: with one element per thread and access the 4646 x 5376 bf16 rows of a video clip took
-// 74 us (1.4 TB/s), now NEW_US (rows are whole 64-column groups and the entry points take
+// 74 us (1.4 TB/s), now 24 us (4.1 TB/s; rows are whole 64-column groups and the entry points take
 // 16-byte aligned activations only).
 constexpr uint32_t kConvertThreads = 256;
 template <bool BF16>

@@ -319,3 +319,76 @@ def test_targets_share_converted_activations(engine, gpu, x_dtype, M):
             gpu.free(pointer)
         for weight in weights:
             weight.destroy()
+
+
+@pytest.mark.parametrize("forced", ["11,1", "11,2", "12,1", "12,2", "12,3", "13,1", "13,2"])
+@pytest.mark.parametrize("N,K,M", [(100, 64, 17), (272, 128, 32), (1102, 192, 33), (1104, 1024, 48), (560, 576, 63),
+                                   (1001, 640, 67), (272, 2176, 80), (1104, 384, 96), (256, 1088, 97), (1102, 256, 128),
+                                   (9000, 1920, 40)])
+def test_rows_kernel(engine, oracle, gpu, force, forced, N, K, M):
+    """17 to 128 rows by blocks of 4, 8 and 16 tiles: fragments of rows partly filled, tiles beyond
+    the matrix, K an odd multiple of 64 (half of the last step does not exist), fewer steps than
+    stages, workgroups that take one step, several blocks, or the end of one block and the
+    beginning of the next."""
+    force("q4_gemm", forced)
+    run_case(engine, oracle, gpu, N, K, M, engine.META_BF16_PLANES, engine.F16, engine.F32, residual=True)
+    run_case(engine, oracle, gpu, N, K, M, engine.META_F16_INTERLEAVED, engine.F16, engine.F16)
+
+
+@pytest.mark.parametrize("forced", ["11,2", "12,1", "13,1", "13,2"])
+@pytest.mark.parametrize("x_dtype,M", [("F32", 9), ("F32", 35), ("F32", 64), ("BF16", 17), ("BF16", 75)])
+def test_rows_kernel_targets_and_converted_activations(engine, gpu, force, forced, x_dtype, M):
+    """Three weights of unequal width as one launch, activations converted: each output equals the
+    same weight's own call under the other GEMM kernels up to the order of the fp32 sums."""
+    K, widths = 448, (272, 1002, 100)
+    x32 = make_x(engine, 101, M, K)
+    x = x32 if x_dtype == "F32" else bf16_bits(x32).reshape(M, K)
+    kind, x_dtype = engine.META_BF16_PLANES, getattr(engine, x_dtype)
+    weights = [gpu.q4_prepare(*engine.synth_q4_affine(102 + i, 0.02, N, K, kind), N, K, kind) for i, N in enumerate(widths)]
+    biases = [gpu.to_device(engine.synth_normal_f32(110 + i, 1.0, N)) for i, N in enumerate(widths)]
+    x_ptr = gpu.to_device(x)
+    outputs = [gpu.alloc(M * N * 4) for N in widths]
+    try:
+        results = []
+        targets = list(zip(weights, outputs, biases))
+        for how, groups in ((forced, [targets]), ("4,1", [[t] for t in targets])):
+            print(f"rows targets M={M} x={x_dtype} forced={how}", flush=True)
+            force("q4_gemm", how)
+            gpu.q4_sequence(engine.make_calls([(g, x_ptr, x_dtype, M, engine.F32, engine.F32, engine.RESIDUAL_IS_BIAS)
+                                               for g in groups]))
+            gpu.sync()
+            results.append([gpu.download(p, (M, N), np.float32) for p, N in zip(outputs, widths)])
+        for here, there in zip(*results):
+            assert np.any(there != 0)
+            # 448 products of one row summed in another order: 448 roundings of 2^-24 at most
+            assert np.max(np.abs(here - there)) <= 448 * 2.0 ** -24 * np.max(np.abs(there))
+    finally:
+        for pointer in [x_ptr] + outputs + biases:
+            gpu.free(pointer)
+        for weight in weights:
+            weight.destroy()
+
+
+@pytest.mark.parametrize("M", [20, 150])
+def test_targets_that_depend_on_each_other(engine, gpu, M):
+    """A call whose second target adds the first one's output runs its targets in order: the same bits as one call per weight."""
+    K = N = 256
+    kind = engine.META_BF16_PLANES
+    weights = [gpu.q4_prepare(*engine.synth_q4_affine(120 + i, 0.02, N, K, kind), N, K, kind) for i in range(2)]
+    x = make_x(engine, 122, M, K).astype(np.float16)
+    x_ptr, first, second = gpu.to_device(x), gpu.alloc(M * N * 2), gpu.alloc(M * N * 2)
+    try:
+        results = []
+        targets = [(weights[0], first, None), (weights[1], second, first)]
+        for groups in ([targets], [[t] for t in targets]):
+            print(f"gemm dependent targets M={M} calls={len(groups)}", flush=True)
+            gpu.q4_sequence(engine.make_calls([(g, x_ptr, engine.F16, M, engine.F16, engine.F16) for g in groups]))
+            gpu.sync()
+            results.append([gpu.download(p, (M, N), np.uint16) for p in (first, second)])
+        for together, alone in zip(*results):
+            assert np.array_equal(together, alone) and np.any(alone != 0)
+    finally:
+        for pointer in (x_ptr, first, second):
+            gpu.free(pointer)
+        for weight in weights:
+            weight.destroy()
