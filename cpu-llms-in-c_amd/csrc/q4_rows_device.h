@@ -7,44 +7,6 @@
 
 namespace mi355q {
 
-// Loads that write LDS directly (uniform base + 32-bit lane offset); lane l's bytes land at
-// lds_base + 16 l (4 l).  NT: use-once data.  m0 is named as clobbered so that the compiler
-// carries no value of its own in it across the statement (it warns that m0 is reserved, which is
-// the point).
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-template <bool NT>
-__device__ __forceinline__ void rows_load_x4(uint32_t lane_offset, const char *base, uint32_t lds_base)
-{
-    if constexpr (NT)
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"
-                     :
-                     : "v"(lane_offset), "s"(base), "s"(lds_base)
-                     : "memory", "m0");
-    else
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                     :
-                     : "v"(lane_offset), "s"(base), "s"(lds_base)
-                     : "memory", "m0");
-}
-__device__ __forceinline__ void rows_load_x1(uint32_t lane_offset, const char *base, uint32_t lds_base)
-{
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
-                 :
-                 : "v"(lane_offset), "s"(base), "s"(lds_base)
-                 : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-// A value that is the same in all lanes, in scalar registers whatever the compiler made of it.
-__device__ __forceinline__ const char *uniform(const char *at)
-{
-    const uint64_t bits = (uint64_t)at;
-    const uint32_t low = __builtin_amdgcn_readfirstlane((uint32_t)bits);  // (the builtin returns a signed word)
-    const uint32_t high = __builtin_amdgcn_readfirstlane((uint32_t)(bits >> 32));
-    return (const char *)((uint64_t)high << 32 | low);
-}
-
 // One stage = one 128-column step of a workgroup: 16 * MF rows of x (256 bytes each), then each
 // wave's own NTW tiles of codes, then their metadata.
 constexpr uint32_t rows_stage_bytes(int mf, int ntw, int waves)
@@ -145,13 +107,13 @@ __global__ void __launch_bounds__(64 * W, 2) q4_rows_kernel(const GemmGroup grou
 #pragma unroll
         for (int j = 0; j < XJ; ++j) {
             const uint32_t octet = r ^ ((x_row[j] + kq) & 15u);
-            rows_load_x4<false>(tail && octet >= 8u ? x_lane[j] - 128u : x_lane[j], x_at, __builtin_amdgcn_readfirstlane(at + x_row[j] * 256u));
+            load_lds_x4<false>(tail && octet >= 8u ? x_lane[j] - 128u : x_lane[j], x_at, __builtin_amdgcn_readfirstlane(at + x_row[j] * 256u));
         }
         const size_t record = (size_t)fetch_step * fetch_NT;
 #pragma unroll
         for (int t = 0; t < NTW; ++t)
-            rows_load_x4<true>(lane * 16u, uniform(fetch_codes + (record + fetch_tile[t]) * 1024u), at + CODES + (wave * NTW + t) * 1024u);
-        rows_load_x1(meta_lane, uniform(fetch_meta + record * 128u), at + METAS + wave * 256u);
+            load_lds_x4<true>(lane * 16u, uniform(fetch_codes + (record + fetch_tile[t]) * 1024u), at + CODES + (wave * NTW + t) * 1024u);
+        load_lds_x1(meta_lane, uniform(fetch_meta + record * 128u), at + METAS + wave * 256u);
         fetched += 1u;
         if (++fetch_step == T) {
             fetch_step = 0;

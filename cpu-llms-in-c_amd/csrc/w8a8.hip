@@ -281,6 +281,204 @@ __global__ void __launch_bounds__(256) w8a8_kernel(const W8a8Params p)
         }
 }
 
+// ---- more work than the kernel above gets through at once ------------------------------------------
+
+// Waits until no more of a wave's loads are out than those of the `younger` steps (at most MOST),
+// PER loads each.
+template <int PER, int MOST>
+__device__ __forceinline__ void wait_for_step(uint32_t younger)
+{
+    if constexpr (MOST > 0) {
+        if (younger < (uint32_t)MOST) {
+            wait_for_step<PER, MOST - 1>(younger);
+            return;
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(PER * MOST) : "memory");
+}
+
+// Block of 32*FM activation rows by 32*FN weight rows, four waves as 2 x 2, each with FM x FN
+// fragments.  The kernel above reads its whole activation block for every sixteen weight rows:
+// at 768 rows and three weights of 4096 x 2048 that is 1.5 GB through the L2s, which bounds it
+// (174 us a pass with the quantizer's, here 49 = 790 TOP/s).  Here the activations and weights
+// of S 64-column steps are written to LDS once per block by LDS-direct loads, R - 1 such stages
+// ahead of the products.  Both lie in LDS as the matrix instruction's operands, 1 KiB a fragment,
+// so every LDS access is sixteen consecutive bytes per lane; the activations get there by the
+// lanes' own addresses.  The loads are asm statements in one in-order queue under one counted wait
+// per stage.  Weights are the first operand: lane (r, kq) then holds activation row r and the four
+// adjacent outputs 4 kq .. + 3 of a tile, one store.  Up to one block per compute unit what bounds
+// it is the chain of a stage (wait, barrier, LDS read, product): two steps a stage instead of one
+// 16.4 -> 14.9 us at 64 rows, 1000 x 2048, while stages further ahead (7 instead of 3) change
+// nothing; above that the output's stores and the loads.  Blocks of 128 x 128: 53.6 against 48.5 us
+// at 768 rows, 4096 x 2048, and 19.8 against 15.4 at 128 rows, 4096 x 1024.
+template <int FM, int FN, int S, int R>
+__global__ void __launch_bounds__(256, 2) w8a8_block_kernel(const W8a8Params p)
+{
+    constexpr int LOADS = (FM + FN) / 2;  // a wave's loads per step
+    constexpr uint32_t STEP = (2u * FM + 2u * FN) * 1024u, STAGE = S * STEP;
+    static_assert((FM + FN) % 2 == 0 && S * LOADS * (R - 1) <= 63, "whole loads per wave; the load counter has six bits");
+    __shared__ uint4 lds[R * STAGE / 16u];
+    typedef __attribute__((address_space(3))) void *lds_ptr;
+
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t r = lane & 15u, kq = lane >> 4;
+    uint32_t target = 0;
+#pragma unroll
+    for (uint32_t t = 1; t < kW8a8Targets; ++t)
+        if (t < p.targets && blockIdx.x >= p.first_group[t]) target = t;
+    const uint32_t N = p.N[target], NT = (N + 15u) / 16u, KS = p.KS, M = p.M, K = p.K;
+    const uint32_t tile0 = (blockIdx.x - p.first_group[target]) * (2u * FN);
+    const uint32_t m0 = blockIdx.y * (32u * FM);
+
+    // Load e of a step is activation fragment e, or weight tile e - 2 FM.  Rows past M repeat the
+    // last row and tiles past the last the last tile: read in bounds, never stored.
+    const char *base[LOADS];
+    uint32_t lane_offset[LOADS];
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) {
+        const uint32_t e = wave * LOADS + j;
+        if (e < 2u * FM) {
+            const uint32_t m = m0 + 16u * e + r;
+            lane_offset[j] = (m < M ? m : M - 1u) * K;
+            base[j] = uniform((const char *)p.q);
+        } else {
+            const uint32_t tile = tile0 + e - 2u * FM;
+            lane_offset[j] = lane * 16u;
+            base[j] = uniform((const char *)(p.tiles[target] + (size_t)(tile < NT ? tile : NT - 1u) * KS * 64u));
+        }
+    }
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr)lds);
+    const uint32_t stages = (KS + S - 1u) / S;
+    auto fetch = [&](uint32_t stage, uint32_t slot) {
+#pragma unroll
+        for (uint32_t u = 0; u < (uint32_t)S; ++u) {
+            const uint32_t ks = stage * S + u < KS ? stage * S + u : KS - 1u;  // past the last: not multiplied
+            // columns past K read the row's last sixteen codes against the tile's zero padding
+            const uint32_t k = ks * 64u + kq * 16u, column = k + 16u <= K ? k : K - 16u;
+#pragma unroll
+            for (int j = 0; j < LOADS; ++j) {
+                const uint32_t e = wave * LOADS + j;
+                load_lds_x4<false>(lane_offset[j] + (e < 2u * FM ? column : ks * 1024u), base[j],
+                                   __builtin_amdgcn_readfirstlane(lds0 + slot * STAGE + u * STEP + e * 1024u));
+            }
+        }
+    };
+
+    const uint32_t row_fragment = (wave & 1u) * FM, tile_fragment = (wave >> 1) * FN;
+    intx4 acc[FN][FM];
+#pragma unroll
+    for (int t = 0; t < FN; ++t)
+#pragma unroll
+        for (int i = 0; i < FM; ++i) acc[t][i] = intx4{0, 0, 0, 0};
+#pragma unroll
+    for (int s = 0; s < R - 1; ++s)
+        if ((uint32_t)s < stages) fetch(s, s);
+    uint32_t slot = 0;
+    for (uint32_t i_stage = 0; i_stage < stages; ++i_stage) {
+        // this wave's loads of the stage have landed once only those of the younger ones are left
+        wait_for_step<S * LOADS, R - 2>(stages - 1u - i_stage);
+        // behind the barrier every wave's have, and every wave has read the last of the stage
+        // before, whose slot is filled next
+        asm volatile("s_barrier" ::: "memory");
+        if (i_stage + R - 1u < stages) fetch(i_stage + R - 1u, slot == 0u ? R - 1u : slot - 1u);
+
+#pragma unroll
+        for (uint32_t u = 0; u < (uint32_t)S; ++u) {
+            if (u > 0u && i_stage * S + u >= KS) break;
+            const uint4 *const step = lds + (slot * STAGE + u * STEP) / 16u + lane;
+            intx4 rows[FM];
+#pragma unroll
+            for (int i = 0; i < FM; ++i) rows[i] = __builtin_bit_cast(intx4, step[(row_fragment + i) * 64u]);
+#pragma unroll
+            for (int t = 0; t < FN; ++t) {
+                const intx4 weights = __builtin_bit_cast(intx4, step[(2u * FM + tile_fragment + t) * 64u]);
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+                    acc[t][i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(weights, rows[i], acc[t][i], 0, 0, 0);
+            }
+        }
+        slot = slot + 1u == (uint32_t)R ? 0u : slot + 1u;
+    }
+
+    typedef float floatx4 __attribute__((ext_vector_type(4)));
+    float *const out = p.out[target];
+    int32_t *const acc_out = p.acc[target];
+    const float *const bias = p.bias[target];
+    const bool wide = N % 4u == 0u && (uintptr_t)out % 16u == 0u && (uintptr_t)acc_out % 16u == 0u;
+#pragma unroll
+    for (int t = 0; t < FN; ++t) {
+        const uint32_t n = (tile0 + tile_fragment + t) * 16u + 4u * kq;
+        float wscale[4], shift[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            wscale[j] = n + j < N ? p.wscales[target][n + j] : 0.0f;
+            shift[j] = bias && n + j < N ? bias[n + j] : 0.0f;
+        }
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            const uint32_t m = m0 + (row_fragment + i) * 16u + r;
+            if (m >= M || n >= N) continue;
+            const float xscale = p.xscales[m];
+            floatx4 value;
+            {
+#pragma clang fp contract(off)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (p.channel_major) {
+                        float product = wscale[j] * xscale;
+                        product = product * (float)acc[t][i][j];
+                        value[j] = shift[j] + product;
+                    } else {
+                        float product = (float)acc[t][i][j] * wscale[j];
+                        product = product * xscale;
+                        value[j] = product + shift[j];
+                    }
+                }
+            }
+            const size_t at = (size_t)m * N + n;
+            if (wide) {
+                if (acc_out) *(intx4 *)(acc_out + at) = acc[t][i];
+                if (!p.channel_major) {
+                    *(floatx4 *)(out + at) = value;
+                    continue;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (n + j >= N) continue;
+                if (acc_out && !wide) acc_out[at + j] = acc[t][i][j];
+                out[p.channel_major ? (size_t)(n + j) * M + m : at + j] = value[j];
+            }
+        }
+    }
+}
+
+// Which kernel takes a call (us of a pass, quantizer included, three weights):
+//   w8a8_kernel while its workgroups - one per weight tile and 64 rows - are fewer than two per
+//     compute unit, and up to 32 rows: its four waves share the columns, so its chain over K is a
+//     quarter as long (64 rows, 1000 x 2048: 12.2 against 15.1; 20 rows, 4096 x 2048: 12.7, 14.7);
+//   blocks of 64 x 64 from there (33 rows, 4096 x 2048: 15.6 -> 15.1, 64: 21.8 -> 15.6, 256: 61.1
+//     -> 25.1; 160 rows, 1000 x 2048: 20.7 -> 15.2; 64 rows, 4096 x 1024: 13.6 -> 11.6);
+//   blocks of 64 x 128 - three loads for eight products where the small ones take two for four -
+//     from four small blocks per compute unit (512 rows, 4096 x 2048: 41.0 -> 33.7; 768: 58 -> 49;
+//     but 256 rows, 4096 x 560, three per compute unit: 13.6 against 15.0).
+enum class W8a8Kernel { tiles, small_blocks, blocks };
+static W8a8Kernel w8a8_choose(mi355q_context *ctx, const W8a8Params &p)
+{
+    // option "w8a8" is about the kernel of tiles; the other one has 32-bit byte offsets into q and a tile
+    if (ctx->w8a8_tiles || (uint64_t)p.M * p.K >= (1ull << 32) || (uint64_t)p.KS * 1024u >= (1ull << 32))
+        return W8a8Kernel::tiles;
+    const uint64_t cus = (uint64_t)ctx->props.multiProcessorCount, m_blocks = (p.M + 63u) / 64u;
+    uint64_t tiles = 0, columns = 0;
+    for (uint32_t t = 0; t < p.targets; ++t) {
+        tiles += (p.N[t] + 15u) / 16u;
+        columns += (p.N[t] + 63u) / 64u;
+    }
+    if (p.M <= 32u || tiles * m_blocks < 2u * cus) return W8a8Kernel::tiles;
+    return columns * m_blocks < 4u * cus ? W8a8Kernel::small_blocks : W8a8Kernel::blocks;
+}
+
 template <int MB>
 static hipError_t launch_w8a8(mi355q_context *ctx, dim3 grid, uint32_t tiles_per_group, const W8a8Params &p)
 {
@@ -546,25 +744,39 @@ int mi355q_w8a8_linear_multi(mi355q_context *ctx, const mi355q_w8a8_target *targ
             }
         }
     }
-    // Tiles per workgroup (they share the workgroup's activation registers).  Measured at
-    // M = 64, K = 1024, three weights of 4096 rows (768 tiles): 10.0 / 10.0 / 11.6 / 10.1 us for
-    // 1 / 2 / 3 / 4 tiles, so a launch takes one unless the option "w8a8" says otherwise.
-    const uint32_t m_blocks = M > 32u ? (M + 63u) / 64u : 1u;
-    uint32_t per_group = ctx->w8a8_tiles ? (uint32_t)ctx->w8a8_tiles : 1u;
-    per_group = per_group < 1u ? 1u : per_group > 4u ? 4u : per_group;
-    uint32_t groups = 0;
-    for (uint32_t t = 0; t < count; ++t) {
-        p.first_group[t] = groups;
-        groups += (targets[t].weight->NT + per_group - 1u) / per_group;
-    }
-    const dim3 grid(groups, m_blocks);
     hipError_t launched;
-    if (M > 32u)
-        launched = launch_w8a8<4>(ctx, grid, per_group, p);
-    else if (M > 16u)
-        launched = launch_w8a8<2>(ctx, grid, per_group, p);
-    else
-        launched = launch_w8a8<1>(ctx, grid, per_group, p);
+    const W8a8Kernel kernel = w8a8_choose(ctx, p);
+    if (kernel != W8a8Kernel::tiles) {
+        const uint32_t tiles = kernel == W8a8Kernel::small_blocks ? 4u : 8u;  // of a block
+        uint32_t groups = 0;
+        for (uint32_t t = 0; t < count; ++t) {
+            p.first_group[t] = groups;
+            groups += (targets[t].weight->NT + tiles - 1u) / tiles;
+        }
+        const dim3 grid(groups, (M + 63u) / 64u);
+        launched = kernel == W8a8Kernel::small_blocks
+                       ? launch(ctx, w8a8_block_kernel<2, 2, 2, 3>, grid, dim3(256), 0, p)
+                       : launch(ctx, w8a8_block_kernel<2, 4, 1, 4>, grid, dim3(256), 0, p);
+    } else {
+        // Tiles per workgroup (they share the workgroup's activation registers).  Measured at
+        // M = 64, K = 1024, three weights of 4096 rows (768 tiles): 10.0 / 10.0 / 11.6 / 10.1 us for
+        // 1 / 2 / 3 / 4 tiles, so a launch takes one unless the option "w8a8" says otherwise.
+        const uint32_t m_blocks = M > 32u ? (M + 63u) / 64u : 1u;
+        uint32_t per_group = ctx->w8a8_tiles ? (uint32_t)ctx->w8a8_tiles : 1u;
+        per_group = per_group < 1u ? 1u : per_group > 4u ? 4u : per_group;
+        uint32_t groups = 0;
+        for (uint32_t t = 0; t < count; ++t) {
+            p.first_group[t] = groups;
+            groups += (targets[t].weight->NT + per_group - 1u) / per_group;
+        }
+        const dim3 grid(groups, m_blocks);
+        if (M > 32u)
+            launched = launch_w8a8<4>(ctx, grid, per_group, p);
+        else if (M > 16u)
+            launched = launch_w8a8<2>(ctx, grid, per_group, p);
+        else
+            launched = launch_w8a8<1>(ctx, grid, per_group, p);
+    }
     if (launched != hipSuccess) return fail_hip(launched, "w8a8 kernel launch", error, error_capacity);
     if (!device) {
         for (uint32_t t = 0; t < count; ++t) {

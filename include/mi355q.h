@@ -122,7 +122,7 @@ int mi355q_context_info(mi355q_context *ctx, mi355q_device_info *info,
  *   "q4_gemm"   = "VARIANT,SPLITS"              forces the GEMM's kernel variant and K split
  *   "trace"     = "1"                           prints every launch's decomposition to stderr
  *   "in_kernel_slices" = "0"                    K slices are added by a second kernel
- *   "w8a8"      = "1" .. "4"                    W8A8: weight tiles per workgroup
+ *   "w8a8"      = "1" .. "4"                    W8A8: the kernel of tiles, with so many per workgroup
  *   "gemm_loads" = "plain"                      GEMM variant 7 built with ordinary weight loads
  *                                               (compiler-placed waits): the cross-check of the
  *                                               hand-scheduled kernel, same bits, slower

@@ -98,6 +98,44 @@ def test_shared_activation_launch_with_several_tiles_per_workgroup(engine, oracl
         assert np.array_equal(results[i][0].view(np.uint32), out_ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("M,K,widths,channel_major", [
+    (33, 16, (8196,), False), (33, 80, (8203,), True), (64, 144, (4096, 2047, 2052), False),
+    (65, 272, (4100,), False), (127, 208, (4093,), True),                        # blocks of 64 x 64
+    (255, 336, (16388,), False), (256, 192, (16400,), True), (257, 64, (9000, 4107), False)])  # 64 x 128
+def test_block_kernel_gives_the_tile_kernels_bits(engine, oracle, gpu, force, M, K, widths, channel_major):
+    """Calls with enough work for the kernel of 64-row blocks: one to six 64-column steps (its ring
+    of stages holds up to four, two steps a stage in the small blocks), columns that end inside a
+    step, ragged rows and weight rows, several weights, both output orders, outputs that end on a
+    16-byte boundary and not (with several weights the accumulators start at any multiple of four
+    bytes).  Integer sums and one order of fp32 operations: the bits of the kernel of tiles
+    (option "w8a8" = "1") and of the oracle."""
+    q, scales = oracle.quantize_i8(engine.synth_normal_f32(41, 1.0, M * K).reshape(M, K))
+    rows = [engine.synth_w8_rows(42 + i, 0.02, N, K) for i, N in enumerate(widths)]
+    biases = [engine.synth_normal_f32(52 + i, 1.0, N) if i != 1 else None for i, N in enumerate(widths)]
+    weights = [gpu.w8a8_prepare(r, N, K) for r, N in zip(rows, widths)]
+    print(f"w8a8 blocks M={M} K={K} widths={widths} channel_major={channel_major}", flush=True)
+
+    def call():
+        if len(widths) == 1:
+            return [gpu.w8a8_linear(weights[0], widths[0], q, scales, biases[0], channel_major=channel_major)]
+        return gpu.w8a8_linear_multi(weights, widths, q, scales, biases)
+
+    try:
+        blocks = call()
+        force("w8a8", "1")
+        tiles = call()
+    finally:
+        for weight in weights:
+            gpu.w8a8_destroy(weight)
+    for i, N in enumerate(widths):
+        out_ref, acc_ref = oracle.w8a8_linear(rows[i], N, K, q, scales, biases[i])
+        if channel_major:
+            out_ref = oracle.w8a8_conv(rows[i], N, K, q, scales, biases[i])
+        assert blocks[i][1].tobytes() == tiles[i][1].tobytes() == acc_ref.tobytes()
+        assert np.array_equal(blocks[i][0].view(np.uint32), out_ref.view(np.uint32))
+        assert np.array_equal(tiles[i][0].view(np.uint32), out_ref.view(np.uint32))
+
+
 def test_reference_golden_vectors(engine, gpu):
     g = np.load(GOLDEN, allow_pickle=False)
     x, rows, bias = g["x"], g["rows"], g["bias"]
