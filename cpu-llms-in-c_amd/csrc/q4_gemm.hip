@@ -73,7 +73,8 @@ __global__ void __launch_bounds__(kReduceThreads) q4_gemm_reduce_kernel(const Ge
     const GemmParams p = SPLITS ? only_target(group) : select_target<true>(group, block);
     const uint32_t n = (block * kReduceThreads + threadIdx.x) * PER;
     if (n >= p.N) return;
-    const size_t stride = (size_t)p.M * p.N;
+    const uint32_t columns = p.units ? padded_columns(p.N) : p.N;  // of a row of partial sums
+    const size_t stride = (size_t)p.M * columns;
     uint32_t splits = p.splits;
     if (!SPLITS && p.units) {  // one workgroup alone has stored the outputs
         const uint32_t begin = (p.first_block + n / p.block_columns) * p.T;
@@ -97,7 +98,15 @@ __global__ void __launch_bounds__(kReduceThreads) q4_gemm_reduce_kernel(const Ge
 #pragma unroll
             for (int s = 0; s < SPLITS; ++s) add(sum, piece[s]);
         } else {
-            for (uint32_t s = 0; s < splits; ++s) add(sum, *(const Piece *)(p.partials + s * stride + from));
+            for (uint32_t s = 0; s < splits; s += 4u) {  // four on their way at once; past the last it is read again
+                Piece piece[4];
+#pragma unroll
+                for (uint32_t i = 0; i < 4u; ++i)
+                    piece[i] = *(const Piece *)(p.partials + (s + i < splits ? s + i : splits - 1u) * stride + from);
+#pragma unroll
+                for (uint32_t i = 0; i < 4u; ++i)
+                    if (s + i < splits) add(sum, piece[i]);
+            }
         }
         return sum;
     };
@@ -105,10 +114,10 @@ __global__ void __launch_bounds__(kReduceThreads) q4_gemm_reduce_kernel(const Ge
     for (uint32_t m = blockIdx.y; m < rows; m += gridDim.y) {
         Piece value;
         if (p.pair) {
-            value = add_splits((size_t)(2u * m) * p.N + n);
-            add(value, add_splits((size_t)(2u * m + 1u) * p.N + n));
+            value = add_splits((size_t)(2u * m) * columns + n);
+            add(value, add_splits((size_t)(2u * m + 1u) * columns + n));
         } else {
-            value = add_splits((size_t)m * p.N + n);
+            value = add_splits((size_t)m * columns + n);
         }
         if constexpr (WIDE) {
             finish_four(p, false, 0, m, n, value);
@@ -189,6 +198,8 @@ static hipError_t launch_reduce(mi355q_context *ctx, GemmGroup &group)
     case 4: return launch(ctx, q4_gemm_reduce_kernel<true, 4>, grid, dim3(kReduceThreads), 0, group);
     case 5: return launch(ctx, q4_gemm_reduce_kernel<true, 5>, grid, dim3(kReduceThreads), 0, group);
     case 6: return launch(ctx, q4_gemm_reduce_kernel<true, 6>, grid, dim3(kReduceThreads), 0, group);
+    case 7: return launch(ctx, q4_gemm_reduce_kernel<true, 7>, grid, dim3(kReduceThreads), 0, group);
+    case 8: return launch(ctx, q4_gemm_reduce_kernel<true, 8>, grid, dim3(kReduceThreads), 0, group);
     default: return launch(ctx, q4_gemm_reduce_kernel<true, 0>, grid, dim3(kReduceThreads), 0, group);
     }
 }
@@ -564,8 +575,8 @@ static int q4_rows_linears(mi355q_context *ctx, const Q4LinearArgs &a, const Row
     const uint32_t sharers = (p.T - 1u) / p.units + 2u;
     if (sharing) {
         size_t columns = 0;
-        for (uint32_t t = 0; t < a.count; ++t) columns += a.targets[t].w->N;
-        status = ensure_stage(ctx, 4, ((size_t)sharers * p.M * columns + 4u * a.count) * sizeof(float), error, error_capacity);
+        for (uint32_t t = 0; t < a.count; ++t) columns += padded_columns(a.targets[t].w->N);
+        status = ensure_stage(ctx, 4, (size_t)sharers * p.M * columns * sizeof(float), error, error_capacity);
         if (status != MI355Q_OK) return status;
     }
     float *partials = (float *)ctx->stage[4];
@@ -584,7 +595,7 @@ static int q4_rows_linears(mi355q_context *ctx, const Q4LinearArgs &a, const Row
         blocks += (w.NT + plan.waves * plan.ntw - 1u) / (plan.waves * plan.ntw);
         if (sharing) {
             target.partials = partials;
-            partials += ((size_t)sharers * p.M * w.N + 3u) / 4u * 4u;  // 16-byte aligned
+            partials += (size_t)sharers * p.M * padded_columns(w.N);
         }
     }
     const uint32_t groups = (p.total_units + p.units - 1u) / p.units;

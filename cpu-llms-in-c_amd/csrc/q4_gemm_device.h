@@ -161,6 +161,10 @@ __device__ __forceinline__ uint32_t bf16_bits(float v)  // round to nearest even
     return (bits + 0x7fffu + ((bits >> 16) & 1u)) >> 16;
 }
 
+// Columns of a row of q4_rows_kernel's partial sums: padded, so that they are 16-byte pieces for
+// every N.
+__host__ __device__ __forceinline__ uint32_t padded_columns(uint32_t N) { return (N + 3u) / 4u * 4u; }
+
 // Four adjacent columns n .. n + 3 of output row m: row scale, residual, conversion, store; or, when
 // partial, of row m of a K split's partial sums.  Columns from N on are not stored.
 __device__ __forceinline__ void finish_four(const GemmParams &p, bool partial, uint32_t split, uint32_t m, uint32_t n,

@@ -188,14 +188,15 @@ __global__ void __launch_bounds__(64 * W, 2) q4_rows_kernel(const GemmGroup grou
         uint32_t local = block;
         const GemmParams p = select_target(group, local);
         const uint32_t sharer = blockIdx.x - block * T / U;  // number among the workgroups that share the block
-        // The two common cases - 16-byte pieces of partial sums, 8-byte pieces of fp16 outputs that
-        // need nothing done to them - as straight code; everything else one fragment after the other
+        // The two common cases - 16-byte pieces of partial sums, fp16 outputs that need nothing done
+        // to them - as straight code; everything else one fragment after the other
         // through one copy of it (straight code for every fragment was 2700 to 10600 lines of
         // assembly, more than the instruction cache holds; one copy for the common cases too made
         // the 27B down projection at 67 rows 40 instead of 33 us).
-        const bool plain = p.wide_stores && !p.pair && p.row_scale == nullptr && p.residual == nullptr && p.y_dtype == MI355Q_F16;
-        if (p.wide_stores && (partial || plain)) {
-            float *const sums = p.partials + (size_t)sharer * M * p.N;
+        const bool plain = !p.pair && p.row_scale == nullptr && p.residual == nullptr && p.y_dtype == MI355Q_F16;
+        if (partial || plain) {
+            const uint32_t columns = padded_columns(p.N);
+            float *const sums = p.partials + (size_t)sharer * M * columns;
 #pragma unroll
             for (int t = 0; t < NTW; ++t) {
                 const uint32_t n = (local * TPB + wave * NTW + t) * kTileRows + 4u * kq;
@@ -205,7 +206,11 @@ __global__ void __launch_bounds__(64 * W, 2) q4_rows_kernel(const GemmGroup grou
                     if (m >= M || n >= p.N) continue;
                     const size_t at = (size_t)m * p.N + n;
                     if (partial) {
-                        *(floatx4 *)(sums + at) = acc[t][f];
+                        *(floatx4 *)(sums + (size_t)m * columns + n) = acc[t][f];
+                    } else if (!p.wide_stores) {
+#pragma unroll
+                        for (uint32_t j = 0; j < 4u; ++j)
+                            if (n + j < p.N) ((_Float16 *)p.y)[at + j] = (_Float16)acc[t][f][j];
                     } else {
                         typedef _Float16 half4v __attribute__((ext_vector_type(4)));
                         const floatx4 v = acc[t][f];
@@ -224,13 +229,13 @@ __global__ void __launch_bounds__(64 * W, 2) q4_rows_kernel(const GemmGroup grou
             const uint32_t n = (local * TPB + wave * NTW + e / MF) * kTileRows + 4u * kq;
             uint32_t m = 16u * (e % MF) + r;
             bool stored = m < M && n < p.N;
-            if (p.pair && !partial) {  // rows 2m and 2m + 1 are adjacent lanes
+            if (p.pair) {  // rows 2m and 2m + 1 are adjacent lanes
 #pragma unroll
                 for (int j = 0; j < 4; ++j) values[j] += __shfl_xor(values[j], 1, 64);
                 stored = stored && (m & 1u) == 0u;
                 m >>= 1;
             }
-            if (stored) finish_four(p, partial, sharer, m, n, values);
+            if (stored) finish_four(p, false, 0, m, n, values);
         }
         // the stores are in the same queue as the fetches under way: with both gone the counts
         // above are fetches again (a builtin, so that the compiler, too, knows that its own loads
