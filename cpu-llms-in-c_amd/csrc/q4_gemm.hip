@@ -60,17 +60,21 @@ extern template __global__ void q4_gemm_pipe_kernel<128, 3, true, false, true>(c
 // A workgroup takes 256 (1024) adjacent columns of one output row: no index is ever divided (a
 // division per thread cost the 27B prefill step's reductions about a microsecond each).
 constexpr uint32_t kReduceThreads = 256;
-// SPLITS: their number when the host knows it and it is small - the loads of all of them are then
+// SPLITS: their number when the host knows it and it is at most eight - the call is then one target's, whose
+// parameters alone are a smaller launch, and the loads of all of them are then
 // on their way before the first is added (the 27B q projection at 512 rows with its four: 50.0 us,
-// with a test of the count in front of every load 50.9); 0: a loop, and the workgroups that share a
+// with a test of the count in front of every load 50.9); 0: a loop over a call's targets, and the workgroups that share a
 // column's block of q4_rows_kernel counted here.
 template <bool WIDE, int SPLITS>
-__global__ void __launch_bounds__(kReduceThreads) q4_gemm_reduce_kernel(const GemmGroup group)
+__global__ void __launch_bounds__(kReduceThreads)
+q4_gemm_reduce_kernel(const std::conditional_t<(SPLITS > 0), GemmParams, GemmGroup> of)
 {
     constexpr int PER = WIDE ? 4 : 1;
     typedef std::conditional_t<WIDE, floatx4, float> Piece;
     uint32_t block = blockIdx.x;
-    const GemmParams p = SPLITS ? only_target(group) : select_target<true>(group, block);
+    GemmParams p;
+    if constexpr (SPLITS > 0) p = of;
+    else p = select_target<true>(of, block);
     const uint32_t n = (block * kReduceThreads + threadIdx.x) * PER;
     if (n >= p.N) return;
     const uint32_t columns = p.units ? padded_columns(p.N) : p.N;  // of a row of partial sums
@@ -191,16 +195,23 @@ static hipError_t launch_reduce(mi355q_context *ctx, GemmGroup &group)
     }
     const uint32_t rows = group.shared.pair ? group.shared.M / 2u : group.shared.M;
     const dim3 grid(blocks, rows < 65535u ? rows : 65535u);
-    if (!wide) return launch(ctx, q4_gemm_reduce_kernel<false, 0>, grid, dim3(kReduceThreads), 0, group);
-    switch (group.targets == 1u && group.shared.units == 0u ? group.shared.splits : 0u) {
-    case 2: return launch(ctx, q4_gemm_reduce_kernel<true, 2>, grid, dim3(kReduceThreads), 0, group);
-    case 3: return launch(ctx, q4_gemm_reduce_kernel<true, 3>, grid, dim3(kReduceThreads), 0, group);
-    case 4: return launch(ctx, q4_gemm_reduce_kernel<true, 4>, grid, dim3(kReduceThreads), 0, group);
-    case 5: return launch(ctx, q4_gemm_reduce_kernel<true, 5>, grid, dim3(kReduceThreads), 0, group);
-    case 6: return launch(ctx, q4_gemm_reduce_kernel<true, 6>, grid, dim3(kReduceThreads), 0, group);
-    case 7: return launch(ctx, q4_gemm_reduce_kernel<true, 7>, grid, dim3(kReduceThreads), 0, group);
-    case 8: return launch(ctx, q4_gemm_reduce_kernel<true, 8>, grid, dim3(kReduceThreads), 0, group);
-    default: return launch(ctx, q4_gemm_reduce_kernel<true, 0>, grid, dim3(kReduceThreads), 0, group);
+    if (group.targets != 1u || group.shared.units != 0u || group.shared.splits > 8u)  // (more than eight: only when forced)
+        return wide ? launch(ctx, q4_gemm_reduce_kernel<true, 0>, grid, dim3(kReduceThreads), 0, group)
+                    : launch(ctx, q4_gemm_reduce_kernel<false, 0>, grid, dim3(kReduceThreads), 0, group);
+    // one target of a K split: the whole of it is in the shared parameters
+    auto one = [&](auto splits) {
+        constexpr int SPLITS = decltype(splits)::value;
+        return wide ? launch(ctx, q4_gemm_reduce_kernel<true, SPLITS>, grid, dim3(kReduceThreads), 0, group.shared)
+                    : launch(ctx, q4_gemm_reduce_kernel<false, SPLITS>, grid, dim3(kReduceThreads), 0, group.shared);
+    };
+    switch (group.shared.splits) {
+    case 2: return one(std::integral_constant<int, 2>());
+    case 3: return one(std::integral_constant<int, 3>());
+    case 4: return one(std::integral_constant<int, 4>());
+    case 5: return one(std::integral_constant<int, 5>());
+    case 6: return one(std::integral_constant<int, 6>());
+    case 7: return one(std::integral_constant<int, 7>());
+    default: return one(std::integral_constant<int, 8>());
     }
 }
 

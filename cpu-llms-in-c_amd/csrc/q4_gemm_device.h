@@ -72,7 +72,6 @@ __device__ __forceinline__ GemmParams target_params(const GemmGroup &group, cons
     p.first_block = target.first_block;
     return p;
 }
-__device__ __forceinline__ GemmParams only_target(const GemmGroup &group) { return target_params(group, group.target[0]); }
 // Those of the target that workgroup `block` works on; `block` becomes its number there.
 template <bool REDUCE = false>
 __device__ __forceinline__ GemmParams select_target(const GemmGroup &group, uint32_t &block)
@@ -117,10 +116,12 @@ __device__ __forceinline__ void static_for(F &&f)
 // Output of one accumulator fragment: lane (r, kq) holds rows row0 + 4*kq + j (j = 0..3) of
 // column n.  MODE 0..2: plain store as fp16 / fp32 / bf16 (no residual, no K split: the common
 // case, with nothing to decide per element); MODE 4: converted activations without a K split;
-// MODE 3: everything else.
+// MODE 3: everything else.  MODE 4 is given its rows' scales and the column's bias (a load of each
+// in front of every store was a chain of memory round trips: 4.4 us of 202 rows x 5219 columns).
 template <int MODE>
 __device__ __forceinline__ void store_fragment(const GemmParams &p, uint32_t split, uint32_t row0,
-                                               uint32_t kq, uint32_t n, const floatx4 &values)
+                                               uint32_t kq, uint32_t n, const floatx4 &values,
+                                               const float (&scale)[4], float bias)
 {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -131,9 +132,9 @@ __device__ __forceinline__ void store_fragment(const GemmParams &p, uint32_t spl
             const float sum = p.pair ? values[j] + values[(j + 1) & 3] : values[j];
             const uint32_t row = p.pair ? m >> 1 : m;
             const size_t at = (size_t)row * p.N + n;
-            float value = sum * p.row_scale[row];
+            float value = sum * scale[j];
             if (p.residual)
-                value += load_as_float(p.residual, p.residual_dtype, p.residual_is_bias ? n : at);
+                value += p.residual_is_bias ? bias : load_as_float(p.residual, p.residual_dtype, at);
             store_from_float(p.y, p.y_dtype, at, value);
             continue;
         }
@@ -364,15 +365,28 @@ __global__ void __launch_bounds__(256, 2) q4_gemm_kernel(const GemmParams p)
 
     // ---- lane (r, kq) holds rows 16*i + 4*kq + j of column tile*16 + r
     auto store_all = [&](auto mode) {
+        float scale[MI][4] = {};
+        if constexpr (decltype(mode)::value == 4) {
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (uint32_t j = 0; j < 4u; ++j) {
+                    const uint32_t m = m0 + 16u * i + 4u * kq + j;
+                    scale[i][j] = p.row_scale[(m < p.M ? m : p.M - 1u) >> (p.pair ? 1 : 0)];
+                }
+        }
 #pragma unroll
         for (int t = 0; t < NTX; ++t) {
             if (t == NTW && !has_extra) continue;
             const uint32_t tile = tile0 + t;
             const uint32_t n = tile * kTileRows + r;
             if (tile >= p.NT || n >= p.N) continue;
+            float bias = 0.0f;
+            if (decltype(mode)::value == 4 && p.residual && p.residual_is_bias)
+                bias = load_as_float(p.residual, p.residual_dtype, n);
 #pragma unroll
             for (int i = 0; i < MI; ++i)
-                store_fragment<decltype(mode)::value>(p, split, m0 + 16u * i, kq, n, acc[i][t]);
+                store_fragment<decltype(mode)::value>(p, split, m0 + 16u * i, kq, n, acc[i][t], scale[i], bias);
         }
     };
     switch (store_mode(p)) {
