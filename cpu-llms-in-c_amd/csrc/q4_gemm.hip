@@ -134,6 +134,13 @@ q4_gemm_reduce_kernel(const std::conditional_t<(SPLITS > 0), GemmParams, GemmGro
     }
 }
 
+template <int BM, int NTW, bool EXTRA>
+static hipError_t launch_gemm(mi355q_context *ctx, dim3 grid, const GemmParams &p)
+{
+    return p.row_scale ? launch(ctx, q4_gemm_kernel<BM, NTW, EXTRA, true>, grid, dim3(256), 0, p)
+                       : launch(ctx, q4_gemm_kernel<BM, NTW, EXTRA, false>, grid, dim3(256), 0, p);
+}
+
 // The pipelined kernel's stage is larger than the 64 KiB a kernel gets without asking: the
 // limit is raised once per device and instantiation.
 template <int NTW, bool XT>
@@ -423,12 +430,12 @@ static int gemm_one_target(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t 
     const dim3 grid(n_blocks, m_blocks, p.splits);
     hipError_t launched = hipErrorInvalidValue;
     switch (best) {
-    case 0: launched = launch(ctx, q4_gemm_kernel<128, 4, false>, grid, dim3(256), 0, p); break;
-    case 1: launched = launch(ctx, q4_gemm_kernel<128, 2, false>, grid, dim3(256), 0, p); break;
-    case 2: launched = launch(ctx, q4_gemm_kernel<64, 4, false>, grid, dim3(256), 0, p); break;
-    case 3: launched = launch(ctx, q4_gemm_kernel<64, 4, true>, grid, dim3(256), 0, p); break;
-    case 4: launched = launch(ctx, q4_gemm_kernel<64, 2, false>, grid, dim3(256), 0, p); break;
-    case 5: launched = launch(ctx, q4_gemm_kernel<64, 2, true>, grid, dim3(256), 0, p); break;
+    case 0: launched = launch_gemm<128, 4, false>(ctx, grid, p); break;
+    case 1: launched = launch_gemm<128, 2, false>(ctx, grid, p); break;
+    case 2: launched = launch_gemm<64, 4, false>(ctx, grid, p); break;
+    case 3: launched = launch_gemm<64, 4, true>(ctx, grid, p); break;
+    case 4: launched = launch_gemm<64, 2, false>(ctx, grid, p); break;
+    case 5: launched = launch_gemm<64, 2, true>(ctx, grid, p); break;
     case 6: launched = launch_pipe<4, false>(ctx, grid, p); break;
     case 7: launched = ctx->gemm_plain_loads ? launch_pipe_plain(ctx, grid, p) : launch_pipe<4, true>(ctx, grid, p); break;
     case 8: launched = launch_pipe<5, false>(ctx, grid, p); break;

@@ -116,8 +116,9 @@ __device__ __forceinline__ void static_for(F &&f)
 // Output of one accumulator fragment: lane (r, kq) holds rows row0 + 4*kq + j (j = 0..3) of
 // column n.  MODE 0..2: plain store as fp16 / fp32 / bf16 (no residual, no K split: the common
 // case, with nothing to decide per element); MODE 4: converted activations without a K split;
-// MODE 3: everything else.  MODE 4 is given its rows' scales and the column's bias (a load of each
-// in front of every store was a chain of memory round trips: 4.4 us of 202 rows x 5219 columns).
+// MODE 5: partial sums of converted activations; MODE 3: everything else.  MODE 4 is given its rows'
+// scales and the column's bias (a load of each in front of every store was a chain of memory round
+// trips: 4.4 us of 202 rows x 5219 columns).
 template <int MODE>
 __device__ __forceinline__ void store_fragment(const GemmParams &p, uint32_t split, uint32_t row0,
                                                uint32_t kq, uint32_t n, const floatx4 &values,
@@ -139,7 +140,9 @@ __device__ __forceinline__ void store_fragment(const GemmParams &p, uint32_t spl
             continue;
         }
         const size_t at = (size_t)m * p.N + n;
-        if (MODE == 0) {
+        if (MODE == 5) {
+            p.partials[(size_t)split * p.M * p.N + at] = values[j];
+        } else if (MODE == 0) {
             ((_Float16 *)p.y)[at] = (_Float16)values[j];
         } else if (MODE == 1) {
             ((float *)p.y)[at] = values[j];
@@ -203,15 +206,16 @@ __device__ __forceinline__ void finish_four(const GemmParams &p, bool partial, u
 
 __device__ __forceinline__ int store_mode(const GemmParams &p)
 {
-    if (p.splits > 1u) return 3;
-    if (p.row_scale != nullptr) return 4;
-    if (p.residual != nullptr) return 3;
+    if (p.splits > 1u || p.residual != nullptr) return 3;
     return p.y_dtype == MI355Q_F16 ? 0 : p.y_dtype == MI355Q_F32 ? 1 : 2;
 }
 
 // BM rows of x per workgroup; every wave owns NTW tiles of 16 weight rows and, when EXTRA,
-// the last wave owns one more (tiles per block = 4*NTW + EXTRA).
-template <int BM, int NTW, bool EXTRA>
+// the last wave owns one more (tiles per block = 4*NTW + EXTRA).  CONVERTED (x was not fp16) is a
+// kernel of its own: its epilogue in the same one made that of fp16 activations slower (fp32 out,
+// 2048 x 2048 at 160 rows 14.1 -> 15.4 us, 8192 x 3200 at 512 rows 40.3 -> 41.5): 62 instead of 39 KB
+// of code, and waits in front of plain stores for loads of the other epilogue.
+template <int BM, int NTW, bool EXTRA, bool CONVERTED>
 __global__ void __launch_bounds__(256, 2) q4_gemm_kernel(const GemmParams p)
 {
     // Activation stage: [buffer][row][slot] of 16-byte pieces, slot = octet ^ (row % 16).
@@ -389,11 +393,15 @@ __global__ void __launch_bounds__(256, 2) q4_gemm_kernel(const GemmParams p)
                 store_fragment<decltype(mode)::value>(p, split, m0 + 16u * i, kq, n, acc[i][t], scale[i], bias);
         }
     };
+    if constexpr (CONVERTED) {
+        if (p.splits > 1u) store_all(std::integral_constant<int, 5>());
+        else store_all(std::integral_constant<int, 4>());
+        return;
+    }
     switch (store_mode(p)) {
     case 0: store_all(std::integral_constant<int, 0>()); break;
     case 1: store_all(std::integral_constant<int, 1>()); break;
     case 2: store_all(std::integral_constant<int, 2>()); break;
-    case 4: store_all(std::integral_constant<int, 4>()); break;
     default: store_all(std::integral_constant<int, 3>()); break;
     }
 }

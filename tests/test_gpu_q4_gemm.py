@@ -392,3 +392,12 @@ def test_targets_that_depend_on_each_other(engine, gpu, M):
             gpu.free(pointer)
         for weight in weights:
             weight.destroy()
+
+
+@pytest.mark.parametrize("forced", ["0,1", "0,2", "1,2", "3,1", "3,2", "5,2"])
+@pytest.mark.parametrize("x_dtype,y_dtype,N", [("F32", "F32", 1101), ("BF16", "F16", 1104)])
+def test_converted_activations_in_every_shape(engine, oracle, gpu, force, forced, x_dtype, y_dtype, N):
+    """The first GEMM kernel's form for converted activations, in the shapes the test above leaves
+    out: its own epilogue and partial sums, a last block of rows partly filled."""
+    force("q4_gemm", forced)
+    run_case(engine, oracle, gpu, N, 256, 75, engine.META_BF16_PLANES, getattr(engine, x_dtype), getattr(engine, y_dtype))
