@@ -60,31 +60,14 @@ extern template __global__ void q4_gemm_pipe_kernel<128, 3, true, false, true>(c
 // A workgroup takes 256 (1024) adjacent columns of one output row: no index is ever divided (a
 // division per thread cost the 27B prefill step's reductions about a microsecond each).
 constexpr uint32_t kReduceThreads = 256;
-// SPLITS: their number when the host knows it and it is at most eight - the call is then one target's, whose
-// parameters alone are a smaller launch, and the loads of all of them are then
-// on their way before the first is added (the 27B q projection at 512 rows with its four: 50.0 us,
-// with a test of the count in front of every load 50.9); 0: a loop over a call's targets, and the workgroups that share a
-// column's block of q4_rows_kernel counted here.
+constexpr uint32_t kReduceRows = 65535;  // of the grid's y; its z counts on
+
+// Columns n (.. n + 3) of output row m from `splits` partial sums (SPLITS of them when that is not 0).
 template <bool WIDE, int SPLITS>
-__global__ void __launch_bounds__(kReduceThreads)
-q4_gemm_reduce_kernel(const std::conditional_t<(SPLITS > 0), GemmParams, GemmGroup> of)
+__device__ __forceinline__ void reduce_columns(const GemmParams &p, uint32_t columns, uint32_t splits, uint32_t m, uint32_t n)
 {
-    constexpr int PER = WIDE ? 4 : 1;
     typedef std::conditional_t<WIDE, floatx4, float> Piece;
-    uint32_t block = blockIdx.x;
-    GemmParams p;
-    if constexpr (SPLITS > 0) p = of;
-    else p = select_target<true>(of, block);
-    const uint32_t n = (block * kReduceThreads + threadIdx.x) * PER;
-    if (n >= p.N) return;
-    const uint32_t columns = p.units ? padded_columns(p.N) : p.N;  // of a row of partial sums
     const size_t stride = (size_t)p.M * columns;
-    uint32_t splits = p.splits;
-    if (!SPLITS && p.units) {  // one workgroup alone has stored the outputs
-        const uint32_t begin = (p.first_block + n / p.block_columns) * p.T;
-        splits = (begin + p.T - 1u) / p.units - begin / p.units + 1u;
-        if (splits == 1u) return;
-    }
     auto add = [](Piece &sum, const Piece &more) {
         if constexpr (WIDE) {
 #pragma unroll
@@ -114,24 +97,80 @@ q4_gemm_reduce_kernel(const std::conditional_t<(SPLITS > 0), GemmParams, GemmGro
         }
         return sum;
     };
-    const uint32_t rows = p.pair ? p.M / 2u : p.M;
-    for (uint32_t m = blockIdx.y; m < rows; m += gridDim.y) {
-        Piece value;
-        if (p.pair) {
-            value = add_splits((size_t)(2u * m) * columns + n);
-            add(value, add_splits((size_t)(2u * m + 1u) * columns + n));
-        } else {
-            value = add_splits((size_t)m * columns + n);
-        }
-        if constexpr (WIDE) {
-            finish_four(p, false, 0, m, n, value);
-        } else {
-            const size_t at = (size_t)m * p.N + n;
-            if (p.row_scale) value *= p.row_scale[m];
-            if (p.residual) value += load_as_float(p.residual, p.residual_dtype, p.residual_is_bias ? n : at);
-            store_from_float(p.y, p.y_dtype, at, value);
-        }
+    Piece value;
+    if (p.pair) {
+        value = add_splits((size_t)(2u * m) * columns + n);
+        add(value, add_splits((size_t)(2u * m + 1u) * columns + n));
+    } else {
+        value = add_splits((size_t)m * columns + n);
     }
+    if constexpr (WIDE) {
+        finish_four(p, false, 0, m, n, value);
+    } else {
+        const size_t at = (size_t)m * p.N + n;
+        if (p.row_scale) value *= p.row_scale[m];
+        if (p.residual) value += load_as_float(p.residual, p.residual_dtype, p.residual_is_bias ? n : at);
+        store_from_float(p.y, p.y_dtype, at, value);
+    }
+}
+
+// One target of a K split into at most eight: the number of splits is the host's, and all their
+// loads are on their way before the first is added.  Launched behind every K split, a few
+// microseconds of which the arguments' way is a good part: they are one cache line, read at once
+// (ReduceParams), and fp16 activations (CONVERTED false) have no code for pairs and row scales.
+// With the GEMM's own parameters and a loop over gridDim.y the arguments came in three round
+// trips, one after the other (GEMM and sum, us: 5216 x 2752 at 96 rows 15.0 -> 14.3, 8192 x 3200 at
+// 67 rows 18.0 -> 17.5, 6144 x 5120 at 200 rows 28.6 -> 28.0; the sum alone of 10000 columns at 200
+// rows 5.2 -> 4.6, of 5120 at 512 rows from five 11.3 -> 10.5).
+struct ReduceParams {
+    const float *partials;
+    void *y;
+    const void *residual;
+    const float *row_scale;
+    uint32_t M, N;
+    uint8_t y_dtype, residual_dtype, residual_is_bias, pair;
+};
+static_assert(sizeof(ReduceParams) <= 64, "one cache line of arguments");
+template <bool WIDE, int SPLITS, bool CONVERTED>
+__global__ void __launch_bounds__(kReduceThreads) q4_gemm_reduce_kernel(const ReduceParams of)
+{
+    GemmParams p = {};
+    p.partials = const_cast<float *>(of.partials);
+    p.y = of.y;
+    p.residual = of.residual;
+    p.M = of.M;
+    p.N = of.N;
+    p.y_dtype = of.y_dtype;
+    p.residual_dtype = of.residual_dtype;
+    p.residual_is_bias = of.residual_is_bias;
+    p.wide_stores = WIDE;
+    if constexpr (CONVERTED) {
+        p.row_scale = of.row_scale;
+        p.pair = of.pair;
+    }
+    const uint32_t n = (blockIdx.x * kReduceThreads + threadIdx.x) * (WIDE ? 4u : 1u);
+    const uint32_t m = blockIdx.z * kReduceRows + blockIdx.y;
+    if (n >= p.N || m >= (p.pair ? p.M / 2u : p.M)) return;
+    reduce_columns<WIDE, SPLITS>(p, p.N, SPLITS, m, n);
+}
+
+// Every other sum: a loop over the splits, a call's targets, and the workgroups that share a
+// column's block of q4_rows_kernel counted here.
+template <bool WIDE>
+__global__ void __launch_bounds__(kReduceThreads) q4_group_reduce_kernel(const GemmGroup group)
+{
+    uint32_t block = blockIdx.x;
+    const GemmParams p = select_target<true>(group, block);
+    const uint32_t n = (block * kReduceThreads + threadIdx.x) * (WIDE ? 4u : 1u);
+    const uint32_t m = blockIdx.z * kReduceRows + blockIdx.y;
+    if (n >= p.N || m >= (p.pair ? p.M / 2u : p.M)) return;
+    uint32_t splits = p.splits;
+    if (p.units) {  // one workgroup alone has stored the outputs
+        const uint32_t begin = (p.first_block + n / p.block_columns) * p.T;
+        splits = (begin + p.T - 1u) / p.units - begin / p.units + 1u;
+        if (splits == 1u) return;
+    }
+    reduce_columns<WIDE, 0>(p, p.units ? padded_columns(p.N) : p.N, splits, m, n);
 }
 
 template <int BM, int NTW, bool EXTRA>
@@ -200,25 +239,31 @@ static hipError_t launch_reduce(mi355q_context *ctx, GemmGroup &group)
         group.target[t].first_reduce = blocks;
         blocks += (group.target[t].N + columns - 1u) / columns;
     }
-    const uint32_t rows = group.shared.pair ? group.shared.M / 2u : group.shared.M;
-    const dim3 grid(blocks, rows < 65535u ? rows : 65535u);
-    if (group.targets != 1u || group.shared.units != 0u || group.shared.splits > 8u)  // (more than eight: only when forced)
-        return wide ? launch(ctx, q4_gemm_reduce_kernel<true, 0>, grid, dim3(kReduceThreads), 0, group)
-                    : launch(ctx, q4_gemm_reduce_kernel<false, 0>, grid, dim3(kReduceThreads), 0, group);
-    // one target of a K split: the whole of it is in the shared parameters
-    auto one = [&](auto splits) {
+    const GemmParams &p = group.shared;
+    const uint32_t rows = p.pair ? p.M / 2u : p.M;
+    const dim3 grid(blocks, std::min(rows, kReduceRows), (rows + kReduceRows - 1u) / kReduceRows);
+    if (group.targets != 1u || p.units != 0u || p.splits > 8u)  // (more than eight: only when forced)
+        return wide ? launch(ctx, q4_group_reduce_kernel<true>, grid, dim3(kReduceThreads), 0, group)
+                    : launch(ctx, q4_group_reduce_kernel<false>, grid, dim3(kReduceThreads), 0, group);
+    const GemmTarget &target = group.target[0];
+    const ReduceParams one = {target.partials, target.y, target.residual, p.row_scale, p.M, target.N, (uint8_t)p.y_dtype,
+                              (uint8_t)p.residual_dtype, (uint8_t)(p.residual_is_bias != 0), (uint8_t)(p.pair != 0)};
+    auto of = [&](auto splits) {
         constexpr int SPLITS = decltype(splits)::value;
-        return wide ? launch(ctx, q4_gemm_reduce_kernel<true, SPLITS>, grid, dim3(kReduceThreads), 0, group.shared)
-                    : launch(ctx, q4_gemm_reduce_kernel<false, SPLITS>, grid, dim3(kReduceThreads), 0, group.shared);
+        if (p.row_scale)
+            return wide ? launch(ctx, q4_gemm_reduce_kernel<true, SPLITS, true>, grid, dim3(kReduceThreads), 0, one)
+                        : launch(ctx, q4_gemm_reduce_kernel<false, SPLITS, true>, grid, dim3(kReduceThreads), 0, one);
+        return wide ? launch(ctx, q4_gemm_reduce_kernel<true, SPLITS, false>, grid, dim3(kReduceThreads), 0, one)
+                    : launch(ctx, q4_gemm_reduce_kernel<false, SPLITS, false>, grid, dim3(kReduceThreads), 0, one);
     };
-    switch (group.shared.splits) {
-    case 2: return one(std::integral_constant<int, 2>());
-    case 3: return one(std::integral_constant<int, 3>());
-    case 4: return one(std::integral_constant<int, 4>());
-    case 5: return one(std::integral_constant<int, 5>());
-    case 6: return one(std::integral_constant<int, 6>());
-    case 7: return one(std::integral_constant<int, 7>());
-    default: return one(std::integral_constant<int, 8>());
+    switch (p.splits) {
+    case 2: return of(std::integral_constant<int, 2>());
+    case 3: return of(std::integral_constant<int, 3>());
+    case 4: return of(std::integral_constant<int, 4>());
+    case 5: return of(std::integral_constant<int, 5>());
+    case 6: return of(std::integral_constant<int, 6>());
+    case 7: return of(std::integral_constant<int, 7>());
+    default: return of(std::integral_constant<int, 8>());
     }
 }
 

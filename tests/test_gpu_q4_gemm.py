@@ -401,3 +401,20 @@ def test_converted_activations_in_every_shape(engine, oracle, gpu, force, forced
     out: its own epilogue and partial sums, a last block of rows partly filled."""
     force("q4_gemm", forced)
     run_case(engine, oracle, gpu, N, 256, 75, engine.META_BF16_PLANES, getattr(engine, x_dtype), getattr(engine, y_dtype))
+
+
+@pytest.mark.parametrize("splits", [2, 3, 4, 5, 6, 7, 8, 9])
+@pytest.mark.parametrize("N,x_dtype,y_dtype", [(1104, "F16", "F16"), (1101, "F16", "F32"), (1104, "F32", "F32"), (1101, "BF16", "F16")])
+def test_k_split_sums(engine, oracle, gpu, force, splits, N, x_dtype, y_dtype):
+    """The kernel behind a K split: every number of splits it is compiled for and one that it counts
+    itself, four columns a thread and one, with and without rows that were converted."""
+    force("q4_gemm", f"4,{splits}")
+    run_case(engine, oracle, gpu, N, 1152, 75, engine.META_BF16_PLANES, getattr(engine, x_dtype), getattr(engine, y_dtype),
+             residual=splits % 2 == 0)
+
+
+@pytest.mark.parametrize("splits", [2, 9])
+def test_k_split_sums_of_many_rows(engine, oracle, gpu, force, splits):
+    """More rows than a grid's second dimension holds (65535)."""
+    force("q4_gemm", f"0,{splits}")
+    run_case(engine, oracle, gpu, 20, 1152, 65600, engine.META_BF16_PLANES, engine.F16, engine.F32)
