@@ -64,9 +64,10 @@ constexpr uint32_t kReduceRows = 65535;  // of the grid's y; its z counts on
 
 // Columns n (.. n + 3) of output row m from `splits` partial sums (SPLITS of them when that is not 0).
 template <bool WIDE, int SPLITS>
-__device__ __forceinline__ void reduce_columns(const GemmParams &p, uint32_t columns, uint32_t splits, uint32_t m, uint32_t n)
+__device__ __forceinline__ void reduce_columns(const GemmParams &p, uint32_t splits, uint32_t m, uint32_t n)
 {
     typedef std::conditional_t<WIDE, floatx4, float> Piece;
+    const uint32_t columns = padded_columns(p.N);
     const size_t stride = (size_t)p.M * columns;
     auto add = [](Piece &sum, const Piece &more) {
         if constexpr (WIDE) {
@@ -105,7 +106,7 @@ __device__ __forceinline__ void reduce_columns(const GemmParams &p, uint32_t col
         value = add_splits((size_t)m * columns + n);
     }
     if constexpr (WIDE) {
-        finish_four(p, false, 0, m, n, value);
+        finish_four(p, m, n, value);
     } else {
         const size_t at = (size_t)m * p.N + n;
         if (p.row_scale) value *= p.row_scale[m];
@@ -151,7 +152,7 @@ __global__ void __launch_bounds__(kReduceThreads) q4_gemm_reduce_kernel(const Re
     const uint32_t n = (blockIdx.x * kReduceThreads + threadIdx.x) * (WIDE ? 4u : 1u);
     const uint32_t m = blockIdx.z * kReduceRows + blockIdx.y;
     if (n >= p.N || m >= (p.pair ? p.M / 2u : p.M)) return;
-    reduce_columns<WIDE, SPLITS>(p, p.N, SPLITS, m, n);
+    reduce_columns<WIDE, SPLITS>(p, SPLITS, m, n);
 }
 
 // Every other sum: a loop over the splits, a call's targets, and the workgroups that share a
@@ -170,7 +171,7 @@ __global__ void __launch_bounds__(kReduceThreads) q4_group_reduce_kernel(const G
         splits = (begin + p.T - 1u) / p.units - begin / p.units + 1u;
         if (splits == 1u) return;
     }
-    reduce_columns<WIDE, 0>(p, p.units ? padded_columns(p.N) : p.N, splits, m, n);
+    reduce_columns<WIDE, 0>(p, splits, m, n);
 }
 
 template <int BM, int NTW, bool EXTRA>
@@ -458,7 +459,7 @@ static int gemm_one_target(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t 
     p.steps_per_split = (T + best_splits - 1) / best_splits;
     p.splits = (T + p.steps_per_split - 1) / p.steps_per_split;
     if (p.splits > 1u) {
-        const size_t bytes = (size_t)p.splits * rows * w.N * sizeof(float);
+        const size_t bytes = (size_t)p.splits * rows * padded_columns(w.N) * sizeof(float);
         status = ensure_stage(ctx, 4, bytes, error, error_capacity);
         if (status != MI355Q_OK) return status;
         p.partials = (float *)ctx->stage[4];

@@ -21,7 +21,7 @@ struct GemmParams {
     uint32_t wrap_steps;
     void *y;
     const void *residual;
-    float *partials;    // [splits][M][N] when splits > 1
+    float *partials;    // [splits, or workgroups that share a block][M][padded_columns(N)] when there is more than one
     uint32_t M, N, K, NT, T;
     uint32_t tiles_per_block;
     uint32_t splits, steps_per_split;
@@ -113,12 +113,15 @@ __device__ __forceinline__ void static_for(F &&f)
     static_for_impl(std::make_integer_sequence<int, N>(), f);
 }
 
+// Columns of a row of partial sums: padded, so that they are 16-byte pieces for every N.
+__host__ __device__ __forceinline__ uint32_t padded_columns(uint32_t N) { return (N + 3u) / 4u * 4u; }
+
 // Output of one accumulator fragment: lane (r, kq) holds rows row0 + 4*kq + j (j = 0..3) of
 // column n.  MODE 0..2: plain store as fp16 / fp32 / bf16 (no residual, no K split: the common
 // case, with nothing to decide per element); MODE 4: converted activations without a K split;
-// MODE 5: partial sums of converted activations; MODE 3: everything else.  MODE 4 is given its rows'
-// scales and the column's bias (a load of each in front of every store was a chain of memory round
-// trips: 4.4 us of 202 rows x 5219 columns).
+// MODE 5: a K split's partial sums; MODE 3: everything else.  MODE 4 is given its rows' scales and the
+// column's bias (a load of each in front of every store was a chain of memory round trips: 4.4 us of
+// 202 rows x 5219 columns).
 template <int MODE>
 __device__ __forceinline__ void store_fragment(const GemmParams &p, uint32_t split, uint32_t row0,
                                                uint32_t kq, uint32_t n, const floatx4 &values,
@@ -141,15 +144,13 @@ __device__ __forceinline__ void store_fragment(const GemmParams &p, uint32_t spl
         }
         const size_t at = (size_t)m * p.N + n;
         if (MODE == 5) {
-            p.partials[(size_t)split * p.M * p.N + at] = values[j];
+            p.partials[((size_t)split * p.M + m) * padded_columns(p.N) + n] = values[j];
         } else if (MODE == 0) {
             ((_Float16 *)p.y)[at] = (_Float16)values[j];
         } else if (MODE == 1) {
             ((float *)p.y)[at] = values[j];
         } else if (MODE == 2) {
             store_from_float(p.y, MI355Q_BF16, at, values[j]);
-        } else if (p.splits > 1u) {
-            p.partials[(size_t)split * p.M * p.N + at] = values[j];
         } else {
             float value = values[j];
             if (p.residual)
@@ -165,35 +166,27 @@ __device__ __forceinline__ uint32_t bf16_bits(float v)  // round to nearest even
     return (bits + 0x7fffu + ((bits >> 16) & 1u)) >> 16;
 }
 
-// Columns of a row of q4_rows_kernel's partial sums: padded, so that they are 16-byte pieces for
-// every N.
-__host__ __device__ __forceinline__ uint32_t padded_columns(uint32_t N) { return (N + 3u) / 4u * 4u; }
-
-// Four adjacent columns n .. n + 3 of output row m: row scale, residual, conversion, store; or, when
-// partial, of row m of a K split's partial sums.  Columns from N on are not stored.
-__device__ __forceinline__ void finish_four(const GemmParams &p, bool partial, uint32_t split, uint32_t m, uint32_t n,
-                                            floatx4 values)
+// Four adjacent columns n .. n + 3 of output row m: row scale, residual, conversion, store.  Columns
+// from N on are not stored.
+__device__ __forceinline__ void finish_four(const GemmParams &p, uint32_t m, uint32_t n, floatx4 values)
 {
     const size_t at = (size_t)m * p.N + n;
-    if (!partial) {
-        if (p.row_scale) {
-            const float scale = p.row_scale[m];
+    if (p.row_scale) {
+        const float scale = p.row_scale[m];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) values[j] *= scale;
-        }
-        if (p.residual) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (n + j < p.N) values[j] += load_as_float(p.residual, p.residual_dtype, p.residual_is_bias ? n + j : at + j);
-        }
+        for (int j = 0; j < 4; ++j) values[j] *= scale;
     }
-    float *const out32 = partial ? p.partials + (size_t)split * p.M * p.N : (float *)p.y;
+    if (p.residual) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (n + j < p.N) values[j] += load_as_float(p.residual, p.residual_dtype, p.residual_is_bias ? n + j : at + j);
+    }
     if (!p.wide_stores) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            if (n + j < p.N) store_from_float(out32, partial ? MI355Q_F32 : p.y_dtype, at + j, values[j]);
-    } else if (partial || p.y_dtype == MI355Q_F32) {
-        *(floatx4 *)(out32 + at) = values;
+            if (n + j < p.N) store_from_float(p.y, p.y_dtype, at + j, values[j]);
+    } else if (p.y_dtype == MI355Q_F32) {
+        *(floatx4 *)((float *)p.y + at) = values;
     } else if (p.y_dtype == MI355Q_F16) {
         typedef _Float16 half4v __attribute__((ext_vector_type(4)));
         const half4v packed = {(_Float16)values[0], (_Float16)values[1], (_Float16)values[2], (_Float16)values[3]};
@@ -204,9 +197,10 @@ __device__ __forceinline__ void finish_four(const GemmParams &p, bool partial, u
     }
 }
 
+// (no K split, fp16 activations)
 __device__ __forceinline__ int store_mode(const GemmParams &p)
 {
-    if (p.splits > 1u || p.residual != nullptr) return 3;
+    if (p.residual != nullptr) return 3;
     return p.y_dtype == MI355Q_F16 ? 0 : p.y_dtype == MI355Q_F32 ? 1 : 2;
 }
 
@@ -399,9 +393,12 @@ __global__ void __launch_bounds__(256, 2) q4_gemm_kernel(const GemmParams p)
                 store_fragment<decltype(mode)::value>(p, split, m0 + 16u * i, kq, n, acc[i][t], scale[i], bias);
         }
     };
+    if (p.splits > 1u) {
+        store_all(std::integral_constant<int, 5>());
+        return;
+    }
     if constexpr (CONVERTED) {
-        if (p.splits > 1u) store_all(std::integral_constant<int, 5>());
-        else store_all(std::integral_constant<int, 4>());
+        store_all(std::integral_constant<int, 4>());
         return;
     }
     switch (store_mode(p)) {
@@ -741,7 +738,7 @@ __global__ void __launch_bounds__(256, 1) q4_gemm_pipe_kernel(const GemmParams p
     auto touch_shared = [&]() { touch(a_shared[0], a_shared[1]); };
     auto multiply = [&](floatx4 &c, const half8 &a, const half2v (&b)[4]) {
         const half8 b8 = {b[0].x, b[0].y, b[1].x, b[1].y, b[2].x, b[2].y, b[3].x, b[3].y};
-        // weights first: the result comes out transposed (see store_columns)
+        // weights first: the result comes out transposed (see the epilogue)
         asm volatile("v_mfma_f32_16x16x32_f16 %0, %2, %1, %0" : "+a"(c) : "v"(a), "v"(b8));
     };
     // Dequantization of one quarter = NTX tiles x 4 pieces (two of a lane's eight weights each),
@@ -992,7 +989,7 @@ __global__ void __launch_bounds__(256, 1) q4_gemm_pipe_kernel(const GemmParams p
     constexpr uint32_t PITCH32 = WIDTH * 4u + 16u;
     static_assert(PITCH32 % 16u == 0u && (PITCH32 / 16u) % 2u == 1u, "rows start 16-byte aligned, an odd number of 16-byte units apart");
     static_assert((size_t)(BM / 2) * PITCH32 <= pipe_lds_bytes(BM), "half a block fits the activation stage");
-    const bool pairs = p.splits <= 1u && p.pair;  // (the kernel that adds K splits adds pairs itself)
+    const bool pairs = p.pair;  // (without a K split: the kernel that adds those adds pairs itself)
     const uint32_t rows_out = pairs ? BM / 4u : BM / 2u;
     constexpr uint32_t FOURS = WIDTH / 4u;  // groups of four columns per row
 #pragma unroll
@@ -1013,11 +1010,21 @@ __global__ void __launch_bounds__(256, 1) q4_gemm_pipe_kernel(const GemmParams p
             }
         }
         __syncthreads();
-        if (p.splits > 1u && p.wide_stores && whole) {  // whole blocks of partial sums: a plain copy
-            float *const out = p.partials + ((size_t)split * p.M + m0 + half * (BM / 2)) * p.N + n_first;
-            for (uint32_t piece = threadIdx.x; piece < BM / 2u * FOURS; piece += 256u) {
-                const uint32_t row = piece / FOURS, column = piece % FOURS * 4u;
-                *(floatx4 *)(out + (size_t)row * p.N + column) = *(const floatx4 *)(stage + row * PITCH32 + column * 4u);
+        if (p.splits > 1u) {  // partial sums: a plain copy
+            const uint32_t columns = padded_columns(p.N), first_row = m0 + half * (BM / 2);
+            float *const out = p.partials + ((size_t)split * p.M + first_row) * columns + n_first;
+            if (whole) {  // (two loops: with the test inside one, whole blocks took 0.5 to 0.7 us more)
+                for (uint32_t piece = threadIdx.x; piece < BM / 2u * FOURS; piece += 256u) {
+                    const uint32_t row = piece / FOURS, column = piece % FOURS * 4u;
+                    *(floatx4 *)(out + (size_t)row * columns + column) = *(const floatx4 *)(stage + row * PITCH32 + column * 4u);
+                }
+            } else {
+                for (uint32_t piece = threadIdx.x; piece < BM / 2u * FOURS; piece += 256u) {
+                    const uint32_t row = piece / FOURS, column = piece % FOURS * 4u;
+                    if (first_row + row < p.M && n_first + column < p.N)
+                        *(floatx4 *)(out + (size_t)row * columns + column) =
+                            *(const floatx4 *)(stage + row * PITCH32 + column * 4u);
+                }
             }
             continue;
         }
@@ -1032,7 +1039,7 @@ __global__ void __launch_bounds__(256, 1) q4_gemm_pipe_kernel(const GemmParams p
 #pragma unroll
                 for (int j = 0; j < 4; ++j) values[j] += remainder[j];
             }
-            finish_four(p, p.splits > 1u, split, (pairs ? m0 / 2u : m0) + half * rows_out + row, n, values);
+            finish_four(p, (pairs ? m0 / 2u : m0) + half * rows_out + row, n, values);
         }
     }
 }

@@ -235,7 +235,7 @@ __global__ void __launch_bounds__(64 * W, 2) q4_rows_kernel(const GemmGroup grou
                 stored = stored && (m & 1u) == 0u;
                 m >>= 1;
             }
-            if (stored) finish_four(p, false, 0, m, n, values);
+            if (stored) finish_four(p, m, n, values);
         }
         // the stores are in the same queue as the fetches under way: with both gone the counts
         // above are fetches again (a builtin, so that the compiler, too, knows that its own loads

@@ -418,3 +418,13 @@ def test_k_split_sums_of_many_rows(engine, oracle, gpu, force, splits):
     """More rows than a grid's second dimension holds (65535)."""
     force("q4_gemm", f"0,{splits}")
     run_case(engine, oracle, gpu, 20, 1152, 65600, engine.META_BF16_PLANES, engine.F16, engine.F32)
+
+
+@pytest.mark.parametrize("forced", ["6,2", "7,3", "8,2"])
+@pytest.mark.parametrize("N", [1101, 1102, 1104])
+@pytest.mark.parametrize("x_dtype,M", [("F16", 150), ("F32", 75), ("BF16", 128)])
+def test_pipelined_k_split_of_any_width(engine, oracle, gpu, force, forced, N, x_dtype, M):
+    """The pipelined kernel's partial sums are rows of 16-byte pieces whatever the width: padded
+    columns, a last block of columns and of rows that is partly filled."""
+    force("q4_gemm", forced)
+    run_case(engine, oracle, gpu, N, 1152, M, engine.META_BF16_PLANES, getattr(engine, x_dtype), engine.F32, residual=M == 75)
