@@ -922,7 +922,7 @@ __global__ void __launch_bounds__(256, 1) q4_gemm_pipe_kernel(const GemmParams p
     const uint32_t n_first = block_first_tile * kTileRows;
     char *const stage = (char *)a_lds_raw;
     const bool through_lds = p.splits <= 1u && p.residual == nullptr && !p.pair && p.y_dtype != MI355Q_F32 &&
-                             p.wide_stores && p.N % 8u == 0u;
+                             p.wide_stores;
     const bool whole = n_first + WIDTH <= p.N && m0 + BM <= p.M;
     if (through_lds) {
         auto put = [&](uint32_t row, uint32_t column, const floatx4 &values) {
@@ -963,17 +963,25 @@ __global__ void __launch_bounds__(256, 1) q4_gemm_pipe_kernel(const GemmParams p
         __syncthreads();
         constexpr uint32_t PIECES = WIDTH / 8u;  // 16-byte pieces per row
         uint16_t *const y = (uint16_t *)p.y;
+        // Rows may start on a multiple of 8 bytes only (N % 8 == 4), which 16-byte stores to memory allow;
+        // through the fp32 halves below 10004 columns of 500 rows took 67.2 us instead of 62.4.
+        typedef uint32_t piece_of_y __attribute__((ext_vector_type(4), aligned(8)));
         if (whole) {
             for (uint32_t piece = threadIdx.x; piece < BM * PIECES; piece += 256u) {
                 const uint32_t row = piece / PIECES, column = piece % PIECES * 8u;
-                *(uint4 *)(y + (size_t)(m0 + row) * p.N + n_first + column) = *(const uint4 *)(stage + row * PITCH + column * 2u);
+                *(piece_of_y *)(y + (size_t)(m0 + row) * p.N + n_first + column) =
+                    *(const u32x4 *)(stage + row * PITCH + column * 2u);
             }
         } else {
             for (uint32_t piece = threadIdx.x; piece < BM * PIECES; piece += 256u) {
-                const uint32_t row = piece / PIECES, column = piece % PIECES * 8u;
-                if (m0 + row < p.M && n_first + column < p.N)
-                    *(uint4 *)(y + (size_t)(m0 + row) * p.N + n_first + column) =
-                        *(const uint4 *)(stage + row * PITCH + column * 2u);
+                const uint32_t row = piece / PIECES, column = piece % PIECES * 8u, n = n_first + column;
+                if (m0 + row >= p.M || n >= p.N) continue;
+                uint16_t *const to = y + (size_t)(m0 + row) * p.N + n;
+                const u32x4 values = *(const u32x4 *)(stage + row * PITCH + column * 2u);
+                if (n + 8u <= p.N)
+                    *(piece_of_y *)to = values;
+                else  // the last four columns of a row
+                    *(uint2 *)to = make_uint2(values.x, values.y);
             }
         }
         return;
@@ -992,6 +1000,10 @@ __global__ void __launch_bounds__(256, 1) q4_gemm_pipe_kernel(const GemmParams p
     const bool pairs = p.pair;  // (without a K split: the kernel that adds those adds pairs itself)
     const uint32_t rows_out = pairs ? BM / 4u : BM / 2u;
     constexpr uint32_t FOURS = WIDTH / 4u;  // groups of four columns per row
+    // Then rows of y are whole 16-byte pieces, as rows of partial sums are, and leave by the same
+    // copy: through finish_four 500 rows of 10000 columns took 68.3 us instead of 64.1, 200 rows of
+    // 17408 by 5120 63.1 instead of 59.6.
+    const bool plain = p.y_dtype == MI355Q_F32 && p.row_scale == nullptr && p.residual == nullptr && p.wide_stores;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
         __syncthreads();  // the stage is free: the main loop's reads, or the first half's
@@ -1010,9 +1022,10 @@ __global__ void __launch_bounds__(256, 1) q4_gemm_pipe_kernel(const GemmParams p
             }
         }
         __syncthreads();
-        if (p.splits > 1u) {  // partial sums: a plain copy
+        if (p.splits > 1u || plain) {  // partial sums, or outputs that need nothing done to them: a plain copy
             const uint32_t columns = padded_columns(p.N), first_row = m0 + half * (BM / 2);
-            float *const out = p.partials + ((size_t)split * p.M + first_row) * columns + n_first;
+            float *const out = (p.splits > 1u ? p.partials + (size_t)split * p.M * columns : (float *)p.y) +
+                               (size_t)first_row * columns + n_first;
             if (whole) {  // (two loops: with the test inside one, whole blocks took 0.5 to 0.7 us more)
                 for (uint32_t piece = threadIdx.x; piece < BM / 2u * FOURS; piece += 256u) {
                     const uint32_t row = piece / FOURS, column = piece % FOURS * 4u;

@@ -428,3 +428,26 @@ def test_pipelined_k_split_of_any_width(engine, oracle, gpu, force, forced, N, x
     columns, a last block of columns and of rows that is partly filled."""
     force("q4_gemm", forced)
     run_case(engine, oracle, gpu, N, 1152, M, engine.META_BF16_PLANES, getattr(engine, x_dtype), engine.F32, residual=M == 75)
+
+
+@pytest.mark.parametrize("forced", ["6,1", "7,1", "8,1"])
+@pytest.mark.parametrize("N", [1100, 1102, 1104])
+@pytest.mark.parametrize("y_dtype", ["F16", "F32", "BF16"])
+@pytest.mark.parametrize("M", [128, 150])
+def test_pipelined_outputs_of_any_width(engine, oracle, gpu, force, forced, N, y_dtype, M):
+    """The pipelined kernel's outputs of fp16 activations without a residual: rows that start on 16
+    bytes, on 8 and on neither, blocks of columns and of rows that are whole and partly filled."""
+    force("q4_gemm", forced)
+    kind, K = engine.META_BF16_PLANES, 256
+    quants, meta_a, meta_b = engine.synth_q4_affine(141, 0.02, N, K, kind)
+    x = make_x(engine, 142, M, K).astype(np.float16)
+    product = oracle.q4_linear(quants, meta_a, meta_b, kind, N, K, x, oracle.X_F16, M, weight_rounding=oracle.W_ROUND_F16)
+    weight = gpu.q4_prepare(quants, meta_a, meta_b, N, K, kind)
+    try:
+        print(f"gemm outputs N={N} M={M} y={y_dtype} forced={forced}", flush=True)
+        y = gpu.q4_linear(weight, x, engine.F16, getattr(engine, y_dtype))
+        y = (y.astype(np.uint32) << 16).view(np.float32) if y_dtype == "BF16" else y
+        # a bf16 output is rounded by at most half a unit of its eight bits: 2^-8 of its value
+        assert q4_relative_error(y, product) <= (2.0 ** -8 if y_dtype == "BF16" else 1e-3)
+    finally:
+        weight.destroy()
