@@ -328,10 +328,25 @@ static bool gemm_pipe_ok(const Q4Device &w, uint32_t rows, uint32_t x_columns)
     return w.K % kStepColumns == 0 && (uint64_t)rows * x_columns * sizeof(_Float16) + 16384u < (1ull << 32);
 }
 
-// The shape and K split with the smallest estimated time for one target, and that time in us.
-static double gemm_decompose(mi355q_context *ctx, uint32_t NT, uint32_t N, uint32_t T, uint32_t rows, bool bytes_native,
-                             bool pipe_ok, int &best, uint32_t &best_splits)
+// How one target of a call is multiplied: the shape and K split with the smallest estimated time.
+struct TargetPlan {
+    bool bytes;       // by the kernel for 8-bit codes
+    int variant;
+    uint32_t splits;
+    double us;        // the estimate
+};
+static TargetPlan plan_target(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, uint32_t rows)
 {
+    const Q4Device &w = *a.targets[target].w;
+    const uint32_t x_columns = a.x_columns ? a.x_columns : w.K, NT = w.NT;
+    // The doubled form of an 8-bit weight whose activation row the kernels would read twice: the
+    // kernel for 8-bit codes reads the bytes themselves instead, one pass over the row, half the
+    // matrix instructions.  It is the pipelined kernel, with that kernel's conditions.
+    const bool bytes = w.codes8 != nullptr && a.x_columns != 0 && !ctx->q8_gemm_doubled &&
+                       (uint64_t)rows * x_columns * sizeof(_Float16) + 16384u < (1ull << 32);
+    const uint32_t T = bytes ? w.T / 2u : w.T;
+    const bool pipe_ok = gemm_pipe_ok(w, rows, x_columns);
+    TargetPlan best = {bytes, 0, 1, 1e30};
     // Decomposition: BM rows x (4*NTW + EXTRA) tiles per workgroup, K split in `splits`.
     // The choice minimises a microsecond estimate fitted to sweeps over every variant
     // and split on this GPU.  Kernels 0-5: a workgroup that has a compute unit to itself
@@ -351,10 +366,9 @@ static double gemm_decompose(mi355q_context *ctx, uint32_t NT, uint32_t N, uint3
         return r <= 0.562 ? 0.771 - 0.081 * r / 0.562 : 1.0 - 0.31 * over * over;
     };
     const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
-    double best_cost = 1e30;
     for (int v = 0; v < (int)(sizeof variants / sizeof variants[0]); ++v) {
         if (v >= 6 && !pipe_ok) continue;
-        if ((v >= kBytesVariant) != bytes_native) continue;
+        if ((v >= kBytesVariant) != bytes) continue;
         const Variant &c = variants[v];
         const uint32_t tpb = 4u * c.ntw + c.extra;
         const uint32_t slots = cus * (uint32_t)c.resident;
@@ -388,19 +402,21 @@ static double gemm_decompose(mi355q_context *ctx, uint32_t NT, uint32_t N, uint3
             else
                 cost = ((double)groups / slots + (groups % slots ? 0.31 : 0.0)) * c.resident * peak_us / c.shared;
             if (splits > 1)  // fp32 partials at 4.6 TB/s and the kernel that adds them
-                cost += (double)splits * rows * (double)N * 4.0 / 4.63e6 + (v >= 6 ? 2.0 : 6.3);
-            if (cost < best_cost) {
-                best_cost = cost;
-                best = v;
-                best_splits = splits;
-            }
+                cost += (double)splits * rows * (double)w.N * 4.0 / 4.63e6 + (v >= 6 ? 2.0 : 6.3);
+            if (cost < best.us) best = {bytes, v, splits, cost};
         }
     }
-    return best_cost;
+    // option "q4_gemm" = "VARIANT,SPLITS" for experiments
+    if (ctx->force_gemm[1] >= 1 && ctx->force_gemm[0] < (int)(sizeof variants / sizeof variants[0]) &&
+        (ctx->force_gemm[0] < 6 || pipe_ok) && (ctx->force_gemm[0] >= kBytesVariant) == bytes) {
+        best.variant = ctx->force_gemm[0];
+        best.splits = (uint32_t)ctx->force_gemm[1];
+    }
+    return best;
 }
 
-static int gemm_one_target(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, char *error,
-                           size_t error_capacity)
+static int gemm_one_target(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, const TargetPlan &plan,
+                           char *error, size_t error_capacity)
 {
     const Q4Device &w = *a.targets[target].w;
     GemmParams p;
@@ -415,13 +431,8 @@ static int gemm_one_target(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t 
     int status = gemm_activations(ctx, a, x_columns, target == 0, p, error, error_capacity);
     if (status != MI355Q_OK) return status;
     const uint32_t rows = p.M;
-    // The doubled form of an 8-bit weight whose activation row the kernels would read twice: the
-    // kernel for 8-bit codes reads the bytes themselves instead, one pass over the row, half the
-    // matrix instructions.  It is the pipelined kernel, with that kernel's conditions.
-    const bool bytes_native = w.codes8 != nullptr && a.x_columns != 0 && !ctx->q8_gemm_doubled &&
-                              (uint64_t)rows * x_columns * sizeof(_Float16) + 16384u < (1ull << 32);
-    const uint32_t T = bytes_native ? w.T / 2u : w.T;
-    if (bytes_native) {
+    const uint32_t T = plan.bytes ? w.T / 2u : w.T;
+    if (plan.bytes) {
         p.codes = w.codes8;
         p.meta = w.meta8;
     }
@@ -429,7 +440,7 @@ static int gemm_one_target(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t 
     p.residual = a.targets[target].residual;
     p.N = w.N;
     p.K = x_columns;
-    p.wrap_steps = a.x_columns && !bytes_native ? a.x_columns / kStepColumns : 0xffffffffu;
+    p.wrap_steps = a.x_columns && !plan.bytes ? a.x_columns / kStepColumns : 0xffffffffu;
     p.NT = w.NT;
     p.T = T;
     p.y_dtype = a.y_dtype;
@@ -437,26 +448,16 @@ static int gemm_one_target(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t 
     p.residual_is_bias = a.residual_is_bias;
     p.wide_stores = w.N % 4u == 0u && (uintptr_t)p.y % 16u == 0u;
 
-    const bool pipe_ok = gemm_pipe_ok(w, rows, x_columns);
-    int best = 0;
-    uint32_t best_splits = 1;
-    (void)gemm_decompose(ctx, w.NT, w.N, T, rows, bytes_native, pipe_ok, best, best_splits);
-    // option "q4_gemm" = "VARIANT,SPLITS" for experiments
-    if (ctx->force_gemm[1] >= 1 && ctx->force_gemm[0] < (int)(sizeof variants / sizeof variants[0]) &&
-        (ctx->force_gemm[0] < 6 || pipe_ok) && (ctx->force_gemm[0] >= kBytesVariant) == bytes_native) {
-        best = ctx->force_gemm[0];
-        best_splits = (uint32_t)ctx->force_gemm[1];
-    }
     if (ctx->trace)
         fprintf(stderr, "mi355q: q4 gemm M=%u N=%u K=%u -> variant %d (BM=%d, %d tiles/wave%s%s), K split %u\n",
-                rows, w.N, w.K, best, variants[best].bm, variants[best].ntw,
-                variants[best].extra ? " +1" : "", bytes_native ? ", 8-bit codes" : "", best_splits);
-    const Variant &chosen = variants[best];
+                rows, w.N, w.K, plan.variant, variants[plan.variant].bm, variants[plan.variant].ntw,
+                variants[plan.variant].extra ? " +1" : "", plan.bytes ? ", 8-bit codes" : "", plan.splits);
+    const Variant &chosen = variants[plan.variant];
     const uint32_t tpb = 4u * chosen.ntw + chosen.extra;
     p.tiles_per_block = tpb;
     const uint32_t n_blocks = (w.NT + tpb - 1) / tpb;
     const uint32_t m_blocks = (rows + chosen.bm - 1) / chosen.bm;
-    p.steps_per_split = (T + best_splits - 1) / best_splits;
+    p.steps_per_split = (T + plan.splits - 1) / plan.splits;
     p.splits = (T + p.steps_per_split - 1) / p.steps_per_split;
     if (p.splits > 1u) {
         const size_t bytes = (size_t)p.splits * rows * padded_columns(w.N) * sizeof(float);
@@ -475,7 +476,7 @@ static int gemm_one_target(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t 
                                        : ((n_blocks % 8u != 0u && m_blocks > 1u) || p.splits > 1u ? 1 : 0);
     const dim3 grid(n_blocks, m_blocks, p.splits);
     hipError_t launched = hipErrorInvalidValue;
-    switch (best) {
+    switch (plan.variant) {
     case 0: launched = launch_gemm<128, 4, false>(ctx, grid, p); break;
     case 1: launched = launch_gemm<128, 2, false>(ctx, grid, p); break;
     case 2: launched = launch_gemm<64, 4, false>(ctx, grid, p); break;
@@ -510,18 +511,24 @@ struct RowsPlan {
 };
 
 // The launch of q4_rows_kernel for a call's targets together; false: not the kernel for it.
+// `others`: what each target would take otherwise.
 // Shape and workgroups minimise a microsecond estimate fitted to 1430 timings on this GPU (three
 // layer shapes, 17 to 128 rows, every block width, whole blocks and 128 to 768 workgroups; 8 % rms,
 // the choice within 8 % of the best timed one in 82 of 84 calls): 4.4 us, then per unit the longer
 // of one workgroup's own chain (0.22 + 0.12 us per 16 rows) and its share of the compute unit,
-// then, where workgroups share blocks, 3.7 us and the partial sums at 2.1 TB/s.  Chosen where that
-// is at most 1 us per target more than the other kernels' estimate, which leaves out the launches
-// behind a K split: at 27B shapes gate|up up to 128 rows (49 -> 33 us at 32, 82 -> 49 at 80, 77 ->
-// 65 at 128) and q|k|v (40 -> 14, 49 -> 23, 52 -> 30); o and down up to 48 and from 65 to 96 rows
-// (27 -> 23 us at 32, 37 -> 34 at 80; the other kernels' 27 against 30 at 64, 38 against 44 at 128).
-static bool rows_plan(mi355q_context *ctx, const Q4LinearArgs &a, RowsPlan &plan)
+// then, where workgroups share blocks, 3.7 us and the partial sums at 2.1 TB/s.
+//
+// Chosen where that is at most 1 us per target more than the other kernels' estimate, which leaves
+// out the launches behind a K split (27B shapes: gate|up up to 128 rows, 49 -> 33 us at 32, 82 -> 49
+// at 80, 77 -> 65 at 128; q|k|v 40 -> 14, 49 -> 23, 52 -> 30).  A call of one weight saves no launch, and
+// both estimates leave out what reading a large one takes: for each MB beyond 20 MB 0.1 us is added to
+// this kernel's and, where two row blocks read it, 0.04 to the other's (twelve weights, 17 to 128
+// rows, each in HBM and in the Infinity Cache).  This kernel against the other, us from HBM (the
+// cache): 17408 x 5120 at 32 rows 23.8 (23.6) and 23.3 (21.3), not chosen, at 80 rows 35.1 (34.5)
+// and 39.8 (37.5), chosen; 5120 x 17408 at 32 rows 23.0 (23.2) and 26.7 (22.7), chosen, at 96 rows
+// 38.9 (37.6) and 37.2 (32.8), not chosen.
+static bool rows_plan(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows, const TargetPlan *others, RowsPlan &plan)
 {
-    const uint32_t rows = a.x_dtype == MI355Q_F32 ? 2u * a.M : a.M;
     const Q4Device &first = *a.targets[0].w;
     const uint32_t T = first.T;
     if (rows > 128u) return false;
@@ -571,15 +578,15 @@ static bool rows_plan(mi355q_context *ctx, const Q4LinearArgs &a, RowsPlan &plan
         }
     }
     plan = best;
-    double others = 0.0;
-    for (uint32_t t = 0; t < a.count; ++t) {
-        const Q4Device &w = *a.targets[t].w;
-        int variant;
-        uint32_t splits;
-        others += gemm_decompose(ctx, w.NT, w.N, T, rows, false, gemm_pipe_ok(w, rows, a.x_columns ? a.x_columns : w.K),
-                                 variant, splits);
+    double others_us = 0.0;
+    for (uint32_t t = 0; t < a.count; ++t) others_us += others[t].us;
+    if (a.count == 1u) {
+        const double megabytes = (double)first.N * first.K * 0.5625e-6;  // 4-bit codes and their metadata
+        const double large = std::min(std::max(megabytes - 20.0, 0.0), 30.0);  // (50 MB: the largest measured)
+        best_cost += 0.1 * large;
+        if (rows > (uint32_t)variants[others[0].variant].bm) others_us += 0.04 * large;
     }
-    return best_cost <= others + 1.0 * a.count;
+    return best_cost <= others_us + 1.0 * a.count;
 }
 
 template <int MF, int NTW, int W>
@@ -713,10 +720,13 @@ int q4_gemm_linears(mi355q_context *ctx, const Q4LinearArgs &a, char *error, siz
         }
         return status;
     }
-    RowsPlan plan;
-    if (rows_plan(ctx, a, plan)) return q4_rows_linears(ctx, a, plan, error, error_capacity);
+    const uint32_t rows = a.x_dtype == MI355Q_F32 ? 2u * a.M : a.M;
+    TargetPlan plans[kMaxTargets];
+    for (uint32_t t = 0; t < a.count; ++t) plans[t] = plan_target(ctx, a, t, rows);
+    RowsPlan together;
+    if (rows_plan(ctx, a, rows, plans, together)) return q4_rows_linears(ctx, a, together, error, error_capacity);
     for (uint32_t t = 0; t < a.count && status == MI355Q_OK; ++t)
-        status = gemm_one_target(ctx, a, t, error, error_capacity);
+        status = gemm_one_target(ctx, a, t, plans[t], error, error_capacity);
     return status;
 }
 

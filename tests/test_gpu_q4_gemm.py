@@ -451,3 +451,19 @@ def test_pipelined_outputs_of_any_width(engine, oracle, gpu, force, forced, N, y
         assert q4_relative_error(y, product) <= (2.0 ** -8 if y_dtype == "BF16" else 1e-3)
     finally:
         weight.destroy()
+
+
+@pytest.mark.parametrize("N,K,M,kernel", [(17408, 5120, 32, "gemm"), (17408, 5120, 80, "rows"), (5120, 17408, 32, "rows"),
+                                          (5120, 17408, 96, "gemm"), (5120, 6144, 32, "rows")])
+def test_kernel_of_one_large_weight(engine, gpu, force, capfd, N, K, M, kernel):
+    """Which kernel takes a large weight alone, as the trace prints it: the ones that timing each
+    with weights in HBM and in the Infinity Cache found faster."""
+    kind = engine.META_BF16_PLANES
+    weight = gpu.q4_prepare(*engine.synth_q4_affine(151, 0.02, N, K, kind), N, K, kind)
+    try:
+        force("trace", "1")
+        y = gpu.q4_linear(weight, make_x(engine, 152, M, K).astype(np.float16), engine.F16, engine.F16)
+        printed = capfd.readouterr().err
+    finally:
+        weight.destroy()
+    assert np.any(y != 0) and ("mi355q: q4 %s M=%d" % (kernel, M)) in printed
