@@ -81,9 +81,11 @@ static int apply_option(mi355q_context *ctx, const char *name, const char *value
         ctx->trace = set && strcmp(value, "0") != 0;
         return MI355Q_OK;
     }
-    if (strcmp(name, "w8a8") == 0) {  // "1" .. "4": tiles per workgroup of the W8A8 kernel, whatever the tile count
-        if (set && (strlen(value) != 1 || value[0] < '1' || value[0] > '4')) return MI355Q_ERROR_INVALID;
-        ctx->w8a8_tiles = set ? value[0] - '0' : 0;
+    if (strcmp(name, "w8a8") == 0) {  // "1" .. "4": the kernel of tiles, so many per workgroup; "small", "blocks": that of blocks
+        const bool small = set && strcmp(value, "small") == 0, blocks = set && strcmp(value, "blocks") == 0;
+        if (set && !small && !blocks && (strlen(value) != 1 || value[0] < '1' || value[0] > '4')) return MI355Q_ERROR_INVALID;
+        ctx->w8a8_tiles = set && !small && !blocks ? value[0] - '0' : 0;
+        ctx->w8a8_blocks = small ? 4 : blocks ? 8 : 0;
         return MI355Q_OK;
     }
     if (strcmp(name, "gemm_loads") == 0) {  // "plain": GEMM variant 7 with ordinary weight loads (a cross-check)

@@ -8,8 +8,9 @@ The log is the compiler's whole diagnostic output; what is not a resource remark
 is passed through to stdout, the remarks themselves are only read.
 
 Budgets (a kernel name is matched after demangling):
-  * every q4_stream_kernel, q4_chain_kernel, q4_rows_kernel and q4_gemm_pipe_kernel instantiation: no scratch memory
-    (a spill inside the streaming loop costs more than any occupancy it buys) and no spilled registers;
+  * every q4_stream_kernel, q4_chain_kernel, q4_rows_kernel, q4_gemm_pipe_kernel and w8a8_block_kernel
+    instantiation: no scratch memory (a spill inside the streaming loop costs more than any occupancy it
+    buys, and its loads would be among those that the kernel's own waits count) and no spilled registers;
   * q4_stream_kernel<1, 1, 2, 16, *, false>: at most 64 vector registers - with sixteen waves a
     workgroup, two workgroups share a compute unit only up to 64 (one more halves the occupancy
     and the launch of the 27B q|k|v group takes a quarter longer);
@@ -73,7 +74,7 @@ def main():
                                text=True, check=True).stdout.splitlines()
     problems = []
     for (mangled, use), name in zip(found, demangled):
-        watched = re.search(r"(q4_stream_kernel|q4_chain_kernel|q4_rows_kernel|q4_gemm_pipe_kernel)<([^>]*)>", name)
+        watched = re.search(r"(q4_stream_kernel|q4_chain_kernel|q4_rows_kernel|q4_gemm_pipe_kernel|w8a8_block_kernel)<([^>]*)>", name)
         if not watched:
             continue
         kind, parameters = watched.group(1), [p.strip() for p in watched.group(2).split(",")]

@@ -94,6 +94,7 @@ struct mi355q_context {
     bool q8_gemm_doubled;   // option "q8_gemm" = "doubled": 8-bit weights take the Q4 GEMM kernels on their doubled form
     bool gemm_plain_loads;  // option "gemm_loads" = "plain": the 17-tile GEMM shape with compiler-managed weight loads
     int w8a8_tiles;       // option "w8a8" = "1" .. "4": tiles per W8A8 workgroup (0: chosen by the launch)
+    int w8a8_blocks;      // the same option = "small" / "blocks": 4 / 8 tiles a block of the kernel of blocks
     bool lds_raised[16];  // q4_gemm_pipe_kernel instantiations whose dynamic LDS limit has been raised
     bool rows_lds_raised[9][5];  // the same for q4_rows_kernel<fragments, tiles per wave>
     // device address of the library's fixed scratch array on this context's device (for the

@@ -401,7 +401,6 @@ __global__ void __launch_bounds__(256, 2) w8a8_block_kernel(const W8a8Params p)
         slot = slot + 1u == (uint32_t)R ? 0u : slot + 1u;
     }
 
-    typedef float floatx4 __attribute__((ext_vector_type(4)));
     float *const out = p.out[target];
     int32_t *const acc_out = p.acc[target];
     const float *const bias = p.bias[target];
@@ -466,9 +465,10 @@ __global__ void __launch_bounds__(256, 2) w8a8_block_kernel(const W8a8Params p)
 enum class W8a8Kernel { tiles, small_blocks, blocks };
 static W8a8Kernel w8a8_choose(mi355q_context *ctx, const W8a8Params &p)
 {
-    // option "w8a8" is about the kernel of tiles; the other one has 32-bit byte offsets into q and a tile
+    // the kernel of blocks has 32-bit byte offsets into q and a tile
     if (ctx->w8a8_tiles || (uint64_t)p.M * p.K >= (1ull << 32) || (uint64_t)p.KS * 1024u >= (1ull << 32))
         return W8a8Kernel::tiles;
+    if (ctx->w8a8_blocks) return ctx->w8a8_blocks == 4 ? W8a8Kernel::small_blocks : W8a8Kernel::blocks;
     const uint64_t cus = (uint64_t)ctx->props.multiProcessorCount, m_blocks = (p.M + 63u) / 64u;
     uint64_t tiles = 0, columns = 0;
     for (uint32_t t = 0; t < p.targets; ++t) {

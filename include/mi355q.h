@@ -123,6 +123,7 @@ int mi355q_context_info(mi355q_context *ctx, mi355q_device_info *info,
  *   "trace"     = "1"                           prints every launch's decomposition to stderr
  *   "in_kernel_slices" = "0"                    K slices are added by a second kernel
  *   "w8a8"      = "1" .. "4"                    W8A8: the kernel of tiles, with so many per workgroup
+ *   "w8a8"      = "small" / "blocks"            W8A8: the kernel of blocks, of 64 x 64 / 64 x 128 outputs
  *   "gemm_loads" = "plain"                      GEMM variant 7 built with ordinary weight loads
  *                                               (compiler-placed waits): the cross-check of the
  *                                               hand-scheduled kernel, same bits, slower

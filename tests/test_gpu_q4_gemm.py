@@ -290,8 +290,9 @@ def test_converted_activations_finish_in_the_kernel(engine, oracle, gpu, force, 
 @pytest.mark.parametrize("x_dtype", ["F32", "BF16"])
 @pytest.mark.parametrize("M", [9, 40, 150])
 def test_targets_share_converted_activations(engine, gpu, x_dtype, M):
-    """Weights of one call multiply activations that were converted once: the same bits as one
-    call per weight."""
+    """Weights of one call multiply activations that were converted once: the results of one call per
+    weight up to the order of the fp32 sums, which at 17 to 128 matrix rows depends on the weights that
+    share the call; above that, where each is multiplied by itself, the same bits."""
     K, widths = 384, (272, 1000, 100)
     x32 = make_x(engine, 81, M, K)
     x = x32 if x_dtype == "F32" else bf16_bits(x32).reshape(M, K)
@@ -314,6 +315,8 @@ def test_targets_share_converted_activations(engine, gpu, x_dtype, M):
             assert np.any(alone != 0)
             close = np.abs(together.view(np.float32) - alone.view(np.float32))
             assert np.max(close) <= 2e-6 * np.max(np.abs(alone.view(np.float32)))
+            if M == 150:
+                assert np.array_equal(together, alone)
     finally:
         for pointer in [x_ptr] + outputs + biases:
             gpu.free(pointer)
@@ -364,6 +367,43 @@ def test_rows_kernel_targets_and_converted_activations(engine, gpu, force, force
             assert np.max(np.abs(here - there)) <= 448 * 2.0 ** -24 * np.max(np.abs(there))
     finally:
         for pointer in [x_ptr] + outputs + biases:
+            gpu.free(pointer)
+        for weight in weights:
+            weight.destroy()
+
+
+@pytest.mark.parametrize("forced", ["11,2", "12,2", "11,1"])
+@pytest.mark.parametrize("x_dtype,M", [("F16", 20), ("F16", 67), ("F32", 40), ("BF16", 128)])
+def test_rows_kernel_runs_that_cross_targets(engine, gpu, force, forced, x_dtype, M):
+    """Runs of steps that begin in one weight and end in the next, in blocks that other workgroups
+    share: five steps a block in runs of three over 10, 16 and 6 blocks of 64 columns ("11,2") and in
+    runs of two over 5, 8 and 3 of 128 ("12,2"), so that 50, 130, 25 and 65 steps precede a weight.  One width is no
+    multiple of 4, the last weight's last block has tiles beyond the matrix.  Under "11,1" every
+    workgroup takes whole blocks and a weight's outputs do not depend on the others, bit for bit."""
+    K, widths = 640, (640, 1002, 330)
+    x32 = make_x(engine, 131, M, K)
+    x = x32 if x_dtype == "F32" else x32.astype(np.float16) if x_dtype == "F16" else bf16_bits(x32).reshape(M, K)
+    kind, x_dtype = engine.META_BF16_PLANES, getattr(engine, x_dtype)
+    weights = [gpu.q4_prepare(*engine.synth_q4_affine(132 + i, 0.02, N, K, kind), N, K, kind) for i, N in enumerate(widths)]
+    x_ptr = gpu.to_device(x)
+    outputs = [gpu.alloc(M * N * 4) for N in widths]
+    try:
+        results = []
+        targets = list(zip(weights, outputs))
+        for how, groups in ((forced, [targets]), ("11,1" if forced == "11,1" else "4,1", [[t] for t in targets])):
+            print(f"rows across targets M={M} x={x_dtype} forced={how}", flush=True)
+            force("q4_gemm", how)
+            gpu.q4_sequence(engine.make_calls([(g, x_ptr, x_dtype, M, engine.F32) for g in groups]))
+            gpu.sync()
+            results.append([gpu.download(p, (M, N), np.float32) for p, N in zip(outputs, widths)])
+        for here, there in zip(*results):
+            assert np.any(there != 0)
+            if forced == "11,1":
+                assert np.array_equal(here, there)
+            # 640 products of one row summed in another order: 640 roundings of 2^-24 at most
+            assert np.max(np.abs(here - there)) <= 640 * 2.0 ** -24 * np.max(np.abs(there))
+    finally:
+        for pointer in [x_ptr] + outputs:
             gpu.free(pointer)
         for weight in weights:
             weight.destroy()

@@ -136,6 +136,35 @@ def test_block_kernel_gives_the_tile_kernels_bits(engine, oracle, gpu, force, M,
         assert np.array_equal(tiles[i][0].view(np.uint32), out_ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("blocks", ["small", "blocks"])
+@pytest.mark.parametrize("M,K,widths,channel_major", [
+    (1, 16, (4,), False), (33, 592, (1000,), True), (64, 1040, (257, 1030), False), (130, 1088, (516,), False),
+    (65, 1104, (131, 70, 64), False)])
+def test_block_kernel_wherever_it_is_asked_for(engine, oracle, gpu, force, blocks, M, K, widths, channel_major):
+    """Both block sizes by option, whatever the sizes would choose: one step, and ten, seventeen and
+    eighteen - odd and even, ragged and whole - which go round the ring of stages more than once."""
+    q, scales = oracle.quantize_i8(engine.synth_normal_f32(61, 1.0, M * K).reshape(M, K))
+    rows = [engine.synth_w8_rows(62 + i, 0.02, N, K) for i, N in enumerate(widths)]
+    biases = [engine.synth_normal_f32(72 + i, 1.0, N) for i, N in enumerate(widths)]
+    weights = [gpu.w8a8_prepare(r, N, K) for r, N in zip(rows, widths)]
+    print(f"w8a8 {blocks} M={M} K={K} widths={widths} channel_major={channel_major}", flush=True)
+    force("w8a8", blocks)
+    try:
+        if len(widths) == 1:
+            results = [gpu.w8a8_linear(weights[0], widths[0], q, scales, biases[0], channel_major=channel_major)]
+        else:
+            results = gpu.w8a8_linear_multi(weights, widths, q, scales, biases)
+    finally:
+        for weight in weights:
+            gpu.w8a8_destroy(weight)
+    for i, N in enumerate(widths):
+        out_ref, acc_ref = oracle.w8a8_linear(rows[i], N, K, q, scales, biases[i])
+        if channel_major:
+            out_ref = oracle.w8a8_conv(rows[i], N, K, q, scales, biases[i])
+        assert results[i][1].tobytes() == acc_ref.tobytes() and np.any(acc_ref != 0)
+        assert np.array_equal(results[i][0].view(np.uint32), out_ref.view(np.uint32))
+
+
 def test_reference_golden_vectors(engine, gpu):
     g = np.load(GOLDEN, allow_pickle=False)
     x, rows, bias = g["x"], g["rows"], g["bias"]
