@@ -14,13 +14,13 @@ constexpr uint32_t rows_stage_bytes(int mf, int ntw, int waves)
     return (uint32_t)mf * 4096u + (uint32_t)waves * ((uint32_t)ntw * 1024u + 256u);
 }
 // Stages in the ring: two workgroups on a compute unit when three stages each fit its 160 KiB (up
-// to four), else one workgroup with up to six.
+// to four), else one workgroup with what fits, three to five.
 constexpr int rows_resident(int mf, int ntw, int waves) { return 3u * rows_stage_bytes(mf, ntw, waves) <= 80u * 1024u ? 2 : 1; }
 constexpr int rows_stages(int mf, int ntw, int waves)
 {
-    const int fit = (int)((rows_resident(mf, ntw, waves) == 2 ? 80u : 160u) * 1024u / rows_stage_bytes(mf, ntw, waves));
-    const int most = rows_resident(mf, ntw, waves) == 2 ? 4 : 6;
-    return fit < most ? fit : most;
+    const int resident = rows_resident(mf, ntw, waves);
+    const int fit = (int)(160u / resident * 1024u / rows_stage_bytes(mf, ntw, waves));
+    return resident == 2 && fit > 4 ? 4 : fit;
 }
 constexpr uint32_t rows_lds_bytes(int mf, int ntw, int waves)
 {
@@ -36,7 +36,7 @@ constexpr uint32_t rows_lds_bytes(int mf, int ntw, int waves)
 // output; the workgroups that share a block leave partial sums, which a second kernel adds in
 // their order.
 // Everything a unit needs - the rows of x, shared by the waves, and each wave's own codes and
-// metadata - is written to LDS by LDS-direct loads, so the units in flight (two to five ahead of
+// metadata - is written to LDS by LDS-direct loads, so the units in flight (two to four ahead of
 // the arithmetic, across the end of a block) cost no registers and one counted wait per unit covers
 // all of them: the loads are asm statements in one in-order queue that the compiler adds nothing
 // to.  Two waves share a SIMD and overlap one's dequantization with the other's matrix

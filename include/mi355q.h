@@ -119,7 +119,10 @@ int mi355q_context_info(mi355q_context *ctx, mi355q_device_info *info,
  * MI355Q_Q4_GEMM, MI355Q_TRACE and MI355Q_NO_ARRIVALS are read once, when the context is
  * created; this call changes the same knobs afterwards.  A NULL or empty value clears one.
  *   "q4_stream" = "TILES,DEPTH,WAVES[,SLICES]"  forces the streaming kernel's launch shape
- *   "q4_gemm"   = "VARIANT,SPLITS"              forces the GEMM's kernel variant and K split
+ *   "q4_gemm"   = "VARIANT,SPLITS"              forces the GEMM's kernel variant and K split; variants 11,
+ *                                               12, 13 are blocks of 4, 8, 16 tiles of the kernel for
+ *                                               17 to 128 rows, whose second number is 1 for whole
+ *                                               blocks, s > 1 for 64 (s - 1) workgroups that share them
  *   "trace"     = "1"                           prints every launch's decomposition to stderr
  *   "in_kernel_slices" = "0"                    K slices are added by a second kernel
  *   "w8a8"      = "1" .. "4"                    W8A8: the kernel of tiles, with so many per workgroup
@@ -417,7 +420,12 @@ int mi355q_q4_linear_noalloc(mi355q_context *ctx, const mi355q_q4_weight *weight
  * so do gate and up (the reference fuses them the same way: one 14336-row
  * q|k|v matrix, qwen38_m3_attention_image.h:11-14; qwen38_q4_gate_up_silu,
  * qwen38_q4.metal:129-151) — and it spares the small matrices their own launch.
- * For M > 16 the targets run one after the other. */
+ * From there to 128 matrix rows (64 of fp32 x) the targets are one launch too
+ * where that is the faster way, and the steps of all of them are divided among
+ * its workgroups: the order in which an output's products are added, and so its
+ * last bits, may then depend on the other targets of the call.  Above that, and
+ * where a target writes what another one reads or writes, they run one after
+ * the other with the results of one call each. */
 typedef struct {
     const mi355q_q4_weight *weight;
     void *y;              /* [M][N_t] of y_dtype */
