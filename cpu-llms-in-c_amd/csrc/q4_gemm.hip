@@ -24,6 +24,11 @@
 //     one launch.
 // The host picks shape and K split by a time estimate fitted on this GPU, e.g.
 // 17 tiles for the 17408-row matrices: 64 x 4 = 256 workgroups at M = 512.
+// Several weights of a call go out as one launch where that is estimated to take less: they
+// fill the chip together (us, a launch each -> one launch: 6144 + 1024 + 1024 x 5120 at 200 rows
+// 51 -> 35, at 512 rows 78 -> 53; 2048 + 512 + 512 x 1024 at 512 rows 26.5 -> 10.8; two of
+// 17408 x 5120 at 200 rows 103 -> 74; two of 8192 x 3072 at 512 rows 68 -> 43; three of 1280 x 1280
+// over 1500 fp32 rows 72 -> 51).
 #include <algorithm>
 #include <cstdio>
 #include "device_util.h"
@@ -39,12 +44,12 @@
 namespace mi355q {
 
 // the pipelined kernel's instantiations live in q4_gemm_pipe_*.hip
-extern template __global__ void q4_gemm_pipe_kernel<128, 4, false, false>(const GemmParams);
-extern template __global__ void q4_gemm_pipe_kernel<128, 4, true, false>(const GemmParams);
-extern template __global__ void q4_gemm_pipe_kernel<128, 4, true, true>(const GemmParams);
-extern template __global__ void q4_gemm_pipe_kernel<128, 5, false, false>(const GemmParams);
-extern template __global__ void q4_gemm_pipe_kernel<128, 4, false, false, true>(const GemmParams);  // 8-bit codes
-extern template __global__ void q4_gemm_pipe_kernel<128, 3, true, false, true>(const GemmParams);   // 8-bit codes
+extern template __global__ void q4_gemm_pipe_kernel<128, 4, false, false>(const GemmGroup);
+extern template __global__ void q4_gemm_pipe_kernel<128, 4, true, false>(const GemmGroup);
+extern template __global__ void q4_gemm_pipe_kernel<128, 4, true, true>(const GemmGroup);
+extern template __global__ void q4_gemm_pipe_kernel<128, 5, false, false>(const GemmGroup);
+extern template __global__ void q4_gemm_pipe_kernel<128, 4, false, false, true>(const GemmGroup);  // 8-bit codes
+extern template __global__ void q4_gemm_pipe_kernel<128, 3, true, false, true>(const GemmGroup);   // 8-bit codes
 
 // Adds the K splits in split order (a fixed order) and applies the epilogue.  WIDE: a thread
 // takes four adjacent outputs of one row (N a multiple of 4, y 16-byte aligned): 16-byte loads
@@ -166,17 +171,21 @@ __global__ void __launch_bounds__(kReduceThreads) q4_group_reduce_kernel(const G
     const uint32_t m = blockIdx.z * kReduceRows + blockIdx.y;
     if (n >= p.N || m >= (p.pair ? p.M / 2u : p.M)) return;
     uint32_t splits = p.splits;
-    if (p.units) {  // one workgroup alone has stored the outputs
+    if (p.units) {
         const uint32_t begin = (p.first_block + n / p.block_columns) * p.T;
         splits = (begin + p.T - 1u) / p.units - begin / p.units + 1u;
-        if (splits == 1u) return;
     }
+    if (splits == 1u) return;  // the outputs are stored: by one workgroup alone, of a target without a K split
     reduce_columns<WIDE, 0>(p, splits, m, n);
 }
 
 template <int BM, int NTW, bool EXTRA>
-static hipError_t launch_gemm(mi355q_context *ctx, dim3 grid, const GemmParams &p)
+static hipError_t launch_gemm(mi355q_context *ctx, dim3 grid, const GemmGroup &group)
 {
+    const GemmParams &p = group.shared;
+    if (p.targets > 1u)
+        return p.row_scale ? launch(ctx, q4_gemm_group_kernel<BM, NTW, EXTRA, true>, grid, dim3(256), 0, group)
+                           : launch(ctx, q4_gemm_group_kernel<BM, NTW, EXTRA, false>, grid, dim3(256), 0, group);
     return p.row_scale ? launch(ctx, q4_gemm_kernel<BM, NTW, EXTRA, true>, grid, dim3(256), 0, p)
                        : launch(ctx, q4_gemm_kernel<BM, NTW, EXTRA, false>, grid, dim3(256), 0, p);
 }
@@ -184,7 +193,7 @@ static hipError_t launch_gemm(mi355q_context *ctx, dim3 grid, const GemmParams &
 // The pipelined kernel's stage is larger than the 64 KiB a kernel gets without asking: the
 // limit is raised once per device and instantiation.
 template <int NTW, bool XT>
-static hipError_t launch_pipe(mi355q_context *ctx, dim3 grid, const GemmParams &p)
+static hipError_t launch_pipe(mi355q_context *ctx, dim3 grid, const GemmGroup &group)
 {
     constexpr size_t bytes = pipe_lds_bytes(128);
     constexpr int slot = 2 * NTW + (XT ? 1 : 0);  // this instantiation's flag in the context
@@ -197,12 +206,12 @@ static hipError_t launch_pipe(mi355q_context *ctx, dim3 grid, const GemmParams &
         if (status != hipSuccess) return status;
         ctx->lds_raised[slot] = true;
     }
-    return launch(ctx, q4_gemm_pipe_kernel<128, NTW, XT>, grid, dim3(256), bytes, p);
+    return launch(ctx, q4_gemm_pipe_kernel<128, NTW, XT>, grid, dim3(256), bytes, group);
 }
 
 // The shapes on 8-bit codes: 16 tiles, or 13 (three per wave and one shared).
 template <int NTW, bool XT>
-static hipError_t launch_pipe_bytes(mi355q_context *ctx, dim3 grid, const GemmParams &p)
+static hipError_t launch_pipe_bytes(mi355q_context *ctx, dim3 grid, const GemmGroup &group)
 {
     constexpr size_t bytes = pipe_lds_bytes(128);
     constexpr int slot = XT ? 13 : 14;
@@ -212,11 +221,11 @@ static hipError_t launch_pipe_bytes(mi355q_context *ctx, dim3 grid, const GemmPa
         if (status != hipSuccess) return status;
         ctx->lds_raised[slot] = true;
     }
-    return launch(ctx, q4_gemm_pipe_kernel<128, NTW, XT, false, true>, grid, dim3(256), bytes, p);
+    return launch(ctx, q4_gemm_pipe_kernel<128, NTW, XT, false, true>, grid, dim3(256), bytes, group);
 }
 
 // The 17-tile shape with compiler-managed weight loads (option "gemm_loads" = "plain").
-static hipError_t launch_pipe_plain(mi355q_context *ctx, dim3 grid, const GemmParams &p)
+static hipError_t launch_pipe_plain(mi355q_context *ctx, dim3 grid, const GemmGroup &group)
 {
     constexpr size_t bytes = pipe_lds_bytes(128);
     constexpr int slot = 15;
@@ -226,24 +235,24 @@ static hipError_t launch_pipe_plain(mi355q_context *ctx, dim3 grid, const GemmPa
         if (status != hipSuccess) return status;
         ctx->lds_raised[slot] = true;
     }
-    return launch(ctx, q4_gemm_pipe_kernel<128, 4, true, true>, grid, dim3(256), bytes, p);
+    return launch(ctx, q4_gemm_pipe_kernel<128, 4, true, true>, grid, dim3(256), bytes, group);
 }
 
 // Adds the K splits of a launch's targets.
 static hipError_t launch_reduce(mi355q_context *ctx, GemmGroup &group)
 {
     bool wide = true;
-    for (uint32_t t = 0; t < group.targets; ++t) wide = wide && group.target[t].wide_stores;
+    for (uint32_t t = 0; t < group.shared.targets; ++t) wide = wide && group.target[t].wide_stores;
     const uint32_t columns = kReduceThreads * (wide ? 4u : 1u);
-    uint32_t blocks = 0;
-    for (uint32_t t = 0; t < group.targets; ++t) {
-        group.target[t].first_reduce = blocks;
-        blocks += (group.target[t].N + columns - 1u) / columns;
-    }
     const GemmParams &p = group.shared;
+    uint32_t blocks = 0;
+    for (uint32_t t = 0; t < group.shared.targets; ++t) {
+        group.target[t].first_reduce = blocks;
+        if (p.units != 0u || group.target[t].splits > 1u) blocks += (group.target[t].N + columns - 1u) / columns;
+    }
     const uint32_t rows = p.pair ? p.M / 2u : p.M;
     const dim3 grid(blocks, std::min(rows, kReduceRows), (rows + kReduceRows - 1u) / kReduceRows);
-    if (group.targets != 1u || p.units != 0u || p.splits > 8u)  // (more than eight: only when forced)
+    if (p.targets != 1u || p.units != 0u || p.splits > 8u)  // (more than eight: only when forced)
         return wide ? launch(ctx, q4_group_reduce_kernel<true>, grid, dim3(kReduceThreads), 0, group)
                     : launch(ctx, q4_group_reduce_kernel<false>, grid, dim3(kReduceThreads), 0, group);
     const GemmTarget &target = group.target[0];
@@ -293,34 +302,42 @@ static int gemm_activations(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t
     return MI355Q_OK;
 }
 
-// One target's parameters as the launches take them.
-static GemmTarget gemm_target(const GemmParams &p)
-{
-    GemmTarget t;
-    memset(&t, 0, sizeof t);
-    t.codes = p.codes;
-    t.meta = p.meta;
-    t.y = p.y;
-    t.residual = p.residual;
-    t.partials = p.partials;
-    t.N = p.N;
-    t.NT = p.NT;
-    t.wide_stores = p.wide_stores;
-    return t;
-}
-
+// The shapes, and what a launch of each is estimated to take: microseconds of a call among others, fitted
+// to timings on this GPU of one weight under every shape and K split (27 weights from 896 x 3584 to
+// 17408 x 5120 at 75 to 4646 rows, ten of them at 17 to 128, six 8-bit weights; 210 to 1130 timings a
+// shape, 4 to 5 % rms).  The shape and split that the estimates choose takes 0.7 % longer than the best
+// timed one on average, 11 % at most (estimates that left out what launches, K splits' second kernels
+// and stores take: 3 %, 26 %).
 struct Variant {
     int bm, ntw, extra;
-    int resident;          // workgroups that fit one compute unit (registers, LDS)
-    double alone, shared;  // fraction of matrix-instruction peak, one / several per CU
-    double step_us;        // pipelined kernel: measured time of one 128-column step, chip full
+    int resident;           // workgroups that fit one compute unit (registers, LDS)
+    double launch;          // once
+    double step, fill;      // a chip full of workgroups: each 128-column step, and once
+    // First kernel: the same of a chip with at most k + 1 workgroups on a compute unit, which the
+    // last workgroups are.  Pipelined kernel, whose last round of workgroups takes the fraction r of
+    // the compute units: {step, + max(0, r - 0.5) of each step}, {fill, + r^2} (the chip is power
+    // limited, and up to about half of it the clock stays near its maximum).
+    double part_step[4], part_fill[4];
+    double split, per_split, sums;  // a K split: its second kernel, more for each split, MB of partial sums
+    double outputs;         // MB of outputs
+    double converted[3];    // activations that are not fp16: once, MB of fp16 rows, MB of outputs
+    double reread;          // MB of fp16 rows beyond an XCD's L2, by each block of tiles
 };
 static const Variant variants[] = {
-    {128, 4, 0, 2, 0.399, 0.491, 0.0}, {128, 2, 0, 2, 0.327, 0.434, 0.0}, {64, 4, 0, 3, 0.333, 0.460, 0.0},
-    {64, 4, 1, 2, 0.347, 0.444, 0.0},  {64, 2, 0, 4, 0.288, 0.422, 0.0},  {64, 2, 1, 2, 0.308, 0.443, 0.0},
-    {128, 4, 0, 1, 0.0, 0.0, 1.493}, {128, 4, 1, 1, 0.0, 0.0, 1.675}, {128, 5, 0, 1, 0.0, 0.0, 1.849},
-    {128, 4, 0, 1, 0.0, 0.0, 1.60}, {128, 3, 1, 1, 0.0, 0.0, 1.40}};  // 9, 10: 16 and 13 tiles on 8-bit codes, and only for them
-constexpr int kBytesVariant = 9;  // the first of them
+    {128, 4, 0, 2, 13.19, 3.208, 5.98, {2.167, 3.026}, {0.0, 1.16}, 0.0, 0.0, 0.192, 0.435, {2.27, 0.36, 0.0}, 0.000},
+    {128, 2, 0, 2, 5.82, 1.628, 0.0, {1.207, 1.595}, {0.0, 0.010}, 2.52, 0.0, 0.304, 0.474, {5.72, 0.40, 0.046}, 0.007},
+    {64, 4, 0, 3, 5.54, 2.755, 0.0, {1.175, 1.820, 2.868}, {0.53, 0.0, 0.0}, 2.60, 0.0, 0.262, 0.566, {5.81, 0.27, 0.0}, 0.000},
+    {64, 4, 1, 2, 8.64, 2.275, 0.0, {1.366, 2.151}, {0.037, 0.0}, 1.82, 0.0, 0.250, 0.206, {3.96, 0.29, 0.31}, 0.002},
+    {64, 2, 0, 4, 4.16, 1.831, 0.0, {0.711, 1.054, 1.516, 1.972}, {0.41, 1.14, 0.61, 0.0}, 2.52, 0.0, 0.280, 0.498, {4.84, 0.37, 0.0}, 0.003},
+    {64, 2, 1, 2, 4.99, 1.240, 0.0, {0.918, 1.294}, {0.0, 0.21}, 2.46, 0.0, 0.279, 0.524, {4.76, 0.36, 0.21}, 0.000},
+    {128, 4, 0, 1, 4.51, 1.363, 5.31, {1.107, 0.117}, {3.93, 2.92}, 2.48, 0.24, 0.207, 0.325, {5.48, 0.18, 0.50}, 0.014},
+    {128, 4, 1, 1, 6.29, 1.545, 6.04, {1.260, 0.291}, {3.64, 1.55}, 2.40, 0.32, 0.182, 0.355, {5.22, 0.19, 0.56}, 0.011},
+    {128, 5, 0, 1, 1.25, 1.747, 6.38, {1.368, 0.627}, {9.07, 0.22}, 2.98, 0.28, 0.175, 0.363, {5.14, 0.23, 0.50}, 0.003},
+    // 16 and 13 tiles on 8-bit codes, and only for them
+    {128, 4, 0, 1, 0.88, 1.544, 9.49, {1.249, 0.535}, {5.21, 6.69}, 4.14, 0.10, 0.172, 0.031, {0.0, 0.0, 0.0}, 0.000},
+    {128, 3, 1, 1, 5.81, 1.436, 6.56, {1.144, 0.482}, {0.0, 4.74}, 4.30, 0.14, 0.208, 0.054, {0.0, 0.0, 0.0}, 0.000}};
+constexpr int kFirstPiped = 6;    // the first shape of the pipelined kernel
+constexpr int kBytesVariant = 9;  // the first on 8-bit codes
 
 // the pipelined kernel addresses x with 32-bit byte offsets and whole 128-column steps
 static bool gemm_pipe_ok(const Q4Device &w, uint32_t rows, uint32_t x_columns)
@@ -335,10 +352,120 @@ struct TargetPlan {
     uint32_t splits;
     double us;        // the estimate
 };
+// One launch as the estimates see it: what each target gives it.
+struct LaunchWork {
+    uint32_t count;
+    uint32_t steps[kMaxTargets];   // of a workgroup
+    uint64_t groups[kMaxTargets];
+    uint32_t splits;               // the most of one target
+    double sums, outputs, reread;  // MB
+    double rows;                   // MB of fp16 rows
+    bool converted;
+};
+static void add_work(LaunchWork &work, const Variant &c, const Q4LinearArgs &a, const Q4Device &w, uint32_t T, uint32_t rows,
+                     uint32_t want_splits)
+{
+    const uint32_t tpb = 4u * c.ntw + c.extra, t = work.count++;
+    work.steps[t] = (T + want_splits - 1) / want_splits;
+    const uint32_t splits = (T + work.steps[t] - 1) / work.steps[t];
+    work.groups[t] = (uint64_t)((w.NT + tpb - 1) / tpb) * ((rows + c.bm - 1) / c.bm) * splits;
+    work.splits = std::max(work.splits, splits);
+    if (splits > 1u) work.sums += (double)splits * rows * w.N * 4e-6;
+    work.outputs += (double)a.M * w.N * dtype_bytes(a.y_dtype) * 1e-6;
+    work.converted = a.x_dtype != MI355Q_F16;
+    work.rows = (double)rows * w.K * sizeof(_Float16) * 1e-6;
+    work.reread += std::max(work.rows - 4.0, 0.0) * ((w.NT + tpb - 1) / tpb);
+}
+
+// Microseconds of the matrix kernel: full rounds of the chip, then what is left.
+static double first_kernel_us(const Variant &c, uint32_t cus, const LaunchWork &work)
+{
+    uint64_t groups = 0, steps = 0;
+    for (uint32_t t = 0; t < work.count; ++t) {
+        groups += work.groups[t];
+        steps += work.groups[t] * work.steps[t];
+    }
+    const double each = (double)steps / (double)groups;
+    const uint64_t slots = (uint64_t)cus * c.resident, rest = groups % slots;
+    double us = (double)(groups / slots) * (each * c.step + c.fill);
+    if (rest != 0u) {
+        const uint64_t k = (rest + cus - 1u) / cus - 1u;
+        us += each * c.part_step[k] + c.part_fill[k];
+    }
+    return us;
+}
+
+// One workgroup per compute unit: the workgroups take the compute units as they come free, the longest
+// first.
+static double pipe_kernel_us(const Variant &c, uint32_t cus, const LaunchWork &work)
+{
+    uint32_t order[kMaxTargets] = {0, 1, 2, 3};
+    std::stable_sort(order, order + work.count, [&](uint32_t l, uint32_t r) { return work.steps[l] > work.steps[r]; });
+    struct Level {
+        double at;  // so many compute units are free from here on
+        uint64_t units;
+    } level[kMaxTargets + 2];  // a target adds at most one
+    int levels = 1;
+    level[0] = {0.0, cus};
+    uint64_t groups = 0, steps = 0;
+    for (uint32_t i = 0; i < work.count; ++i) {
+        const double time = c.fill + (double)work.steps[order[i]] * c.step;
+        uint64_t left = work.groups[order[i]];
+        groups += left;
+        steps += left * work.steps[order[i]];
+        while (left > 0u) {
+            if (levels == 1 && left >= cus) {  // whole rounds
+                level[0].at += time * (double)(left / cus);
+                left %= cus;
+                continue;
+            }
+            const uint64_t taken = std::min(left, level[0].units);  // those that are free first
+            const Level busy = {level[0].at + time, taken};
+            left -= taken;
+            level[0].units -= taken;
+            if (level[0].units == 0u) {
+                for (int l = 1; l < levels; ++l) level[l - 1] = level[l];
+                --levels;
+            }
+            int at = levels;
+            while (at > 0 && level[at - 1].at > busy.at + 1e-9) --at;
+            if (at > 0 && level[at - 1].at > busy.at - 1e-9) {
+                level[at - 1].units += taken;
+            } else {
+                for (int l = levels; l > at; --l) level[l] = level[l - 1];
+                level[at] = busy;
+                ++levels;
+            }
+        }
+    }
+    double us = level[0].at, busy = 0.0;  // busy: of all compute units together, from the first one's end on
+    for (int l = 0; l < levels; ++l) busy += (level[l].at - level[0].at) * (double)level[l].units;
+    const double rest = level[levels - 1].at - level[0].at;
+    if (rest > 0.0) {
+        const double r = busy / (rest * cus), each = (double)steps / (double)groups;
+        us += rest * (each * (c.part_step[0] + c.part_step[1] * std::max(0.0, r - 0.5)) + c.part_fill[0] + c.part_fill[1] * r * r) /
+              (each * c.step + c.fill);
+    }
+    return us;
+}
+
+static double launch_us(int variant, uint32_t cus, const LaunchWork &work)
+{
+    const Variant &c = variants[variant];
+    double us = c.launch + (variant >= kFirstPiped ? pipe_kernel_us(c, cus, work) : first_kernel_us(c, cus, work));
+    if (work.splits > 1u) us += c.split + c.per_split * work.splits + c.sums * work.sums;
+    if (work.converted) us += c.converted[0] + c.converted[1] * work.rows + c.converted[2] * work.outputs;
+    return us + c.outputs * work.outputs + c.reread * work.reread;
+}
+
+// A target splits K the same way in company as alone, and two weights that each take more than half of
+// the chip without a split fill it together: such a weight splits only where that gains 12 % (17408 x 5120 at
+// 200 rows 54.3 instead of 51.7 us; a pair of them 81 instead of 101).
+constexpr double kSplitWeight = 1.12;
 static TargetPlan plan_target(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, uint32_t rows)
 {
     const Q4Device &w = *a.targets[target].w;
-    const uint32_t x_columns = a.x_columns ? a.x_columns : w.K, NT = w.NT;
+    const uint32_t x_columns = a.x_columns ? a.x_columns : w.K;
     // The doubled form of an 8-bit weight whose activation row the kernels would read twice: the
     // kernel for 8-bit codes reads the bytes themselves instead, one pass over the row, half the
     // matrix instructions.  It is the pipelined kernel, with that kernel's conditions.
@@ -347,155 +474,181 @@ static TargetPlan plan_target(mi355q_context *ctx, const Q4LinearArgs &a, uint32
     const uint32_t T = bytes ? w.T / 2u : w.T;
     const bool pipe_ok = gemm_pipe_ok(w, rows, x_columns);
     TargetPlan best = {bytes, 0, 1, 1e30};
+    double best_weighed = 1e30;
     // Decomposition: BM rows x (4*NTW + EXTRA) tiles per workgroup, K split in `splits`.
-    // The choice minimises a microsecond estimate fitted to sweeps over every variant
-    // and split on this GPU.  Kernels 0-5: a workgroup that has a compute unit to itself
-    // sustains `alone` of the matrix-instruction peak, co-resident workgroups `shared`
-    // together; a grid that is not a whole number of resident sets pays ~0.3 of a workgroup
-    // time for its ragged end.  The pipelined kernel (6, 7, 8; one workgroup per compute unit)
-    // runs in rounds of `step_us` per 128-column step; a round that does not fill the chip is
-    // shorter (partial_round).  A K split pays for writing its fp32
-    // partials and for the kernel that adds them.
-    // A round of the pipelined kernel that fills only the fraction r of the compute units runs
-    // faster than a full one: the chip is power limited, and up to about half of it the clock
-    // stays near its maximum, from there it falls to the sustained clock of a full chip
-    // (fitted, like the other figures here, to interleaved timings of every variant and split
-    // at M = 128 .. 4096 on the 27B shapes: 3 % rms over 78 timings of the pipelined variants).
-    auto partial_round = [](double r) {
-        const double over = (1.0 - r) / 0.438;
-        return r <= 0.562 ? 0.771 - 0.081 * r / 0.562 : 1.0 - 0.31 * over * over;
-    };
     const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
+    const bool half_filled = (uint64_t)((w.NT + 15u) / 16u) * ((rows + 127u) / 128u) * 2u > cus;  // in blocks of 128 rows x 16 tiles
     for (int v = 0; v < (int)(sizeof variants / sizeof variants[0]); ++v) {
-        if (v >= 6 && !pipe_ok) continue;
+        if (v >= kFirstPiped && !pipe_ok) continue;
         if ((v >= kBytesVariant) != bytes) continue;
-        const Variant &c = variants[v];
-        const uint32_t tpb = 4u * c.ntw + c.extra;
-        const uint32_t slots = cus * (uint32_t)c.resident;
-        const uint32_t m_blocks = (rows + c.bm - 1) / c.bm;
-        const uint32_t n_blocks = (NT + tpb - 1) / tpb;
         for (uint32_t want = 1; want <= 8u && want * 8u <= T + 7u; ++want) {
-            const uint32_t steps = (T + want - 1) / want;
-            const uint32_t splits = (T + steps - 1) / steps;
-            const uint64_t groups = (uint64_t)n_blocks * m_blocks * splits;
-            // one workgroup at peak: 64 matrix-instruction cycles per (tile, 16-row
-            // fragment, step) and wave, at 2.4 GHz
-            // (the pipelined kernel spreads its odd tile over the four waves)
-            const double tiles_per_wave = v >= 6 ? c.ntw + 0.25 * c.extra : c.ntw + c.extra;
-            const double peak_us = (double)steps * tiles_per_wave * (c.bm / 16.0) * 64.0 / 2400.0;
-            double cost;
-            if (v >= 6) {
-                // 6.0 us per launch; a round = 5.5 us (fill, and the burst of stores at its end)
-                // plus its steps
-                const uint64_t rest = groups % cus;
-                const double round = 5.5 + (double)steps * c.step_us;
-                cost = 6.0 + round * ((double)(groups / cus) + (rest ? partial_round((double)rest / cus) : 0.0));
+            LaunchWork work = {};
+            add_work(work, variants[v], a, w, T, rows, want);
+            const double us = launch_us(v, cus, work), weighed = us * (want > 1u && half_filled ? kSplitWeight : 1.0);
+            if (weighed < best_weighed) {
+                best_weighed = weighed;
+                best = {bytes, v, want, us};
             }
-            else if (groups <= cus)
-                cost = peak_us / c.alone;
-            else if (groups <= slots) {
-                // k of the `resident` workgroups a compute unit could hold: in between
-                const double k = (double)((groups + cus - 1) / cus);
-                const double sustained = c.alone + (c.shared - c.alone) * (k - 1.0) / (c.resident - 1.0);
-                cost = k * peak_us / sustained;
-            }
-            else
-                cost = ((double)groups / slots + (groups % slots ? 0.31 : 0.0)) * c.resident * peak_us / c.shared;
-            if (splits > 1)  // fp32 partials at 4.6 TB/s and the kernel that adds them
-                cost += (double)splits * rows * (double)w.N * 4.0 / 4.63e6 + (v >= 6 ? 2.0 : 6.3);
-            if (cost < best.us) best = {bytes, v, splits, cost};
         }
     }
     // option "q4_gemm" = "VARIANT,SPLITS" for experiments
     if (ctx->force_gemm[1] >= 1 && ctx->force_gemm[0] < (int)(sizeof variants / sizeof variants[0]) &&
-        (ctx->force_gemm[0] < 6 || pipe_ok) && (ctx->force_gemm[0] >= kBytesVariant) == bytes) {
+        (ctx->force_gemm[0] < kFirstPiped || pipe_ok) && (ctx->force_gemm[0] >= kBytesVariant) == bytes) {
         best.variant = ctx->force_gemm[0];
         best.splits = (uint32_t)ctx->force_gemm[1];
     }
     return best;
 }
 
-static int gemm_one_target(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, const TargetPlan &plan,
-                           char *error, size_t error_capacity)
+// How a call's targets go out: as one launch of one shape, or each by its own plan (variant -1).  In one
+// launch, too, each has the K split of its own plan, and so its own call's bits.
+struct CallPlan {
+    int variant;
+    double us;
+};
+static CallPlan plan_call(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows, const TargetPlan *plans)
 {
-    const Q4Device &w = *a.targets[target].w;
-    GemmParams p;
-    memset(&p, 0, sizeof p);
-    p.codes = w.codes;
-    p.meta = w.meta16;  // fp16 {scale, bias}: the weight is evaluated in fp16 here
-    if (a.x_columns != 0 && (a.x_columns * 2u != w.K || a.x_columns % kStepColumns != 0)) {
+    CallPlan best = {-1, 0.0};
+    bool alike = a.count > 1u;
+    for (uint32_t t = 0; t < a.count; ++t) {
+        best.us += plans[t].us;
+        if (t != 0u && a.x_dtype != MI355Q_F16) {  // one conversion serves them all
+            const Variant &c = variants[plans[t].variant];
+            best.us -= c.converted[0] + c.converted[1] * (double)rows * a.targets[t].w->K * sizeof(_Float16) * 1e-6;
+        }
+        alike = alike && plans[t].bytes == plans[0].bytes;
+    }
+    if (!alike) return best;
+    if (ctx->force_gemm[1] >= 1) {
+        if (plans[0].variant == ctx->force_gemm[0]) best.variant = plans[0].variant;
+        return best;
+    }
+    const double alone_us = best.us;
+    const Q4Device &first = *a.targets[0].w;
+    const bool bytes = plans[0].bytes, pipe_ok = gemm_pipe_ok(first, rows, a.x_columns ? a.x_columns : first.K);
+    const uint32_t T = bytes ? first.T / 2u : first.T, cus = (uint32_t)ctx->props.multiProcessorCount;
+    for (int v = 0; v < (int)(sizeof variants / sizeof variants[0]); ++v) {
+        if ((v >= kFirstPiped && !pipe_ok) || (v >= kBytesVariant) != bytes) continue;
+        LaunchWork work = {};
+        for (uint32_t t = 0; t < a.count; ++t) add_work(work, variants[v], a, *a.targets[t].w, T, rows, plans[t].splits);
+        const double us = launch_us(v, cus, work);
+        if (us < 0.95 * alone_us && us < best.us) best = {v, us};
+    }
+    return best;
+}
+
+// Targets first .. first + count - 1 of a call in one launch: the shape `variant`, each target with the
+// K split of its own plan.
+static int gemm_targets(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t first, uint32_t count, const TargetPlan *plans,
+                        int variant, char *error, size_t error_capacity)
+{
+    const Q4Device &shape = *a.targets[first].w;  // columns and kind are the same for all
+    const bool bytes_kernel = plans[first].bytes;
+    if (a.x_columns != 0 && (a.x_columns * 2u != shape.K || a.x_columns % kStepColumns != 0)) {
         set_error(error, error_capacity, "q4 gemm: a repeated activation row is half the weight's columns, whole 128-column steps");
         return MI355Q_ERROR_INVALID;
     }
-    const uint32_t x_columns = a.x_columns ? a.x_columns : w.K;
-    int status = gemm_activations(ctx, a, x_columns, target == 0, p, error, error_capacity);
+    const uint32_t x_columns = a.x_columns ? a.x_columns : shape.K;
+    GemmGroup group;
+    memset(&group, 0, sizeof group);
+    GemmParams &p = group.shared;
+    int status = gemm_activations(ctx, a, x_columns, first == 0, p, error, error_capacity);
     if (status != MI355Q_OK) return status;
-    const uint32_t rows = p.M;
-    const uint32_t T = plan.bytes ? w.T / 2u : w.T;
-    if (plan.bytes) {
-        p.codes = w.codes8;
-        p.meta = w.meta8;
-    }
-    p.y = a.targets[target].y;
-    p.residual = a.targets[target].residual;
-    p.N = w.N;
+    const Variant &chosen = variants[variant];
+    const uint32_t tpb = 4u * chosen.ntw + chosen.extra;
+    const uint32_t rows = p.M, m_blocks = (rows + chosen.bm - 1) / chosen.bm;
     p.K = x_columns;
-    p.wrap_steps = a.x_columns && !plan.bytes ? a.x_columns / kStepColumns : 0xffffffffu;
-    p.NT = w.NT;
-    p.T = T;
+    p.T = bytes_kernel ? shape.T / 2u : shape.T;
+    p.wrap_steps = a.x_columns && !bytes_kernel ? a.x_columns / kStepColumns : 0xffffffffu;
     p.y_dtype = a.y_dtype;
     p.residual_dtype = a.residual_dtype;
     p.residual_is_bias = a.residual_is_bias;
-    p.wide_stores = w.N % 4u == 0u && (uintptr_t)p.y % 16u == 0u;
-
-    if (ctx->trace)
-        fprintf(stderr, "mi355q: q4 gemm M=%u N=%u K=%u -> variant %d (BM=%d, %d tiles/wave%s%s), K split %u\n",
-                rows, w.N, w.K, plan.variant, variants[plan.variant].bm, variants[plan.variant].ntw,
-                variants[plan.variant].extra ? " +1" : "", plan.bytes ? ", 8-bit codes" : "", plan.splits);
-    const Variant &chosen = variants[plan.variant];
-    const uint32_t tpb = 4u * chosen.ntw + chosen.extra;
     p.tiles_per_block = tpb;
-    const uint32_t n_blocks = (w.NT + tpb - 1) / tpb;
-    const uint32_t m_blocks = (rows + chosen.bm - 1) / chosen.bm;
-    p.steps_per_split = (T + plan.splits - 1) / plan.splits;
-    p.splits = (T + p.steps_per_split - 1) / p.steps_per_split;
-    if (p.splits > 1u) {
-        const size_t bytes = (size_t)p.splits * rows * padded_columns(w.N) * sizeof(float);
-        status = ensure_stage(ctx, 4, bytes, error, error_capacity);
-        if (status != MI355Q_OK) return status;
-        p.partials = (float *)ctx->stage[4];
+    p.targets = count;
+    size_t sums = 0;  // floats of partial sums
+    bool split = false;
+    for (uint32_t t = 0; t < count; ++t) {
+        const Q4Device &w = *a.targets[first + t].w;
+        GemmTarget &target = group.target[t];
+        target.codes = bytes_kernel ? w.codes8 : w.codes;
+        target.meta = bytes_kernel ? w.meta8 : w.meta16;  // fp16 {scale, bias}: the weight is evaluated in fp16 here
+        target.y = a.targets[first + t].y;
+        target.residual = a.targets[first + t].residual;
+        target.N = w.N;
+        target.NT = w.NT;
+        target.wide_stores = w.N % 4u == 0u && (uintptr_t)target.y % 16u == 0u;
+        target.steps_per_split = (p.T + plans[first + t].splits - 1) / plans[first + t].splits;
+        target.splits = (p.T + target.steps_per_split - 1) / target.steps_per_split;
+        if (target.splits > 1u) {
+            split = true;
+            sums += (size_t)target.splits * rows * padded_columns(w.N);
+        }
+        if (ctx->trace)
+            fprintf(stderr, "mi355q: q4 gemm M=%u N=%u K=%u -> variant %d (BM=%d, %d tiles/wave%s%s), K split %u%s\n",
+                    rows, w.N, w.K, variant, chosen.bm, chosen.ntw, chosen.extra ? " +1" : "",
+                    bytes_kernel ? ", 8-bit codes" : "", target.splits, t ? ", same launch" : "");
     }
-    // Workgroups go to the XCDs in turn: when the number of tile blocks is a multiple of eight, the
-    // row blocks of one tile block already meet on one XCD and read their weights through one L2;
-    // otherwise the pipelined kernel renumbers its blocks so that they do (2-3 % on the 100-block
-    // 8-bit gate, about 1 % on the 20-block down projection, nothing or slightly worse where the
-    // launch order was already right).  With K splits the renumbering also gives every XCD one
-    // split's columns of the activations instead of all of them (down at M = 512: 193 -> 86 MB
-    // fetched, 0.7 % faster).
-    p.xcd_order = ctx->gemm_order >= 0 ? ctx->gemm_order
-                                       : ((n_blocks % 8u != 0u && m_blocks > 1u) || p.splits > 1u ? 1 : 0);
-    const dim3 grid(n_blocks, m_blocks, p.splits);
+    if (split) {
+        status = ensure_stage(ctx, 4, sums * sizeof(float), error, error_capacity);
+        if (status != MI355Q_OK) return status;
+    }
+    // the longest first: what is left to start late is short
+    std::stable_sort(group.target, group.target + count,
+                     [](const GemmTarget &l, const GemmTarget &r) { return l.steps_per_split > r.steps_per_split; });
+    float *partials = (float *)ctx->stage[4];
+    uint32_t blocks = 0;
+    for (uint32_t t = 0; t < count; ++t) {
+        GemmTarget &target = group.target[t];
+        const uint32_t n_blocks = (target.NT + tpb - 1) / tpb;
+        target.first_block = blocks;
+        blocks += (n_blocks * m_blocks * target.splits + 7u) / 8u * 8u;
+        if (target.splits > 1u) {
+            target.partials = partials;
+            partials += (size_t)target.splits * rows * padded_columns(target.N);
+        }
+    }
+    dim3 grid(blocks);
+    if (count == 1u) {
+        const GemmTarget &target = group.target[0];
+        p.codes = target.codes;
+        p.meta = target.meta;
+        p.y = target.y;
+        p.residual = target.residual;
+        p.partials = target.partials;
+        p.N = target.N;
+        p.NT = target.NT;
+        p.wide_stores = target.wide_stores;
+        p.splits = target.splits;
+        p.steps_per_split = target.steps_per_split;
+        // Workgroups go to the XCDs in turn: when the number of tile blocks is a multiple of eight, the
+        // row blocks of one tile block already meet on one XCD and read their weights through one L2;
+        // otherwise the pipelined kernel renumbers its blocks so that they do (2-3 % on the 100-block
+        // 8-bit gate, about 1 % on the 20-block down projection, nothing or slightly worse where the
+        // launch order was already right).  With K splits the renumbering also gives every XCD one
+        // split's columns of the activations instead of all of them (down at M = 512: 193 -> 86 MB
+        // fetched, 0.7 % faster).
+        const uint32_t n_blocks = (target.NT + tpb - 1) / tpb;
+        p.xcd_order = ctx->gemm_order >= 0 ? ctx->gemm_order
+                                           : ((n_blocks % 8u != 0u && m_blocks > 1u) || p.splits > 1u ? 1 : 0);
+        grid = dim3(n_blocks, m_blocks, p.splits);
+    }
     hipError_t launched = hipErrorInvalidValue;
-    switch (plan.variant) {
-    case 0: launched = launch_gemm<128, 4, false>(ctx, grid, p); break;
-    case 1: launched = launch_gemm<128, 2, false>(ctx, grid, p); break;
-    case 2: launched = launch_gemm<64, 4, false>(ctx, grid, p); break;
-    case 3: launched = launch_gemm<64, 4, true>(ctx, grid, p); break;
-    case 4: launched = launch_gemm<64, 2, false>(ctx, grid, p); break;
-    case 5: launched = launch_gemm<64, 2, true>(ctx, grid, p); break;
-    case 6: launched = launch_pipe<4, false>(ctx, grid, p); break;
-    case 7: launched = ctx->gemm_plain_loads ? launch_pipe_plain(ctx, grid, p) : launch_pipe<4, true>(ctx, grid, p); break;
-    case 8: launched = launch_pipe<5, false>(ctx, grid, p); break;
-    case 9: launched = launch_pipe_bytes<4, false>(ctx, grid, p); break;
-    default: launched = launch_pipe_bytes<3, true>(ctx, grid, p); break;
+    switch (variant) {
+    case 0: launched = launch_gemm<128, 4, false>(ctx, grid, group); break;
+    case 1: launched = launch_gemm<128, 2, false>(ctx, grid, group); break;
+    case 2: launched = launch_gemm<64, 4, false>(ctx, grid, group); break;
+    case 3: launched = launch_gemm<64, 4, true>(ctx, grid, group); break;
+    case 4: launched = launch_gemm<64, 2, false>(ctx, grid, group); break;
+    case 5: launched = launch_gemm<64, 2, true>(ctx, grid, group); break;
+    case 6: launched = launch_pipe<4, false>(ctx, grid, group); break;
+    case 7: launched = ctx->gemm_plain_loads ? launch_pipe_plain(ctx, grid, group) : launch_pipe<4, true>(ctx, grid, group); break;
+    case 8: launched = launch_pipe<5, false>(ctx, grid, group); break;
+    case 9: launched = launch_pipe_bytes<4, false>(ctx, grid, group); break;
+    default: launched = launch_pipe_bytes<3, true>(ctx, grid, group); break;
     }
     if (launched != hipSuccess)
         return fail_hip(launched, "q4 gemm kernel launch", error, error_capacity);
-    if (p.splits > 1u) {
-        GemmGroup group;
-        group.shared = p;
-        group.targets = 1;
-        group.target[0] = gemm_target(p);
+    if (split) {
         launched = launch_reduce(ctx, group);
         if (launched != hipSuccess)
             return fail_hip(launched, "q4 gemm reduce launch", error, error_capacity);
@@ -512,22 +665,22 @@ struct RowsPlan {
 
 // The launch of q4_rows_kernel for a call's targets together; false: not the kernel for it.
 // `others`: what each target would take otherwise.
-// Shape and workgroups minimise a microsecond estimate fitted to 1430 timings on this GPU (three
-// layer shapes, 17 to 128 rows, every block width, whole blocks and 128 to 768 workgroups; 8 % rms,
-// the choice within 8 % of the best timed one in 82 of 84 calls): 4.4 us, then per unit the longer
-// of one workgroup's own chain (0.22 + 0.12 us per 16 rows) and its share of the compute unit,
-// then, where workgroups share blocks, 3.7 us and the partial sums at 2.1 TB/s.
+// Shape and workgroups minimise a microsecond estimate fitted to 2100 timings on this GPU (14 calls
+// from 1024 x 3584 to two weights of 17408 x 5120, 17 to 128 rows, every block width, whole blocks
+// and 128 to 512 workgroups; 6 % rms): 5.2 us, 0.02 for each MB of weights, then per unit the longer of one
+// workgroup's own chain (0.26 + 0.11 us per 16 rows) and its share of the compute unit, then, where
+// workgroups share blocks, 2.9 us and the partial sums at 2 TB/s.
 //
-// Chosen where that is at most 1 us per target more than the other kernels' estimate, which leaves
-// out the launches behind a K split (27B shapes: gate|up up to 128 rows, 49 -> 33 us at 32, 82 -> 49
-// at 80, 77 -> 65 at 128; q|k|v 40 -> 14, 49 -> 23, 52 -> 30).  A call of one weight saves no launch, and
-// both estimates leave out what reading a large one takes: for each MB beyond 20 MB 0.1 us is added to
-// this kernel's and, where two row blocks read it, 0.04 to the other's (twelve weights, 17 to 128
-// rows, each in HBM and in the Infinity Cache).  This kernel against the other, us from HBM (the
-// cache): 17408 x 5120 at 32 rows 23.8 (23.6) and 23.3 (21.3), not chosen, at 80 rows 35.1 (34.5)
-// and 39.8 (37.5), chosen; 5120 x 17408 at 32 rows 23.0 (23.2) and 26.7 (22.7), chosen, at 96 rows
-// 38.9 (37.6) and 37.2 (32.8), not chosen.
-static bool rows_plan(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows, const TargetPlan *others, RowsPlan &plan)
+// Chosen where that is less than the other kernels' estimate (one weight), or less than 1.08 times it and
+// 1 us (several: theirs for small and for large calls of several weights is that much too low; us, this
+// kernel and the other: 2048 + 512 + 512 x 1024 at 48 rows 8.0 and 10.0, two of 17408 x 5120 at 64 rows 41 and
+// 50, two of 8192 x 3072 at 48 rows 17.7 and 19.7).  One weight of more than 20 MB, from HBM (the Infinity
+// Cache), this kernel and the other: 17408 x 5120 at 32 rows 24.4 (23.5) and 23.5 (21.3), not chosen, at
+// 80 rows 34.8 (33.1) and 33.0 (31.9), chosen all the same; 5120 x 17408 at 32 rows 23.3 (23.3) and 27.1
+// (23.2), chosen, at 96 rows 34.7 (34.8) and 36.5 (34.0), not chosen; 14336 x 5376 at 32 rows 23.2 (22.1) and
+// 20.9 (19.6), not chosen.
+static bool rows_plan(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows, double others_us, int other_variant,
+                      RowsPlan &plan)
 {
     const Q4Device &first = *a.targets[0].w;
     const uint32_t T = first.T;
@@ -553,8 +706,11 @@ static bool rows_plan(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows,
         return true;
     }
     const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
-    double outputs = 0.0, best_cost = 1e30;
-    for (uint32_t t = 0; t < a.count; ++t) outputs += (double)rows * a.targets[t].w->N;
+    double outputs = 0.0, megabytes = 0.0, best_cost = 1e30;  // megabytes: 4-bit codes and their metadata
+    for (uint32_t t = 0; t < a.count; ++t) {
+        outputs += (double)rows * a.targets[t].w->N;
+        megabytes += (double)a.targets[t].w->N * first.K * 0.5625e-6;
+    }
     RowsPlan best = plan;
     for (int which = 0; which < 3; ++which) {
         if (!shape(which)) return false;
@@ -567,10 +723,10 @@ static bool rows_plan(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows,
             const uint32_t together = std::min(places, (groups + cus - 1u) / cus);
             const uint32_t rounds = (groups + cus * together - 1u) / (cus * together);
             const double tiles = plan.waves * plan.ntw, mf = plan.mf;
-            const double alone = 0.222 + 0.119 * mf, sharing = together * (tiles * (0.0344 + 0.0075 * mf) + 0.0282 * mf);
-            double cost = 4.4 + (double)rounds * plan.units * (alone > sharing ? alone : sharing);
+            const double alone = 0.262 + 0.107 * mf, sharing = together * (tiles * (0.0345 + 0.0058 * mf) + 0.0378 * mf);
+            double cost = 5.2 + 0.02 * megabytes + (double)rounds * plan.units * (alone > sharing ? alone : sharing);
             if (plan.units % T != 0u && plan.units < total)
-                cost += 3.7 + 0.466e-6 * 4.0 * outputs * (T + plan.units - 1.0) / plan.units;
+                cost += 2.9 + 2.0e-6 * outputs * (T + plan.units - 1.0) / plan.units;
             if (cost < best_cost) {
                 best_cost = cost;
                 best = plan;
@@ -578,15 +734,14 @@ static bool rows_plan(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows,
         }
     }
     plan = best;
-    double others_us = 0.0;
-    for (uint32_t t = 0; t < a.count; ++t) others_us += others[t].us;
     if (a.count == 1u) {
-        const double megabytes = (double)first.N * first.K * 0.5625e-6;  // 4-bit codes and their metadata
         const double large = std::min(std::max(megabytes - 20.0, 0.0), 30.0);  // (50 MB: the largest measured)
-        best_cost += 0.1 * large;
-        if (rows > (uint32_t)variants[others[0].variant].bm) others_us += 0.04 * large;
+        if (large == 0.0) others_us *= 1.04;  // both estimates' error, and one launch rather than two
+        else if (rows <= 64u) best_cost += 0.03 * large;
+        else if (variants[other_variant].bm > 64) others_us += 0.05 * large;
     }
-    return best_cost <= others_us + 1.0 * a.count;
+    if (a.x_dtype != MI355Q_F16) best_cost += 5.0 + 0.3 * (double)rows * first.K * sizeof(_Float16) * 1e-6;
+    return best_cost <= (a.count == 1u ? others_us : 1.08 * others_us + 1.0);
 }
 
 template <int MF, int NTW, int W>
@@ -640,7 +795,7 @@ static int q4_rows_linears(mi355q_context *ctx, const Q4LinearArgs &a, const Row
     p.units = plan.units;
     p.total_units = plan.blocks * p.T;
     p.block_columns = (uint32_t)(plan.waves * plan.ntw) * kTileRows;
-    group.targets = a.count;
+    p.targets = a.count;
     // blocks are shared unless every workgroup takes whole ones; a block meets at most this many
     const bool sharing = p.units % p.T != 0u && p.units < p.total_units;
     const uint32_t sharers = (p.T - 1u) / p.units + 2u;
@@ -724,9 +879,11 @@ int q4_gemm_linears(mi355q_context *ctx, const Q4LinearArgs &a, char *error, siz
     TargetPlan plans[kMaxTargets];
     for (uint32_t t = 0; t < a.count; ++t) plans[t] = plan_target(ctx, a, t, rows);
     RowsPlan together;
-    if (rows_plan(ctx, a, rows, plans, together)) return q4_rows_linears(ctx, a, together, error, error_capacity);
+    const CallPlan call = plan_call(ctx, a, rows, plans);
+    if (rows_plan(ctx, a, rows, call.us, plans[0].variant, together)) return q4_rows_linears(ctx, a, together, error, error_capacity);
+    if (call.variant >= 0) return gemm_targets(ctx, a, 0, a.count, plans, call.variant, error, error_capacity);
     for (uint32_t t = 0; t < a.count && status == MI355Q_OK; ++t)
-        status = gemm_one_target(ctx, a, t, plans[t], error, error_capacity);
+        status = gemm_targets(ctx, a, t, 1, plans, plans[t].variant, error, error_capacity);
     return status;
 }
 

@@ -13,6 +13,7 @@ namespace mi355q {
 
 
 struct GemmParams {
+    uint32_t targets;   // of the launch (GemmGroup)
     const uint4 *codes;
     const uint2 *meta;
     const _Float16 *x;  // [M][K] fp16
@@ -49,12 +50,12 @@ struct GemmTarget {
     float *partials;
     uint32_t N, NT, first_block;
     uint32_t first_reduce;  // the same for the kernel that adds K splits
+    uint32_t splits, steps_per_split;
     int wide_stores;
 };
 struct GemmGroup {
-    GemmParams shared;  // everything else; its per-target fields are not read
+    GemmParams shared;  // everything else; its per-target fields are read where targets is 1
     GemmTarget target[kMaxTargets];
-    uint32_t targets;
 };
 
 // The parameters of one target.
@@ -70,6 +71,8 @@ __device__ __forceinline__ GemmParams target_params(const GemmGroup &group, cons
     p.NT = target.NT;
     p.wide_stores = target.wide_stores;
     p.first_block = target.first_block;
+    p.splits = target.splits;
+    p.steps_per_split = target.steps_per_split;
     return p;
 }
 // Those of the target that workgroup `block` works on; `block` becomes its number there.
@@ -79,10 +82,56 @@ __device__ __forceinline__ GemmParams select_target(const GemmGroup &group, uint
     uint32_t t = 0;
 #pragma unroll
     for (uint32_t i = 1; i < kMaxTargets; ++i)
-        if (i < group.targets && block >= (REDUCE ? group.target[i].first_reduce : group.target[i].first_block)) t = i;
+        if (i < group.shared.targets && block >= (REDUCE ? group.target[i].first_reduce : group.target[i].first_block)) t = i;
     const GemmTarget &target = group.target[t];
     block -= REDUCE ? target.first_reduce : target.first_block;
     return target_params(group, target);
+}
+
+// Workgroup `index` of `total`, and the XCD it runs on is index % 8: its number when XCD i works
+// through a contiguous run of the numbers, XCDs in turn.  `total` or more: none is left for it.
+__device__ __forceinline__ uint32_t number_by_xcd(uint32_t index, uint32_t total)
+{
+    const uint32_t xcd = index % 8u, base = total / 8u, longer = total % 8u;  // XCDs 0 .. longer-1 get base + 1
+    if (index / 8u >= base + (xcd < longer ? 1u : 0u)) return total;
+    return (xcd < longer ? xcd * (base + 1u) : longer * (base + 1u) + (xcd - longer) * base) + index / 8u;
+}
+
+// The block of the problem that a workgroup of the GEMM kernels takes, and its target's parameters;
+// false: none.  One target has a grid of tile blocks, row blocks and K splits, in launch order
+// or, by xcd_order, so that the row blocks that multiply the same weights meet in one XCD's L2:
+// each XCD works through a contiguous run of the blocks numbered row block fastest, then tile
+// block, then K split.  Several targets share a grid of one dimension: each has a range of it, a multiple
+// of eight workgroups, in which its blocks are numbered that way.
+__device__ __forceinline__ bool locate_block(const GemmGroup &group, uint32_t tiles_per_block, uint32_t rows_per_block,
+                                             GemmParams &p, uint32_t &block_n, uint32_t &block_m, uint32_t &split)
+{
+    p = group.shared;
+    // one target's parameters are asked for with the number of targets: one round trip, not two
+    asm volatile("" ::"s"(p.codes), "s"(p.meta), "s"(p.y), "s"(p.residual), "s"(p.partials), "s"(p.N), "s"(p.NT), "s"(p.splits),
+                 "s"(p.steps_per_split), "s"(p.wide_stores));
+    block_n = blockIdx.x;
+    block_m = blockIdx.y;
+    split = blockIdx.z;
+    uint32_t n_blocks = gridDim.x, m_blocks = gridDim.y, number;
+    if (p.targets > 1u) {
+        uint32_t index = blockIdx.x;
+        p = select_target(group, index);
+        n_blocks = (p.NT + tiles_per_block - 1u) / tiles_per_block;
+        m_blocks = (p.M + rows_per_block - 1u) / rows_per_block;
+        const uint32_t total = n_blocks * m_blocks * p.splits;
+        number = number_by_xcd(index, total);
+        if (number >= total) return false;
+    } else if (p.xcd_order) {
+        number = number_by_xcd(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z),
+                               gridDim.x * gridDim.y * gridDim.z);
+    } else {
+        return true;
+    }
+    block_m = number % m_blocks;
+    block_n = number / m_blocks % n_blocks;
+    split = number / (m_blocks * n_blocks);
+    return true;
 }
 
 __device__ __forceinline__ half8 dequant8(uint32_t word, const NibbleMasks &masks, half8 scale,
@@ -210,7 +259,7 @@ __device__ __forceinline__ int store_mode(const GemmParams &p)
 // 2048 x 2048 at 160 rows 14.1 -> 15.4 us, 8192 x 3200 at 512 rows 40.3 -> 41.5): 62 instead of 39 KB
 // of code, and waits in front of plain stores for loads of the other epilogue.
 template <int BM, int NTW, bool EXTRA, bool CONVERTED>
-__global__ void __launch_bounds__(256, 2) q4_gemm_kernel(const GemmParams p)
+__device__ __forceinline__ void gemm_workgroup(const GemmParams &p, uint32_t block_n, uint32_t block_m, uint32_t split)
 {
     // Activation stage: [buffer][row][slot] of 16-byte pieces, slot = octet ^ (row % 16).
     // It is filled by LDS-direct loads (no registers): one wave instruction brings four
@@ -228,10 +277,9 @@ __global__ void __launch_bounds__(256, 2) q4_gemm_kernel(const GemmParams p)
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t r = lane & 15u;
     const uint32_t kq = lane >> 4;
-    const uint32_t m0 = blockIdx.y * BM;
-    const uint32_t tile0 = blockIdx.x * TPB + wave * NTW;
+    const uint32_t m0 = block_m * BM;
+    const uint32_t tile0 = block_n * TPB + wave * NTW;
     const bool has_extra = EXTRA && wave == 3u;  // its tile index is tile0 + NTW
-    const uint32_t split = blockIdx.z;
     const uint32_t step_begin = split * p.steps_per_split;
     const uint32_t step_end = step_begin + p.steps_per_split < p.T ? step_begin + p.steps_per_split : p.T;
 
@@ -409,6 +457,23 @@ __global__ void __launch_bounds__(256, 2) q4_gemm_kernel(const GemmParams p)
     }
 }
 
+// One weight, and several: the choice of the target in the same kernel made one weight's launches, the
+// smallest most of all, 0.5 to 0.9 us longer (2048 x 1024 at 256 rows 12.0 -> 12.5, 1280 x 1280 at 150
+// fp32 rows 15.1 -> 16.0; the pipelined kernel's did not change).
+template <int BM, int NTW, bool EXTRA, bool CONVERTED>
+__global__ void __launch_bounds__(256, 2) q4_gemm_kernel(const GemmParams p)
+{
+    gemm_workgroup<BM, NTW, EXTRA, CONVERTED>(p, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+template <int BM, int NTW, bool EXTRA, bool CONVERTED>
+__global__ void __launch_bounds__(256, 2) q4_gemm_group_kernel(const GemmGroup group)
+{
+    GemmParams p;
+    uint32_t block_n, block_m, split;
+    if (!locate_block(group, 4 * NTW + (EXTRA ? 1 : 0), BM, p, block_n, block_m, split)) return;
+    gemm_workgroup<BM, NTW, EXTRA, CONVERTED>(p, block_n, block_m, split);
+}
+
 // One of the three dependent instructions that dequantize piece PIECE (tile PIECE/4, weights
 // 2*(PIECE%4) and +1 of a lane's eight) of quarter D: mask-and-merge into an fp16 with the code
 // in its mantissa, subtract the offset, fused multiply-add with the group's {scale, bias}.  They
@@ -574,7 +639,7 @@ __device__ __forceinline__ void load_x2(u32x2 &to, uint32_t lane_offset, const c
 // of a quarter in order), with the same fp16 {scale, bias} records: one code register more per
 // tile and step, the same three vector instructions per pair of weights.
 template <int BM, int NTW, bool XT, bool PLAIN = false, bool Q8 = false>
-__global__ void __launch_bounds__(256, 1) q4_gemm_pipe_kernel(const GemmParams p)
+__global__ void __launch_bounds__(256, 1) q4_gemm_pipe_kernel(const GemmGroup group)
 {
     extern __shared__ uint4 a_lds_raw[];  // [buffer][row][slot], slot = octet ^ (row % 16)
     typedef uint4 (*stage_rows)[16];
@@ -595,21 +660,9 @@ __global__ void __launch_bounds__(256, 1) q4_gemm_pipe_kernel(const GemmParams p
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t r = lane & 15u;
     const uint32_t kq = lane >> 4;
-    // Which block of the problem this workgroup takes.  Workgroups go to the eight XCDs in turn
-    // (workgroup L of the launch to XCD L % 8), and the row blocks that multiply the same weights
-    // should meet in one XCD's L2: with xcd_order, XCD i works through a contiguous run of the
-    // problem's blocks numbered row block fastest, then tile block, then K split.
-    uint32_t block_n = blockIdx.x, block_m = blockIdx.y, split = blockIdx.z;
-    if (p.xcd_order) {
-        const uint32_t total = gridDim.x * gridDim.y * gridDim.z;
-        const uint32_t launch_index = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-        const uint32_t xcd = launch_index % 8u, base = total / 8u, longer = total % 8u;  // XCDs 0 .. longer-1 get base + 1
-        const uint32_t first = xcd < longer ? xcd * (base + 1u) : longer * (base + 1u) + (xcd - longer) * base;
-        const uint32_t number = first + launch_index / 8u;
-        block_m = number % gridDim.y;
-        block_n = number / gridDim.y % gridDim.x;
-        split = number / (gridDim.y * gridDim.x);
-    }
+    GemmParams p;
+    uint32_t block_n, block_m, split;
+    if (!locate_block(group, TPB, BM, p, block_n, block_m, split)) return;
     const uint32_t m0 = block_m * BM;
     const uint32_t block_first_tile = block_n * TPB;
     const uint32_t tile0 = block_first_tile + wave * NTW;

@@ -4,6 +4,6 @@
 
 namespace mi355q {
 
-template __global__ void q4_gemm_pipe_kernel<128, 4, false, false>(const GemmParams);
+template __global__ void q4_gemm_pipe_kernel<128, 4, false, false>(const GemmGroup);
 
 }  // namespace mi355q

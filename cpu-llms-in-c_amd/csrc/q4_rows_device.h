@@ -89,7 +89,7 @@ __global__ void __launch_bounds__(64 * W, 2) q4_rows_kernel(const GemmGroup grou
         uint32_t t = 0;
 #pragma unroll
         for (uint32_t i = 1; i < kMaxTargets; ++i)
-            if (i < group.targets && fetch_block >= group.target[i].first_block) t = i;
+            if (i < group.shared.targets && fetch_block >= group.target[i].first_block) t = i;
         fetch_codes = (const char *)group.target[t].codes;
         fetch_meta = (const char *)group.target[t].meta;
         fetch_NT = group.target[t].NT;

@@ -423,9 +423,10 @@ int mi355q_q4_linear_noalloc(mi355q_context *ctx, const mi355q_q4_weight *weight
  * From there to 128 matrix rows (64 of fp32 x) the targets are one launch too
  * where that is the faster way, and the steps of all of them are divided among
  * its workgroups: the order in which an output's products are added, and so its
- * last bits, may then depend on the other targets of the call.  Above that, and
- * where a target writes what another one reads or writes, they run one after
- * the other with the results of one call each. */
+ * last bits, may then depend on the other targets of the call.  Above that they
+ * have the results of one call each, as one launch where that is the faster way;
+ * where a target writes what another one reads or writes, they run one after the
+ * other with the results of one call each. */
 typedef struct {
     const mi355q_q4_weight *weight;
     void *y;              /* [M][N_t] of y_dtype */

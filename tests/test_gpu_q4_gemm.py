@@ -507,3 +507,41 @@ def test_kernel_of_one_large_weight(engine, gpu, force, capfd, N, K, M, kernel):
     finally:
         weight.destroy()
     assert np.any(y != 0) and ("mi355q: q4 %s M=%d" % (kernel, M)) in printed
+
+
+@pytest.mark.parametrize("forced", [None, "0,1", "1,2", "2,1", "3,3", "4,2", "5,1", "6,1", "6,3", "7,2", "8,1"])
+@pytest.mark.parametrize("x_dtype,y_dtype,M", [("F16", "F16", 130), ("F16", "F32", 257), ("BF16", "BF16", 300), ("F32", "F32", 81)])
+def test_targets_in_one_launch(engine, gpu, force, forced, x_dtype, y_dtype, M):
+    """Weights of one call in one launch of the GEMM kernels: each output has the bits of its weight's
+    own call.  Numbers of blocks that are and are not multiples of eight, ragged last tiles, a width that
+    is no multiple of 4, fewer blocks than XCDs, more weights than one with and without a K split."""
+    K, widths = 3072, (1280, 1002, 64, 100)
+    x32 = make_x(engine, 141, M, K)
+    x = x32 if x_dtype == "F32" else x32.astype(np.float16) if x_dtype == "F16" else bf16_bits(x32).reshape(M, K)
+    kind, x_dtype, y_dtype = engine.META_BF16_PLANES, getattr(engine, x_dtype), getattr(engine, y_dtype)
+    cell = np.uint32 if y_dtype == engine.F32 else np.uint16
+    weights = [gpu.q4_prepare(*engine.synth_q4_affine(142 + i, 0.02, N, K, kind), N, K, kind) for i, N in enumerate(widths)]
+    biases = [gpu.to_device(engine.synth_normal_f32(150 + i, 1.0, N)) for i, N in enumerate(widths)]
+    x_ptr = gpu.to_device(x)
+    outputs = [gpu.alloc(M * N * np.dtype(cell).itemsize) for N in widths]
+    if forced:
+        force("q4_gemm", forced)
+    try:
+        results = []
+        targets = list(zip(weights, outputs, biases))
+        for groups in ([targets[::-1]], [targets[:2], targets[2:]], [[t] for t in targets]):
+            print(f"gemm one launch M={M} x={x_dtype} forced={forced} calls={len(groups)}", flush=True)
+            for pointer, N in zip(outputs, widths):
+                gpu.upload(pointer, np.full((M, N), 0x7FFF, cell))
+            gpu.q4_sequence(engine.make_calls([(g, x_ptr, x_dtype, M, y_dtype, engine.F32, engine.RESIDUAL_IS_BIAS)
+                                               for g in groups]))
+            gpu.sync()
+            results.append([gpu.download(p, (M, N), cell) for p, N in zip(outputs, widths)])
+        for one, two, alone in zip(*results):
+            assert np.any(alone != 0) and not np.any(alone == 0x7FFF)
+            assert np.array_equal(one, alone) and np.array_equal(two, alone)
+    finally:
+        for pointer in [x_ptr] + outputs + biases:
+            gpu.free(pointer)
+        for weight in weights:
+            weight.destroy()
