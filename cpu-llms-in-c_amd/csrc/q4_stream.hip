@@ -125,70 +125,96 @@ __global__ void __launch_bounds__(256) q4_stream_reduce_kernel(const StreamParam
 // whose results the kernel adds (about 22 significant bits relative to the row's maximum).
 // Infinities saturate at the largest fp16 value, NaN stays NaN.
 //
-// Bound by memory (each row is read once from HBM and once more from the compute unit's vector
-// cache).  A thread takes eight adjacent columns at a time, 16- and 32-byte loads and 16-byte
-// stores: with one element per thread and access the 4646 x 5376 bf16 rows of a video clip took
-// 74 us (1.4 TB/s), now 24 us (4.1 TB/s; rows are whole 64-column groups and the entry points take
-// 16-byte aligned activations only).
+// Bound by memory, and for the smaller calls by the chain load, maximum, store.  A row is held in
+// registers between its maximum and its conversion, PIECES times eight adjacent columns a thread with
+// all their 16-byte loads on their way at once; up to 2048 columns a wave takes a row by itself (no
+// barrier), up to 18432 a workgroup of four.  PIECES 0: longer rows are read twice.
+// The stores go past the L2 (what they write is read by other XCDs): left dirty there, it is written
+// back when the kernel ends, and nothing overlaps that.  Kernel time before / held in registers / stored
+// past the L2, us: 1500 rows of 1280 fp32 8.7 / 8.2 / 6.9, of 512 5.4 / 5.0 / 4.3, of 5120 13.1 / 10.9 / 11.0,
+// 150 of 5120 6.2 / 5.7 / 5.1, 4646 of 5376 bf16 19.4 / 16.8 / 16.0 (6.2 TB/s), 1000 of 2752 6.8 / 6.5 / 5.1.
+// Loading past the L2 too: 6.9, 5.2, 14.3, 5.6, 18.8, 5.7.
 constexpr uint32_t kConvertThreads = 256;
-template <bool BF16>
+template <bool BF16, bool WAVE, int PIECES>
 __global__ void __launch_bounds__(kConvertThreads)
 q4_convert_x_kernel(const void *__restrict__ x, _Float16 *__restrict__ out, float *__restrict__ row_scale,
-                    uint32_t K)
+                    uint32_t M, uint32_t K)
 {
-    __shared__ float wave_max[kConvertThreads / 64u];
-    const uint32_t m = blockIdx.x, pieces = K / 8u;
+    constexpr uint32_t kLanes = WAVE ? 64u : kConvertThreads;  // threads of a row
+    typedef std::conditional_t<BF16, u32x4, floatx4> Part;
+    constexpr int PARTS = BF16 ? 1 : 2;  // of a piece
+    struct Piece {
+        Part part[PARTS];
+    };
+    const uint32_t m = WAVE ? blockIdx.x * (kConvertThreads / 64u) + threadIdx.x / 64u : blockIdx.x;
+    if (m >= M) return;  // (a whole wave, and only without a barrier)
+    const uint32_t pieces = K / 8u, first = threadIdx.x % kLanes;
     const size_t row_at = (size_t)m * K;
-    auto load = [&](uint32_t piece, float (&v)[8]) {
-        if constexpr (BF16) {
-            const u32x4 bits = *(const u32x4 *)((const uint16_t *)x + row_at + 8u * piece);
+    const Part *const row = (const Part *)((const char *)x + row_at * (BF16 ? 2u : 4u));
+    auto load = [&](uint32_t piece) {
+        Piece of;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                v[2 * j] = __builtin_bit_cast(float, bits[j] << 16);
-                v[2 * j + 1] = __builtin_bit_cast(float, bits[j] & 0xffff0000u);
-            }
-        } else {
-            const floatx4 *from = (const floatx4 *)((const float *)x + row_at + 8u * piece);
-            const floatx4 low = from[0], high = from[1];
+        for (int i = 0; i < PARTS; ++i) of.part[i] = row[(size_t)piece * PARTS + i];
+        return of;
+    };
+    auto values = [&](const Piece &of, float (&v)[8]) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                v[j] = low[j];
-                v[j + 4] = high[j];
+        for (int j = 0; j < 4; ++j) {
+            if constexpr (BF16) {
+                v[2 * j] = __builtin_bit_cast(float, of.part[0][j] << 16);
+                v[2 * j + 1] = __builtin_bit_cast(float, of.part[0][j] & 0xffff0000u);
+            } else {
+                v[j] = of.part[0][j];
+                v[j + 4] = of.part[PARTS - 1][j];
             }
         }
     };
     float biggest = 0.0f;
-#pragma unroll 4
-    for (uint32_t piece = threadIdx.x; piece < pieces; piece += kConvertThreads) {
+    auto look_at = [&](const Piece &of) {
         float v[8];
-        load(piece, v);
+        values(of, v);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const float magnitude = __builtin_fabsf(v[j]);
             if (magnitude > biggest && magnitude <= 3.4028234e38f) biggest = magnitude;  // finite values only
         }
+    };
+    Piece held[PIECES > 0 ? PIECES : 1];
+    if constexpr (PIECES > 0) {
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {  // past the row's end: its last piece again
+            const uint32_t piece = first + i * kLanes;
+            held[i] = load(piece < pieces ? piece : pieces - 1u);
+        }
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) look_at(held[i]);
+    } else {
+#pragma unroll 4
+        for (uint32_t piece = first; piece < pieces; piece += kLanes) look_at(load(piece));
     }
 #pragma unroll
     for (int offset = 32; offset > 0; offset >>= 1) {
         const float other = __shfl_xor(biggest, offset, 64);
         biggest = other > biggest ? other : biggest;
     }
-    if ((threadIdx.x & 63u) == 0u) wave_max[threadIdx.x >> 6] = biggest;
-    __syncthreads();
-    biggest = wave_max[0];
+    if constexpr (!WAVE) {
+        __shared__ float wave_max[kConvertThreads / 64u];
+        if ((threadIdx.x & 63u) == 0u) wave_max[threadIdx.x >> 6] = biggest;
+        __syncthreads();
+        biggest = wave_max[0];
 #pragma unroll
-    for (uint32_t w = 1; w < kConvertThreads / 64u; ++w) biggest = wave_max[w] > biggest ? wave_max[w] : biggest;
+        for (uint32_t w = 1; w < kConvertThreads / 64u; ++w) biggest = wave_max[w] > biggest ? wave_max[w] : biggest;
+    }
     int exponent = 0;
     (void)__builtin_frexpf(biggest, &exponent);  // biggest = f * 2^exponent, f in [0.5, 1)
     int shift = biggest > 0.0f ? 14 - exponent : 0;
     shift = shift < -126 ? -126 : shift > 126 ? 126 : shift;  // both powers stay normal numbers
     const float forward = __builtin_ldexpf(1.0f, shift), back = __builtin_ldexpf(1.0f, -shift);
-    if (threadIdx.x == 0) row_scale[m] = back;
+    if (first == 0u) row_scale[m] = back;
     const float limit = 65504.0f;
-#pragma unroll 2
-    for (uint32_t piece = threadIdx.x; piece < pieces; piece += kConvertThreads) {
+    auto convert = [&](uint32_t piece, const Piece &of) {
         float v[8];
-        load(piece, v);
+        values(of, v);
         half8 heads, rests;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -199,11 +225,19 @@ q4_convert_x_kernel(const void *__restrict__ x, _Float16 *__restrict__ out, floa
             rests[j] = (_Float16)(rest > limit ? limit : rest < -limit ? -limit : rest);
         }
         if constexpr (BF16) {
-            *(half8 *)(out + row_at + 8u * piece) = heads;
+            __builtin_nontemporal_store(heads, (half8 *)(out + row_at + 8u * piece));
         } else {
-            *(half8 *)(out + 2u * row_at + 8u * piece) = heads;
-            *(half8 *)(out + 2u * row_at + K + 8u * piece) = rests;
+            __builtin_nontemporal_store(heads, (half8 *)(out + 2u * row_at + 8u * piece));
+            __builtin_nontemporal_store(rests, (half8 *)(out + 2u * row_at + K + 8u * piece));
         }
+    };
+    if constexpr (PIECES > 0) {
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i)
+            if (first + i * kLanes < pieces) convert(first + i * kLanes, held[i]);
+    } else {
+#pragma unroll 2
+        for (uint32_t piece = first; piece < pieces; piece += kLanes) convert(piece, load(piece));
     }
 }
 
@@ -413,12 +447,33 @@ StreamShape choose_shape(const mi355q_context *ctx, uint32_t NT_total, uint32_t 
     return shape;
 }
 
+template <bool BF16>
+static hipError_t convert_x_launch(mi355q_context *ctx, const void *x, _Float16 *out, float *row_scale, uint32_t M, uint32_t K)
+{
+    auto rows = [&](auto wave_c, auto pieces_c) {
+        constexpr bool WAVE = decltype(wave_c)::value;
+        constexpr uint32_t kRows = WAVE ? kConvertThreads / 64u : 1u;  // of a workgroup
+        return launch(ctx, q4_convert_x_kernel<BF16, WAVE, decltype(pieces_c)::value>, dim3((M + kRows - 1u) / kRows),
+                      dim3(kConvertThreads), 0, x, out, row_scale, M, K);
+    };
+    typedef std::true_type wave;
+    typedef std::false_type workgroup;
+    if (K <= 512u) return rows(wave(), std::integral_constant<int, 1>());
+    if (K <= 1024u) return rows(wave(), std::integral_constant<int, 2>());
+    if (K <= 1536u) return rows(wave(), std::integral_constant<int, 3>());
+    if (K <= 2048u) return rows(wave(), std::integral_constant<int, 4>());
+    if (K <= 4096u) return rows(workgroup(), std::integral_constant<int, 2>());
+    if (K <= 6144u) return rows(workgroup(), std::integral_constant<int, 3>());
+    if (K <= 8192u) return rows(workgroup(), std::integral_constant<int, 4>());
+    if (K <= 18432u) return rows(workgroup(), std::integral_constant<int, 9>());
+    return rows(workgroup(), std::integral_constant<int, 0>());
+}
+
 hipError_t q4_convert_x_launch(mi355q_context *ctx, const void *x, int x_dtype, _Float16 *out, float *row_scale,
                                uint32_t M, uint32_t K)
 {
-    if (x_dtype == MI355Q_BF16)
-        return launch(ctx, q4_convert_x_kernel<true>, dim3(M), dim3(kConvertThreads), 0, x, out, row_scale, K);
-    return launch(ctx, q4_convert_x_kernel<false>, dim3(M), dim3(kConvertThreads), 0, x, out, row_scale, K);
+    return x_dtype == MI355Q_BF16 ? convert_x_launch<true>(ctx, x, out, row_scale, M, K)
+                                  : convert_x_launch<false>(ctx, x, out, row_scale, M, K);
 }
 
 hipError_t zero_words_launch(mi355q_context *ctx, uint32_t *words, uint32_t count)

@@ -545,3 +545,25 @@ def test_targets_in_one_launch(engine, gpu, force, forced, x_dtype, y_dtype, M):
             gpu.free(pointer)
         for weight in weights:
             weight.destroy()
+
+
+@pytest.mark.parametrize("K", [64, 512, 576, 1024, 1088, 1536, 1600, 2048, 2112, 4096, 4160, 6144, 6208, 8192, 8256, 18432, 18496])
+def test_row_lengths_of_converted_activations(engine, oracle, gpu, K):
+    """The conversion's forms by row length (a wave or a workgroup a row, so many columns a thread, a row
+    read twice): five rows, whose largest value is the first, the last, or stands in the last octet but one."""
+    N, M, kind = 16, 5, engine.META_BF16_PLANES
+    quants, meta_a, meta_b = engine.synth_q4_affine(161, 0.02, N, K, kind)
+    x = make_x(engine, 162, M, K).copy()
+    x[0, 0], x[1, K - 1], x[2, K - 9], x[4] = 1e5, -3e6, 2e5, 0.0
+    weight = gpu.q4_prepare(quants, meta_a, meta_b, N, K, kind)
+    try:
+        print(f"converted rows K={K}", flush=True)
+        y = gpu.q4_linear(weight, x, engine.F32, engine.F32)
+        y_bf = gpu.q4_linear(weight, bf16_bits(x).reshape(M, K), engine.BF16, engine.F32)
+    finally:
+        weight.destroy()
+    exact_rows = oracle.q4_linear(quants, meta_a, meta_b, kind, N, K, bf16_bits(x).reshape(M, K), oracle.X_BF16, M)
+    # five fp32 rows are ten rows of the streaming kernel, which keeps the weight exact
+    exact = oracle.q4_linear(quants, meta_a, meta_b, kind, N, K, x, oracle.X_F32, M)
+    assert q4_relative_error(y[:4], exact[:4]) <= 1e-3 and q4_relative_error(y_bf[:4], exact_rows[:4]) <= 1e-3
+    assert np.all(y[4] == 0.0) and np.all(y_bf[4] == 0.0)
