@@ -247,6 +247,7 @@ void mi355q_context_destroy(mi355q_context *ctx)
         for (hipEvent_t event : *ctx->profile_events) (void)hipEventDestroy(event);
         delete ctx->profile_events;
     }
+    host_outputs_free(ctx);
     if (ctx->arrivals) (void)hipFree(ctx->arrivals);
     if (ctx->chain_ready) (void)hipFree(ctx->chain_ready);
     if (ctx->chain_gave_up) (void)hipHostFree(ctx->chain_gave_up);
@@ -862,9 +863,8 @@ int q4_linear_multi_repeated(mi355q_context *ctx, const mi355q_q4_target *target
 
     if (!y_dev)
         for (uint32_t t = 0; t < outputs; ++t)
-            MI355Q_HIP(hipMemcpyAsync(targets[t].y, args.targets[t].y,
-                                      (size_t)M * targets[t].weight->dev.N * dtype_bytes(y_dtype),
-                                      hipMemcpyDeviceToHost, ctx->stream),
+            MI355Q_HIP(copy_outputs(ctx, targets[t].y, args.targets[t].y,
+                                    (size_t)M * targets[t].weight->dev.N * dtype_bytes(y_dtype)),
                        "output download");
     if (!(flags & MI355Q_ASYNC))
         MI355Q_HIP(hipStreamSynchronize(ctx->stream), "q4_linear sync");

@@ -54,6 +54,7 @@ struct Q4Device {
 
 namespace mi355q {
 constexpr int kStageSlots = 6;
+struct HostOutputs;
 }
 struct mi355q_context {
     int device;
@@ -115,6 +116,7 @@ struct mi355q_context {
     uint64_t chain_total;     // chained launches of this context so far
     uint32_t chain_spin_limit;
     bool chain_enabled, chain_withhold;
+    mi355q::HostOutputs *host_outputs;  // pinned memory outputs pass through; null until the first large ones
     bool chain_pending;  // a chained launch has been queued since the host last looked at chain_gave_up
 };
 namespace mi355q {
@@ -144,6 +146,11 @@ int fail_hip(hipError_t status, const char *what, char *error, size_t capacity);
 
 int ensure_stage(mi355q_context *ctx, int slot, size_t bytes,
                  char *error, size_t error_capacity);
+
+// Outputs from a staging buffer to memory of the caller's, on the context's stream (host_copy.hip): they may
+// be read once the stream has been waited for.
+hipError_t copy_outputs(mi355q_context *ctx, void *host, const void *device, size_t bytes);
+void host_outputs_free(mi355q_context *ctx);
 
 // Every compute kernel goes through here so that profiling sees it.
 template <typename Kernel, typename... Args>

@@ -515,7 +515,7 @@ extern "C" int mi355q_q8_linear(mi355q_context *ctx, const mi355q_q8_weight *wei
                                  (int)is_bias, y_on_device, y_dtype, M, N);
     if (launched != hipSuccess) return fail_hip(launched, "q8 rows finish launch", error, error_capacity);
     if (!y_dev)
-        MI355Q_HIP(hipMemcpyAsync(y, y_on_device, y_bytes, hipMemcpyDeviceToHost, ctx->stream), "output download");
+        MI355Q_HIP(copy_outputs(ctx, y, y_on_device, y_bytes), "output download");
     if (!(flags & MI355Q_ASYNC)) MI355Q_HIP(hipStreamSynchronize(ctx->stream), "q8_linear sync");
     return MI355Q_OK;
 }

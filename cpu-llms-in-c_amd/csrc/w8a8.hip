@@ -781,12 +781,9 @@ int mi355q_w8a8_linear_multi(mi355q_context *ctx, const mi355q_w8a8_target *targ
     if (!device) {
         for (uint32_t t = 0; t < count; ++t) {
             const size_t o_bytes = (size_t)M * p.N[t] * 4u;
-            MI355Q_HIP(hipMemcpyAsync(targets[t].out, p.out[t], o_bytes, hipMemcpyDeviceToHost, ctx->stream),
-                       "output download");
+            MI355Q_HIP(copy_outputs(ctx, targets[t].out, p.out[t], o_bytes), "output download");
             if (targets[t].acc)
-                MI355Q_HIP(hipMemcpyAsync(targets[t].acc, p.acc[t], o_bytes, hipMemcpyDeviceToHost,
-                                          ctx->stream),
-                           "accumulator download");
+                MI355Q_HIP(copy_outputs(ctx, targets[t].acc, p.acc[t], o_bytes), "accumulator download");
         }
     }
     if (!(flags & MI355Q_ASYNC)) MI355Q_HIP(hipStreamSynchronize(ctx->stream), "w8a8_linear sync");
