@@ -32,13 +32,13 @@ constexpr uint32_t kCopyGroups = 16;
 
 struct HostOutputs {
     unsigned char *memory;   // two halves, pinned
-    uint32_t *flags;         // one a chunk, pinned: the number of the last copy that has filled it
-    uint32_t copies[2];      // of each half so far
+    uint64_t *flags;         // one a chunk, pinned: the number of the last copy that has filled it
+    uint64_t copies[2];      // of each half so far (64 bits: a number never comes again)
 };
 
 // bytes <= kHalfBytes from `from` (16-byte aligned) to `to`.
 __global__ void __launch_bounds__(kChunkThreads) host_chunks_kernel(unsigned char *to, const unsigned char *from, uint32_t bytes,
-                                                                   uint32_t *flags, uint32_t number)
+                                                                   uint64_t *flags, uint64_t number)
 {
     for (uint32_t chunk = blockIdx.x; chunk * kChunkBytes < bytes; chunk += gridDim.x) {
         const uint32_t begin = chunk * kChunkBytes, end = bytes - begin < kChunkBytes ? bytes : begin + kChunkBytes;
@@ -88,9 +88,9 @@ static bool host_outputs_serve(mi355q_context *ctx, const void *host, const void
     ctx->host_outputs = outputs;
     hipError_t status = hipHostMalloc((void **)&outputs->memory, 2u * kHalfBytes, hipHostMallocCoherent);
     if (status == hipSuccess)
-        status = hipHostMalloc((void **)&outputs->flags, 2u * kHalfChunks * sizeof(uint32_t), hipHostMallocCoherent);
+        status = hipHostMalloc((void **)&outputs->flags, 2u * kHalfChunks * sizeof(uint64_t), hipHostMallocCoherent);
     if (status == hipSuccess) {
-        memset(outputs->flags, 0, 2u * kHalfChunks * sizeof(uint32_t));
+        memset(outputs->flags, 0, 2u * kHalfChunks * sizeof(uint64_t));
         return true;
     }
     (void)hipGetLastError();
@@ -99,7 +99,7 @@ static bool host_outputs_serve(mi355q_context *ctx, const void *host, const void
 }
 
 // Waits for a chunk's flag; a stream that has ended, or failed, without raising it is an error.
-static hipError_t wait_for_flag(hipStream_t stream, const uint32_t *flag, uint32_t number)
+static hipError_t wait_for_flag(hipStream_t stream, const uint64_t *flag, uint64_t number)
 {
     for (;;) {
         for (uint32_t poll = 0; poll < 4096u; ++poll) {
