@@ -48,8 +48,8 @@ extern template __global__ void q4_gemm_pipe_kernel<128, 4, false, false>(const 
 extern template __global__ void q4_gemm_pipe_kernel<128, 4, true, false>(const GemmGroup);
 extern template __global__ void q4_gemm_pipe_kernel<128, 4, true, true>(const GemmGroup);
 extern template __global__ void q4_gemm_pipe_kernel<128, 5, false, false>(const GemmGroup);
-extern template __global__ void q4_gemm_pipe_kernel<128, 4, false, false, true>(const GemmGroup);  // 8-bit codes
-extern template __global__ void q4_gemm_pipe_kernel<128, 3, true, false, true>(const GemmGroup);   // 8-bit codes
+extern template __global__ void q4_gemm_pipe_kernel<128, 4, false, false, true>(const GemmParams);  // 8-bit codes
+extern template __global__ void q4_gemm_pipe_kernel<128, 3, true, false, true>(const GemmParams);   // 8-bit codes
 
 // Adds the K splits in split order (a fixed order) and applies the epilogue.  WIDE: a thread
 // takes four adjacent outputs of one row (N a multiple of 4, y 16-byte aligned): 16-byte loads
@@ -221,7 +221,7 @@ static hipError_t launch_pipe_bytes(mi355q_context *ctx, dim3 grid, const GemmGr
         if (status != hipSuccess) return status;
         ctx->lds_raised[slot] = true;
     }
-    return launch(ctx, q4_gemm_pipe_kernel<128, NTW, XT, false, true>, grid, dim3(256), bytes, group);
+    return launch(ctx, q4_gemm_pipe_kernel<128, NTW, XT, false, true>, grid, dim3(256), bytes, group.shared);
 }
 
 // The 17-tile shape with compiler-managed weight loads (option "gemm_loads" = "plain").
@@ -509,14 +509,14 @@ struct CallPlan {
 static CallPlan plan_call(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows, const TargetPlan *plans)
 {
     CallPlan best = {-1, 0.0};
-    bool alike = a.count > 1u;
+    bool alike = a.count > 1u && !plans[0].bytes;  // (the kernel of 8-bit codes takes one target)
     for (uint32_t t = 0; t < a.count; ++t) {
         best.us += plans[t].us;
         if (t != 0u && a.x_dtype != MI355Q_F16) {  // one conversion serves them all
             const Variant &c = variants[plans[t].variant];
             best.us -= c.converted[0] + c.converted[1] * (double)rows * a.targets[t].w->K * sizeof(_Float16) * 1e-6;
         }
-        alike = alike && plans[t].bytes == plans[0].bytes;
+        alike = alike && !plans[t].bytes;
     }
     if (!alike) return best;
     if (ctx->force_gemm[1] >= 1) {
@@ -525,12 +525,12 @@ static CallPlan plan_call(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t r
     }
     const double alone_us = best.us;
     const Q4Device &first = *a.targets[0].w;
-    const bool bytes = plans[0].bytes, pipe_ok = gemm_pipe_ok(first, rows, a.x_columns ? a.x_columns : first.K);
-    const uint32_t T = bytes ? first.T / 2u : first.T, cus = (uint32_t)ctx->props.multiProcessorCount;
-    for (int v = 0; v < (int)(sizeof variants / sizeof variants[0]); ++v) {
-        if ((v >= kFirstPiped && !pipe_ok) || (v >= kBytesVariant) != bytes) continue;
+    const bool pipe_ok = gemm_pipe_ok(first, rows, a.x_columns ? a.x_columns : first.K);
+    const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
+    for (int v = 0; v < kBytesVariant; ++v) {
+        if (v >= kFirstPiped && !pipe_ok) continue;
         LaunchWork work = {};
-        for (uint32_t t = 0; t < a.count; ++t) add_work(work, variants[v], a, *a.targets[t].w, T, rows, plans[t].splits);
+        for (uint32_t t = 0; t < a.count; ++t) add_work(work, variants[v], a, *a.targets[t].w, first.T, rows, plans[t].splits);
         const double us = launch_us(v, cus, work);
         if (us < 0.95 * alone_us && us < best.us) best = {v, us};
     }

@@ -5,6 +5,6 @@
 
 namespace mi355q {
 
-template __global__ void q4_gemm_pipe_kernel<128, 3, true, false, true>(const GemmGroup);
+template __global__ void q4_gemm_pipe_kernel<128, 3, true, false, true>(const GemmParams);
 
 }  // namespace mi355q

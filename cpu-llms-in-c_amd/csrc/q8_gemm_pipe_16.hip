@@ -4,6 +4,6 @@
 
 namespace mi355q {
 
-template __global__ void q4_gemm_pipe_kernel<128, 4, false, false, true>(const GemmGroup);
+template __global__ void q4_gemm_pipe_kernel<128, 4, false, false, true>(const GemmParams);
 
 }  // namespace mi355q
