@@ -54,7 +54,59 @@ w8a8_repack_kernel(const uint8_t *__restrict__ rows, uint4 *__restrict__ tiles,
     tiles[index] = make_uint4(words[0], words[1], words[2], words[3]);
 }
 
-// One workgroup per activation row: absmax, then the codes.
+// Rows of whole 4-column pieces, x 16-byte and q 4-byte aligned: a row's pieces are held in registers
+// between its maximum and its codes, all their loads on their way at once, four codes a store; a wave takes
+// a row by itself up to 2048 columns (no barrier), a workgroup of four above.
+// Bound by the chain load, maximum, store.  Kernel time, one column a thread and access -> this, us: 64 rows of 512
+// 2.7 -> 2.3, of 1024 3.2 -> 2.4, of 2048 4.1 -> 2.7, of 4096 5.9 -> 2.8; 768 of 2048 4.8 -> 3.0; 300 of 8192 10.5 -> 3.6.
+// Quantizer and three weights: 768 rows of 2048 x 4096 46.8 -> 44.4, 300 of 2048 x 1024 14.7 -> 13.3, 64 of 1024 x 4096
+// 11.6 -> 11.2.  Stores past the L2 take the kernel as long, and the codes out of the caches that the matrix kernel
+// reads them through: 768 rows 51.
+template <bool WAVE, int PIECES>
+__global__ void __launch_bounds__(WAVE ? 64 : 256)
+quantize_i8_rows_kernel(const float *__restrict__ x, uint32_t K, int8_t *__restrict__ q, float *__restrict__ scales)
+{
+    constexpr uint32_t kLanes = WAVE ? 64u : 256u;
+    typedef float Piece __attribute__((ext_vector_type(4)));
+    const Piece *const row = (const Piece *)(x + (size_t)blockIdx.x * K);
+    uint32_t *const out = (uint32_t *)(q + (size_t)blockIdx.x * K);
+    const uint32_t pieces = K / 4u;
+    Piece held[PIECES];
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {  // past the row's end: its last piece again
+        const uint32_t piece = threadIdx.x + i * kLanes;
+        held[i] = row[piece < pieces ? piece : pieces - 1u];
+    }
+    float maximum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) maximum = fmaxf(maximum, fabsf(held[i][j]));
+#pragma unroll
+    for (int offset = 32; offset > 0; offset >>= 1) maximum = fmaxf(maximum, __shfl_xor(maximum, offset));
+    if constexpr (!WAVE) {
+        __shared__ float wave_max[4];
+        if ((threadIdx.x & 63u) == 0u) wave_max[threadIdx.x >> 6] = maximum;
+        __syncthreads();
+        maximum = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
+    }
+    const bool codes = maximum > 0.0f;  // else all zero (or NaN): zero codes, scale 0
+    const float scale = maximum / 127.0f;  // IEEE division, as the reference's
+    const float inverse = 1.0f / scale;
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+        const uint32_t piece = threadIdx.x + i * kLanes;
+        uint32_t word = 0u;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)  // round half to even
+            word |= (uint32_t)(uint8_t)(int8_t)(int)__builtin_rintf(held[i][j] * inverse) << (8 * j);
+        if (piece < pieces) out[piece] = codes ? word : 0u;
+    }
+    if (threadIdx.x == 0u) scales[blockIdx.x] = codes ? scale : 0.0f;
+}
+
+// Every other row (longer than 8192 columns, a number of columns that is no multiple of 4, x or q not
+// aligned): one workgroup per activation row, absmax, then the codes, read a second time.
 __global__ void __launch_bounds__(256)
 quantize_i8_kernel(const float *__restrict__ x, uint32_t K, int8_t *__restrict__ q,
                    float *__restrict__ scales)
@@ -490,6 +542,19 @@ static hipError_t launch_w8a8(mi355q_context *ctx, dim3 grid, uint32_t tiles_per
     }
 }
 
+// The lines between the kernels: where a lane's pieces would be more than eight (the figures above: a row
+// held by one wave, 2048 columns, and by four, 4096 and 8192, gains alike); one reads what none may hold.
+static hipError_t quantize_launch(mi355q_context *ctx, const float *x, uint32_t M, uint32_t K, int8_t *q, float *scales)
+{
+    const bool whole = K % 4u == 0u && (uintptr_t)x % 16u == 0u && (uintptr_t)q % 4u == 0u;
+    if (!whole || K > 8192u) return launch(ctx, quantize_i8_kernel, dim3(M), dim3(256), 0, x, K, q, scales);
+    if (K <= 512u) return launch(ctx, quantize_i8_rows_kernel<true, 2>, dim3(M), dim3(64), 0, x, K, q, scales);
+    if (K <= 1024u) return launch(ctx, quantize_i8_rows_kernel<true, 4>, dim3(M), dim3(64), 0, x, K, q, scales);
+    if (K <= 2048u) return launch(ctx, quantize_i8_rows_kernel<true, 8>, dim3(M), dim3(64), 0, x, K, q, scales);
+    if (K <= 4096u) return launch(ctx, quantize_i8_rows_kernel<false, 4>, dim3(M), dim3(256), 0, x, K, q, scales);
+    return launch(ctx, quantize_i8_rows_kernel<false, 8>, dim3(M), dim3(256), 0, x, K, q, scales);
+}
+
 }  // namespace mi355q
 
 using namespace mi355q;
@@ -592,7 +657,7 @@ int mi355q_quantize_i8(mi355q_context *ctx, const float *x, uint32_t M, uint32_t
         q_dev = (int8_t *)ctx->stage[1];
         s_dev = (float *)((char *)ctx->stage[1] + ((q_bytes + 15u) & ~(size_t)15u));
     }
-    hipError_t launched = launch(ctx, quantize_i8_kernel, dim3(M), dim3(256), 0, x_dev, K, q_dev, s_dev);
+    hipError_t launched = quantize_launch(ctx, x_dev, M, K, q_dev, s_dev);
     if (launched != hipSuccess) return fail_hip(launched, "quantize_i8 launch", error, error_capacity);
     if (!device) {
         MI355Q_HIP(hipMemcpyAsync(q, q_dev, q_bytes, hipMemcpyDeviceToHost, ctx->stream), "code download");

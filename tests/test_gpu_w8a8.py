@@ -246,3 +246,31 @@ def test_shared_activation_needs_equal_columns(engine, gpu):
     finally:
         gpu.w8a8_destroy(a)
         gpu.w8a8_destroy(b)
+
+
+@pytest.mark.parametrize("K", [1, 4, 252, 510, 512, 516, 1024, 1028, 2044, 2048, 2052, 2049, 4096, 4100, 8192, 8196])
+@pytest.mark.parametrize("M", [1, 7])
+def test_quantizer_row_lengths(engine, oracle, gpu, M, K):
+    """Rows held in registers and rows read twice, at the edges of each kernel's range: the oracle's codes
+    and scales, for aligned rows and for rows whose first column is at 4 bytes of 16, with nothing written
+    past the codes.  The first row's largest value stands at its end, one row is zero."""
+    x = engine.synth_normal_f32(K, 1.0, M * K).reshape(M, K)
+    x[0, K - 1] = -9.5
+    x[M // 2 + 1:M // 2 + 2] = 0.0
+    q_ref, s_ref = oracle.quantize_i8(x)
+    x_ptr, q_ptr, s_ptr = gpu.alloc(M * K * 4 + 16), gpu.alloc(M * K + 16), gpu.alloc(M * 4)
+    try:
+        for shift in (0, 4):
+            print(f"quantizer M={M} K={K} at {shift} bytes", flush=True)
+            padded = np.zeros(M * K + 4, np.float32)
+            padded[shift // 4:shift // 4 + M * K] = x.reshape(-1)
+            gpu.upload(x_ptr, padded)
+            gpu.upload(q_ptr, np.full(M * K + 16, 85, np.int8))
+            gpu.quantize_i8_device(x_ptr + shift, M, K, q_ptr, s_ptr)
+            gpu.sync()
+            got = gpu.download(q_ptr, (M * K + 16,), np.int8)
+            assert np.array_equal(got[:M * K].reshape(M, K), q_ref) and np.all(got[M * K:] == 85)
+            assert np.array_equal(gpu.download(s_ptr, (M,), np.uint32), s_ref.view(np.uint32))
+    finally:
+        for pointer in (x_ptr, q_ptr, s_ptr):
+            gpu.free(pointer)
