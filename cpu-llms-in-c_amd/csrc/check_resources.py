@@ -8,9 +8,12 @@ The log is the compiler's whole diagnostic output; what is not a resource remark
 is passed through to stdout, the remarks themselves are only read.
 
 Budgets (a kernel name is matched after demangling):
-  * every q4_stream_kernel, q4_chain_kernel, q4_rows_kernel, q4_gemm_pipe_kernel and w8a8_block_kernel
-    instantiation: no scratch memory (a spill inside the streaming loop costs more than any occupancy it
-    buys, and its loads would be among those that the kernel's own waits count) and no spilled registers;
+  * every q4_stream_kernel, q4_chain_kernel, q4_rows_kernel, q4_gemm_kernel, q4_gemm_group_kernel,
+    q4_gemm_pipe_kernel and w8a8_block_kernel instantiation: no scratch memory (a spill inside the streaming
+    loop costs more than any occupancy it buys, and its loads would be among those that the kernel's own
+    waits count) and no spilled registers;
+  * q4_gemm_kernel and q4_gemm_group_kernel: at least the workgroups a compute unit that the table of
+    shapes in q4_gemm.hip counts on (a workgroup is one wave a SIMD);
   * q4_stream_kernel<1, 1, 2, 16, *, false>: at most 64 vector registers - with sixteen waves a
     workgroup, two workgroups share a compute unit only up to 64 (one more halves the occupancy
     and the launch of the 27B q|k|v group takes a quarter longer);
@@ -23,6 +26,9 @@ import sys
 
 PIPE_DYNAMIC_LDS = 4 * 128 * 16 * 16
 LDS_PER_CU = 160 * 1024
+# rows of x, tiles a wave, one tile more: `resident` of the same line of `variants` in q4_gemm.hip
+GEMM_RESIDENT = {("128", "4", "false"): 2, ("128", "2", "false"): 2, ("64", "4", "false"): 3, ("64", "4", "true"): 2,
+                 ("64", "2", "false"): 4, ("64", "2", "true"): 2}
 
 
 def kernels(text):
@@ -35,7 +41,8 @@ def kernels(text):
 
         yield name, {"vgprs": field("VGPRs"), "agprs": field("AGPRs"),
                      "scratch": field("ScratchSize [bytes/lane]"), "vgpr_spill": field("VGPRs Spill"),
-                     "sgpr_spill": field("SGPRs Spill"), "lds": field("LDS Size [bytes/block]")}
+                     "sgpr_spill": field("SGPRs Spill"), "lds": field("LDS Size [bytes/block]"),
+                     "waves": field("Occupancy [waves/SIMD]")}
 
 
 def split_log(text):
@@ -74,7 +81,8 @@ def main():
                                text=True, check=True).stdout.splitlines()
     problems = []
     for (mangled, use), name in zip(found, demangled):
-        watched = re.search(r"(q4_stream_kernel|q4_chain_kernel|q4_rows_kernel|q4_gemm_pipe_kernel|w8a8_block_kernel)<([^>]*)>", name)
+        watched = re.search(r"(q4_stream_kernel|q4_chain_kernel|q4_rows_kernel|q4_gemm_kernel|q4_gemm_group_kernel|q4_gemm_pipe_kernel|"
+                            r"w8a8_block_kernel)<([^>]*)>", name)
         if not watched:
             continue
         kind, parameters = watched.group(1), [p.strip() for p in watched.group(2).split(",")]
@@ -85,6 +93,11 @@ def main():
         if kind == "q4_stream_kernel" and parameters[:4] == ["1", "1", "2", "16"] and parameters[5:6] != ["true"] \
                 and use["vgprs"] > 64:
             problems.append("%s: %d vector registers, the sixteen-wave launch needs at most 64" % (label, use["vgprs"]))
+        if kind in ("q4_gemm_kernel", "q4_gemm_group_kernel"):
+            resident = GEMM_RESIDENT.get(tuple(parameters[:3]))
+            if resident is None or use["waves"] < resident:
+                problems.append("%s: %d waves a SIMD, its line of the table of shapes counts on %s"
+                                % (label, use["waves"], resident))
         if kind == "q4_gemm_pipe_kernel":
             if use["lds"] + PIPE_DYNAMIC_LDS > LDS_PER_CU:
                 problems.append("%s: %d bytes of static LDS + %d at launch exceed %d"

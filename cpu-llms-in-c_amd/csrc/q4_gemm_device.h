@@ -489,6 +489,14 @@ __global__ void __launch_bounds__(256, 2) q4_gemm_group_kernel(const GemmGroup g
     GemmParams p;
     uint32_t block_n, block_m, split;
     if (!locate_block(group, 4 * NTW + (EXTRA ? 1 : 0), BM, p, block_n, block_m, split)) return;
+    // The divisions leave the three in vector registers, where the compiler no longer knows that a workgroup
+    // has one of each: 128 rows x 16 tiles then spilled 22 registers and 64 x 17 four, and 64 x 16 fitted two
+    // to a compute unit where the estimates count on three.  In scalar registers they take what one weight's
+    // kernels take (us: two of 6080 x 3008 at 331 rows 58.3 -> 46.6; two of 6000 x 4096 at 400 rows, 128 x 16
+    // 145 -> 75, 64 x 17 76.6 -> 74.1, the other shapes 0 to 3 % less).
+    block_n = __builtin_amdgcn_readfirstlane(block_n);
+    block_m = __builtin_amdgcn_readfirstlane(block_m);
+    split = __builtin_amdgcn_readfirstlane(split);
     gemm_workgroup<BM, NTW, EXTRA, CONVERTED>(p, block_n, block_m, split);
 }
 
