@@ -13,7 +13,7 @@ Budgets (a kernel name is matched after demangling):
     loop costs more than any occupancy it buys, and its loads would be among those that the kernel's own
     waits count) and no spilled registers;
   * q4_gemm_kernel and q4_gemm_group_kernel: at least the workgroups a compute unit that the table of
-    shapes in q4_gemm.hip counts on (a workgroup is one wave a SIMD);
+    shapes in q4_gemm_plan.h counts on (a workgroup is one wave a SIMD);
   * q4_stream_kernel<1, 1, 2, 16, *, false>: at most 64 vector registers - with sixteen waves a
     workgroup, two workgroups share a compute unit only up to 64 (one more halves the occupancy
     and the launch of the 27B q|k|v group takes a quarter longer);
@@ -26,7 +26,7 @@ import sys
 
 PIPE_DYNAMIC_LDS = 4 * 128 * 16 * 16
 LDS_PER_CU = 160 * 1024
-# rows of x, tiles a wave, one tile more: `resident` of the same line of `variants` in q4_gemm.hip
+# rows of x, tiles a wave, one tile more: `resident` of the same line of `variants` in q4_gemm_plan.h
 GEMM_RESIDENT = {("128", "4", "false"): 2, ("128", "2", "false"): 2, ("64", "4", "false"): 3, ("64", "4", "true"): 2,
                  ("64", "2", "false"): 4, ("64", "2", "true"): 2}
 

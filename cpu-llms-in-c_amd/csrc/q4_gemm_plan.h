@@ -1,0 +1,400 @@
+// How a call of the GEMM kernels goes out: shapes, K splits, launches.  Host code that runs on every call before
+// its first launch: on one core, us, a 27B layer's q|k|v at 32 and at 512 rows 0.9 and 0.8, gate|up 0.5, down 0.4
+// (the K splits of one weight estimated like a launch of several, whose workgroups take compute units in turn:
+// 7.9, 7.2, 4.8, 3.5).
+#pragma once
+#include <algorithm>
+
+#include "internal.h"
+#include "q4_rows_device.h"
+
+namespace mi355q {
+
+// The shapes, and what a launch of each is estimated to take: microseconds of a call among others, fitted
+// to timings on this GPU of one weight under every shape and K split (27 weights from 896 x 3584 to
+// 17408 x 5120 at 75 to 4646 rows, ten of them at 17 to 128, six 8-bit weights; 210 to 1130 timings a
+// shape, 4 to 5 % rms).  The shape and split that the estimates choose takes 0.7 % longer than the best
+// timed one on average, 11 % at most (estimates that left out what launches, K splits' second kernels
+// and stores take: 3 %, 26 %).
+struct Variant {
+    int bm, ntw, extra;
+    int resident;           // workgroups that fit one compute unit (registers, LDS)
+    double launch;          // once
+    double step, fill;      // a chip full of workgroups: each 128-column step, and once
+    // First kernel: the same of a chip with at most k + 1 workgroups on a compute unit, which the
+    // last workgroups are.  Pipelined kernel, whose last round of workgroups takes the fraction r of
+    // the compute units: {step, + max(0, r - 0.5) of each step}, {fill, + r^2} (the chip is power
+    // limited, and up to about half of it the clock stays near its maximum).
+    double part_step[4], part_fill[4];
+    double split, per_split, sums;  // a K split: its second kernel, more for each split, MB of partial sums
+    double outputs;         // MB of outputs
+    double converted[3];    // activations that are not fp16: once, MB of fp16 rows, MB of outputs
+    double reread;          // MB of fp16 rows beyond an XCD's L2, by each block of tiles
+};
+constexpr Variant variants[] = {
+    {128, 4, 0, 2, 13.19, 3.208, 5.98, {2.167, 3.026}, {0.0, 1.16}, 0.0, 0.0, 0.192, 0.435, {2.27, 0.36, 0.0}, 0.000},
+    {128, 2, 0, 2, 5.82, 1.628, 0.0, {1.207, 1.595}, {0.0, 0.010}, 2.52, 0.0, 0.304, 0.474, {5.72, 0.40, 0.046}, 0.007},
+    {64, 4, 0, 3, 5.54, 2.755, 0.0, {1.175, 1.820, 2.868}, {0.53, 0.0, 0.0}, 2.60, 0.0, 0.262, 0.566, {5.81, 0.27, 0.0}, 0.000},
+    {64, 4, 1, 2, 8.64, 2.275, 0.0, {1.366, 2.151}, {0.037, 0.0}, 1.82, 0.0, 0.250, 0.206, {3.96, 0.29, 0.31}, 0.002},
+    {64, 2, 0, 4, 4.16, 1.831, 0.0, {0.711, 1.054, 1.516, 1.972}, {0.41, 1.14, 0.61, 0.0}, 2.52, 0.0, 0.280, 0.498, {4.84, 0.37, 0.0}, 0.003},
+    {64, 2, 1, 2, 4.99, 1.240, 0.0, {0.918, 1.294}, {0.0, 0.21}, 2.46, 0.0, 0.279, 0.524, {4.76, 0.36, 0.21}, 0.000},
+    {128, 4, 0, 1, 4.51, 1.363, 5.31, {1.107, 0.117}, {3.93, 2.92}, 2.48, 0.24, 0.207, 0.325, {5.48, 0.18, 0.50}, 0.014},
+    {128, 4, 1, 1, 6.29, 1.545, 6.04, {1.260, 0.291}, {3.64, 1.55}, 2.40, 0.32, 0.182, 0.355, {5.22, 0.19, 0.56}, 0.011},
+    {128, 5, 0, 1, 1.25, 1.747, 6.38, {1.368, 0.627}, {9.07, 0.22}, 2.98, 0.28, 0.175, 0.363, {5.14, 0.23, 0.50}, 0.003},
+    // 16 and 13 tiles on 8-bit codes, and only for them
+    {128, 4, 0, 1, 0.88, 1.544, 9.49, {1.249, 0.535}, {5.21, 6.69}, 4.14, 0.10, 0.172, 0.031, {0.0, 0.0, 0.0}, 0.000},
+    {128, 3, 1, 1, 5.81, 1.436, 6.56, {1.144, 0.482}, {0.0, 4.74}, 4.30, 0.14, 0.208, 0.054, {0.0, 0.0, 0.0}, 0.000}};
+constexpr int kVariants = sizeof variants / sizeof variants[0];
+constexpr int kFirstPiped = 6;    // the first shape of the pipelined kernel
+constexpr int kBytesVariant = 9;  // the first on 8-bit codes
+
+// the pipelined kernel addresses x with 32-bit byte offsets and whole 128-column steps
+inline bool gemm_pipe_ok(const Q4Device &w, uint32_t rows, uint32_t x_columns)
+{
+    return w.K % kStepColumns == 0 && (uint64_t)rows * x_columns * sizeof(_Float16) + 16384u < (1ull << 32);
+}
+
+// What a launch takes besides its matrix kernel.
+struct Around {
+    uint32_t splits;       // the most of one target
+    double sums, outputs;  // MB
+    double rows;           // MB of fp16 rows
+    double reread;         // MB
+    bool converted;
+};
+inline double launch_us(const Variant &c, double kernel_us, const Around &around)
+{
+    double us = c.launch + kernel_us;
+    if (around.splits > 1u) us += c.split + c.per_split * around.splits + c.sums * around.sums;
+    if (around.converted) us += c.converted[0] + c.converted[1] * around.rows + c.converted[2] * around.outputs;
+    return us + c.outputs * around.outputs + c.reread * around.reread;
+}
+
+// Microseconds of the first kernel, `each` steps a workgroup: full rounds of the chip, then what is left.
+inline double first_kernel_us(const Variant &c, uint32_t cus, uint64_t groups, double each)
+{
+    const uint64_t slots = (uint64_t)cus * c.resident, rounds = groups < slots ? 0u : groups / slots;
+    uint64_t rest = groups - rounds * slots;
+    double us = (double)rounds * (each * c.step + c.fill);
+    if (rest != 0u) {
+        int k = 0;
+        for (; rest > cus; rest -= cus) ++k;
+        us += each * c.part_step[k] + c.part_fill[k];
+    }
+    return us;
+}
+
+// The last round of the pipelined kernel, on the fraction r of the compute units.
+inline double pipe_rest_us(const Variant &c, double each, double r)
+{
+    return each * (c.part_step[0] + c.part_step[1] * std::max(0.0, r - 0.5)) + c.part_fill[0] + c.part_fill[1] * r * r;
+}
+
+// Microseconds of the pipelined kernel, one workgroup per compute unit: one target, whole rounds and a rest.
+inline double pipe_kernel_us(const Variant &c, uint32_t cus, uint64_t groups, uint32_t steps)
+{
+    const uint64_t rounds = groups < cus ? 0u : groups / cus, rest = groups - rounds * cus;
+    double us = (double)rounds * (c.fill + (double)steps * c.step);
+    if (rest != 0u) us += pipe_rest_us(c, (double)steps, (double)rest / (double)cus);
+    return us;
+}
+
+// What each target gives a launch of several, the longest workgroups first.
+struct GroupWork {
+    uint32_t count;
+    uint32_t steps[kMaxTargets];   // of a workgroup
+    uint64_t groups[kMaxTargets];
+};
+
+// The same of several targets: the workgroups take the compute units as they come free.
+inline double pipe_group_us(const Variant &c, uint32_t cus, const GroupWork &work)
+{
+    struct Level {
+        double at;  // so many compute units are free from here on
+        uint64_t units;
+    } level[kMaxTargets + 2];  // a target adds at most one
+    int levels = 1;
+    level[0] = {0.0, cus};
+    uint64_t groups = 0, steps = 0;
+    for (uint32_t i = 0; i < work.count; ++i) {
+        const double time = c.fill + (double)work.steps[i] * c.step;
+        uint64_t left = work.groups[i];
+        groups += left;
+        steps += left * work.steps[i];
+        while (left > 0u) {
+            if (levels == 1 && left >= cus) {  // whole rounds
+                level[0].at += time * (double)(left / cus);
+                left %= cus;
+                continue;
+            }
+            const uint64_t taken = std::min(left, level[0].units);  // those that are free first
+            const Level busy = {level[0].at + time, taken};
+            left -= taken;
+            level[0].units -= taken;
+            if (level[0].units == 0u) {
+                for (int l = 1; l < levels; ++l) level[l - 1] = level[l];
+                --levels;
+            }
+            int at = levels;
+            while (at > 0 && level[at - 1].at > busy.at + 1e-9) --at;
+            if (at > 0 && level[at - 1].at > busy.at - 1e-9) {
+                level[at - 1].units += taken;
+            } else {
+                for (int l = levels; l > at; --l) level[l] = level[l - 1];
+                level[at] = busy;
+                ++levels;
+            }
+        }
+    }
+    double us = level[0].at, busy = 0.0;  // busy: of all compute units together, from the first one's end on
+    for (int l = 0; l < levels; ++l) busy += (level[l].at - level[0].at) * (double)level[l].units;
+    const double rest = level[levels - 1].at - level[0].at;
+    if (rest > 0.0) {
+        const double r = busy / (rest * cus), each = (double)steps / (double)groups;
+        us += rest * pipe_rest_us(c, each, r) / (each * c.step + c.fill);
+    }
+    return us;
+}
+
+// How one target of a call is multiplied: the shape and K split with the smallest estimated time.
+struct TargetPlan {
+    bool bytes;       // by the kernel for 8-bit codes
+    int variant;
+    uint32_t splits;
+    double us;        // the estimate
+};
+
+// A target splits K the same way in company as alone, and two weights that each take more than half of
+// the chip without a split fill it together: such a weight splits only where that gains 12 % (17408 x 5120 at
+// 200 rows 54.3 instead of 51.7 us; a pair of them 81 instead of 101).
+constexpr double kSplitWeight = 1.12;
+inline TargetPlan plan_target(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, uint32_t rows)
+{
+    const Q4Device &w = *a.targets[target].w;
+    const uint32_t x_columns = a.x_columns ? a.x_columns : w.K;
+    // The doubled form of an 8-bit weight whose activation row the kernels would read twice: the
+    // kernel for 8-bit codes reads the bytes themselves instead, one pass over the row, half the
+    // matrix instructions.  It is the pipelined kernel, with that kernel's conditions.
+    const bool bytes = w.codes8 != nullptr && a.x_columns != 0 && !ctx->q8_gemm_doubled &&
+                       (uint64_t)rows * x_columns * sizeof(_Float16) + 16384u < (1ull << 32);
+    const uint32_t T = bytes ? w.T / 2u : w.T;
+    const bool pipe_ok = gemm_pipe_ok(w, rows, x_columns);
+    TargetPlan best = {bytes, 0, 1, 1e30};
+    double best_weighed = 1e30;
+    // Decomposition: BM rows x (4*NTW + EXTRA) tiles per workgroup, K split in `splits`: up to eight, of eight
+    // steps or so at least.
+    uint32_t ways = 0, want[8], steps[8], splits[8];
+    for (uint32_t s = 1; s <= 8u && s * 8u <= T + 7u; ++s) {
+        const uint32_t of_steps = (T + s - 1u) / s;
+        if (ways != 0u && of_steps == steps[ways - 1u]) continue;  // the split before it again
+        want[ways] = s;
+        steps[ways] = of_steps;
+        splits[ways++] = (T + of_steps - 1u) / of_steps;
+    }
+    const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
+    const bool half_filled = (uint64_t)((w.NT + 15u) / 16u) * ((rows + 127u) / 128u) * 2u > cus;  // in blocks of 128 rows x 16 tiles
+    Around around;
+    around.outputs = (double)a.M * w.N * dtype_bytes(a.y_dtype) * 1e-6;
+    around.converted = a.x_dtype != MI355Q_F16;
+    around.rows = (double)rows * w.K * sizeof(_Float16) * 1e-6;
+    const double sums = (double)rows * w.N * 4e-6;
+    for (int v = bytes ? kBytesVariant : 0; v < (bytes ? kVariants : kBytesVariant); ++v) {
+        if (v >= kFirstPiped && !pipe_ok) break;
+        const Variant &c = variants[v];
+        const uint32_t tpb = 4u * c.ntw + c.extra, n_blocks = (w.NT + tpb - 1u) / tpb;
+        const uint64_t blocks = (uint64_t)n_blocks * ((rows + c.bm - 1u) / c.bm);
+        around.reread = std::max(around.rows - 4.0, 0.0) * n_blocks;
+        for (uint32_t i = 0; i < ways; ++i) {
+            around.splits = splits[i];
+            around.sums = splits[i] > 1u ? splits[i] * sums : 0.0;
+            const double us = launch_us(c, v >= kFirstPiped ? pipe_kernel_us(c, cus, blocks * splits[i], steps[i])
+                                                            : first_kernel_us(c, cus, blocks * splits[i], steps[i]), around);
+            const double weighed = us * (splits[i] > 1u && half_filled ? kSplitWeight : 1.0);
+            if (weighed < best_weighed) {
+                best_weighed = weighed;
+                best = {bytes, v, want[i], us};
+            }
+        }
+    }
+    // option "q4_gemm" = "VARIANT,SPLITS" for experiments
+    if (ctx->force_gemm[1] >= 1 && ctx->force_gemm[0] < kVariants && (ctx->force_gemm[0] < kFirstPiped || pipe_ok) &&
+        (ctx->force_gemm[0] >= kBytesVariant) == bytes) {
+        best.variant = ctx->force_gemm[0];
+        best.splits = (uint32_t)ctx->force_gemm[1];
+    }
+    return best;
+}
+
+// The targets above 128 rows: as one launch of one shape, or each by its own plan (variant -1).  In one
+// launch, too, each has the K split of its own plan, and so its own call's bits.
+struct GroupPlan {
+    int variant;
+    double us;
+};
+inline GroupPlan plan_group(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows, const TargetPlan *plans)
+{
+    GroupPlan best = {-1, 0.0};
+    bool alike = a.count > 1u;
+    for (uint32_t t = 0; t < a.count; ++t) {
+        best.us += plans[t].us;
+        if (t != 0u && a.x_dtype != MI355Q_F16) {  // one conversion serves them all
+            const Variant &c = variants[plans[t].variant];
+            best.us -= c.converted[0] + c.converted[1] * (double)rows * a.targets[t].w->K * sizeof(_Float16) * 1e-6;
+        }
+        alike = alike && !plans[t].bytes;  // (the kernel of 8-bit codes takes one target)
+    }
+    if (!alike) return best;
+    if (ctx->force_gemm[1] >= 1) {
+        if (plans[0].variant == ctx->force_gemm[0]) best.variant = plans[0].variant;
+        return best;
+    }
+    const double alone_us = best.us;
+    const Q4Device &first = *a.targets[0].w;
+    const bool pipe_ok = gemm_pipe_ok(first, rows, a.x_columns ? a.x_columns : first.K);
+    const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
+    GroupWork work = {};
+    work.count = a.count;
+    uint32_t splits[kMaxTargets], NT[kMaxTargets];
+    Around around = {};
+    around.converted = a.x_dtype != MI355Q_F16;
+    around.rows = (double)rows * first.K * sizeof(_Float16) * 1e-6;
+    for (uint32_t t = 0; t < a.count; ++t) {
+        const Q4Device &w = *a.targets[t].w;
+        const uint32_t steps = (first.T + plans[t].splits - 1u) / plans[t].splits, ways = (first.T + steps - 1u) / steps;
+        around.splits = std::max(around.splits, ways);
+        if (ways > 1u) around.sums += (double)ways * rows * w.N * 4e-6;
+        around.outputs += (double)a.M * w.N * dtype_bytes(a.y_dtype) * 1e-6;
+        uint32_t at = t;
+        for (; at > 0u && work.steps[at - 1u] < steps; --at) {
+            work.steps[at] = work.steps[at - 1u];
+            splits[at] = splits[at - 1u];
+            NT[at] = NT[at - 1u];
+        }
+        work.steps[at] = steps;
+        splits[at] = ways;
+        NT[at] = w.NT;
+    }
+    for (int v = 0; v < kBytesVariant; ++v) {
+        if (v >= kFirstPiped && !pipe_ok) break;
+        const Variant &c = variants[v];
+        const uint32_t tpb = 4u * c.ntw + c.extra, m_blocks = (rows + c.bm - 1u) / c.bm;
+        uint64_t groups = 0, steps = 0;
+        around.reread = 0.0;
+        for (uint32_t t = 0; t < a.count; ++t) {
+            const uint32_t n_blocks = (NT[t] + tpb - 1u) / tpb;
+            work.groups[t] = (uint64_t)n_blocks * m_blocks * splits[t];
+            groups += work.groups[t];
+            steps += work.groups[t] * work.steps[t];
+            around.reread += std::max(around.rows - 4.0, 0.0) * n_blocks;
+        }
+        const double us = launch_us(c, v >= kFirstPiped ? pipe_group_us(c, cus, work)
+                                                        : first_kernel_us(c, cus, groups, (double)steps / (double)groups), around);
+        if (us < 0.95 * alone_us && us < best.us) best = {v, us};
+    }
+    return best;
+}
+
+// ---- 17..128 rows: q4_rows_kernel (q4_rows_device.h) ---------------------------------------
+
+struct RowsPlan {
+    int mf, ntw, waves;            // 16-row fragments, tiles per wave, waves
+    uint32_t blocks, units;        // blocks in all, units per workgroup
+};
+
+// The launch of q4_rows_kernel for a call's targets together; false: not the kernel for it.
+// `others`: what each target would take otherwise.
+// Shape and workgroups minimise a microsecond estimate fitted to 2100 timings on this GPU (14 calls
+// from 1024 x 3584 to two weights of 17408 x 5120, 17 to 128 rows, every block width, whole blocks
+// and 128 to 512 workgroups; 6 % rms): 5.2 us, 0.02 for each MB of weights, then per unit the longer of one
+// workgroup's own chain (0.26 + 0.11 us per 16 rows) and its share of the compute unit, then, where
+// workgroups share blocks, 2.9 us and the partial sums at 2 TB/s.
+//
+// Chosen where that is less than the other kernels' estimate (one weight), or less than 1.08 times it and
+// 1 us (several: theirs for small and for large calls of several weights is that much too low; us, this
+// kernel and the other: 2048 + 512 + 512 x 1024 at 48 rows 8.0 and 10.0, two of 17408 x 5120 at 64 rows 41 and
+// 50, two of 8192 x 3072 at 48 rows 17.7 and 19.7).  One weight of more than 20 MB, from HBM (the Infinity
+// Cache), this kernel and the other: 17408 x 5120 at 32 rows 24.4 (23.5) and 23.5 (21.3), not chosen, at
+// 80 rows 34.8 (33.1) and 33.0 (31.9), chosen all the same; 5120 x 17408 at 32 rows 23.3 (23.3) and 27.1
+// (23.2), chosen, at 96 rows 34.7 (34.8) and 36.5 (34.0), not chosen; 14336 x 5376 at 32 rows 23.2 (22.1) and
+// 20.9 (19.6), not chosen.
+inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows, double others_us, int other_variant,
+                      RowsPlan &plan)
+{
+    const Q4Device &first = *a.targets[0].w;
+    const uint32_t T = first.T;
+    if (rows > 128u) return false;
+    // 8-bit weights with byte tiles have a kernel that reads those
+    if (a.x_columns != 0 && first.codes8 != nullptr && !ctx->q8_gemm_doubled) return false;
+    plan.mf = (int)((rows + 15u) / 16u);
+    if (plan.mf < 2) plan.mf = 2;
+    if (plan.mf == 7) plan.mf = 8;
+    auto shape = [&](int which) {
+        plan.waves = which == 0 ? 4 : 8;
+        plan.ntw = which == 2 ? 2 : 1;
+        plan.blocks = 0;
+        for (uint32_t t = 0; t < a.count; ++t)
+            plan.blocks += (a.targets[t].w->NT + plan.waves * plan.ntw - 1u) / (plan.waves * plan.ntw);
+        return (uint64_t)plan.blocks * T < (1ull << 31);
+    };
+    if (ctx->force_gemm[1] >= 1) {
+        // option "q4_gemm": 11, 12, 13 = 4, 8, 16 tiles a block; 1 = whole blocks, s = 64 (s - 1) workgroups
+        if (ctx->force_gemm[0] < 11 || ctx->force_gemm[0] > 13 || !shape(ctx->force_gemm[0] - 11)) return false;
+        const uint32_t groups = ctx->force_gemm[1] == 1 ? plan.blocks : 64u * (uint32_t)(ctx->force_gemm[1] - 1);
+        plan.units = (plan.blocks * T + groups - 1u) / groups;
+        return true;
+    }
+    const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
+    double outputs = 0.0, megabytes = 0.0, best_cost = 1e30;  // megabytes: 4-bit codes and their metadata
+    for (uint32_t t = 0; t < a.count; ++t) {
+        outputs += (double)rows * a.targets[t].w->N;
+        megabytes += (double)a.targets[t].w->N * first.K * 0.5625e-6;
+    }
+    RowsPlan best = plan;
+    for (int which = 0; which < 3; ++which) {
+        if (!shape(which)) return false;
+        const uint32_t total = plan.blocks * T;
+        const uint32_t lds = rows_stages(plan.mf, plan.ntw, plan.waves) * rows_stage_bytes(plan.mf, plan.ntw, plan.waves);
+        const uint32_t places = std::min(160u * 1024u / lds, 2048u / (64u * plan.waves));  // on a compute unit
+        for (const uint32_t want : {plan.blocks, cus / 2u, cus, cus + cus / 2u, 2u * cus}) {
+            plan.units = (total + want - 1u) / want;
+            const uint32_t groups = (total + plan.units - 1u) / plan.units;
+            const uint32_t together = std::min(places, (groups + cus - 1u) / cus);
+            const uint32_t rounds = (groups + cus * together - 1u) / (cus * together);
+            const double tiles = plan.waves * plan.ntw, mf = plan.mf;
+            const double alone = 0.262 + 0.107 * mf, sharing = together * (tiles * (0.0345 + 0.0058 * mf) + 0.0378 * mf);
+            double cost = 5.2 + 0.02 * megabytes + (double)rounds * plan.units * (alone > sharing ? alone : sharing);
+            if (plan.units % T != 0u && plan.units < total)
+                cost += 2.9 + 2.0e-6 * outputs * (T + plan.units - 1.0) / plan.units;
+            if (cost < best_cost) {
+                best_cost = cost;
+                best = plan;
+            }
+        }
+    }
+    plan = best;
+    if (a.count == 1u) {
+        const double large = std::min(std::max(megabytes - 20.0, 0.0), 30.0);  // (50 MB: the largest measured)
+        if (large == 0.0) others_us *= 1.04;  // both estimates' error, and one launch rather than two
+        else if (rows <= 64u) best_cost += 0.03 * large;
+        else if (variants[other_variant].bm > 64) others_us += 0.05 * large;
+    }
+    if (a.x_dtype != MI355Q_F16) best_cost += 5.0 + 0.3 * (double)rows * first.K * sizeof(_Float16) * 1e-6;
+    return best_cost <= (a.count == 1u ? others_us : 1.08 * others_us + 1.0);
+}
+
+// The call: by q4_rows_kernel as `rows_launch` says (true), else by `group` and `plans`.
+inline bool plan_gemm(const mi355q_context *ctx, const Q4LinearArgs &a, TargetPlan *plans, GroupPlan &group, RowsPlan &rows_launch)
+{
+    const uint32_t rows = a.x_dtype == MI355Q_F32 ? 2u * a.M : a.M;
+    for (uint32_t t = 0; t < a.count; ++t) {
+        uint32_t same = 0;  // gate and up, k and v: planned once
+        while (same < t && (a.targets[same].w->N != a.targets[t].w->N || a.targets[same].w->codes8 != nullptr ||
+                            a.targets[t].w->codes8 != nullptr))
+            ++same;
+        plans[t] = same < t ? plans[same] : plan_target(ctx, a, t, rows);
+    }
+    group = plan_group(ctx, a, rows, plans);
+    return rows_plan(ctx, a, rows, group.us, plans[0].variant, rows_launch);
+}
+
+}  // namespace mi355q
