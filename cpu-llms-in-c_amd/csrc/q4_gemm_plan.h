@@ -164,10 +164,17 @@ struct TargetPlan {
     double us;        // the estimate
 };
 
-// A target splits K the same way in company as alone, and two weights that each take more than half of
-// the chip without a split fill it together: such a weight splits only where that gains 12 % (17408 x 5120 at
-// 200 rows 54.3 instead of 51.7 us; a pair of them 81 instead of 101).
+// A target splits K the same way in company as alone, so that it has the same bits, and two weights that each
+// take more than half of the chip fill it together, in one round of the pipelined kernel, without splits.
+// Such a weight of up to 48 steps takes a split of the pipelined kernel only where that is estimated to gain
+// 12 %.  Seventeen pairs were 30 % faster than as launches with splits of their own, us: two of 17408 x 5120 at 200
+// rows 74 instead of 96, of 8368 x 5248 at 487 75 instead of 97.  The weight alone pays for it: up to a tenth of
+// its time with the split, a quarter where its width is no multiple of 4 (17408 x 5120 at 200 rows 52 instead of 50,
+// 6144 x 6144 at 726 61 instead of 60, 10943 x 4224 at 333 56 instead of 45).  From 52 steps on, and held back from
+// splits of the first kernel, it pays more than a pair gains (13312 x 8064 at 351 rows 90 instead of 79, 5696 x
+// 7424 at 687 77 instead of 65, 8512 x 8064 at 401 83 instead of 69).
 constexpr double kSplitWeight = 1.12;
+constexpr uint32_t kWholeSteps = 48;
 inline TargetPlan plan_target(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t target, uint32_t rows)
 {
     const Q4Device &w = *a.targets[target].w;
@@ -179,8 +186,7 @@ inline TargetPlan plan_target(const mi355q_context *ctx, const Q4LinearArgs &a, 
                        (uint64_t)rows * x_columns * sizeof(_Float16) + 16384u < (1ull << 32);
     const uint32_t T = bytes ? w.T / 2u : w.T;
     const bool pipe_ok = gemm_pipe_ok(w, rows, x_columns);
-    TargetPlan best = {bytes, 0, 1, 1e30};
-    double best_weighed = 1e30;
+    TargetPlan best = {bytes, 0, 1, 1e30}, whole = best;  // whole: without a split
     // Decomposition: BM rows x (4*NTW + EXTRA) tiles per workgroup, K split in `splits`: up to eight, of eight
     // steps or so at least.
     uint32_t ways = 0, want[8], steps[8], splits[8];
@@ -192,7 +198,6 @@ inline TargetPlan plan_target(const mi355q_context *ctx, const Q4LinearArgs &a, 
         splits[ways++] = (T + of_steps - 1u) / of_steps;
     }
     const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
-    const bool half_filled = (uint64_t)((w.NT + 15u) / 16u) * ((rows + 127u) / 128u) * 2u > cus;  // in blocks of 128 rows x 16 tiles
     Around around;
     around.outputs = (double)a.M * w.N * dtype_bytes(a.y_dtype) * 1e-6;
     around.converted = a.x_dtype != MI355Q_F16;
@@ -209,13 +214,14 @@ inline TargetPlan plan_target(const mi355q_context *ctx, const Q4LinearArgs &a, 
             around.sums = splits[i] > 1u ? splits[i] * sums : 0.0;
             const double us = launch_us(c, v >= kFirstPiped ? pipe_kernel_us(c, cus, blocks * splits[i], steps[i])
                                                             : first_kernel_us(c, cus, blocks * splits[i], steps[i]), around);
-            const double weighed = us * (splits[i] > 1u && half_filled ? kSplitWeight : 1.0);
-            if (weighed < best_weighed) {
-                best_weighed = weighed;
-                best = {bytes, v, want[i], us};
-            }
+            if (us < best.us) best = {bytes, v, want[i], us};
+            if (i == 0u && us < whole.us) whole = {bytes, v, 1u, us};
         }
     }
+    const uint64_t pipe_blocks = (uint64_t)((w.NT + 15u) / 16u) * ((rows + 127u) / 128u);  // of 128 rows x 16 tiles
+    if (best.splits > 1u && best.variant >= kFirstPiped && !bytes && T <= kWholeSteps && 2u * pipe_blocks > cus &&
+        pipe_blocks <= cus && whole.us < kSplitWeight * best.us)
+        best = whole;
     // option "q4_gemm" = "VARIANT,SPLITS" for experiments
     if (ctx->force_gemm[1] >= 1 && ctx->force_gemm[0] < kVariants && (ctx->force_gemm[0] < kFirstPiped || pipe_ok) &&
         (ctx->force_gemm[0] >= kBytesVariant) == bytes) {

@@ -1,6 +1,6 @@
 // The planner of the GEMM calls (csrc/q4_gemm_plan.h) on the host: its estimates of the pipelined kernel
-// against a schedule that hands out every workgroup, and what planning a call takes.
-//   gemm_plan            prints "schedule ok" and, a line a call, its name and microseconds
+// against a schedule that hands out every workgroup, the choice for one weight, and what planning a call takes.
+//   gemm_plan            prints "schedule ok", "choices ok" and, a line a call, its name and microseconds
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -77,21 +77,68 @@ static int check_schedules()
     return 0;
 }
 
+struct Call {
+    std::vector<Q4Device> weights;
+    Q4LinearArgs a;
+    Call(uint32_t M, uint32_t K, const std::vector<uint32_t> &widths) : weights(widths.size())
+    {
+        memset(&a, 0, sizeof a);
+        a.M = M;
+        a.count = (uint32_t)widths.size();
+        for (size_t t = 0; t < widths.size(); ++t) {
+            memset(&weights[t], 0, sizeof weights[t]);
+            weights[t].N = widths[t];
+            weights[t].K = K;
+            weights[t].NT = (widths[t] + kTileRows - 1u) / kTileRows;
+            weights[t].T = (K + kStepColumns - 1u) / kStepColumns;
+            a.targets[t].w = &weights[t];
+        }
+    }
+    Call(const Call &) = delete;
+};
+
+// The plan of a weight is what that weight alone is estimated to be fastest with, of every shape and split; only a
+// weight of up to 48 steps that takes more than half of the chip in one round of the pipelined kernel may go
+// without a split, as the fastest shape that does, for up to 12 % more.
+static int check_choices(const mi355q_context *ctx)
+{
+    std::mt19937 random(2);
+    for (int round = 0; round < 4000; ++round) {
+        const uint32_t N = round == 0 ? 13312u : 64u + (uint32_t)(random() % 17408u), T = round == 0 ? 63u : 4u + (uint32_t)(random() % 132u);
+        const uint32_t M = round == 0 ? 351u : 129u + (uint32_t)(random() % 1000u);
+        Call call(M, T * kStepColumns, {N});
+        const TargetPlan plan = plan_target(ctx, call.a, 0, M);
+        for (int v = 0; v < kBytesVariant; ++v)
+            for (uint32_t want = 1; want <= 8u && want * 8u <= T + 7u; ++want) {
+                const Variant &c = variants[v];
+                const uint32_t tpb = 4u * c.ntw + c.extra, n_blocks = (call.weights[0].NT + tpb - 1u) / tpb;
+                const uint32_t steps = (T + want - 1u) / want, splits = (T + steps - 1u) / steps;
+                const uint64_t groups = (uint64_t)n_blocks * ((M + c.bm - 1u) / c.bm) * splits;
+                Around around = {};
+                around.splits = splits;
+                around.sums = splits > 1u ? (double)splits * M * N * 4e-6 : 0.0;
+                around.outputs = (double)M * N * 2e-6;
+                around.rows = (double)M * call.weights[0].K * 2e-6;
+                around.reread = std::fmax(around.rows - 4.0, 0.0) * n_blocks;
+                const double us = launch_us(c, v >= kFirstPiped ? pipe_kernel_us(c, kCus, groups, steps)
+                                                                : first_kernel_us(c, kCus, groups, steps), around);
+                const uint32_t blocks = (call.weights[0].NT + 15u) / 16u * ((M + 127u) / 128u);
+                const bool whole = plan.splits == 1u && splits > 1u && v >= kFirstPiped && T <= 48u && 2u * blocks > kCus && blocks <= kCus;
+                if (us * (whole ? 1.12 : 1.0) < plan.us * (1.0 - 1e-9)) {
+                    printf("%u x %u at %u rows: shape %d, %u splits, %.2f us; shape %d, %u splits is estimated at %.2f\n", N,
+                           call.weights[0].K, M, plan.variant, plan.splits, plan.us, v, want, us);
+                    return 1;
+                }
+            }
+    }
+    printf("choices ok\n");
+    return 0;
+}
+
 static double planning_us(const mi355q_context *ctx, uint32_t M, uint32_t K, const std::vector<uint32_t> &widths)
 {
-    std::vector<Q4Device> weights(widths.size());
-    Q4LinearArgs a;
-    memset(&a, 0, sizeof a);
-    a.M = M;
-    a.count = (uint32_t)widths.size();
-    for (size_t t = 0; t < widths.size(); ++t) {
-        memset(&weights[t], 0, sizeof weights[t]);
-        weights[t].N = widths[t];
-        weights[t].K = K;
-        weights[t].NT = (widths[t] + kTileRows - 1u) / kTileRows;
-        weights[t].T = (K + kStepColumns - 1u) / kStepColumns;
-        a.targets[t].w = &weights[t];
-    }
+    Call call(M, K, widths);
+    const Q4LinearArgs &a = call.a;
     constexpr int kCalls = 200;
     double best = 1e30;
     volatile uint32_t sink = 0;
@@ -114,6 +161,7 @@ int main()
     mi355q_context *const ctx = (mi355q_context *)calloc(1, sizeof(mi355q_context));  // no device: what the planner reads
     if (ctx == nullptr) return 1;
     ctx->props.multiProcessorCount = (int)kCus;
+    if (check_choices(ctx) != 0) return 1;
     printf("q_k_v_32_rows %.2f\n", planning_us(ctx, 32, 5120, {6144, 1024, 1024}));
     printf("q_k_v_512_rows %.2f\n", planning_us(ctx, 512, 5120, {6144, 1024, 1024}));
     printf("gate_up_512_rows %.2f\n", planning_us(ctx, 512, 5120, {17408, 17408}));

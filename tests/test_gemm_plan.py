@@ -1,6 +1,7 @@
 """The planner of the GEMM calls (csrc/q4_gemm_plan.h) on the host, by tests/c/gemm_plan.cpp: its closed
-form for one weight and its levels for several give what handing out every workgroup gives, and a call's
-plan takes a fraction of its smallest kernel (0.4 to 0.9 us on one core; a simulated schedule for every K split of
+form for one weight and its levels for several give what handing out every workgroup gives, a weight alone takes
+the shape and K split that are estimated to be its fastest (held back for calls of several only where the
+weight fills more than half of the chip without a split and has a short chain), and a call's plan takes a fraction of its smallest kernel (0.4 to 0.9 us on one core; a simulated schedule for every K split of
 every weight took 3.5 to 7.9)."""
 import os
 import subprocess
@@ -14,8 +15,8 @@ def test_gemm_plans():
     subprocess.run(["make", "-C", os.fspath(HERE / "c"), program], check=True, capture_output=True)
     done = subprocess.run([program], capture_output=True, text=True, timeout=120)
     assert done.returncode == 0, done.stdout
-    first, *calls = done.stdout.splitlines()
-    assert first == "schedule ok" and len(calls) == 4
+    schedule, choices, *calls = done.stdout.splitlines()
+    assert schedule == "schedule ok" and choices == "choices ok" and len(calls) == 4
     for line in calls:
         name, us = line.split()
         assert float(us) < 2.5, line
