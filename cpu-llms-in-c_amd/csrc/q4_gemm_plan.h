@@ -240,7 +240,7 @@ struct GroupPlan {
 inline GroupPlan plan_group(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows, const TargetPlan *plans)
 {
     GroupPlan best = {-1, 0.0};
-    bool alike = a.count > 1u;
+    bool alike = a.count > 1u && ctx->gemm_order < 0;  // (an order asked for is that of a weight's own launch)
     for (uint32_t t = 0; t < a.count; ++t) {
         best.us += plans[t].us;
         if (t != 0u && a.x_dtype != MI355Q_F16) {  // one conversion serves them all

@@ -141,7 +141,9 @@ int mi355q_context_info(mi355q_context *ctx, mi355q_device_info *info,
  *                                               workgroup (unset: where two would not fit one round)
  *   "gemm_order" = "xcd" / "launch"             the pipelined GEMM numbers its blocks so that the row
  *                                               blocks of one tile block share an XCD's L2 / takes them
- *                                               in launch order; unset: by the number of tile blocks
+ *                                               in launch order, and above 128 rows every weight of a
+ *                                               call has a launch of its own; unset: by the number of
+ *                                               tile blocks, and the first of them in shared launches
  *   "q8_gemm"   = "doubled" / "native"          8-bit weights above 16 rows: the Q4 GEMM kernels on
  *                                               the doubled weight / the kernel on the bytes
  *                                               themselves where it applies (the default)

@@ -1,6 +1,6 @@
 // The planner of the GEMM calls (csrc/q4_gemm_plan.h) on the host: its estimates of the pipelined kernel
 // against a schedule that hands out every workgroup, the choice for one weight, and what planning a call takes.
-//   gemm_plan            prints "schedule ok", "choices ok" and, a line a call, its name and microseconds
+//   gemm_plan            prints "schedule ok", "choices ok", "order ok" and, a line a call, its name and microseconds
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -135,6 +135,25 @@ static int check_choices(const mi355q_context *ctx)
     return 0;
 }
 
+// Weights that share a launch go out one by one under option "gemm_order", whose two orders are one weight's.
+static int check_order(mi355q_context *ctx)
+{
+    Call call(512, 5120, {6144, 1024, 1024});
+    for (const int order : {-1, 0, 1}) {
+        ctx->gemm_order = order;
+        TargetPlan plans[kMaxTargets];
+        GroupPlan group;
+        RowsPlan rows;
+        if (plan_gemm(ctx, call.a, plans, group, rows) || (group.variant >= 0) != (order < 0)) {
+            printf("order %d: shape %d for the weights together\n", order, group.variant);
+            return 1;
+        }
+    }
+    ctx->gemm_order = -1;
+    printf("order ok\n");
+    return 0;
+}
+
 static double planning_us(const mi355q_context *ctx, uint32_t M, uint32_t K, const std::vector<uint32_t> &widths)
 {
     Call call(M, K, widths);
@@ -161,7 +180,8 @@ int main()
     mi355q_context *const ctx = (mi355q_context *)calloc(1, sizeof(mi355q_context));  // no device: what the planner reads
     if (ctx == nullptr) return 1;
     ctx->props.multiProcessorCount = (int)kCus;
-    if (check_choices(ctx) != 0) return 1;
+    ctx->gemm_order = -1;
+    if (check_choices(ctx) != 0 || check_order(ctx) != 0) return 1;
     printf("q_k_v_32_rows %.2f\n", planning_us(ctx, 32, 5120, {6144, 1024, 1024}));
     printf("q_k_v_512_rows %.2f\n", planning_us(ctx, 512, 5120, {6144, 1024, 1024}));
     printf("gate_up_512_rows %.2f\n", planning_us(ctx, 512, 5120, {17408, 17408}));
