@@ -11,6 +11,7 @@
 #include <emmintrin.h>
 
 #include <algorithm>
+#include <cstdio>
 #include <cstring>
 #include <new>
 
@@ -72,8 +73,9 @@ void host_outputs_free(mi355q_context *ctx)
 }
 
 // Whether a copy takes this way: a large one, to memory that the runtime does not know (it reaches pinned
-// and managed memory directly), outside of a graph's recording.  The pinned memory is made on the first
-// such copy and kept by the context; without it the runtime's copy does it.
+// and managed memory directly), outside of a graph's recording, from 16-byte aligned memory (every output's
+// place in a staging buffer is).  The pinned memory is made on the first such copy and kept by the context; without
+// it the runtime's copy does it.
 static bool host_outputs_serve(mi355q_context *ctx, const void *host, const void *device, size_t bytes)
 {
     if (bytes < kHostCopyMin || ctx->capturing || (uintptr_t)device % 16u != 0u) return false;
@@ -120,6 +122,7 @@ hipError_t copy_outputs(mi355q_context *ctx, void *host, const void *device, siz
 {
     if (!host_outputs_serve(ctx, host, device, bytes))
         return hipMemcpyAsync(host, device, bytes, hipMemcpyDeviceToHost, ctx->stream);
+    if (ctx->trace) fprintf(stderr, "mi355q: host outputs, %zu bytes in chunks of %u\n", bytes, kChunkBytes);
     HostOutputs &outputs = *ctx->host_outputs;
     const size_t parts = (bytes + kHalfBytes - 1) / kHalfBytes;  // part i passes through half i % 2
     auto part_bytes = [&](size_t i) { return (uint32_t)std::min(kHalfBytes, bytes - i * kHalfBytes); };

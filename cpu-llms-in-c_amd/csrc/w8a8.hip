@@ -778,7 +778,7 @@ int mi355q_w8a8_linear_multi(mi355q_context *ctx, const mi355q_w8a8_target *targ
         p.N[t] = weight->N;
 
         bias_bytes += (size_t)weight->N * 4u;
-        out_bytes += (size_t)M * weight->N * 4u * (targets[t].acc ? 2u : 1u);
+        out_bytes += (((size_t)M * weight->N * 4u + 15u) & ~(size_t)15u) * (targets[t].acc ? 2u : 1u);
     }
     if (!device) {
         int status = ensure_stage(ctx, 0, q_bytes + s_bytes + bias_bytes, error, error_capacity);
@@ -801,11 +801,12 @@ int mi355q_w8a8_linear_multi(mi355q_context *ctx, const mi355q_w8a8_target *targ
                 p.bias[t] = (const float *)in;
                 in += b_bytes;
             }
+            const size_t o_step = (o_bytes + 15u) & ~(size_t)15u;  // copy_outputs takes whole 16-byte pieces from its start
             p.out[t] = (float *)back;
-            back += o_bytes;
+            back += o_step;
             if (targets[t].acc) {
                 p.acc[t] = (int32_t *)back;
-                back += o_bytes;
+                back += o_step;
             }
         }
     }

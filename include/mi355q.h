@@ -166,7 +166,9 @@ int mi355q_context_set_option(mi355q_context *ctx, const char *name, const char 
                               char *error, size_t error_capacity);
 /* Counters of one context, for tests and reports (no counterpart in the reference):
  *   "chained_launches"    pairs of linears that went out as one launch (see mi355q_q4_linear_sequence)
- *   "staging_bytes"       bytes of the context's growable staging buffers
+ *   "staging_bytes"       bytes of the context's growable staging buffers (4 MiB of pinned host memory
+ *                         are not among them: the first linear with a host output of 512 KiB or
+ *                         more makes them, and they are the context's until it is destroyed)
  *   "staging_generation"  how often a staging buffer has been reallocated
  * Unknown names: status 2. */
 int mi355q_context_get(mi355q_context *ctx, const char *name, uint64_t *value,

@@ -42,3 +42,33 @@ def test_host_outputs_are_the_device_outputs(engine, gpu, N, M, y_dtype):
         gpu.free(y_device)
         gpu.free(x_device)
         weight.destroy()
+
+
+def test_w8a8_outputs_leave_in_chunks(engine, gpu, force, capfd):
+    """Every large output of a W8A8 call goes through the pinned chunks, whatever the sizes of those staged before
+    it (odd widths and an odd number of rows: multiples of 4 bytes), accumulators too."""
+    K, M, widths = 32, 331, (1001, 1003, 998)
+    rows = [engine.synth_w8_rows(5 + i, 0.02, N, K) for i, N in enumerate(widths)]
+    weights = [gpu.w8a8_prepare(r, N, K) for r, N in zip(rows, widths)]
+    q, scales = gpu.quantize_i8(engine.synth_normal_f32(9, 1.0, M * K).reshape(M, K))
+    biases = [engine.synth_normal_f32(20 + i, 1.0, N) for i, N in enumerate(widths)]
+    pointers = [[gpu.alloc(M * N * 4) for N in widths] for _ in range(2)]
+    on_device = [gpu.to_device(q), gpu.to_device(scales)] + [gpu.to_device(b) for b in biases]
+    force("trace", "1")
+    try:
+        print(f"w8a8 host outputs {M} x {widths}", flush=True)
+        capfd.readouterr()
+        got = gpu.w8a8_linear_multi(weights, widths, q, scales, biases)
+        printed = capfd.readouterr().err
+        gpu.w8a8_linear_multi_device(weights, on_device[0], on_device[1], M, on_device[2:], *pointers)
+        gpu.sync()
+        expected = [[gpu.download(p, (M, N), np.uint32) for p, N in zip(kind, widths)] for kind in pointers]
+    finally:
+        for pointer in pointers[0] + pointers[1] + on_device:
+            gpu.free(pointer)
+        for weight in weights:
+            gpu.w8a8_destroy(weight)
+    for (out, acc), out_ref, acc_ref, N in zip(got, *expected, widths):
+        assert np.any(acc_ref != 0)
+        assert np.array_equal(out.view(np.uint32), out_ref) and np.array_equal(acc.view(np.uint32), acc_ref)
+        assert printed.count(f"host outputs, {M * N * 4} bytes in chunks") == 2
