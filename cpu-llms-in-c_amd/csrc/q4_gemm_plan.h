@@ -30,20 +30,25 @@ struct Variant {
     double outputs;         // MB of outputs
     double converted[3];    // activations that are not fp16: once, MB of fp16 rows, MB of outputs
     double reread;          // MB of fp16 rows beyond an XCD's L2, by each block of tiles
+    // Pipelined kernel without a K split, outputs whose width is no multiple of 4 and which it stores one by one:
+    // a round of the chip with fp16, fp32, bf16 activations.  (One more column than 10208, 4096, 14336 by 2688, 4096,
+    // 5120 at 440, 300, 700 rows; 25 and 12 more of 8-bit codes.  Left out, 10214 x 2688 at 440 rows took 45.6 us in a
+    // shape estimated at 39, where one of the first kernel takes 34, and 23677 8-bit x 1728 at 154 rows 58 instead of 46.)
+    double narrow[3];
 };
 constexpr Variant variants[] = {
-    {128, 4, 0, 2, 13.19, 3.208, 5.98, {2.167, 3.026}, {0.0, 1.16}, 0.0, 0.0, 0.192, 0.435, {2.27, 0.36, 0.0}, 0.000},
-    {128, 2, 0, 2, 5.82, 1.628, 0.0, {1.207, 1.595}, {0.0, 0.010}, 2.52, 0.0, 0.304, 0.474, {5.72, 0.40, 0.046}, 0.007},
-    {64, 4, 0, 3, 5.54, 2.755, 0.0, {1.175, 1.820, 2.868}, {0.53, 0.0, 0.0}, 2.60, 0.0, 0.262, 0.566, {5.81, 0.27, 0.0}, 0.000},
-    {64, 4, 1, 2, 8.64, 2.275, 0.0, {1.366, 2.151}, {0.037, 0.0}, 1.82, 0.0, 0.250, 0.206, {3.96, 0.29, 0.31}, 0.002},
-    {64, 2, 0, 4, 4.16, 1.831, 0.0, {0.711, 1.054, 1.516, 1.972}, {0.41, 1.14, 0.61, 0.0}, 2.52, 0.0, 0.280, 0.498, {4.84, 0.37, 0.0}, 0.003},
-    {64, 2, 1, 2, 4.99, 1.240, 0.0, {0.918, 1.294}, {0.0, 0.21}, 2.46, 0.0, 0.279, 0.524, {4.76, 0.36, 0.21}, 0.000},
-    {128, 4, 0, 1, 4.51, 1.363, 5.31, {1.107, 0.117}, {3.93, 2.92}, 2.48, 0.24, 0.207, 0.325, {5.48, 0.18, 0.50}, 0.014},
-    {128, 4, 1, 1, 6.29, 1.545, 6.04, {1.260, 0.291}, {3.64, 1.55}, 2.40, 0.32, 0.182, 0.355, {5.22, 0.19, 0.56}, 0.011},
-    {128, 5, 0, 1, 1.25, 1.747, 6.38, {1.368, 0.627}, {9.07, 0.22}, 2.98, 0.28, 0.175, 0.363, {5.14, 0.23, 0.50}, 0.003},
+    {128, 4, 0, 2, 13.19, 3.208, 5.98, {2.167, 3.026}, {0.0, 1.16}, 0.0, 0.0, 0.192, 0.435, {2.27, 0.36, 0.0}, 0.000, {}},
+    {128, 2, 0, 2, 5.82, 1.628, 0.0, {1.207, 1.595}, {0.0, 0.010}, 2.52, 0.0, 0.304, 0.474, {5.72, 0.40, 0.046}, 0.007, {}},
+    {64, 4, 0, 3, 5.54, 2.755, 0.0, {1.175, 1.820, 2.868}, {0.53, 0.0, 0.0}, 2.60, 0.0, 0.262, 0.566, {5.81, 0.27, 0.0}, 0.000, {}},
+    {64, 4, 1, 2, 8.64, 2.275, 0.0, {1.366, 2.151}, {0.037, 0.0}, 1.82, 0.0, 0.250, 0.206, {3.96, 0.29, 0.31}, 0.002, {}},
+    {64, 2, 0, 4, 4.16, 1.831, 0.0, {0.711, 1.054, 1.516, 1.972}, {0.41, 1.14, 0.61, 0.0}, 2.52, 0.0, 0.280, 0.498, {4.84, 0.37, 0.0}, 0.003, {}},
+    {64, 2, 1, 2, 4.99, 1.240, 0.0, {0.918, 1.294}, {0.0, 0.21}, 2.46, 0.0, 0.279, 0.524, {4.76, 0.36, 0.21}, 0.000, {}},
+    {128, 4, 0, 1, 4.51, 1.363, 5.31, {1.107, 0.117}, {3.93, 2.92}, 2.48, 0.24, 0.207, 0.325, {5.48, 0.18, 0.50}, 0.014, {10.8, 3.7, 13.5}},
+    {128, 4, 1, 1, 6.29, 1.545, 6.04, {1.260, 0.291}, {3.64, 1.55}, 2.40, 0.32, 0.182, 0.355, {5.22, 0.19, 0.56}, 0.011, {12.4, 4.2, 16.0}},
+    {128, 5, 0, 1, 1.25, 1.747, 6.38, {1.368, 0.627}, {9.07, 0.22}, 2.98, 0.28, 0.175, 0.363, {5.14, 0.23, 0.50}, 0.003, {15.5, 5.3, 18.7}},
     // 16 and 13 tiles on 8-bit codes, and only for them
-    {128, 4, 0, 1, 0.88, 1.544, 9.49, {1.249, 0.535}, {5.21, 6.69}, 4.14, 0.10, 0.172, 0.031, {0.0, 0.0, 0.0}, 0.000},
-    {128, 3, 1, 1, 5.81, 1.436, 6.56, {1.144, 0.482}, {0.0, 4.74}, 4.30, 0.14, 0.208, 0.054, {0.0, 0.0, 0.0}, 0.000}};
+    {128, 4, 0, 1, 0.88, 1.544, 9.49, {1.249, 0.535}, {5.21, 6.69}, 4.14, 0.10, 0.172, 0.031, {0.0, 0.0, 0.0}, 0.000, {10.0, 3.5, 13.4}},
+    {128, 3, 1, 1, 5.81, 1.436, 6.56, {1.144, 0.482}, {0.0, 4.74}, 4.30, 0.14, 0.208, 0.054, {0.0, 0.0, 0.0}, 0.000, {9.8, 2.4, 10.0}}};
 constexpr int kVariants = sizeof variants / sizeof variants[0];
 constexpr int kFirstPiped = 6;    // the first shape of the pipelined kernel
 constexpr int kBytesVariant = 9;  // the first on 8-bit codes
@@ -97,6 +102,13 @@ inline double pipe_kernel_us(const Variant &c, uint32_t cus, uint64_t groups, ui
     double us = (double)rounds * (c.fill + (double)steps * c.step);
     if (rest != 0u) us += pipe_rest_us(c, (double)steps, (double)rest / (double)cus);
     return us;
+}
+
+// Its stores of narrow outputs (Variant::narrow), beside that.
+inline double narrow_us(const Variant &c, uint32_t cus, int x_dtype, uint64_t groups)
+{
+    const uint64_t rounds = groups <= cus ? groups != 0u : (groups + cus - 1u) / cus;
+    return c.narrow[x_dtype == MI355Q_F16 ? 0 : x_dtype == MI355Q_F32 ? 1 : 2] * (double)rounds;
 }
 
 // What each target gives a launch of several, the longest workgroups first.
@@ -169,8 +181,7 @@ struct TargetPlan {
 // Such a weight of up to 48 steps takes a split of the pipelined kernel only where that is estimated to gain
 // 12 %.  Seventeen pairs were 30 % faster than as launches with splits of their own, us: two of 17408 x 5120 at 200
 // rows 74 instead of 96, of 8368 x 5248 at 487 75 instead of 97.  The weight alone pays for it: up to a tenth of
-// its time with the split, a quarter where its width is no multiple of 4 (17408 x 5120 at 200 rows 52 instead of 50,
-// 6144 x 6144 at 726 61 instead of 60, 10943 x 4224 at 333 56 instead of 45).  From 52 steps on, and held back from
+// its time with the split (17408 x 5120 at 200 rows 52 instead of 50, 6144 x 6144 at 726 61 instead of 60).  From 52 steps on, and held back from
 // splits of the first kernel, it pays more than a pair gains (13312 x 8064 at 351 rows 90 instead of 79, 5696 x
 // 7424 at 687 77 instead of 65, 8512 x 8064 at 401 83 instead of 69).
 constexpr double kSplitWeight = 1.12;
@@ -212,8 +223,9 @@ inline TargetPlan plan_target(const mi355q_context *ctx, const Q4LinearArgs &a, 
         for (uint32_t i = 0; i < ways; ++i) {
             around.splits = splits[i];
             around.sums = splits[i] > 1u ? splits[i] * sums : 0.0;
-            const double us = launch_us(c, v >= kFirstPiped ? pipe_kernel_us(c, cus, blocks * splits[i], steps[i])
-                                                            : first_kernel_us(c, cus, blocks * splits[i], steps[i]), around);
+            double us = launch_us(c, v >= kFirstPiped ? pipe_kernel_us(c, cus, blocks * splits[i], steps[i])
+                                                      : first_kernel_us(c, cus, blocks * splits[i], steps[i]), around);
+            if (w.N % 4u != 0u && splits[i] == 1u) us += narrow_us(c, cus, a.x_dtype, blocks);
             if (us < best.us) best = {bytes, v, want[i], us};
             if (i == 0u && us < whole.us) whole = {bytes, v, 1u, us};
         }
@@ -261,6 +273,7 @@ inline GroupPlan plan_group(const mi355q_context *ctx, const Q4LinearArgs &a, ui
     GroupWork work = {};
     work.count = a.count;
     uint32_t splits[kMaxTargets], NT[kMaxTargets];
+    bool odd[kMaxTargets];  // of a width that is no multiple of 4
     Around around = {};
     around.converted = a.x_dtype != MI355Q_F16;
     around.rows = (double)rows * first.K * sizeof(_Float16) * 1e-6;
@@ -275,26 +288,30 @@ inline GroupPlan plan_group(const mi355q_context *ctx, const Q4LinearArgs &a, ui
             work.steps[at] = work.steps[at - 1u];
             splits[at] = splits[at - 1u];
             NT[at] = NT[at - 1u];
+            odd[at] = odd[at - 1u];
         }
         work.steps[at] = steps;
         splits[at] = ways;
         NT[at] = w.NT;
+        odd[at] = w.N % 4u != 0u;
     }
     for (int v = 0; v < kBytesVariant; ++v) {
         if (v >= kFirstPiped && !pipe_ok) break;
         const Variant &c = variants[v];
         const uint32_t tpb = 4u * c.ntw + c.extra, m_blocks = (rows + c.bm - 1u) / c.bm;
-        uint64_t groups = 0, steps = 0;
+        uint64_t groups = 0, steps = 0, narrow = 0;
         around.reread = 0.0;
         for (uint32_t t = 0; t < a.count; ++t) {
             const uint32_t n_blocks = (NT[t] + tpb - 1u) / tpb;
             work.groups[t] = (uint64_t)n_blocks * m_blocks * splits[t];
             groups += work.groups[t];
             steps += work.groups[t] * work.steps[t];
+            if (odd[t] && splits[t] == 1u) narrow += work.groups[t];
             around.reread += std::max(around.rows - 4.0, 0.0) * n_blocks;
         }
         const double us = launch_us(c, v >= kFirstPiped ? pipe_group_us(c, cus, work)
-                                                        : first_kernel_us(c, cus, groups, (double)steps / (double)groups), around);
+                                                        : first_kernel_us(c, cus, groups, (double)steps / (double)groups), around) +
+                          narrow_us(c, cus, a.x_dtype, narrow);
         if (us < 0.95 * alone_us && us < best.us) best = {v, us};
     }
     return best;

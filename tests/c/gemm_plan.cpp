@@ -1,6 +1,6 @@
 // The planner of the GEMM calls (csrc/q4_gemm_plan.h) on the host: its estimates of the pipelined kernel
 // against a schedule that hands out every workgroup, the choice for one weight, and what planning a call takes.
-//   gemm_plan            prints "schedule ok", "choices ok", "order ok" and, a line a call, its name and microseconds
+//   gemm_plan            prints "schedule ok", "choices ok", "widths ok", "order ok" and, a line a call, its name and microseconds
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -120,10 +120,11 @@ static int check_choices(const mi355q_context *ctx)
                 around.outputs = (double)M * N * 2e-6;
                 around.rows = (double)M * call.weights[0].K * 2e-6;
                 around.reread = std::fmax(around.rows - 4.0, 0.0) * n_blocks;
-                const double us = launch_us(c, v >= kFirstPiped ? pipe_kernel_us(c, kCus, groups, steps)
-                                                                : first_kernel_us(c, kCus, groups, steps), around);
+                double us = launch_us(c, v >= kFirstPiped ? pipe_kernel_us(c, kCus, groups, steps)
+                                                          : first_kernel_us(c, kCus, groups, steps), around);
+                if (N % 4u != 0u && splits == 1u) us += narrow_us(c, kCus, MI355Q_F16, groups);
                 const uint32_t blocks = (call.weights[0].NT + 15u) / 16u * ((M + 127u) / 128u);
-                const bool whole = plan.splits == 1u && splits > 1u && v >= kFirstPiped && T <= 48u && 2u * blocks > kCus && blocks <= kCus;
+                const bool whole = plan.splits == 1u && splits > 1u && T <= 48u && 2u * blocks > kCus && blocks <= kCus;
                 if (us * (whole ? 1.12 : 1.0) < plan.us * (1.0 - 1e-9)) {
                     printf("%u x %u at %u rows: shape %d, %u splits, %.2f us; shape %d, %u splits is estimated at %.2f\n", N,
                            call.weights[0].K, M, plan.variant, plan.splits, plan.us, v, want, us);
@@ -132,6 +133,23 @@ static int check_choices(const mi355q_context *ctx)
             }
     }
     printf("choices ok\n");
+    return 0;
+}
+
+// Outputs that the pipelined kernel stores one by one (a width that is no multiple of 4) count: 10212 columns
+// take it without a split, 10214 do not.
+static int check_widths(const mi355q_context *ctx)
+{
+    for (const uint32_t N : {10212u, 10214u}) {
+        Call call(440, 2688, {N});
+        const TargetPlan plan = plan_target(ctx, call.a, 0, 440);
+        const bool piped = plan.variant >= kFirstPiped && plan.splits == 1u;
+        if (piped != (N % 4u == 0u)) {
+            printf("%u columns: shape %d, %u splits\n", N, plan.variant, plan.splits);
+            return 1;
+        }
+    }
+    printf("widths ok\n");
     return 0;
 }
 
@@ -181,7 +199,7 @@ int main()
     if (ctx == nullptr) return 1;
     ctx->props.multiProcessorCount = (int)kCus;
     ctx->gemm_order = -1;
-    if (check_choices(ctx) != 0 || check_order(ctx) != 0) return 1;
+    if (check_choices(ctx) != 0 || check_widths(ctx) != 0 || check_order(ctx) != 0) return 1;
     printf("q_k_v_32_rows %.2f\n", planning_us(ctx, 32, 5120, {6144, 1024, 1024}));
     printf("q_k_v_512_rows %.2f\n", planning_us(ctx, 512, 5120, {6144, 1024, 1024}));
     printf("gate_up_512_rows %.2f\n", planning_us(ctx, 512, 5120, {17408, 17408}));
