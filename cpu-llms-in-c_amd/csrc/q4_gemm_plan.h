@@ -111,6 +111,10 @@ inline double narrow_us(const Variant &c, uint32_t cus, int x_dtype, uint64_t gr
     return c.narrow[x_dtype == MI355Q_F16 ? 0 : x_dtype == MI355Q_F32 ? 1 : 2] * (double)rounds;
 }
 
+// What the kernel that adds K splits takes more for each narrow output, whose row it also stores one value at a time
+// (10210, 4098, 14338 columns against four-column multiples at 150 to 700 rows: 0.5 to 5.5 us).
+constexpr double kNarrowSumUs = 0.45e-6;
+
 // What each target gives a launch of several, the longest workgroups first.
 struct GroupWork {
     uint32_t count;
@@ -225,7 +229,7 @@ inline TargetPlan plan_target(const mi355q_context *ctx, const Q4LinearArgs &a, 
             around.sums = splits[i] > 1u ? splits[i] * sums : 0.0;
             double us = launch_us(c, v >= kFirstPiped ? pipe_kernel_us(c, cus, blocks * splits[i], steps[i])
                                                       : first_kernel_us(c, cus, blocks * splits[i], steps[i]), around);
-            if (w.N % 4u != 0u && splits[i] == 1u) us += narrow_us(c, cus, a.x_dtype, blocks);
+            if (w.N % 4u != 0u) us += splits[i] == 1u ? narrow_us(c, cus, a.x_dtype, blocks) : kNarrowSumUs * a.M * w.N;
             if (us < best.us) best = {bytes, v, want[i], us};
             if (i == 0u && us < whole.us) whole = {bytes, v, 1u, us};
         }
@@ -274,6 +278,7 @@ inline GroupPlan plan_group(const mi355q_context *ctx, const Q4LinearArgs &a, ui
     work.count = a.count;
     uint32_t splits[kMaxTargets], NT[kMaxTargets];
     bool odd[kMaxTargets];  // of a width that is no multiple of 4
+    double narrow_sums = 0.0;
     Around around = {};
     around.converted = a.x_dtype != MI355Q_F16;
     around.rows = (double)rows * first.K * sizeof(_Float16) * 1e-6;
@@ -283,6 +288,7 @@ inline GroupPlan plan_group(const mi355q_context *ctx, const Q4LinearArgs &a, ui
         around.splits = std::max(around.splits, ways);
         if (ways > 1u) around.sums += (double)ways * rows * w.N * 4e-6;
         around.outputs += (double)a.M * w.N * dtype_bytes(a.y_dtype) * 1e-6;
+        if (w.N % 4u != 0u && ways > 1u) narrow_sums += kNarrowSumUs * a.M * w.N;
         uint32_t at = t;
         for (; at > 0u && work.steps[at - 1u] < steps; --at) {
             work.steps[at] = work.steps[at - 1u];
@@ -311,7 +317,7 @@ inline GroupPlan plan_group(const mi355q_context *ctx, const Q4LinearArgs &a, ui
         }
         const double us = launch_us(c, v >= kFirstPiped ? pipe_group_us(c, cus, work)
                                                         : first_kernel_us(c, cus, groups, (double)steps / (double)groups), around) +
-                          narrow_us(c, cus, a.x_dtype, narrow);
+                          narrow_us(c, cus, a.x_dtype, narrow) + narrow_sums;
         if (us < 0.95 * alone_us && us < best.us) best = {v, us};
     }
     return best;

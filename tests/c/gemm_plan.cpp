@@ -122,7 +122,7 @@ static int check_choices(const mi355q_context *ctx)
                 around.reread = std::fmax(around.rows - 4.0, 0.0) * n_blocks;
                 double us = launch_us(c, v >= kFirstPiped ? pipe_kernel_us(c, kCus, groups, steps)
                                                           : first_kernel_us(c, kCus, groups, steps), around);
-                if (N % 4u != 0u && splits == 1u) us += narrow_us(c, kCus, MI355Q_F16, groups);
+                if (N % 4u != 0u) us += splits == 1u ? narrow_us(c, kCus, MI355Q_F16, groups) : kNarrowSumUs * M * N;
                 const uint32_t blocks = (call.weights[0].NT + 15u) / 16u * ((M + 127u) / 128u);
                 const bool whole = plan.splits == 1u && splits > 1u && T <= 48u && 2u * blocks > kCus && blocks <= kCus;
                 if (us * (whole ? 1.12 : 1.0) < plan.us * (1.0 - 1e-9)) {
@@ -136,16 +136,16 @@ static int check_choices(const mi355q_context *ctx)
     return 0;
 }
 
-// Outputs that the pipelined kernel stores one by one (a width that is no multiple of 4) count: 10212 columns
-// take it without a split, 10214 do not.
+// Outputs that the pipelined kernel and the kernel that adds K splits store one by one (a width that is no
+// multiple of 4) count: 10212 columns take the first without a split, 3064 a split, two columns less or more neither.
 static int check_widths(const mi355q_context *ctx)
 {
-    for (const uint32_t N : {10212u, 10214u}) {
-        Call call(440, 2688, {N});
-        const TargetPlan plan = plan_target(ctx, call.a, 0, 440);
-        const bool piped = plan.variant >= kFirstPiped && plan.splits == 1u;
-        if (piped != (N % 4u == 0u)) {
-            printf("%u columns: shape %d, %u splits\n", N, plan.variant, plan.splits);
+    const struct { uint32_t M, K, N; } calls[] = {{440, 2688, 10212}, {440, 2688, 10214}, {345, 2560, 3064}, {345, 2560, 3062}};
+    for (const auto &of : calls) {
+        Call call(of.M, of.K, {of.N});
+        const TargetPlan plan = plan_target(ctx, call.a, 0, of.M);
+        if ((plan.variant >= kFirstPiped || plan.splits > 1u) != (of.N % 4u == 0u)) {
+            printf("%u columns: shape %d, %u splits\n", of.N, plan.variant, plan.splits);
             return 1;
         }
     }
