@@ -331,23 +331,28 @@ struct RowsPlan {
 };
 
 // The launch of q4_rows_kernel for a call's targets together; false: not the kernel for it.
-// `others`: what each target would take otherwise.
+// `others_us`: what they would take otherwise.
 // Shape and workgroups minimise a microsecond estimate fitted to 2100 timings on this GPU (14 calls
 // from 1024 x 3584 to two weights of 17408 x 5120, 17 to 128 rows, every block width, whole blocks
 // and 128 to 512 workgroups; 6 % rms): 5.2 us, 0.02 for each MB of weights, then per unit the longer of one
 // workgroup's own chain (0.26 + 0.11 us per 16 rows) and its share of the compute unit, then, where
 // workgroups share blocks, 2.9 us and the partial sums at 2 TB/s.
 //
-// Chosen where that is less than the other kernels' estimate (one weight), or less than 1.08 times it and
-// 1 us (several: theirs for small and for large calls of several weights is that much too low; us, this
-// kernel and the other: 2048 + 512 + 512 x 1024 at 48 rows 8.0 and 10.0, two of 17408 x 5120 at 64 rows 41 and
-// 50, two of 8192 x 3072 at 48 rows 17.7 and 19.7).  One weight of more than 20 MB, from HBM (the Infinity
-// Cache), this kernel and the other: 17408 x 5120 at 32 rows 24.4 (23.5) and 23.5 (21.3), not chosen, at
-// 80 rows 34.8 (33.1) and 33.0 (31.9), chosen all the same; 5120 x 17408 at 32 rows 23.3 (23.3) and 27.1
-// (23.2), chosen, at 96 rows 34.7 (34.8) and 36.5 (34.0), not chosen; 14336 x 5376 at 32 rows 23.2 (22.1) and
-// 20.9 (19.6), not chosen.
-inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows, double others_us, int other_variant,
-                      RowsPlan &plan)
+// Several weights take it where that is less than 1.08 times the other kernels' estimate and 1 us (theirs is that much too
+// low for small and for large calls of several weights; us, this kernel and the other: 2048 + 512 + 512 x 1024
+// at 48 rows 8.0 and 10.0, two of 17408 x 5120 at 64 rows 41 and 50, two of 8192 x 3072 at 48 rows 17.7 and 19.7).
+//
+// One weight takes it where that is less than 0.9 times the others' estimate, which is 1.9 us too high for one weight where
+// this one is 0.5; above 30 us, where that is little, 0.98 times.  With bf16 x, whose conversion both estimates
+// make too long, 0.98 and above 64 rows 0.95 times.  Up to 64 fp16 rows it takes it up to 1.04 times the others'
+// estimate: they lose more when the weight comes from HBM (5120 x 6144 at 32 rows, this kernel and the other from the
+// Infinity Cache 13.4 and 13.2 us, from HBM 13.7 and 14.2; 5120 x 17408 22.7 and 22.4, 22.5 and 26.3), though not
+// weights of more than 20 MB with fewer steps (17408 x 5120 at 32 rows from HBM 24.4 and 23.5, 14336 x 5376 23.2 and
+// 20.9): 0.03 us for each MB more.
+// Of 960 random calls of one weight with both kernels timed, the choice is 0.8 % slower than the better one, and 18
+// times 10 % or more (chosen up to 1.04 times the others at any number of rows and for every type: 2.4 %, 91 times; e.g.
+// 2928 x 2944 at 36 fp32 rows 18.7 instead of 16.0, 14336 x 5376 at 80 fp16 rows 31.3 instead of 28.6).
+inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows, double others_us, RowsPlan &plan)
 {
     const Q4Device &first = *a.targets[0].w;
     const uint32_t T = first.T;
@@ -401,14 +406,12 @@ inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t
         }
     }
     plan = best;
-    if (a.count == 1u) {
-        const double large = std::min(std::max(megabytes - 20.0, 0.0), 30.0);  // (50 MB: the largest measured)
-        if (large == 0.0) others_us *= 1.04;  // both estimates' error, and one launch rather than two
-        else if (rows <= 64u) best_cost += 0.03 * large;
-        else if (variants[other_variant].bm > 64) others_us += 0.05 * large;
-    }
     if (a.x_dtype != MI355Q_F16) best_cost += 5.0 + 0.3 * (double)rows * first.K * sizeof(_Float16) * 1e-6;
-    return best_cost <= (a.count == 1u ? others_us : 1.08 * others_us + 1.0);
+    if (a.count != 1u) return best_cost <= 1.08 * others_us + 1.0;
+    if (a.x_dtype == MI355Q_BF16) return best_cost <= (rows > 64u ? 0.95 : 0.98) * others_us;
+    if (a.x_dtype == MI355Q_F32 || rows > 64u) return best_cost <= (others_us < 30.0 ? 0.9 : 0.98) * others_us;
+    const double large = std::min(std::max(megabytes - 20.0, 0.0), 30.0);  // (50 MB: the largest measured)
+    return large == 0.0 ? best_cost <= 1.04 * others_us : best_cost + 0.03 * large <= others_us;
 }
 
 // The call: by q4_rows_kernel as `rows_launch` says (true), else by `group` and `plans`.
@@ -423,7 +426,7 @@ inline bool plan_gemm(const mi355q_context *ctx, const Q4LinearArgs &a, TargetPl
         plans[t] = same < t ? plans[same] : plan_target(ctx, a, t, rows);
     }
     group = plan_group(ctx, a, rows, plans);
-    return rows_plan(ctx, a, rows, group.us, plans[0].variant, rows_launch);
+    return rows_plan(ctx, a, rows, group.us, rows_launch);
 }
 
 }  // namespace mi355q

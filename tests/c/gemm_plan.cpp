@@ -1,6 +1,6 @@
 // The planner of the GEMM calls (csrc/q4_gemm_plan.h) on the host: its estimates of the pipelined kernel
 // against a schedule that hands out every workgroup, the choice for one weight, and what planning a call takes.
-//   gemm_plan            prints "schedule ok", "choices ok", "widths ok", "order ok" and, a line a call, its name and microseconds
+//   gemm_plan            prints "schedule ok", "choices ok", "widths ok", "rows ok", "order ok" and, a line a call, its name and microseconds
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -153,6 +153,29 @@ static int check_widths(const mi355q_context *ctx)
     return 0;
 }
 
+// One weight at 17 to 128 rows takes the kernel that was timed faster for it, q4_rows_kernel or another.
+static int check_rows(const mi355q_context *ctx)
+{
+    const struct { uint32_t M, K, N; int x; bool by_rows; } calls[] = {
+        {36, 2944, 2928, MI355Q_F32, false}, {28, 5120, 1280, MI355Q_F32, false}, {80, 5376, 14336, MI355Q_F16, false},
+        {96, 5376, 14336, MI355Q_BF16, false}, {100, 3584, 1024, MI355Q_F16, false}, {32, 6144, 5120, MI355Q_F16, true}, {32, 17408, 5120, MI355Q_F16, true},
+        {67, 17408, 5120, MI355Q_F16, true}, {48, 2048, 1024, MI355Q_F16, true}, {36, 1152, 12000, MI355Q_BF16, true}};
+    for (const auto &of : calls) {
+        Call call(of.M, of.K, {of.N});
+        call.a.x_dtype = of.x;
+        call.a.y_dtype = of.x;
+        TargetPlan plans[kMaxTargets];
+        GroupPlan group;
+        RowsPlan rows;
+        if (plan_gemm(ctx, call.a, plans, group, rows) != of.by_rows) {
+            printf("%u x %u at %u rows of type %d: the other kernel\n", of.N, of.K, of.M, of.x);
+            return 1;
+        }
+    }
+    printf("rows ok\n");
+    return 0;
+}
+
 // Weights that share a launch go out one by one under option "gemm_order", whose two orders are one weight's.
 static int check_order(mi355q_context *ctx)
 {
@@ -199,7 +222,7 @@ int main()
     if (ctx == nullptr) return 1;
     ctx->props.multiProcessorCount = (int)kCus;
     ctx->gemm_order = -1;
-    if (check_choices(ctx) != 0 || check_widths(ctx) != 0 || check_order(ctx) != 0) return 1;
+    if (check_choices(ctx) != 0 || check_widths(ctx) != 0 || check_rows(ctx) != 0 || check_order(ctx) != 0) return 1;
     printf("q_k_v_32_rows %.2f\n", planning_us(ctx, 32, 5120, {6144, 1024, 1024}));
     printf("q_k_v_512_rows %.2f\n", planning_us(ctx, 512, 5120, {6144, 1024, 1024}));
     printf("gate_up_512_rows %.2f\n", planning_us(ctx, 512, 5120, {17408, 17408}));
