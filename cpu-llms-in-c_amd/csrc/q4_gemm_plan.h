@@ -342,17 +342,20 @@ struct RowsPlan {
 // low for small and for large calls of several weights; us, this kernel and the other: 2048 + 512 + 512 x 1024
 // at 48 rows 8.0 and 10.0, two of 17408 x 5120 at 64 rows 41 and 50, two of 8192 x 3072 at 48 rows 17.7 and 19.7).
 //
-// One weight takes it where that is less than 0.9 times the others' estimate, which is 1.9 us too high for one weight where
-// this one is 0.5; above 30 us, where that is little, 0.98 times.  With bf16 x, whose conversion both estimates
-// make too long, 0.98 and above 64 rows 0.95 times.  Up to 64 fp16 rows it takes it up to 1.04 times the others'
-// estimate: they lose more when the weight comes from HBM (5120 x 6144 at 32 rows, this kernel and the other from the
-// Infinity Cache 13.4 and 13.2 us, from HBM 13.7 and 14.2; 5120 x 17408 22.7 and 22.4, 22.5 and 26.3), though not
-// weights of more than 20 MB with fewer steps (17408 x 5120 at 32 rows from HBM 24.4 and 23.5, 14336 x 5376 23.2 and
-// 20.9): 0.03 us for each MB more.
+// One weight takes it where that is less than 0.9 times the others' estimate, which is 1.9 us too high for one weight
+// where this one is 0.5; above 30 us, where that is little, 0.98 times.  With bf16 x, whose conversion both
+// estimates make too long, 0.98 and above 64 rows 0.95 times.  More than 64 fp16 rows, a weight of more than 45 MB
+// and the pipelined kernel otherwise: up to 1.5 us more (17408 x 5120 at 67 rows, this kernel and the other from HBM 30.7
+// and 31.3 us, though at 80 33.8 and 32.2; 14336 x 5376 at 67 30.3 and 28.4).  Up to 64 fp16 rows: up to 1.04 times the
+// others' estimate, for they lose more when the weight comes from HBM (5120 x 6144 at 32 rows from the Infinity
+// Cache 13.4 and 13.2, from HBM 13.7 and 14.2; 5120 x 17408 22.7 and 22.4, 22.5 and 26.3), though not weights of
+// more than 20 MB with fewer steps (17408 x 5120 at 32 rows from HBM 24.4 and 23.5, 14336 x 5376 23.2 and 20.9):
+// 0.03 us for each MB more.
 // Of 960 random calls of one weight with both kernels timed, the choice is 0.8 % slower than the better one, and 18
 // times 10 % or more (chosen up to 1.04 times the others at any number of rows and for every type: 2.4 %, 91 times; e.g.
 // 2928 x 2944 at 36 fp32 rows 18.7 instead of 16.0, 14336 x 5376 at 80 fp16 rows 31.3 instead of 28.6).
-inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows, double others_us, RowsPlan &plan)
+inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows, double others_us, int other_variant,
+                      RowsPlan &plan)
 {
     const Q4Device &first = *a.targets[0].w;
     const uint32_t T = first.T;
@@ -409,6 +412,8 @@ inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t
     if (a.x_dtype != MI355Q_F16) best_cost += 5.0 + 0.3 * (double)rows * first.K * sizeof(_Float16) * 1e-6;
     if (a.count != 1u) return best_cost <= 1.08 * others_us + 1.0;
     if (a.x_dtype == MI355Q_BF16) return best_cost <= (rows > 64u ? 0.95 : 0.98) * others_us;
+    if (a.x_dtype == MI355Q_F16 && rows > 64u && megabytes > 45.0 && other_variant >= kFirstPiped)
+        return best_cost <= others_us + 1.5;
     if (a.x_dtype == MI355Q_F32 || rows > 64u) return best_cost <= (others_us < 30.0 ? 0.9 : 0.98) * others_us;
     const double large = std::min(std::max(megabytes - 20.0, 0.0), 30.0);  // (50 MB: the largest measured)
     return large == 0.0 ? best_cost <= 1.04 * others_us : best_cost + 0.03 * large <= others_us;
@@ -426,7 +431,7 @@ inline bool plan_gemm(const mi355q_context *ctx, const Q4LinearArgs &a, TargetPl
         plans[t] = same < t ? plans[same] : plan_target(ctx, a, t, rows);
     }
     group = plan_group(ctx, a, rows, plans);
-    return rows_plan(ctx, a, rows, group.us, rows_launch);
+    return rows_plan(ctx, a, rows, group.us, plans[0].variant, rows_launch);
 }
 
 }  // namespace mi355q

@@ -159,7 +159,7 @@ static int check_rows(const mi355q_context *ctx)
     const struct { uint32_t M, K, N; int x; bool by_rows; } calls[] = {
         {36, 2944, 2928, MI355Q_F32, false}, {28, 5120, 1280, MI355Q_F32, false}, {80, 5376, 14336, MI355Q_F16, false},
         {96, 5376, 14336, MI355Q_BF16, false}, {100, 3584, 1024, MI355Q_F16, false}, {32, 6144, 5120, MI355Q_F16, true}, {32, 17408, 5120, MI355Q_F16, true},
-        {67, 17408, 5120, MI355Q_F16, true}, {48, 2048, 1024, MI355Q_F16, true}, {36, 1152, 12000, MI355Q_BF16, true}};
+        {67, 17408, 5120, MI355Q_F16, true}, {67, 5120, 17408, MI355Q_F16, true}, {48, 2048, 1024, MI355Q_F16, true}, {36, 1152, 12000, MI355Q_BF16, true}};
     for (const auto &of : calls) {
         Call call(of.M, of.K, {of.N});
         call.a.x_dtype = of.x;
