@@ -547,6 +547,29 @@ def test_targets_in_one_launch(engine, gpu, force, forced, x_dtype, y_dtype, M):
             weight.destroy()
 
 
+@pytest.mark.parametrize("forced", ["7,1", "7,3"])
+def test_load_forms_of_targets_in_one_launch(engine, gpu, force, forced):
+    """The 17-tile shape for several weights, like the one for one weight, gives the same bits with hand-scheduled and
+    with compiler-managed weight loads, and those of each weight alone."""
+    K, M, widths, kind = 1152, 260, (560, 1104), engine.META_BF16_PLANES
+    weights = [gpu.q4_prepare(*engine.synth_q4_affine(171 + i, 0.02, N, K, kind), N, K, kind) for i, N in enumerate(widths)]
+    x = make_x(engine, 173, M, K).astype(np.float16)
+    force("q4_gemm", forced)
+    try:
+        print(f"gemm load forms of two weights forced={forced}", flush=True)
+        scheduled = gpu.q4_linear_multi(weights, x, engine.F16, engine.F32)
+        force("gemm_loads", "plain")
+        plain = gpu.q4_linear_multi(weights, x, engine.F16, engine.F32)
+        alone = [gpu.q4_linear(w, x, engine.F16, engine.F32) for w in weights]
+    finally:
+        for weight in weights:
+            weight.destroy()
+    for one, other, by_itself in zip(scheduled, plain, alone):
+        assert np.any(by_itself != 0)
+        assert np.array_equal(one.view(np.uint32), by_itself.view(np.uint32))
+        assert np.array_equal(other.view(np.uint32), by_itself.view(np.uint32))
+
+
 @pytest.mark.parametrize("K", [64, 512, 576, 1024, 1088, 1536, 1600, 2048, 2112, 4096, 4160, 6144, 6208, 8192, 8256, 18432, 18496])
 def test_row_lengths_of_converted_activations(engine, oracle, gpu, K):
     """The conversion's forms by row length (a wave or a workgroup a row, so many columns a thread, a row
