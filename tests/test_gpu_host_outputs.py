@@ -1,7 +1,7 @@
 """Outputs that leave for the caller's memory in chunks (512 KiB and more) are the bytes that the same call
 leaves in device memory: at the smallest such output and one below it, at whole halves of the pinned memory
 they pass through and one output beyond, at ends that are no multiple of 16 bytes, through each half more
-than once, and for two calls one after the other."""
+than once, and for two calls one after the other; and so with every entry point that has them."""
 import numpy as np
 import pytest
 
@@ -13,10 +13,10 @@ HALF = 2 << 20
 @pytest.mark.parametrize("N,M,y_dtype", [
     (4096, 32, "F32"),        # 512 KiB
     (4095, 32, "F32"),        # below: the runtime's own copy
-    (1023, 513, "F16"),       # odd fp16 columns: the last chunk ends at 2 bytes of 16
+    (1023, 513, "F16"),       # odd fp16 columns: the last chunk ends at 14 bytes of 16
     (4096, 128, "F32"),       # one half
     (HALF // 4 + 1, 1, "F32"),  # one half and 4 bytes
-    (HALF // 2 - 3, 1, "F16"),  # half a half less 6 bytes, one row
+    (HALF // 2 - 3, 1, "F16"),  # one half less 6 bytes, one row
     (4097, 256, "F32"),       # two halves and 1 KiB
     (3001, 700, "BF16"),
     (2049, 1100, "F32"),      # five parts
@@ -72,3 +72,51 @@ def test_w8a8_outputs_leave_in_chunks(engine, gpu, force, capfd):
         assert np.any(acc_ref != 0)
         assert np.array_equal(out.view(np.uint32), out_ref) and np.array_equal(acc.view(np.uint32), acc_ref)
         assert printed.count(f"host outputs, {M * N * 4} bytes in chunks") == 2
+
+
+def test_several_q4_outputs_leave_in_chunks(engine, gpu, force, capfd):
+    """Outputs of one call one after the other through the same pinned halves: the first of more than one half, the
+    second of two and more."""
+    K, M, widths, kind = 128, 521, (1003, 2049), engine.META_F16_INTERLEAVED
+    weights = [gpu.q4_prepare(*engine.synth_q4_affine(31 + i, 0.02, N, K, kind), N, K, kind) for i, N in enumerate(widths)]
+    x = engine.synth_normal_f16(33, 1.0, M * K).reshape(M, K)
+    x_ptr, pointers = gpu.to_device(x), [gpu.alloc(M * N * 4) for N in widths]
+    force("trace", "1")
+    try:
+        for _ in range(2):
+            print(f"q4 host outputs {M} x {widths}", flush=True)
+            capfd.readouterr()
+            got = gpu.q4_linear_multi(weights, x, engine.F16, engine.F32)
+            printed = capfd.readouterr().err
+            gpu.q4_sequence(engine.make_calls([(list(zip(weights, pointers)), x_ptr, engine.F16, M, engine.F32)]))
+            gpu.sync()
+            for y, pointer, N in zip(got, pointers, widths):
+                assert np.array_equal(y.view(np.uint32), gpu.download(pointer, (M, N), np.uint32))
+                assert printed.count(f"host outputs, {M * N * 4} bytes in chunks") == 1
+    finally:
+        for pointer in pointers + [x_ptr]:
+            gpu.free(pointer)
+        for weight in weights:
+            weight.destroy()
+
+
+@pytest.mark.parametrize("M", [12, 150])  # the streaming kernel's rows, the GEMM's
+def test_q8_outputs_leave_in_chunks(engine, gpu, force, capfd, M):
+    N, K = 16411, 128
+    records = engine.synth_w8_rows(41, 0.02, N, K)
+    weight = gpu.q8rows_prepare(records, N, K)
+    x = engine.synth_normal_f16(42, 1.0, M * K).reshape(M, K)
+    x_ptr, pointer = gpu.to_device(x), gpu.alloc(M * N * 4)
+    force("trace", "1")
+    try:
+        print(f"q8 host outputs {M} x {N}", flush=True)
+        capfd.readouterr()
+        got = gpu.q8_linear(weight, N, x, engine.F16, engine.F32)
+        printed = capfd.readouterr().err
+        gpu.q8_linear_device(weight, x_ptr, engine.F16, M, pointer, engine.F32, asynchronous=False)
+        assert np.array_equal(got.view(np.uint32), gpu.download(pointer, (M, N), np.uint32)) and np.any(got != 0)
+        assert printed.count(f"host outputs, {M * N * 4} bytes in chunks") == 1
+    finally:
+        gpu.free(pointer)
+        gpu.free(x_ptr)
+        gpu.q8_destroy(weight)

@@ -5,6 +5,8 @@ The GEMM rounds each weight to fp16 before an fp16 x fp16 multiply with fp32 acc
 the gate compares with the oracle's fp16-weight flavour in double accumulation:
 max_i |y_i - ref_i| / max(|ref_i|, 1e-2*rms(ref)) <= 1e-3.  The distance to the exact-weight
 result is reported against rms(ref) (the weight rounding itself, ~2^-12 per weight)."""
+import re
+
 import numpy as np
 import pytest
 
@@ -547,6 +549,53 @@ def test_targets_in_one_launch(engine, gpu, force, forced, x_dtype, y_dtype, M):
             weight.destroy()
 
 
+@pytest.mark.parametrize("x_dtype,y_dtype,M,K,widths,moved", [
+    ("F16", "F16", 200, 3072, (17408, 64), True),           # no split beside three, first kernel -> pipelined
+    ("F16", "F32", 512, 5120, (6144, 1024, 1024), True),    # two splits beside four
+    ("BF16", "BF16", 300, 3072, (6144, 102), False),        # a width that is no multiple of 4
+    ("F16", "F32", 300, 1088, (5120, 64), False),           # K an odd multiple of 64
+    ("F32", "F32", 130, 2112, (5120, 64), False),           # the same, pairs of rows
+    ("F32", "F16", 200, 1600, (5120, 100, 64), True)])      # three weights, 17 tiles alone
+def test_targets_whose_plans_differ(engine, gpu, force, capfd, x_dtype, y_dtype, M, K, widths, moved):
+    """Weights of one launch whose own plans have different K splits, and (moved) another shape or kernel than the
+    launch they share: the bits of each weight's own call, in both orders, with full residual rows."""
+    x32 = make_x(engine, 181, M, K)
+    x = x32 if x_dtype == "F32" else x32.astype(np.float16) if x_dtype == "F16" else bf16_bits(x32).reshape(M, K)
+    kind, x_dtype, y_dtype = engine.META_BF16_PLANES, getattr(engine, x_dtype), getattr(engine, y_dtype)
+    cell = np.uint32 if y_dtype == engine.F32 else np.uint16
+    weights = [gpu.q4_prepare(*engine.synth_q4_affine(182 + i, 0.02, N, K, kind), N, K, kind) for i, N in enumerate(widths)]
+    residuals = [gpu.to_device(engine.synth_normal_f32(190 + i, 1.0, M * N)) for i, N in enumerate(widths)]
+    x_ptr = gpu.to_device(x)
+    outputs = [gpu.alloc(M * N * np.dtype(cell).itemsize) for N in widths]
+    force("trace", "1")
+    try:
+        results, plans = [], []
+        targets = list(zip(weights, outputs, residuals))
+        for groups in ([targets], [targets[::-1]], [[t] for t in targets]):
+            print(f"gemm differing plans M={M} K={K} widths={widths} calls={len(groups)}", flush=True)
+            for pointer, N in zip(outputs, widths):
+                gpu.upload(pointer, np.full((M, N), 0x7FFF, cell))
+            capfd.readouterr()
+            gpu.q4_sequence(engine.make_calls([(g, x_ptr, x_dtype, M, y_dtype, engine.F32) for g in groups]))
+            gpu.sync()
+            printed = capfd.readouterr().err
+            plans.append([(int(v), int(s), same != "") for v, s, same in
+                          re.findall(r"q4 gemm .* -> variant (\d+) .*, K split (\d+)(, same launch)?\n", printed)])
+            results.append([gpu.download(p, (M, N), cell) for p, N in zip(outputs, widths)])
+    finally:
+        for pointer in [x_ptr] + outputs + residuals:
+            gpu.free(pointer)
+        for weight in weights:
+            weight.destroy()
+    together, reverse, alone = plans
+    assert [p[2] for p in together] == [False] + [True] * (len(widths) - 1) and not any(p[2] for p in alone)
+    assert [p[1] for p in together] == [p[1] for p in alone] == [p[1] for p in reverse[::-1]]
+    assert len({p[1] for p in alone}) > 1 and any(p[0] != together[0][0] for p in alone) == moved
+    for one, other, by_itself in zip(*results):
+        assert np.any(by_itself != 0) and not np.any(by_itself == 0x7FFF)
+        assert np.array_equal(one, by_itself) and np.array_equal(other, by_itself)
+
+
 @pytest.mark.parametrize("forced", ["7,1", "7,3"])
 def test_load_forms_of_targets_in_one_launch(engine, gpu, force, forced):
     """The 17-tile shape for several weights, like the one for one weight, gives the same bits with hand-scheduled and
@@ -583,10 +632,15 @@ def test_row_lengths_of_converted_activations(engine, oracle, gpu, K):
         print(f"converted rows K={K}", flush=True)
         y = gpu.q4_linear(weight, x, engine.F32, engine.F32)
         y_bf = gpu.q4_linear(weight, bf16_bits(x).reshape(M, K), engine.BF16, engine.F32)
+        rows = gpu.q4_dequant_rows(weight, np.arange(N, dtype=np.uint32))
     finally:
         weight.destroy()
     exact_rows = oracle.q4_linear(quants, meta_a, meta_b, kind, N, K, bf16_bits(x).reshape(M, K), oracle.X_BF16, M)
     # five fp32 rows are ten rows of the streaming kernel, which keeps the weight exact
     exact = oracle.q4_linear(quants, meta_a, meta_b, kind, N, K, x, oracle.X_F32, M)
     assert q4_relative_error(y[:4], exact[:4]) <= 1e-3 and q4_relative_error(y_bf[:4], exact_rows[:4]) <= 1e-3
+    # value and remainder keep a row's numbers to 2^-22 of its largest, whose errors add like noise: 8 of that scale
+    # at most.  Without the remainders the oracle's row without outliers is 290 to 970 of it off
+    scale = 2.0 ** -22 * np.abs(x).max(axis=1, keepdims=True) * np.sqrt(np.sum(rows.astype(np.float64) ** 2, axis=1))
+    assert np.all(np.abs(y[:4] - exact[:4]) <= 8.0 * scale[:4])
     assert np.all(y[4] == 0.0) and np.all(y_bf[4] == 0.0)
