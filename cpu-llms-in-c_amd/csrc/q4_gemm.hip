@@ -44,14 +44,10 @@
 namespace mi355q {
 
 // the pipelined kernel's instantiations live in q4_gemm_pipe_*.hip
-extern template __global__ void q4_gemm_pipe_kernel<128, 4, false, false>(const GemmParams);
-extern template __global__ void q4_gemm_pipe_kernel<128, 4, true, false>(const GemmParams);
-extern template __global__ void q4_gemm_pipe_kernel<128, 4, true, true>(const GemmParams);
-extern template __global__ void q4_gemm_pipe_kernel<128, 5, false, false>(const GemmParams);
-extern template __global__ void q4_gemm_pipe_kernel<128, 4, false, false, false, true>(const GemmGroup);
-extern template __global__ void q4_gemm_pipe_kernel<128, 4, true, false, false, true>(const GemmGroup);
-extern template __global__ void q4_gemm_pipe_kernel<128, 4, true, true, false, true>(const GemmGroup);
-extern template __global__ void q4_gemm_pipe_kernel<128, 5, false, false, false, true>(const GemmGroup);
+extern template __global__ void q4_gemm_pipe_kernel<128, 4, false, false>(const GemmGroup);
+extern template __global__ void q4_gemm_pipe_kernel<128, 4, true, false>(const GemmGroup);
+extern template __global__ void q4_gemm_pipe_kernel<128, 4, true, true>(const GemmGroup);
+extern template __global__ void q4_gemm_pipe_kernel<128, 5, false, false>(const GemmGroup);
 extern template __global__ void q4_gemm_pipe_kernel<128, 4, false, false, true>(const GemmParams);  // 8-bit codes
 extern template __global__ void q4_gemm_pipe_kernel<128, 3, true, false, true>(const GemmParams);   // 8-bit codes
 
@@ -194,37 +190,52 @@ static hipError_t launch_gemm(mi355q_context *ctx, dim3 grid, const GemmGroup &g
                        : launch(ctx, q4_gemm_kernel<BM, NTW, EXTRA, false>, grid, dim3(256), 0, p);
 }
 
-// The pipelined kernel's stage is larger than the 64 KiB a kernel gets without asking: the limit is raised once
-// per context (a context belongs to one device and serialises its calls) and build, whose flag there is SLOT: no
-// process-wide state, so contexts on different threads do not meet here; raising the limit twice is harmless.
-template <int SLOT, typename Args>
-static hipError_t launch_pipe_build(mi355q_context *ctx, void (*kernel)(Args), dim3 grid, const Args &args)
-{
-    constexpr size_t bytes = pipe_lds_bytes(128);
-    static_assert(SLOT < 16, "mi355q_context::lds_raised holds sixteen flags");
-    if (!ctx->lds_raised[SLOT]) {
-        hipError_t status = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-        if (status != hipSuccess) return status;
-        ctx->lds_raised[SLOT] = true;
-    }
-    return launch(ctx, kernel, grid, dim3(256), bytes, args);
-}
-
-// 16, 17 or 20 tiles; PLAIN: compiler-managed weight loads (option "gemm_loads" = "plain").
-template <int NTW, bool XT, bool PLAIN = false>
+// The pipelined kernel's stage is larger than the 64 KiB a kernel gets without asking: the
+// limit is raised once per device and instantiation.
+template <int NTW, bool XT>
 static hipError_t launch_pipe(mi355q_context *ctx, dim3 grid, const GemmGroup &group)
 {
-    constexpr int slot = 2 * (NTW - 4) + (PLAIN ? 3 : XT ? 1 : 0);  // 0 .. 3
-    if (group.shared.targets > 1u)
-        return launch_pipe_build<slot>(ctx, q4_gemm_pipe_kernel<128, NTW, XT, PLAIN, false, true>, grid, group);
-    return launch_pipe_build<4 + slot>(ctx, q4_gemm_pipe_kernel<128, NTW, XT, PLAIN>, grid, group.shared);
+    constexpr size_t bytes = pipe_lds_bytes(128);
+    constexpr int slot = 2 * NTW + (XT ? 1 : 0);  // this instantiation's flag in the context
+    static_assert(slot < 16, "mi355q_context::lds_raised holds sixteen flags");
+    // per context (a context belongs to one device and serialises its calls): no process-wide
+    // state, so contexts on different threads do not meet here; raising the limit twice is harmless
+    if (!ctx->lds_raised[slot]) {
+        hipError_t status = hipFuncSetAttribute((const void *)q4_gemm_pipe_kernel<128, NTW, XT>,
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        if (status != hipSuccess) return status;
+        ctx->lds_raised[slot] = true;
+    }
+    return launch(ctx, q4_gemm_pipe_kernel<128, NTW, XT>, grid, dim3(256), bytes, group);
 }
 
 // The shapes on 8-bit codes: 16 tiles, or 13 (three per wave and one shared).
 template <int NTW, bool XT>
 static hipError_t launch_pipe_bytes(mi355q_context *ctx, dim3 grid, const GemmGroup &group)
 {
-    return launch_pipe_build<XT ? 8 : 9>(ctx, q4_gemm_pipe_kernel<128, NTW, XT, false, true>, grid, group.shared);
+    constexpr size_t bytes = pipe_lds_bytes(128);
+    constexpr int slot = XT ? 13 : 14;
+    if (!ctx->lds_raised[slot]) {
+        hipError_t status = hipFuncSetAttribute((const void *)q4_gemm_pipe_kernel<128, NTW, XT, false, true>,
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        if (status != hipSuccess) return status;
+        ctx->lds_raised[slot] = true;
+    }
+    return launch(ctx, q4_gemm_pipe_kernel<128, NTW, XT, false, true>, grid, dim3(256), bytes, group.shared);
+}
+
+// The 17-tile shape with compiler-managed weight loads (option "gemm_loads" = "plain").
+static hipError_t launch_pipe_plain(mi355q_context *ctx, dim3 grid, const GemmGroup &group)
+{
+    constexpr size_t bytes = pipe_lds_bytes(128);
+    constexpr int slot = 15;
+    if (!ctx->lds_raised[slot]) {
+        hipError_t status = hipFuncSetAttribute((const void *)q4_gemm_pipe_kernel<128, 4, true, true>,
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        if (status != hipSuccess) return status;
+        ctx->lds_raised[slot] = true;
+    }
+    return launch(ctx, q4_gemm_pipe_kernel<128, 4, true, true>, grid, dim3(256), bytes, group);
 }
 
 // Adds the K splits of a launch's targets.
@@ -395,7 +406,7 @@ static int gemm_targets(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t fir
     case 4: launched = launch_gemm<64, 2, false>(ctx, grid, group); break;
     case 5: launched = launch_gemm<64, 2, true>(ctx, grid, group); break;
     case 6: launched = launch_pipe<4, false>(ctx, grid, group); break;
-    case 7: launched = ctx->gemm_plain_loads ? launch_pipe<4, true, true>(ctx, grid, group) : launch_pipe<4, true>(ctx, grid, group); break;
+    case 7: launched = ctx->gemm_plain_loads ? launch_pipe_plain(ctx, grid, group) : launch_pipe<4, true>(ctx, grid, group); break;
     case 8: launched = launch_pipe<5, false>(ctx, grid, group); break;
     case 9: launched = launch_pipe_bytes<4, false>(ctx, grid, group); break;
     default: launched = launch_pipe_bytes<3, true>(ctx, grid, group); break;

@@ -89,10 +89,11 @@ __device__ __forceinline__ GemmParams select_target(const GemmGroup &group, uint
 }
 
 // Workgroup `index` of `total`, and the XCD it runs on is index % 8: its number when XCD i works
-// through a contiguous run of the numbers, XCDs in turn.
+// through a contiguous run of the numbers, XCDs in turn.  `total` or more: none is left for it.
 __device__ __forceinline__ uint32_t number_by_xcd(uint32_t index, uint32_t total)
 {
     const uint32_t xcd = index % 8u, base = total / 8u, longer = total % 8u;  // XCDs 0 .. longer-1 get base + 1
+    if (index / 8u >= base + (xcd < longer ? 1u : 0u)) return total;
     return (xcd < longer ? xcd * (base + 1u) : longer * (base + 1u) + (xcd - longer) * base) + index / 8u;
 }
 
@@ -119,8 +120,8 @@ __device__ __forceinline__ bool locate_block(const GemmGroup &group, uint32_t ti
         n_blocks = (p.NT + tiles_per_block - 1u) / tiles_per_block;
         m_blocks = (p.M + rows_per_block - 1u) / rows_per_block;
         const uint32_t total = n_blocks * m_blocks * p.splits;
-        if (index / 8u >= total / 8u + (index % 8u < total % 8u ? 1u : 0u)) return false;  // the range's last, rounded up to eight
         number = number_by_xcd(index, total);
+        if (number >= total) return false;
     } else if (p.xcd_order) {
         number = number_by_xcd(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z),
                                gridDim.x * gridDim.y * gridDim.z);
@@ -476,12 +477,7 @@ __device__ __forceinline__ void gemm_workgroup(const GemmParams &p, uint32_t blo
 
 // One weight, and several: the choice of the target in the same kernel made one weight's launches, the
 // smallest most of all, 0.5 to 0.9 us longer (2048 x 1024 at 256 rows 12.0 -> 12.5, 1280 x 1280 at 150
-// fp32 rows 15.1 -> 16.0).
-// The block's numbers are moved to scalar registers (their divisions leave them in vector registers, where the
-// compiler no longer knows that a workgroup has one of each): without that 128 rows x 16 tiles spilled 22 registers and
-// 64 x 17 four, and 64 x 16 fitted two to a compute unit where the estimates count on three.  Now the kernels take what
-// one weight's take (us: two of 6080 x 3008 at 331 rows 58.3 -> 46.6; two of 6000 x 4096 at 400 rows, 128 x 16
-// 145 -> 75, 64 x 17 76.6 -> 74.1, the other shapes 0 to 3 % less).
+// fp32 rows 15.1 -> 16.0; the pipelined kernel's did not change).
 template <int BM, int NTW, bool EXTRA, bool CONVERTED>
 __global__ void __launch_bounds__(256, 2) q4_gemm_kernel(const GemmParams p)
 {
@@ -493,6 +489,11 @@ __global__ void __launch_bounds__(256, 2) q4_gemm_group_kernel(const GemmGroup g
     GemmParams p;
     uint32_t block_n, block_m, split;
     if (!locate_block(group, 4 * NTW + (EXTRA ? 1 : 0), BM, p, block_n, block_m, split)) return;
+    // The divisions leave the three in vector registers, where the compiler no longer knows that a workgroup
+    // has one of each: 128 rows x 16 tiles then spilled 22 registers and 64 x 17 four, and 64 x 16 fitted two
+    // to a compute unit where the estimates count on three.  In scalar registers they take what one weight's
+    // kernels take (us: two of 6080 x 3008 at 331 rows 58.3 -> 46.6; two of 6000 x 4096 at 400 rows, 128 x 16
+    // 145 -> 75, 64 x 17 76.6 -> 74.1, the other shapes 0 to 3 % less).
     block_n = __builtin_amdgcn_readfirstlane(block_n);
     block_m = __builtin_amdgcn_readfirstlane(block_m);
     split = __builtin_amdgcn_readfirstlane(split);
@@ -662,16 +663,12 @@ __device__ __forceinline__ void load_x2(u32x2 &to, uint32_t lane_offset, const c
 // Q8: the weights are 8-bit codes in tiles of the same rows and columns (2 KiB per tile and step:
 // [step][tile][half][lane] of 16 bytes, half h = quarters 2h and 2h + 1, a lane's eight columns
 // of a quarter in order), with the same fp16 {scale, bias} records: one code register more per
-// tile and step, the same three vector instructions per pair of weights.
-//
-// SEVERAL: the weights of a call in one launch.  One weight has a build of its own, whose parameters are fewer and
-// asked for at once: with a group's its launches, of any shape, took 0.3 to 0.6 us more (16 tiles, us: 8320 x 3968 at
-// 464 rows 42.2 -> 42.8, 6144 x 1024 at 300 15.4 -> 15.7; 8-bit codes, whose calls have one weight, 25600 x 5120 at
-// 256 rows 70.7 -> 71.25).
-template <bool SEVERAL>
-using PipeArgs = std::conditional_t<SEVERAL, GemmGroup, GemmParams>;
-template <int BM, int NTW, bool XT, bool PLAIN = false, bool Q8 = false, bool SEVERAL = false>
-__global__ void __launch_bounds__(256, 1) q4_gemm_pipe_kernel(const PipeArgs<SEVERAL> args)
+// tile and step, the same three vector instructions per pair of weights.  Its calls have one
+// weight (with a group's parameters 25600 x 5120 at 256 rows took 0.7 % longer: 71.25 us, not 70.7).
+template <bool Q8>
+using PipeArgs = std::conditional_t<Q8, GemmParams, GemmGroup>;
+template <int BM, int NTW, bool XT, bool PLAIN = false, bool Q8 = false>
+__global__ void __launch_bounds__(256, 1) q4_gemm_pipe_kernel(const PipeArgs<Q8> args)
 {
     extern __shared__ uint4 a_lds_raw[];  // [buffer][row][slot], slot = octet ^ (row % 16)
     typedef uint4 (*stage_rows)[16];

@@ -1,9 +1,9 @@
-// The pipelined affine-Q4 GEMM kernel, 17 tiles per workgroup with compiler-managed weight loads (option
-// "gemm_loads" = "plain"), for one weight: one instantiation per file so that they compile side by side.
+// The pipelined affine-Q4 GEMM kernel, 17 tiles per workgroup with compiler-managed weight loads (option "gemm_loads" = "plain"): one instantiation per file so that they
+// compile side by side.
 #include "q4_gemm_device.h"
 
 namespace mi355q {
 
-template __global__ void q4_gemm_pipe_kernel<128, 4, true, true>(const GemmParams);
+template __global__ void q4_gemm_pipe_kernel<128, 4, true, true>(const GemmGroup);
 
 }  // namespace mi355q
