@@ -114,7 +114,7 @@ __device__ __forceinline__ bool locate_block(const GemmGroup &group, uint32_t ti
     block_m = blockIdx.y;
     split = blockIdx.z;
     uint32_t n_blocks = gridDim.x, m_blocks = gridDim.y, number;
-    if (p.targets > 1u) {
+    if (__builtin_expect(p.targets > 1u, 0)) {  // out of one weight's way
         uint32_t index = blockIdx.x;
         p = select_target(group, index);
         n_blocks = (p.NT + tiles_per_block - 1u) / tiles_per_block;
@@ -477,7 +477,10 @@ __device__ __forceinline__ void gemm_workgroup(const GemmParams &p, uint32_t blo
 
 // One weight, and several: the choice of the target in the same kernel made one weight's launches, the
 // smallest most of all, 0.5 to 0.9 us longer (2048 x 1024 at 256 rows 12.0 -> 12.5, 1280 x 1280 at 150
-// fp32 rows 15.1 -> 16.0; the pipelined kernel's did not change).
+// fp32 rows 15.1 -> 16.0).  The pipelined kernel's became 0.3 to 0.8 us longer (8320 x 3968 at 464 rows 42.0 -> 42.7, and
+// 42.4 with the code of several weights behind the rest); but a build for each of its shapes costs a decoder layer,
+// which alternates between them, more than it gives: another kernel in the instruction caches, the four calls of a 27B
+// layer at 512 rows 336.1 -> 337.5.
 template <int BM, int NTW, bool EXTRA, bool CONVERTED>
 __global__ void __launch_bounds__(256, 2) q4_gemm_kernel(const GemmParams p)
 {
