@@ -487,7 +487,7 @@ def measure_w8a8(engine, ctx, steps, warmup, preheat_ms, with_cpu=True):
             "unit": "TOP/s",
             "frac": round(achieved / I8_MFMA_PEAK_TOPS, 5),
             "traffic": None,
-            "kernel": "w8a8_block_kernel (quantize_i8_kernel included in the time)",
+            "kernel": "w8a8_block_kernel (quantize_i8_rows_kernel included in the time)",
             "launches": timed["launches"],
             "avg_kernel_us": round(timed["kernel_ms"] * 1e3 / max(timed["launches"], 1), 3),
         },

@@ -19,15 +19,15 @@
 //   q4_gemm_kernel: two workgroups per compute unit overlap each other's
 //     dequantization and matrix instructions (six tile shapes);
 //   q4_gemm_pipe_kernel: one workgroup per compute unit, software pipelined by
-//     hand (128 rows x 16 or 17 tiles);
+//     hand (128 rows x 16, 17 or 20 tiles);
 //   q4_rows_kernel (q4_rows_device.h): up to 128 rows, all weights of a call as
 //     one launch.
-// The host picks shape and K split by a time estimate fitted on this GPU, e.g.
-// 17 tiles for the 17408-row matrices: 64 x 4 = 256 workgroups at M = 512.
+// The host picks shape and K split by a time estimate fitted on this GPU (q4_gemm_plan.h), e.g.
+// 20 tiles for the 17408-row matrices: 55 x 4 = 220 workgroups at M = 512.
 // Several weights of a call go out as one launch where that is estimated to take less: they
 // fill the chip together (us, a launch each -> one launch: 6144 + 1024 + 1024 x 5120 at 200 rows
-// 51 -> 35, at 512 rows 78 -> 53; 2048 + 512 + 512 x 1024 at 512 rows 26.5 -> 10.8; two of
-// 17408 x 5120 at 200 rows 103 -> 74; two of 8192 x 3072 at 512 rows 68 -> 43; three of 1280 x 1280
+// 51 -> 35, at 512 rows 78 -> 53; 2048 + 512 + 512 x 1024 at 512 rows 26.5 -> 10.5; two of
+// 17408 x 5120 at 200 rows 106 -> 74; two of 8192 x 3072 at 512 rows 68 -> 43; three of 1280 x 1280
 // over 1500 fp32 rows 72 -> 51).
 #include <algorithm>
 #include <cstdio>
@@ -328,7 +328,6 @@ static int gemm_targets(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t fir
     p.y_dtype = a.y_dtype;
     p.residual_dtype = a.residual_dtype;
     p.residual_is_bias = a.residual_is_bias;
-    p.tiles_per_block = tpb;
     p.targets = count;
     size_t sums = 0;  // floats of partial sums
     bool split = false;

@@ -24,7 +24,6 @@ struct GemmParams {
     const void *residual;
     float *partials;    // [splits, or workgroups that share a block][M][padded_columns(N)] when there is more than one
     uint32_t M, N, K, NT, T;
-    uint32_t tiles_per_block;
     uint32_t splits, steps_per_split;
     int y_dtype, residual_dtype;
     int residual_is_bias;  // residual is one row [N], added to every activation row

@@ -133,7 +133,11 @@ __global__ void __launch_bounds__(256) q4_stream_reduce_kernel(const StreamParam
 // back when the kernel ends, and nothing overlaps that.  Kernel time before / held in registers / stored
 // past the L2, us: 1500 rows of 1280 fp32 8.7 / 8.2 / 6.9, of 512 5.4 / 5.0 / 4.3, of 5120 13.1 / 10.9 / 11.0,
 // 150 of 5120 6.2 / 5.7 / 5.1, 4646 of 5376 bf16 19.4 / 16.8 / 16.0 (6.2 TB/s), 1000 of 2752 6.8 / 6.5 / 5.1.
-// Loading past the L2 too: 6.9, 5.2, 14.3, 5.6, 18.8, 5.7.
+// Loading past the L2 too: 6.9, 5.2, 14.3, 5.6, 18.8, 5.7.  (Behind a launch whose outputs still leave the L2s, as in an
+// encoder layer, the 1500 rows of 5120 take 15.6.)  The streaming kernel, which reads up to 16 of such rows on every
+// XCD at once, loses nothing by it: whole calls at 1 to 16 rows before and now, us: 5120 x 5120 bf16 at one row 10.6 and
+// 10.3, at eight 13.1 and 12.4, 5120 x 17408 at four 20.3 and 19.7, at eight fp32 27.6 and 27.5; 1024 and 2048 x 1024 5.6 to
+// 7.8 either way.
 constexpr uint32_t kConvertThreads = 256;
 template <bool BF16, bool WAVE, int PIECES>
 __global__ void __launch_bounds__(kConvertThreads)
