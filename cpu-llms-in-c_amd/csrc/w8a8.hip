@@ -60,7 +60,7 @@ w8a8_repack_kernel(const uint8_t *__restrict__ rows, uint4 *__restrict__ tiles,
 // Bound by the chain load, maximum, store.  Kernel time, one column a thread and access -> this, us: 64 rows of 512
 // 2.7 -> 2.3, of 1024 3.2 -> 2.4, of 2048 4.1 -> 2.7, of 4096 5.9 -> 2.8; 768 of 2048 4.8 -> 3.0; 300 of 8192 10.5 -> 3.6.
 // Quantizer and three weights: 768 rows of 2048 x 4096 46.8 -> 44.4, 300 of 2048 x 1024 14.7 -> 13.3, 64 of 1024 x 4096
-// 11.6 -> 11.2.  Stores past the L2 take the kernel as long, and the codes out of the caches that the matrix kernel
+// 11.2 -> 11.0 (two runs of one side differ by 0.2).  Stores past the L2 take the kernel as long, and the codes out of the caches that the matrix kernel
 // reads them through: 768 rows 51.
 template <bool WAVE, int PIECES>
 __global__ void __launch_bounds__(WAVE ? 64 : 256)

@@ -596,6 +596,46 @@ def test_targets_whose_plans_differ(engine, gpu, force, capfd, x_dtype, y_dtype,
         assert np.array_equal(one, by_itself) and np.array_equal(other, by_itself)
 
 
+def test_targets_in_one_launch_replayed(engine, gpu):
+    """Shared launches, their conversion and the sums behind their K splits from a recorded graph: every replay, with
+    eager calls of other sizes and new inputs between them, has the bits of the eager calls."""
+    kind, K = engine.META_BF16_PLANES, 3072
+    weights = [gpu.q4_prepare(*engine.synth_q4_affine(201 + i, 0.02, N, K, kind), N, K, kind) for i, N in enumerate((6144, 100, 1001))]
+    shapes = [(300, engine.F16, np.float16), (150, engine.F32, np.float32)]
+    x_ptrs = [gpu.alloc(M * K * 4) for M, _, _ in shapes]
+    outputs = [[gpu.alloc(M * w.N * 4) for w in weights] for M, _, _ in shapes]
+    calls = engine.make_calls([(list(zip(weights, ys)), x, dtype, M, engine.F32)
+                               for (M, dtype, _), x, ys in zip(shapes, x_ptrs, outputs)])
+    other = engine.make_calls([([(weights[1], outputs[0][1])], x_ptrs[0], engine.F16, 40, engine.F32)])
+
+    def fill(seed):
+        for (M, _, cell), pointer in zip(shapes, x_ptrs):
+            gpu.upload(pointer, make_x(engine, seed, M, K).astype(cell))
+
+    def downloaded():
+        gpu.sync()
+        return [gpu.download(y, (M, w.N), np.uint32) for (M, _, _), ys in zip(shapes, outputs) for w, y in zip(weights, ys)]
+
+    fill(1)
+    graph = gpu.q4_sequence_record(calls)
+    try:
+        for replay in range(4):
+            print(f"replay {replay} of shared launches", flush=True)
+            fill(10 + replay)
+            gpu.q4_sequence(calls)
+            eager = downloaded()
+            gpu.q4_sequence(other)
+            gpu.graph_launch(graph)
+            for one, two in zip(eager, downloaded()):
+                assert np.any(one != 0) and np.array_equal(one, two)
+    finally:
+        gpu.graph_destroy(graph)
+        for pointer in x_ptrs + outputs[0] + outputs[1]:
+            gpu.free(pointer)
+        for weight in weights:
+            weight.destroy()
+
+
 @pytest.mark.parametrize("forced", ["7,1", "7,3"])
 def test_load_forms_of_targets_in_one_launch(engine, gpu, force, forced):
     """The 17-tile shape for several weights, like the one for one weight, gives the same bits with hand-scheduled and
