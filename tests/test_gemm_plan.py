@@ -19,6 +19,7 @@ def test_gemm_plans():
     assert done.returncode == 0, done.stdout
     *checks, a, b, c, d = done.stdout.splitlines()
     assert checks == ["schedule ok", "choices ok", "widths ok", "rows ok", "order ok"]
-    for line in (a, b, c, d):
+    # between what they take (0.9, 0.8, 0.5, 0.4) and what that schedule took (7.9, 7.2, 4.8, 3.5), for a slower host's sake
+    for line, most in zip((a, b, c, d), (5.0, 4.5, 3.0, 2.2)):
         name, us = line.split()
-        assert float(us) < 2.5, line
+        assert float(us) < most, line
