@@ -97,7 +97,7 @@ struct mi355q_context {
     int w8a8_tiles;       // option "w8a8" = "1" .. "4": tiles per W8A8 workgroup (0: chosen by the launch)
     int w8a8_blocks;      // the same option = "small" / "blocks": 4 / 8 tiles a block of the kernel of blocks
     bool lds_raised[16];  // q4_gemm_pipe_kernel instantiations whose dynamic LDS limit has been raised
-    bool rows_lds_raised[9][5];  // the same for q4_rows_kernel<fragments, tiles per wave>
+    bool rows_lds_raised[8][2][4];  // the same for q4_rows_kernel: fragments, pairs, tiles a block
     // device address of the library's fixed scratch array on this context's device (for the
     // entry point that allocates nothing); every context on the device sees the same array
     unsigned char *fixed_scratch;

@@ -422,33 +422,6 @@ static int gemm_targets(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t fir
 
 // ---- 17..128 rows: q4_rows_kernel (q4_rows_device.h) ---------------------------------------
 
-template <int MF, int NTW, int W>
-static hipError_t launch_rows(mi355q_context *ctx, uint32_t groups, const GemmGroup &group)
-{
-    constexpr uint32_t bytes = rows_lds_bytes(MF, NTW, W);
-    bool &raised = ctx->rows_lds_raised[MF][W == 4 ? 0 : NTW];
-    if (!raised) {  // per context, as in launch_pipe
-        hipError_t status = hipFuncSetAttribute((const void *)q4_rows_kernel<MF, NTW, W>,
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-        if (status != hipSuccess) return status;
-        raised = true;
-    }
-    return launch(ctx, q4_rows_kernel<MF, NTW, W>, dim3(groups), dim3(64u * W), bytes, group);
-}
-
-template <int NTW, int W>
-static hipError_t launch_rows_of(mi355q_context *ctx, int mf, uint32_t groups, const GemmGroup &group)
-{
-    switch (mf) {
-    case 2: return launch_rows<2, NTW, W>(ctx, groups, group);
-    case 3: return launch_rows<3, NTW, W>(ctx, groups, group);
-    case 4: return launch_rows<4, NTW, W>(ctx, groups, group);
-    case 5: return launch_rows<5, NTW, W>(ctx, groups, group);
-    case 6: return launch_rows<6, NTW, W>(ctx, groups, group);
-    default: return launch_rows<8, NTW, W>(ctx, groups, group);
-    }
-}
-
 static int q4_rows_linears(mi355q_context *ctx, const Q4LinearArgs &a, const RowsPlan &plan, char *error,
                            size_t error_capacity)
 {
@@ -463,6 +436,8 @@ static int q4_rows_linears(mi355q_context *ctx, const Q4LinearArgs &a, const Row
     GemmParams &p = group.shared;
     int status = gemm_activations(ctx, a, x_columns, true, p, error, error_capacity);
     if (status != MI355Q_OK) return status;
+    p.M = a.M;  // the kernel adds value and remainder rows up in one accumulator
+    p.pair = 0;
     p.K = x_columns;
     p.T = first.T;
     p.wrap_steps = a.x_columns ? a.x_columns / kStepColumns : 0xffffffffu;
@@ -472,7 +447,7 @@ static int q4_rows_linears(mi355q_context *ctx, const Q4LinearArgs &a, const Row
     p.splits = 1;
     p.units = plan.units;
     p.total_units = plan.blocks * p.T;
-    p.block_columns = (uint32_t)(plan.waves * plan.ntw) * kTileRows;
+    p.block_columns = (uint32_t)plan.tiles * kTileRows;
     p.targets = a.count;
     // blocks are shared unless every workgroup takes whole ones; a block meets at most this many
     const bool sharing = p.units % p.T != 0u && p.units < p.total_units;
@@ -496,7 +471,7 @@ static int q4_rows_linears(mi355q_context *ctx, const Q4LinearArgs &a, const Row
         target.NT = w.NT;
         target.wide_stores = w.N % 4u == 0u && (uintptr_t)target.y % 16u == 0u;
         target.first_block = blocks;
-        blocks += (w.NT + plan.waves * plan.ntw - 1u) / (plan.waves * plan.ntw);
+        blocks += (w.NT + plan.tiles - 1u) / plan.tiles;
         if (sharing) {
             target.partials = partials;
             partials += (size_t)sharers * p.M * padded_columns(w.N);
@@ -504,11 +479,11 @@ static int q4_rows_linears(mi355q_context *ctx, const Q4LinearArgs &a, const Row
     }
     const uint32_t groups = (p.total_units + p.units - 1u) / p.units;
     if (ctx->trace)
-        fprintf(stderr, "mi355q: q4 rows M=%u K=%u -> %d rows x %u columns, %u workgroups of %d waves, %u steps each\n", p.M,
-                p.K, 16 * plan.mf, p.block_columns, groups, plan.waves, p.units);
-    hipError_t launched = plan.waves == 4 ? launch_rows_of<1, 4>(ctx, plan.mf, groups, group)
-                          : plan.ntw == 1 ? launch_rows_of<1, 8>(ctx, plan.mf, groups, group)
-                                          : launch_rows_of<2, 8>(ctx, plan.mf, groups, group);
+        fprintf(stderr, "mi355q: q4 rows M=%u K=%u -> %d fragments%s x %u columns, %u workgroups, %u steps each\n", p.M, p.K,
+                plan.mf, plan.pair ? " of pairs" : "", p.block_columns, groups, p.units);
+    hipError_t launched = plan.tiles == 4    ? q4_rows_launch_4(ctx, plan.mf, plan.pair, groups, group)
+                          : plan.tiles == 8  ? q4_rows_launch_8(ctx, plan.mf, plan.pair, groups, group)
+                                             : q4_rows_launch_16(ctx, plan.mf, plan.pair, groups, group);
     if (launched != hipSuccess) return fail_hip(launched, "q4 rows kernel launch", error, error_capacity);
     if (sharing) {
         launched = launch_reduce(ctx, group);

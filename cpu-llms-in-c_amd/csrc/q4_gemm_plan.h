@@ -327,34 +327,33 @@ inline GroupPlan plan_group(const mi355q_context *ctx, const Q4LinearArgs &a, ui
 // ---- 17..128 rows: q4_rows_kernel (q4_rows_device.h) ---------------------------------------
 
 struct RowsPlan {
-    int mf, ntw, waves;            // 16-row fragments, tiles per wave, waves
+    int mf, tiles;                 // 16-row fragments of fp16 rows, tiles a block
+    bool pair;                     // fp32 activations: pairs of fp16 rows
     uint32_t blocks, units;        // blocks in all, units per workgroup
 };
 
 // The launch of q4_rows_kernel for a call's targets together; false: not the kernel for it.
 // `others_us`: what they would take otherwise.
-// Shape and workgroups minimise a microsecond estimate fitted to 2100 timings on this GPU (14 calls
-// from 1024 x 3584 to two weights of 17408 x 5120, 17 to 128 rows, every block width, whole blocks
-// and 128 to 512 workgroups; 6 % rms): 5.2 us, 0.02 for each MB of weights, then per unit the longer of one
-// workgroup's own chain (0.26 + 0.11 us per 16 rows) and its share of the compute unit, then, where
-// workgroups share blocks, 2.9 us and the partial sums at 2 TB/s.
+// Shape and workgroups minimise a microsecond estimate fitted to 2400 timings on this GPU (270 calls of one to three
+// weights from 448 x 512 to two of 17408 x 5120, 17 to 128 rows of fp16, fp32 and bf16, every block width, whole blocks
+// and 128 and 256 workgroups; 7 % rms, and the launch it chooses takes 0.6 % more than the best timed one): 5 us, each
+// unit, where workgroups share blocks 3.8 us and the partial sums at 1.8 TB/s, the conversion of activations that are not
+// fp16, the outputs.
 //
-// Several weights take it where that is less than 1.08 times the other kernels' estimate and 1 us (theirs is that much too
-// low for small and for large calls of several weights; us, this kernel and the other: 2048 + 512 + 512 x 1024
-// at 48 rows 8.0 and 10.0, two of 17408 x 5120 at 64 rows 41 and 50, two of 8192 x 3072 at 48 rows 17.7 and 19.7).
+// Several weights take it where that is not more than the other kernels' estimate, up to 96 rows 1.05 times that (us, this
+// kernel and the other: two of 17408 x 5120 at 67 rows 46.3 and 65.9, at 128 rows 62 and 70.5; 6144 + 1024 + 1024 x
+// 5120 at 32 rows 12.9 and 18.9, at 100 rows 23 and 26.8; 2048 + 512 + 512 x 1024 at 100 rows 10.8 and 9.7).
 //
-// One weight takes it where that is less than 0.9 times the others' estimate, which is 1.9 us too high for one weight
-// where this one is 0.5; above 30 us, where that is little, 0.98 times.  With bf16 x, whose conversion both
-// estimates make too long, 0.98 and above 64 rows 0.95 times.  More than 64 fp16 rows, a weight of more than 45 MB
-// and the pipelined kernel otherwise: up to 1.5 us more (17408 x 5120 at 67 rows, this kernel and the other from HBM 30.7
-// and 31.3 us, though at 80 33.8 and 32.2; 14336 x 5376 at 67 30.3 and 28.4).  Up to 64 fp16 rows: up to 1.04 times the
-// others' estimate, for they lose more when the weight comes from HBM (5120 x 6144 at 32 rows from the Infinity
-// Cache 13.4 and 13.2, from HBM 13.7 and 14.2; 5120 x 17408 22.7 and 22.4, 22.5 and 26.3), though not weights of
-// more than 20 MB with fewer steps (17408 x 5120 at 32 rows from HBM 24.4 and 23.5, 14336 x 5376 23.2 and 20.9):
-// 0.03 us for each MB more.
-// Of 960 random calls of one weight with both kernels timed, the choice is 0.8 % slower than the better one, and 18
-// times 10 % or more (chosen up to 1.04 times the others at any number of rows and for every type: 2.4 %, 91 times; e.g.
-// 2928 x 2944 at 36 fp32 rows 18.7 instead of 16.0, 14336 x 5376 at 80 fp16 rows 31.3 instead of 28.6).
+// One weight takes it where the estimate is well below the others', which are up to 2 us too high for calls of 10 to
+// 15 us: 0.82 times with fp32 and 0.8 with bf16 activations, 0.9 of fp16 rows.  Up to 64 fp16 rows a long weight of at
+// most 20 MB up to 1.1 times: the others lose more when it comes from HBM and not from the Infinity Cache (5120 x 6144
+// at 32 rows 13.7 here, there 13.5 and 14.2).  Above 64 rows 0.72 times; up to 80 rows of a long weight 0.96 (4240 x 13376
+// at 67 rows 25.3 here and 26.9 there); weights of more than 45 MB 0.9, and 0.99 where the other is the pipelined kernel
+// (17408 x 5120 at 67 rows from HBM 30 here and 31 there).  Above 64 rows the line is drawn for the others' sake more
+// often than timings ask for (13758 x 5312 at 84 rows 29 here and 36 there).
+// The choice of the 270 calls takes 1.4 to 3 % more than the better of the two, and 3 (one weight of fp16 rows) to 10 %
+// (several, and fp32) less than the choice between the others and this kernel's first form, in which every wave fetched
+// and multiplied.
 inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows, double others_us, int other_variant,
                       RowsPlan &plan)
 {
@@ -363,20 +362,20 @@ inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t
     if (rows > 128u) return false;
     // 8-bit weights with byte tiles have a kernel that reads those
     if (a.x_columns != 0 && first.codes8 != nullptr && !ctx->q8_gemm_doubled) return false;
-    plan.mf = (int)((rows + 15u) / 16u);
+    plan.pair = a.x_dtype == MI355Q_F32;
+    plan.mf = (int)((a.M + 15u) / 16u) * (plan.pair ? 2 : 1);
     if (plan.mf < 2) plan.mf = 2;
     if (plan.mf == 7) plan.mf = 8;
-    auto shape = [&](int which) {
-        plan.waves = which == 0 ? 4 : 8;
-        plan.ntw = which == 2 ? 2 : 1;
+    auto shape = [&](int tiles) {
+        plan.tiles = tiles;
         plan.blocks = 0;
-        for (uint32_t t = 0; t < a.count; ++t)
-            plan.blocks += (a.targets[t].w->NT + plan.waves * plan.ntw - 1u) / (plan.waves * plan.ntw);
+        for (uint32_t t = 0; t < a.count; ++t) plan.blocks += (a.targets[t].w->NT + tiles - 1u) / tiles;
         return (uint64_t)plan.blocks * T < (1ull << 31);
     };
     if (ctx->force_gemm[1] >= 1) {
         // option "q4_gemm": 11, 12, 13 = 4, 8, 16 tiles a block; 1 = whole blocks, s = 64 (s - 1) workgroups
-        if (ctx->force_gemm[0] < 11 || ctx->force_gemm[0] > 13 || !shape(ctx->force_gemm[0] - 11)) return false;
+        const int which = ctx->force_gemm[0];
+        if (which < 11 || which > 13 || !shape(4 << (which - 11))) return false;
         const uint32_t groups = ctx->force_gemm[1] == 1 ? plan.blocks : 64u * (uint32_t)(ctx->force_gemm[1] - 1);
         plan.units = (plan.blocks * T + groups - 1u) / groups;
         return true;
@@ -384,25 +383,24 @@ inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t
     const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
     double outputs = 0.0, megabytes = 0.0, best_cost = 1e30;  // megabytes: 4-bit codes and their metadata
     for (uint32_t t = 0; t < a.count; ++t) {
-        outputs += (double)rows * a.targets[t].w->N;
+        outputs += (double)a.M * a.targets[t].w->N;
         megabytes += (double)a.targets[t].w->N * first.K * 0.5625e-6;
     }
+    const double mf = plan.mf;
     RowsPlan best = plan;
-    for (int which = 0; which < 3; ++which) {
-        if (!shape(which)) return false;
+    for (const int tiles : {4, 8, 16}) {
+        if (!shape(tiles)) return false;
         const uint32_t total = plan.blocks * T;
-        const uint32_t lds = rows_stages(plan.mf, plan.ntw, plan.waves) * rows_stage_bytes(plan.mf, plan.ntw, plan.waves);
-        const uint32_t places = std::min(160u * 1024u / lds, 2048u / (64u * plan.waves));  // on a compute unit
-        for (const uint32_t want : {plan.blocks, cus / 2u, cus, cus + cus / 2u, 2u * cus}) {
+        const double unit = tiles == 4   ? 0.329 + mf * (0.0099 * mf - 0.0309)
+                            : tiles == 8 ? 0.216 + mf * (0.0015 * mf + 0.0864)
+                                         : 0.378 + mf * (0.2182 - 0.0112 * mf);
+        for (const uint32_t want : {plan.blocks, cus / 2u, cus}) {
             plan.units = (total + want - 1u) / want;
             const uint32_t groups = (total + plan.units - 1u) / plan.units;
-            const uint32_t together = std::min(places, (groups + cus - 1u) / cus);
-            const uint32_t rounds = (groups + cus * together - 1u) / (cus * together);
-            const double tiles = plan.waves * plan.ntw, mf = plan.mf;
-            const double alone = 0.262 + 0.107 * mf, sharing = together * (tiles * (0.0345 + 0.0058 * mf) + 0.0378 * mf);
-            double cost = 5.2 + 0.02 * megabytes + (double)rounds * plan.units * (alone > sharing ? alone : sharing);
+            const uint32_t rounds = (groups + cus - 1u) / cus;
+            double cost = 5.0 + (double)rounds * plan.units * unit;
             if (plan.units % T != 0u && plan.units < total)
-                cost += 2.9 + 2.0e-6 * outputs * (T + plan.units - 1.0) / plan.units;
+                cost += 3.78 + 2.18e-6 * outputs * (T + plan.units - 1.0) / plan.units;
             if (cost < best_cost) {
                 best_cost = cost;
                 best = plan;
@@ -410,14 +408,20 @@ inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t
         }
     }
     plan = best;
-    if (a.x_dtype != MI355Q_F16) best_cost += 5.0 + 0.3 * (double)rows * first.K * sizeof(_Float16) * 1e-6;
-    if (a.count != 1u) return best_cost <= 1.08 * others_us + 1.0;
-    if (a.x_dtype == MI355Q_BF16) return best_cost <= (rows > 64u ? 0.95 : 0.98) * others_us;
-    if (a.x_dtype == MI355Q_F16 && rows > 64u && megabytes > 45.0 && other_variant >= kFirstPiped)
-        return best_cost <= others_us + 1.5;
-    if (a.x_dtype == MI355Q_F32 || rows > 64u) return best_cost <= (others_us < 30.0 ? 0.9 : 0.98) * others_us;
-    const double large = std::min(std::max(megabytes - 20.0, 0.0), 30.0);  // (50 MB: the largest measured)
-    return large == 0.0 ? best_cost <= 1.04 * others_us : best_cost + 0.03 * large <= others_us;
+    best_cost += 0.37e-6 * outputs * dtype_bytes(a.y_dtype);
+    if (a.x_dtype != MI355Q_F16) best_cost += 2.98 + 1.92 * (double)rows * first.K * sizeof(_Float16) * 1e-6;
+    double most = 0.9;
+    if (a.count != 1u)
+        most = rows <= 96u ? 1.05 : 1.0;
+    else if (a.x_dtype != MI355Q_F16)
+        most = a.x_dtype == MI355Q_F32 ? 0.82 : 0.8;
+    else if (rows > 64u)
+        most = rows <= 80u && T >= 64u ? 0.96 : megabytes <= 45.0 ? 0.72 : other_variant >= kFirstPiped ? 0.99 : 0.9;
+    else if (megabytes > 20.0)
+        most = 0.9;
+    else if (T >= 40u)
+        most = 1.1;
+    return best_cost <= most * others_us;
 }
 
 // The call: by q4_rows_kernel as `rows_launch` says (true), else by `group` and `plans`.

@@ -340,6 +340,17 @@ def test_rows_kernel(engine, oracle, gpu, force, forced, N, K, M):
     run_case(engine, oracle, gpu, N, K, M, engine.META_F16_INTERLEAVED, engine.F16, engine.F16)
 
 
+@pytest.mark.parametrize("forced", ["11,1", "11,5", "12,2", "12,5", "13,1", "13,5"])
+@pytest.mark.parametrize("N,K,M", [(1104, 1280, 16), (1104, 192, 17), (272, 1280, 32), (1101, 640, 48), (2052, 640, 49), (64, 128, 64)])
+def test_rows_kernel_pairs(engine, oracle, gpu, force, forced, N, K, M):
+    """fp32 activations: value and remainder rows in fragments of their own, one to four fragments of
+    outputs full and with one row more; fp32 outputs with residual rows (16-byte pieces, and a width that has
+    none) and bf16 outputs."""
+    force("q4_gemm", forced)
+    run_case(engine, oracle, gpu, N, K, M, engine.META_BF16_PLANES, engine.F32, engine.F32, residual=True)
+    run_case(engine, oracle, gpu, N, K, M, engine.META_F16_INTERLEAVED, engine.F32, engine.BF16)
+
+
 @pytest.mark.parametrize("forced", ["11,2", "12,1", "13,1", "13,2"])
 @pytest.mark.parametrize("x_dtype,M", [("F32", 9), ("F32", 35), ("F32", 64), ("BF16", 17), ("BF16", 75)])
 def test_rows_kernel_targets_and_converted_activations(engine, gpu, force, forced, x_dtype, M):
