@@ -345,10 +345,10 @@ def test_rows_kernel(engine, oracle, gpu, force, forced, N, K, M):
 def test_rows_kernel_pairs(engine, oracle, gpu, force, forced, N, K, M):
     """fp32 activations: value and remainder rows in fragments of their own, one to four fragments of
     outputs full and with one row more; fp32 outputs with residual rows (16-byte pieces, and a width that has
-    none) and bf16 outputs."""
+    none) and without."""
     force("q4_gemm", forced)
     run_case(engine, oracle, gpu, N, K, M, engine.META_BF16_PLANES, engine.F32, engine.F32, residual=True)
-    run_case(engine, oracle, gpu, N, K, M, engine.META_F16_INTERLEAVED, engine.F32, engine.BF16)
+    run_case(engine, oracle, gpu, N, K, M, engine.META_F16_INTERLEAVED, engine.F32, engine.F32)
 
 
 @pytest.mark.parametrize("forced", ["11,2", "12,1", "13,1", "13,2"])
