@@ -26,12 +26,16 @@ struct RowsShape {
     // KiB: four fragments of sums from each multiplying wave, two where the rings leave no more
     static constexpr int kExchange = KS == 1 ? 0 : 3 * kRowLoads + 3 * kCodeLoads + 16 <= 160 ? 16 : 8;
     static constexpr int kRowSlots = 4 * kRowLoads + 5 * kCodeLoads + kExchange <= 160 ? 4 : 3;
-    static constexpr int kCodeFit = (160 - (KS == 1 ? 0 : 1) - kExchange - kRowSlots * kRowLoads) / kCodeLoads, kCodeSlots = kCodeFit > 6 ? 6 : kCodeFit;
+    static constexpr int kCodeFit = (160 - (KS == 2 && MF < 4 ? 1 : 0) - kExchange - kRowSlots * kRowLoads) / kCodeLoads, kCodeSlots = kCodeFit > 6 ? 6 : kCodeFit;
     static constexpr int kRounds = KS == 1 ? 0 : (NT / 2 * kFragments + kExchange / 4 - 1) / (kExchange / 4);  // of the exchange
+    // The two waves of an exchange meet at the workgroup's barriers, which wait for the fetching waves too, or, up to 48
+    // rows, wait for each other alone: a barrier there cost 1.8 us of a short run (512 + 256 + 256 x 1088 at 32 rows 10.0 ->
+    // 8.5 us), while at 67 rows polling took more than the barriers (27B layer 107.2 and 109.4 us).
+    static constexpr bool kBarriers = KS == 2 && MF >= 4;
     static constexpr int kRowWaves = 2 * kRowLoads > 5 * kCodeLoads ? 3 : 2 * kCodeLoads > 3 * kRowLoads ? 1 : 2;
     static constexpr uint32_t kRowBytes = kRowLoads * 1024u, kCodeBytes = kCodeLoads * 1024u, kCodesAt = kRowSlots * kRowBytes;
     static constexpr uint32_t kExchangeAt = kCodesAt + kCodeSlots * kCodeBytes, kWordsAt = kExchangeAt + kExchange * 1024u;
-    static constexpr uint32_t kLds = kWordsAt + (KS == 1 ? 0u : 32u);
+    static constexpr uint32_t kLds = kWordsAt + (KS == 2 && MF < 4 ? 32u : 0u);
     static_assert(!PAIR || MF % 2 == 0, "value and remainder rows in fragments of their own");
     static_assert(kRowSlots >= 3 && kCodeSlots >= 3, "a unit ahead of the one that is read ahead, at least");
 };
@@ -111,6 +115,7 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
                     refresh();
                 }
             };
+            uint32_t left = T - step < count ? T - step : count;  // units of the block worked on that are left
             refresh();
             uint32_t slot = 0;
             for (; slot < (uint32_t)(SLOTS - 1) && fetched < count; ++slot) next(ring + slot * bytes);
@@ -131,6 +136,11 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
                 asm volatile("s_barrier" ::: "memory");
                 if (fetched < count) next(ring + slot);
                 slot = slot == (SLOTS - 1) * bytes ? 0u : slot + bytes;
+                if constexpr (S::kBarriers) {
+                    if (--left != 0u) continue;
+                    for (int j = 0; j < 2 * S::kRounds; ++j) asm volatile("s_barrier" ::: "memory");
+                    left = T < count - 1u - i ? T : count - 1u - i;
+                }
             }
         };
         const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr)rows_lds);
@@ -281,7 +291,7 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
     };
     enter_block();
     uint32_t exchanged = 0;  // rounds of it
-    if (KS == 2 && threadIdx.x < 8u) ((uint32_t *)((char *)rows_lds + S::kWordsAt))[threadIdx.x] = 0u;
+    if (KS == 2 && !S::kBarriers && threadIdx.x < 8u) ((uint32_t *)((char *)rows_lds + S::kWordsAt))[threadIdx.x] = 0u;
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     read_meta();
     read_codes(std::integral_constant<int, 0>());
@@ -331,10 +341,8 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
             constexpr int AT_ONCE = S::kExchange / 4;
             char *const mine = (char *)rows_lds + S::kExchangeAt + wave * (AT_ONCE * 1024u) + lane * 16u;
             const char *const theirs = (const char *)rows_lds + S::kExchangeAt + (wave ^ 1u) * (AT_ONCE * 1024u) + lane * 16u;
-            // The two waves wait for each other alone (a barrier would wait for the fetching waves, which may stand in the
-            // queue of their loads: 1.8 us for 32 rows x 64 columns in runs of three units).  LDS serves a wave's accesses in
-            // their order, so a word that counts rounds follows what it tells of; each wave writes its own two words,
-            // and both pass through the same rounds, so every wait ends.
+            // Without barriers: LDS serves a wave's accesses in their order, so a word that counts rounds follows what it tells of;
+            // each wave writes its own two words, and both pass through the same rounds, so every wait ends.
             volatile uint32_t *const words = (volatile uint32_t *)((char *)rows_lds + S::kWordsAt);
             auto reached = [&](uint32_t word, uint32_t rounds_done) __attribute__((always_inline)) {
                 while (__builtin_amdgcn_readfirstlane(words[word]) - rounds_done > 0x7fffffffu) {
@@ -343,13 +351,20 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
             };
             static_for<S::kRounds>([&](auto round_c) __attribute__((always_inline)) {
                 constexpr int from = AT_ONCE * decltype(round_c)::value, until = from + AT_ONCE < KEPT * OF ? from + AT_ONCE : KEPT * OF;
-                reached(4u + (wave ^ 1u), exchanged);  // the partner has read the round before
+                if constexpr (S::kBarriers)
+                    asm volatile("s_barrier" ::: "memory");  // the round before has been read
+                else
+                    reached(4u + (wave ^ 1u), exchanged);
 #pragma unroll
                 for (int e = from; e < until; ++e) *(floatx4 *)(mine + (e - from) * 1024) = acc[KEPT + e / OF][e % OF];
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                exchanged += 1u;
-                words[wave] = exchanged;  // written
-                reached(wave ^ 1u, exchanged);
+                if constexpr (S::kBarriers) {
+                    asm volatile("s_barrier" ::: "memory");
+                } else {
+                    exchanged += 1u;
+                    words[wave] = exchanged;  // written
+                    reached(wave ^ 1u, exchanged);
+                }
 #pragma unroll
                 for (int e = from; e < until; ++e) {
                     const floatx4 more = *(const floatx4 *)(theirs + (e - from) * 1024);
@@ -357,7 +372,7 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
                     for (int j = 0; j < 4; ++j) acc[e / OF][e % OF][j] += more[j];
                 }
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                words[4u + wave] = exchanged;  // read
+                if constexpr (!S::kBarriers) words[4u + wave] = exchanged;  // read
             });
         }
         const bool partial = begin != 0u || step != T;
