@@ -438,6 +438,7 @@ static int q4_rows_linears(mi355q_context *ctx, const Q4LinearArgs &a, const Row
     if (status != MI355Q_OK) return status;
     p.M = a.M;  // the kernel adds value and remainder rows up in one accumulator
     p.pair = 0;
+    p.m_blocks = plan.m_blocks;
     p.K = x_columns;
     p.T = first.T;
     p.wrap_steps = a.x_columns ? a.x_columns / kStepColumns : 0xffffffffu;
@@ -471,7 +472,7 @@ static int q4_rows_linears(mi355q_context *ctx, const Q4LinearArgs &a, const Row
         target.NT = w.NT;
         target.wide_stores = w.N % 4u == 0u && (uintptr_t)target.y % 16u == 0u;
         target.first_block = blocks;
-        blocks += (w.NT + plan.tiles - 1u) / plan.tiles;
+        blocks += (w.NT + plan.tiles - 1u) / plan.tiles * plan.m_blocks;
         if (sharing) {
             target.partials = partials;
             partials += (size_t)sharers * p.M * padded_columns(w.N);
@@ -532,6 +533,19 @@ int q4_gemm_linears(mi355q_context *ctx, const Q4LinearArgs &a, char *error, siz
     RowsPlan together;
     GroupPlan group;
     if (plan_gemm(ctx, a, plans, group, together)) return q4_rows_linears(ctx, a, together, error, error_capacity);
+    bool taken[kMaxTargets];
+    const uint32_t pairs = plan_pairs(ctx, a, plans, taken, together);
+    if (pairs == a.count) return q4_rows_linears(ctx, a, together, error, error_capacity);
+    if (pairs != 0u) {  // those targets by q4_rows_kernel, the others as a call of their own
+        Q4LinearArgs part[2] = {a, a};
+        part[0].count = part[1].count = 0;
+        for (uint32_t t = 0; t < a.count; ++t) {
+            Q4LinearArgs &to = part[taken[t] ? 0 : 1];
+            to.targets[to.count++] = a.targets[t];
+        }
+        status = q4_rows_linears(ctx, part[0], together, error, error_capacity);
+        return status == MI355Q_OK ? q4_gemm_linears(ctx, part[1], error, error_capacity) : status;
+    }
     if (group.variant >= 0) return gemm_targets(ctx, a, 0, a.count, plans, group.variant, error, error_capacity);
     for (uint32_t t = 0; t < a.count && status == MI355Q_OK; ++t)
         status = gemm_targets(ctx, a, t, 1, plans, plans[t].variant, error, error_capacity);

@@ -36,6 +36,7 @@ struct GemmParams {
     // q4_rows_kernel: units (128-column steps of a block) per workgroup and in all, columns of a
     // block, and the target's first block (set by select_target); units 0: K splits as above
     uint32_t units, total_units, block_columns, first_block;
+    uint32_t m_blocks;     // q4_rows_kernel: blocks of rows, which number a target's blocks fastest
     int xcd_order;         // pipelined kernel: blocks that share weights are placed on one XCD (see there)
 };
 

@@ -329,6 +329,7 @@ inline GroupPlan plan_group(const mi355q_context *ctx, const Q4LinearArgs &a, ui
 struct RowsPlan {
     int mf, tiles;                 // 16-row fragments of fp16 rows, tiles a block
     bool pair;                     // fp32 activations: pairs of fp16 rows
+    uint32_t m_blocks;             // blocks of rows
     uint32_t blocks, units;        // blocks in all, units per workgroup
 };
 
@@ -363,6 +364,7 @@ inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t
     // 8-bit weights with byte tiles have a kernel that reads those
     if (a.x_columns != 0 && first.codes8 != nullptr && !ctx->q8_gemm_doubled) return false;
     plan.pair = a.x_dtype == MI355Q_F32;
+    plan.m_blocks = 1;
     plan.mf = (int)((a.M + 15u) / 16u) * (plan.pair ? 2 : 1);
     if (plan.mf < 2) plan.mf = 2;
     if (plan.mf == 7) plan.mf = 8;
@@ -422,6 +424,64 @@ inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t
     else if (T >= 40u)
         most = 1.1;
     return best_cost <= most * others_us;
+}
+
+// ---- more than 128 rows, fp32 activations: q4_rows_kernel on whole blocks of 64 rows or less -----------
+
+// A call of targets 0 .. count - 1, whole blocks dealt to workgroups as evenly as they come: microseconds, and the blocks'
+// width.  Fitted to 600 timings on this GPU (210 calls from 512 x 512 to 6144 x 1536 and three of 1536 x 1536, 70 to
+// 1500 rows; 7 % rms): the conversion, then for every block of a workgroup its steps and its outputs.
+inline double pairs_us(uint32_t cus, const Q4LinearArgs &a, const uint32_t *of, uint32_t count, RowsPlan &plan)
+{
+    const uint32_t T = a.targets[0].w->T, block_rows = (a.M + (a.M + 63u) / 64u - 1u) / ((a.M + 63u) / 64u);
+    plan.pair = true;
+    plan.m_blocks = (a.M + 63u) / 64u;
+    plan.mf = 2 * (int)((block_rows + 15u) / 16u);
+    double best = 1e30, outputs = 0.0;
+    for (uint32_t i = 0; i < count; ++i) outputs += (double)a.M * a.targets[of[i]].w->N * dtype_bytes(a.y_dtype) * 1e-6;
+    RowsPlan at = plan;
+    for (const int tiles : {4, 8, 16}) {
+        at.tiles = tiles;
+        uint64_t blocks = 0;
+        for (uint32_t i = 0; i < count; ++i) blocks += (uint64_t)((a.targets[of[i]].w->NT + tiles - 1u) / tiles) * plan.m_blocks;
+        if (blocks * T >= (1ull << 31)) continue;
+        const uint32_t rounds = (uint32_t)((blocks + cus - 1u) / cus);
+        at.blocks = (uint32_t)blocks;
+        at.units = rounds * T;
+        const double mf = plan.mf, filled = (double)((blocks + rounds - 1u) / rounds) / cus;
+        const double alone = 0.1192 * mf + 0.0753 * tiles - 0.0044 * mf * tiles - 0.412;
+        const double share = (0.2807 * mf - 0.1142 * tiles + 0.0194 * mf * tiles - 1.64) * (0.649 + 0.351 * filled);
+        const double us = 6.75 + 1.777e-6 * a.M * 2.0 * a.targets[0].w->K + rounds * (T * std::max(alone, share) + 0.0317 * mf * tiles) +
+                          0.188 * outputs;
+        if (us < best) {
+            best = us;
+            plan = at;
+        }
+    }
+    return best;
+}
+
+// Which targets of the call it takes (their number): those whose own call is estimated to take 2 % less, so that a weight
+// has the bits of its own call in company too.  Outputs do not depend on the blocks' width.  Rows of a few steps have
+// the most to gain: the other kernels multiply value and remainder rows like rows of their own, in blocks whose
+// fill and stores nothing hides (us, those and this kernel: three of 1280 x 1280 at 150 rows 21.9 and 16.1, at 1500 rows 50.7 and 47.3;
+// 5120 x 1280 at 700 rows 36.2 and 29.5, 1280 x 1280 at 300 rows 17.3 and 16.9, at 100 rows 14.2 and 15.5).  With
+// more steps than about sixteen they have K splits for weights that do not fill the chip (1280 x 5120 at 300 rows 26 and 46).
+// Of 58 calls of three weights 10 % less time, of 155 of one 2 %.
+inline uint32_t plan_pairs(const mi355q_context *ctx, const Q4LinearArgs &a, const TargetPlan *plans, bool *taken, RowsPlan &plan)
+{
+    const Q4Device &first = *a.targets[0].w;
+    if (a.x_dtype != MI355Q_F32 || a.M <= 64u || a.x_columns != 0u || first.K % kStepColumns != 0u || ctx->force_gemm[1] >= 1 ||
+        ctx->gemm_order >= 0 || (uint64_t)128u * first.K * sizeof(_Float16) >= (1ull << 32))
+        return 0;
+    const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
+    uint32_t of[kMaxTargets], count = 0;
+    for (uint32_t t = 0; t < a.count; ++t) {
+        taken[t] = a.targets[t].w->N % 4u == 0u && pairs_us(cus, a, &t, 1, plan) <= 0.98 * plans[t].us;
+        if (taken[t]) of[count++] = t;
+    }
+    if (count != 0u && pairs_us(cus, a, of, count, plan) >= 1e30) return 0;
+    return count;
 }
 
 // The call: by q4_rows_kernel as `rows_launch` says (true), else by `group` and `plans`.

@@ -1,5 +1,5 @@
 // Device code of the affine-Q4 linear for 17..128 rows of x: more rows than the streaming kernel
-// takes, too few to keep the matrix cores busy.  Bound by memory, by what a launch costs besides (the
+// takes, too few to keep the matrix cores busy; and for more rows of fp32 activations by weights of short rows.  Bound by memory, by what a launch costs besides (the
 // second kernel behind shared blocks 4 to 6 us), and by power: with random operands a unit of 80 rows x 256 columns
 // takes 1.45 us, with zeros in x 1.35, with zeros in both 1.15, at which its loads and its arithmetic each take
 // 0.7 and 1.1 alone.
@@ -46,6 +46,8 @@ struct RowsShape {
 // steps each; whole blocks would keep 120 of them idle, thirds of blocks would run in two rounds).
 // A block that one workgroup finishes alone is stored as output; the workgroups that share a block
 // leave partial sums, which a second kernel adds in their order.  The workgroups of one XCD are neighbours on the line.
+// More rows than a block has make several blocks of a group of tiles, numbered next to each other, and U a multiple of a
+// block's steps.
 // The fetching waves run ahead, across the ends of blocks: their loads are asm statements, each wave's in one in-order
 // queue of which a counted wait takes the oldest unit.  At barrier i the units up to i + 1 have landed and unit i - 1
 // has been read: the multiplying waves read their operands a quarter of a unit ahead, the next unit's first ones
@@ -70,7 +72,7 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t r = lane & 15u, kq = lane >> 4;
     const GemmParams &shared = group.shared;
-    const uint32_t M = shared.M, K = shared.K, T = shared.T, U = shared.units;
+    const uint32_t M = shared.M, K = shared.K, T = shared.T, U = shared.units, m_blocks = shared.m_blocks;
     const uint32_t number = __builtin_amdgcn_readfirstlane(number_by_xcd(blockIdx.x, gridDim.x));
     const uint32_t first_unit = number * U;
     const uint32_t count = first_unit + U < shared.total_units ? U : shared.total_units - first_unit;  // never 0
@@ -162,12 +164,20 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
                 [&]() __attribute__((always_inline)) {
                     const uint32_t x_step = step >= wrap_steps ? step - wrap_steps : step;
                     const bool tail = odd_tail && step + 1u == T;
-                    rows = (const char *)(shared.x + (size_t)x_step * kStepColumns);
+                    uint32_t m0 = 0;
+                    if (m_blocks > 1u) {
+                        uint32_t first = first_of[0];
+#pragma unroll
+                        for (uint32_t t = 1; t < kMaxTargets; ++t)
+                            if (t < shared.targets && block >= first_of[t]) first = first_of[t];
+                        m0 = (block - first) % m_blocks * OUT_ROWS;
+                    }
+                    rows = (const char *)(shared.x + (size_t)(PAIR ? 2u * m0 : m0) * K + (size_t)x_step * kStepColumns);
 #pragma unroll
                     for (int j = 0; j < LOADS; ++j) {
                         const uint32_t row = at[j] / 256u + kq, octet = r ^ (row & 15u);  // of the stage
                         uint32_t m = PAIR ? row % OUT_ROWS : row;
-                        m = m < M ? m : M - 1u;
+                        m = m0 + m < M ? m : M - 1u - m0;
                         from[j] = ((PAIR ? 2u * m + row / OUT_ROWS : m) * K + 8u * octet) * (uint32_t)sizeof(_Float16) -
                                   (tail && octet >= 8u ? 128u : 0u);
                     }
@@ -204,7 +214,7 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
                             codes = codes_of[t];
                             metas = meta_of[t];
                         }
-                    const uint32_t tile0 = (block - first) * TPB;
+                    const uint32_t tile0 = (m_blocks > 1u ? (block - first) / m_blocks : block - first) * TPB;
                     stride = all * 1024u;
                     codes += (size_t)step * stride;
                     metas += (size_t)step * (stride / 8u);
@@ -377,9 +387,14 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
         }
         const bool partial = begin != 0u || step != T;
         const uint32_t sharer = number - block * T / U;  // number among the workgroups that share the block
-        uint32_t m0 = 0;  // unknown to the compiler, which would else keep every row's address in registers all the time
+        uint32_t m0 = 0, block_n = local;
+        if (m_blocks > 1u) {
+            m0 = __builtin_amdgcn_readfirstlane(local % m_blocks * OUT_ROWS);
+            block_n = local / m_blocks;
+        }
+        // unknown to the compiler, which would else keep every row's address in registers all the time
         asm volatile("" : "+s"(m0));
-        const uint32_t n0 = (local * TPB + group0 + part * KEPT) * kTileRows + 4u * kq;
+        const uint32_t n0 = (block_n * TPB + group0 + part * KEPT) * kTileRows + 4u * kq;
         // The common cases - 16-byte pieces of partial sums, fp16 outputs that need nothing done to them, fp32
         // outputs - as straight code; everything else one fragment after the other
         // through one copy of it (straight code for every fragment was 2700 to 10600 lines of

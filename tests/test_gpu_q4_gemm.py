@@ -351,6 +351,51 @@ def test_rows_kernel_pairs(engine, oracle, gpu, force, forced, N, K, M):
     run_case(engine, oracle, gpu, N, K, M, engine.META_F16_INTERLEAVED, engine.F32, engine.F32)
 
 
+@pytest.mark.parametrize("K,widths,by_rows", [(1280, (1280, 1280, 1280), 3), (640, (2048, 516, 1002), 2), (1152, (3072,), 1)])
+@pytest.mark.parametrize("M", [65, 129, 150, 193, 450])
+def test_pairs_of_many_rows(engine, oracle, gpu, force, capfd, K, widths, by_rows, M):
+    """fp32 activations beyond 128 matrix rows by q4_rows_kernel: two to eight blocks of rows, the last with one row or full,
+    more blocks than compute units and fewer, weights it takes beside one it does not (a width that is no multiple of
+    4).  Each output has the bits of its weight's own call, agrees with another kernel up to the order of
+    the sums, and the first weight's with the oracle."""
+    kind = engine.META_BF16_PLANES
+    x = make_x(engine, 201, M, K)
+    planes = [engine.synth_q4_affine(202 + i, 0.02, N, K, kind) for i, N in enumerate(widths)]
+    weights = [gpu.q4_prepare(*p, N, K, kind) for p, N in zip(planes, widths)]
+    biases = [gpu.to_device(engine.synth_normal_f32(210 + i, 1.0, N)) for i, N in enumerate(widths)]
+    x_ptr = gpu.to_device(x)
+    outputs = [gpu.alloc(M * N * 4) for N in widths]
+    try:
+        results, printed = [], []
+        targets = list(zip(weights, outputs, biases))
+        for how, groups in (("", [targets]), ("", [[t] for t in targets]), ("4,1", [[t] for t in targets])):
+            print(f"pairs M={M} K={K} widths={widths} forced={how}", flush=True)
+            force("q4_gemm", how)
+            force("trace", "1")
+            for pointer, N in zip(outputs, widths):
+                gpu.upload(pointer, np.full((M, N), np.nan, np.float32))
+            capfd.readouterr()
+            gpu.q4_sequence(engine.make_calls([(g, x_ptr, engine.F32, M, engine.F32, engine.F32, engine.RESIDUAL_IS_BIAS)
+                                               for g in groups]))
+            gpu.sync()
+            printed.append(capfd.readouterr().err)
+            results.append([gpu.download(p, (M, N), np.float32) for p, N in zip(outputs, widths)])
+        if M == 150:  # (other numbers of rows are the estimates' choice)
+            assert printed[1].count("q4 rows M=150") == by_rows and printed[0].count("q4 rows M=150") == 1
+        for together, alone, other in zip(*results):
+            assert np.array_equal(together, alone)
+            # K products of one row, of values and of remainders, summed in another order
+            assert np.max(np.abs(alone - other)) <= 2 * K * 2.0 ** -24 * np.max(np.abs(other))
+        ref = oracle.q4_linear(*planes[0], kind, widths[0], K, x, oracle.X_F32, M, weight_rounding=oracle.W_ROUND_F16)
+        ref = ref + gpu.download(biases[0], (1, widths[0]), np.float32)
+        assert q4_relative_error(np.asarray(results[1][0], np.float64), ref) <= 1e-3
+    finally:
+        for pointer in [x_ptr] + outputs + biases:
+            gpu.free(pointer)
+        for weight in weights:
+            weight.destroy()
+
+
 @pytest.mark.parametrize("forced", ["11,2", "12,1", "13,1", "13,2"])
 @pytest.mark.parametrize("x_dtype,M", [("F32", 9), ("F32", 35), ("F32", 64), ("BF16", 17), ("BF16", 75)])
 def test_rows_kernel_targets_and_converted_activations(engine, gpu, force, forced, x_dtype, M):
