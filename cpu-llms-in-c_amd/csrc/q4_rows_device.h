@@ -72,7 +72,8 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t r = lane & 15u, kq = lane >> 4;
     const GemmParams &shared = group.shared;
-    const uint32_t M = shared.M, K = shared.K, T = shared.T, U = shared.units, m_blocks = shared.m_blocks;
+    const uint32_t M = shared.M, K = shared.K, T = shared.T, U = shared.units;
+    const uint32_t m_blocks = PAIR ? shared.m_blocks : 1u;  // of rows; up to 128 rows of other activations are one
     const uint32_t number = __builtin_amdgcn_readfirstlane(number_by_xcd(blockIdx.x, gridDim.x));
     const uint32_t first_unit = number * U;
     const uint32_t count = first_unit + U < shared.total_units ? U : shared.total_units - first_unit;  // never 0
@@ -89,7 +90,7 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
         meta_of[t] = (const char *)group.target[t].meta;
         asm volatile("" ::"s"(first_of[t]), "s"(NT_of[t]), "s"(codes_of[t]), "s"(meta_of[t]));
     }
-    asm volatile("" ::"s"(M), "s"(K), "s"(T), "s"(U), "s"(shared.total_units), "s"(shared.targets), "s"(shared.wrap_steps), "s"(shared.x));
+    asm volatile("" ::"s"(M), "s"(K), "s"(T), "s"(U), "s"(m_blocks), "s"(shared.total_units), "s"(shared.targets), "s"(shared.wrap_steps), "s"(shared.x));
 
     if (wave >= 4u) {
         // ---- A fetching wave.  Pointers run on by a step, and only at the end of a `run` of units (a block, the half step
