@@ -21,7 +21,7 @@
 //   q4_gemm_pipe_kernel: one workgroup per compute unit, software pipelined by
 //     hand (128 rows x 16, 17 or 20 tiles);
 //   q4_rows_kernel (q4_rows_device.h): up to 128 rows, all weights of a call as
-//     one launch.
+//     one launch; of fp32 activations also more, in blocks of 64 rows' pairs.
 // The host picks shape and K split by a time estimate fitted on this GPU (q4_gemm_plan.h), e.g.
 // 20 tiles for the 17408-row matrices: 55 x 4 = 220 workgroups at M = 512.
 // Several weights of a call go out as one launch where that is estimated to take less: they
