@@ -436,7 +436,7 @@ static int q4_rows_linears(mi355q_context *ctx, const Q4LinearArgs &a, const Row
     GemmParams &p = group.shared;
     int status = gemm_activations(ctx, a, x_columns, true, p, error, error_capacity);
     if (status != MI355Q_OK) return status;
-    p.M = a.M;  // the kernel adds value and remainder rows up in one accumulator
+    p.M = a.M;  // the kernel adds the sums of value and remainder rows itself
     p.pair = 0;
     p.m_blocks = plan.m_blocks;
     p.K = x_columns;

@@ -440,7 +440,7 @@ inline double pairs_us(uint32_t cus, const Q4LinearArgs &a, const uint32_t *of, 
     double best = 1e30, outputs = 0.0;
     for (uint32_t i = 0; i < count; ++i) outputs += (double)a.M * a.targets[of[i]].w->N * dtype_bytes(a.y_dtype) * 1e-6;
     RowsPlan at = plan;
-    for (const int tiles : {4, 8, 16}) {
+    for (const int tiles : {4, 8}) {  // (16 tiles of so many rows add a row's products up in another order)
         at.tiles = tiles;
         uint64_t blocks = 0;
         for (uint32_t i = 0; i < count; ++i) blocks += (uint64_t)((a.targets[of[i]].w->NT + tiles - 1u) / tiles) * plan.m_blocks;

@@ -58,8 +58,9 @@ struct RowsShape {
 // adjacent bytes 16 (16 d + r) + 4 j: lane (r, j) reads one word of codes and the word of metadata of its group
 // j / 2.
 // PAIR: x is 2 M rows, value and rounding remainder of each of the M rows (of fp32 activations);
-// a block's value rows lie in the first half of its stage, their remainders in the second, and both
-// are added up in one accumulator.
+// a block's value rows lie in the first half of its stage, their remainders in the second.  Each has accumulators of its
+// own, which are added when the block is done: in one accumulator a row's products were rounded twice as often (relative
+// error against 64 bits of 1.8 to 2.8e-7 where it is 1.3 to 2.0e-7 now, K of 1216 to 2112; 0.6 % of a call's time).
 template <int MF, int NT, int KS, bool PAIR>
 __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
 {
@@ -246,12 +247,12 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
     }
 
     // ---- a multiplying wave
-    floatx4 acc[NT][OF];
+    floatx4 acc[NT][MF];
     auto clear = [&]() {
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int i = 0; i < OF; ++i) acc[t][i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int i = 0; i < MF; ++i) acc[t][i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
     };
     clear();
     const NibbleMasks masks = nibble_masks();
@@ -333,12 +334,12 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
             }
 #pragma unroll
             for (int m = 0; m < MF; ++m)
-                acc[t][m % OF] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w16, x_frag[d % 2][m], acc[t][m % OF], 0, 0, 0);
+                acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w16, x_frag[d % 2][m], acc[t][m], 0, 0, 0);
             w16 = next;
             // the weights' vector instructions between the matrix instructions: a wave issues in order, and one of those
             // waits for the one before it
 #pragma unroll
-            for (int m = 0; m < (MF * NT < 32 || PAIR ? MF : 0); ++m) {
+            for (int m = 0; m < (MF * NT < 32 ? MF : 0); ++m) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x002, (14 + MF - 1) / MF, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
@@ -348,6 +349,14 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
         if (left != 0u) continue;
 
         // ---- the last unit of this block here: outputs, or partial sums
+        if constexpr (PAIR) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int f = 0; f < OF; ++f)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[t][f][j] += acc[t][f + OF][j];
+        }
         if constexpr (KS == 2) {
             constexpr int AT_ONCE = S::kExchange / 4;
             char *const mine = (char *)rows_lds + S::kExchangeAt + wave * (AT_ONCE * 1024u) + lane * 16u;
@@ -488,7 +497,7 @@ static hipError_t launch_rows_of(mi355q_context *ctx, int mf, bool pair, uint32_
         // whole columns to a wave: up to 48 rows by 8 and 16 tiles, whose reading from LDS is cheaper than an exchange (us,
         // 5120 x 6144 at 32 rows 13.6 and 14.4, 512 + 256 + 256 x 1088 8.1 and 10.3), and 96 and 128 rows by 16 tiles, for the
         // accumulators' sake
-        constexpr int SPLIT = (NT >= 4 && MF <= 3) || (NT == 8 && MF >= 6 && !PAIR) ? 2 : 1;
+        constexpr int SPLIT = (NT >= 4 && MF <= 3) || (NT == 8 && MF >= 6) ? 2 : 1;
         typedef RowsShape<MF, NT / SPLIT, KS / SPLIT, PAIR> S;
         bool &raised = ctx->rows_lds_raised[MF - 1][PAIR][S::kTiles / 8];
         const auto kernel = q4_rows_kernel<MF, NT / SPLIT, KS / SPLIT, PAIR>;

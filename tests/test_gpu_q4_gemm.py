@@ -351,6 +351,31 @@ def test_rows_kernel_pairs(engine, oracle, gpu, force, forced, N, K, M):
     run_case(engine, oracle, gpu, N, K, M, engine.META_F16_INTERLEAVED, engine.F32, engine.F32)
 
 
+@pytest.mark.parametrize("forced,M,parts", [("11,1", 16, 2), ("12,1", 16, 1), ("13,1", 16, 1), ("11,1", 32, 2), ("12,1", 32, 2),
+                                            ("13,1", 32, 2), ("11,1", 48, 2), ("12,1", 64, 2), ("13,1", 64, 1)])
+@pytest.mark.parametrize("K", [1280, 5120])
+def test_rows_kernel_pairs_precision(engine, oracle, gpu, force, forced, parts, M, K):
+    """fp32 activations on whole blocks: an output is as near to 64 bits as sums of a row's K value products alone, in
+    `parts` accumulators.  An addition of the matrix instruction (eight products; four of them an instruction) is off by
+    0.424 * 2^-24 of the sum (rms over mantissas), and n of them into a sum that grows like a random walk by that times
+    sqrt(n / 2); n additions in two halves by sqrt(n / 4).  A tenth more for the pieces of x and for the sample."""
+    N, kind = 1024, engine.META_BF16_PLANES
+    force("q4_gemm", forced)
+    planes = engine.synth_q4_affine(221, 0.02, N, K, kind)
+    x = make_x(engine, 222, M, K)
+    weight = gpu.q4_prepare(*planes, N, K, kind)
+    try:
+        print(f"pairs precision M={M} K={K} forced={forced}", flush=True)
+        y = gpu.q4_linear(weight, x, engine.F32, engine.F32).astype(np.float64)
+    finally:
+        weight.destroy()
+    exact = oracle.q4_linear(*planes, kind, N, K, x, oracle.X_F32, M, weight_rounding=oracle.W_ROUND_F16)
+    error = np.sqrt(np.sum((y - exact) ** 2) / np.sum(exact ** 2))
+    bound = 1.1 * 0.424 * 2.0 ** -24 * np.sqrt(K / 8 / (2 * parts))
+    print(f"relative error {error:.3e}, bound {bound:.3e}", flush=True)
+    assert error <= bound
+
+
 @pytest.mark.parametrize("K,widths,by_rows", [(1280, (1280, 1280, 1280), 3), (640, (2048, 516, 1002), 2), (1152, (3072,), 1)])
 @pytest.mark.parametrize("M", [65, 129, 150, 193, 450])
 def test_pairs_of_many_rows(engine, oracle, gpu, force, capfd, K, widths, by_rows, M):
