@@ -20,13 +20,15 @@ struct RowsShape {
     static constexpr int kTiles = 4 / KS * NT, kQuarters = 4 / KS;
     static constexpr int kFragments = PAIR ? MF / 2 : MF;  // of outputs
     // One unit in LDS, a load brings 1 KiB: four rows of x; a tile's codes, eight tiles' metadata.  The rows, which
-    // come from the L2, and the codes, which come from HBM, have rings and waves of their own, so that more
-    // units of codes are on their way.
+    // come from the L2, and the codes, which come from HBM, have rings and waves of their own.
     static constexpr int kRowLoads = 4 * MF, kCodeLoads = kTiles + (kTiles + 7) / 8;
     // KiB: four fragments of sums from each multiplying wave, two where the rings leave no more
     static constexpr int kExchange = KS == 1 ? 0 : 3 * kRowLoads + 3 * kCodeLoads + 16 <= 160 ? 16 : 8;
-    static constexpr int kRowSlots = 4 * kRowLoads + 5 * kCodeLoads + kExchange <= 160 ? 4 : 3;
-    static constexpr int kCodeFit = (160 - (KS == 2 && MF < 4 ? 1 : 0) - kExchange - kRowSlots * kRowLoads) / kCodeLoads, kCodeSlots = kCodeFit > 6 ? 6 : kCodeFit;
+    static constexpr int kRowSlots = 4 * kRowLoads + 4 * kCodeLoads + kExchange <= 160 ? 4 : 3;
+    // Four units of codes: with up to six, requests to HBM run further ahead of the multiplying waves than they are of use
+    // (us, six and four units: two of 17408 x 5120 at 32 rows 32.7 and 31.5, at 67 rows 45 and 43.7; 5120 x 17408 at 67
+    // rows 28.2 and 27.4), and three are too few (6144 + 1024 + 1024 x 5120 at 48 rows 15.4 and, three, 19.8).
+    static constexpr int kCodeFit = (160 - (KS == 2 && MF < 4 ? 1 : 0) - kExchange - kRowSlots * kRowLoads) / kCodeLoads, kCodeSlots = kCodeFit > 4 ? 4 : kCodeFit;
     static constexpr int kRounds = KS == 1 ? 0 : (NT / 2 * kFragments + kExchange / 4 - 1) / (kExchange / 4);  // of the exchange
     // The two waves of an exchange meet at the workgroup's barriers, which wait for the fetching waves too, or, up to 48
     // rows, wait for each other alone: a barrier there cost 1.8 us of a short run (512 + 256 + 256 x 1088 at 32 rows 10.0 ->
