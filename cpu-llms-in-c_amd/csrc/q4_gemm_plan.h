@@ -335,28 +335,26 @@ struct RowsPlan {
 
 // The launch of q4_rows_kernel for a call's targets together; false: not the kernel for it.
 // `others_us`: what they would take otherwise.
-// Shape and workgroups minimise a microsecond estimate fitted to 2400 timings on this GPU (270 calls of one to three
-// weights from 448 x 512 to two of 17408 x 5120, 17 to 128 rows of fp16, fp32 and bf16, every block width, whole blocks
-// and 128 and 256 workgroups; 7 % rms, and the launch it chooses takes 0.6 % more than the best timed one): 5 us, each
-// unit, where workgroups share blocks 3.8 us and the partial sums at 1.8 TB/s, the conversion of activations that are not
-// fp16, the outputs.
+// Shape and workgroups minimise a microsecond estimate fitted to 14000 timings on this GPU (526 calls of one to three
+// weights from 128 x 512 to two of 17408 x 5120, 9 to 64 rows of fp32, 17 to 128 of fp16 and bf16, every block width, whole
+// blocks and 128 and 256 workgroups; each with weights from HBM, from the Infinity Cache, and between two large calls,
+// where the chip runs slower; 5 % rms; the launch it chooses takes 0.5 % more than the best timed one on average): a
+// unit's arithmetic, longer the more of the chip works (power), or its bytes; the end of every block in a workgroup's run,
+// which is why runs that divide a block are worth more; where workgroups share blocks the second kernel and the partial
+// sums; the conversion of activations that are not fp16; the outputs.  (Without the power and the ends: 1.3 %; two of
+// 17408 x 5120 at 32 rows took 128 columns a block, 33.0 us, and not 256, 31.5.)
 //
-// Several weights take it where that is not more than the other kernels' estimate, up to 96 rows 1.05 times that (us, this
-// kernel and the other: two of 17408 x 5120 at 67 rows 46.3 and 65.9, at 128 rows 62 and 70.5; 6144 + 1024 + 1024 x
-// 5120 at 32 rows 12.9 and 18.9, at 100 rows 23 and 26.8; 2048 + 512 + 512 x 1024 at 100 rows 10.8 and 9.7).
-//
-// One weight takes it where the estimate is well below the others', which are up to 2 us too high for calls of 10 to
-// 15 us: 0.82 times with fp32 and 0.8 with bf16 activations, 0.9 of fp16 rows.  Up to 64 fp16 rows a long weight of at
-// most 20 MB up to 1.1 times: the others lose more when it comes from HBM and not from the Infinity Cache (5120 x 6144
-// at 32 rows 13.7 here, there 13.5 and 14.2).  Above 64 rows 0.72 times; up to 80 rows of a long weight 0.96 (4240 x 13376
-// at 67 rows 25.3 here and 26.9 there); weights of more than 45 MB 0.9, and 0.99 where the other is the pipelined kernel
-// (17408 x 5120 at 67 rows from HBM 30 here and 31 there).  Above 64 rows the line is drawn for the others' sake more
-// often than timings ask for (13758 x 5312 at 84 rows 29 here and 36 there).
-// The choice of the 270 calls takes 1.4 to 3 % more than the better of the two, and 3 (one weight of fp16 rows) to 10 %
-// (several, and fp32) less than the choice between the others and this kernel's first form, in which every wave fetched
-// and multiplied.
-inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows, double others_us, int other_variant,
-                      RowsPlan &plan)
+// It is taken up to 1.05 times the other kernels' estimate for several weights of up to 96 matrix rows, 0.98 times of more
+// where they are large, and up to 0.89 times otherwise, 0.95 of 16-bit outputs of up to 64 rows: 0.1 to 0.7 % more time than
+// with the better of the two, above 96 rows 1 to 2 % (us from HBM and between large calls, this kernel and the others: 14336 x 5376 at 67 rows 24.3 and 30.7, 21.5 and
+// 29.4; 5120 x 6144 at 48 rows 15.4 and 16.0, 14.7 and 13.5; 17408 x 5120 at 112 rows 41 and 37; 6144 + 1024 + 1024 x 5120
+// at 67 rows 18.0 and 26.2, 17.9 and 23.0; two of 3584 x 1024 at 128 rows from the Infinity Cache 10.8 and 9.9, of 17408 x 5120 61.5 and 65.4
+// between large calls).
+// A unit, by tiles a block (4, 8, 16) and fragments:
+constexpr double kRowsUnitUs[3][9] = {{0, 0, 0.327, 0.380, 0.389, 0.434, 0.483, 0, 0.733},
+                                      {0, 0, 0.425, 0.506, 0.622, 0.647, 0.733, 0, 0.971},
+                                      {0, 0, 0.782, 0.873, 0.991, 1.123, 1.186, 0, 1.382}};
+inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows, double others_us, RowsPlan &plan)
 {
     const Q4Device &first = *a.targets[0].w;
     const uint32_t T = first.T;
@@ -383,26 +381,24 @@ inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t
         return true;
     }
     const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
-    double outputs = 0.0, megabytes = 0.0, best_cost = 1e30;  // megabytes: 4-bit codes and their metadata
-    for (uint32_t t = 0; t < a.count; ++t) {
-        outputs += (double)a.M * a.targets[t].w->N;
-        megabytes += (double)a.targets[t].w->N * first.K * 0.5625e-6;
-    }
+    double outputs = 0.0, best_cost = 1e30;
+    for (uint32_t t = 0; t < a.count; ++t) outputs += (double)a.M * a.targets[t].w->N;
     const double mf = plan.mf;
     RowsPlan best = plan;
     for (const int tiles : {4, 8, 16}) {
         if (!shape(tiles)) return false;
         const uint32_t total = plan.blocks * T;
-        const double unit = tiles == 4   ? 0.329 + mf * (0.0099 * mf - 0.0309)
-                            : tiles == 8 ? 0.216 + mf * (0.0015 * mf + 0.0864)
-                                         : 0.378 + mf * (0.2182 - 0.0112 * mf);
         for (const uint32_t want : {plan.blocks, cus / 2u, cus}) {
             plan.units = (total + want - 1u) / want;
-            const uint32_t groups = (total + plan.units - 1u) / plan.units;
-            const uint32_t rounds = (groups + cus - 1u) / cus;
-            double cost = 5.0 + (double)rounds * plan.units * unit;
-            if (plan.units % T != 0u && plan.units < total)
-                cost += 3.78 + 2.18e-6 * outputs * (T + plan.units - 1.0) / plan.units;
+            const uint32_t units = plan.units, groups = (total + units - 1u) / units, rounds = (groups + cus - 1u) / cus;
+            const bool sharing = units % T != 0u && units < total;
+            const double filled = (double)groups / ((double)rounds * cus);
+            const double unit = std::max(kRowsUnitUs[tiles / 8][plan.mf] * (1.0 + 0.0227 * mf * (filled - 0.75)), 0.051 * tiles * filled + 0.0483 * mf);
+            // ends of blocks in the longest run, and workgroups that share a block
+            const double ends = !sharing ? std::max(1u, units / T) : T % units == 0u ? 1.0 : (units - 2u) / T + 2u;
+            const double sharers = T % units == 0u ? T / units : (T + units - 1.0) / units;
+            double cost = 3.78 + rounds * (units * unit + ends * (plan.pair ? 0.0119 : 0.0237) * mf * tiles);
+            if (sharing) cost += 3.21 + sharers * (0.0781 + 1.53e-6 * outputs);
             if (cost < best_cost) {
                 best_cost = cost;
                 best = plan;
@@ -410,19 +406,13 @@ inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t
         }
     }
     plan = best;
-    best_cost += 0.37e-6 * outputs * dtype_bytes(a.y_dtype);
-    if (a.x_dtype != MI355Q_F16) best_cost += 2.98 + 1.92 * (double)rows * first.K * sizeof(_Float16) * 1e-6;
-    double most = 0.9;
-    if (a.count != 1u)
-        most = rows <= 96u ? 1.05 : 1.0;
-    else if (a.x_dtype != MI355Q_F16)
-        most = a.x_dtype == MI355Q_F32 ? 0.82 : 0.8;
-    else if (rows > 64u)
-        most = rows <= 80u && T >= 64u ? 0.96 : megabytes <= 45.0 ? 0.72 : other_variant >= kFirstPiped ? 0.99 : 0.9;
-    else if (megabytes > 20.0)
-        most = 0.9;
-    else if (T >= 40u)
-        most = 1.1;
+    best_cost += 0.107e-6 * outputs * dtype_bytes(a.y_dtype);
+    if (a.x_dtype != MI355Q_F16) best_cost += 3.24 + 1.86e-6 * rows * first.K * sizeof(_Float16);
+    double most = 0.89;
+    if (a.count != 1u && (rows <= 96u || others_us > 20.0))
+        most = rows <= 96u ? 1.05 : 0.98;
+    else if (a.count == 1u && rows <= 64u && a.y_dtype != MI355Q_F32)
+        most = 0.95;
     return best_cost <= most * others_us;
 }
 
@@ -496,7 +486,7 @@ inline bool plan_gemm(const mi355q_context *ctx, const Q4LinearArgs &a, TargetPl
         plans[t] = same < t ? plans[same] : plan_target(ctx, a, t, rows);
     }
     group = plan_group(ctx, a, rows, plans);
-    return rows_plan(ctx, a, rows, group.us, plans[0].variant, rows_launch);
+    return rows_plan(ctx, a, rows, group.us, rows_launch);
 }
 
 }  // namespace mi355q

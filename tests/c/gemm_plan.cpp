@@ -153,13 +153,26 @@ static int check_widths(const mi355q_context *ctx)
     return 0;
 }
 
-// One weight at 17 to 128 rows takes the kernel that was timed faster for it, q4_rows_kernel or another.
+// One weight at 17 to 128 rows takes the kernel that was timed faster for it, q4_rows_kernel or another (us, weights from
+// HBM), and two large ones at 32 rows the width of block that was.
 static int check_rows(const mi355q_context *ctx)
 {
     const struct { uint32_t M, K, N; int x; bool by_rows; } calls[] = {
-        {36, 2944, 2928, MI355Q_F32, false}, {28, 5120, 1280, MI355Q_F32, false}, {80, 5376, 14336, MI355Q_F16, false},
-        {96, 5376, 14336, MI355Q_BF16, false}, {100, 3584, 1024, MI355Q_F16, false}, {32, 6144, 5120, MI355Q_F16, true}, {32, 17408, 5120, MI355Q_F16, true},
-        {67, 17408, 5120, MI355Q_F16, true}, {67, 5120, 17408, MI355Q_F16, true}, {48, 2048, 1024, MI355Q_F16, true}, {36, 1152, 12000, MI355Q_BF16, true}};
+        {36, 2944, 2928, MI355Q_F32, true},     // 16.1 by q4_rows_kernel, 17.1 by the other
+        {28, 5120, 1280, MI355Q_F32, true},     // 14.8, 16.7
+        {80, 5376, 14336, MI355Q_F16, true},    // 22.9, 33.0
+        {84, 5312, 13758, MI355Q_F16, true},    // 25.6, 33.4
+        {96, 5376, 14336, MI355Q_BF16, true},   // 30.4, 35.6
+        {112, 5376, 14336, MI355Q_F16, false},  // 38.1, 33.7
+        {112, 5120, 17408, MI355Q_F16, false},  // 41.0, 36.8
+        {128, 6144, 5120, MI355Q_F16, false},   // 25.4, 21.3
+        {100, 3584, 1024, MI355Q_F16, false},   // 12.7, 11.5
+        {32, 6144, 5120, MI355Q_F16, true},     // 14.6, 14.8
+        {32, 17408, 5120, MI355Q_F16, true},    // 22.5, 27.3
+        {67, 17408, 5120, MI355Q_F16, true},    // 28.7, 35.8
+        {67, 5120, 17408, MI355Q_F16, true},    // 29.0, 33.1
+        {48, 2048, 1024, MI355Q_F16, true},     // 9.7, 11.6
+        {36, 1152, 12000, MI355Q_BF16, true}};  // 11.8, 16.1
     for (const auto &of : calls) {
         Call call(of.M, of.K, {of.N});
         call.a.x_dtype = of.x;
@@ -171,6 +184,14 @@ static int check_rows(const mi355q_context *ctx)
             printf("%u x %u at %u rows of type %d: the other kernel\n", of.N, of.K, of.M, of.x);
             return 1;
         }
+    }
+    Call pair(32, 5120, {17408, 17408});  // 128 columns a block 33.0 us, 256 31.5
+    TargetPlan plans[kMaxTargets];
+    GroupPlan group;
+    RowsPlan rows;
+    if (!plan_gemm(ctx, pair.a, plans, group, rows) || rows.tiles != 16) {
+        printf("two of 17408 x 5120 at 32 rows: %d tiles a block\n", rows.tiles);
+        return 1;
     }
     printf("rows ok\n");
     return 0;
