@@ -21,7 +21,7 @@
 //   q4_gemm_pipe_kernel: one workgroup per compute unit, software pipelined by
 //     hand (128 rows x 16, 17 or 20 tiles);
 //   q4_rows_kernel (q4_rows_device.h): up to 128 rows, all weights of a call as
-//     one launch; of fp32 activations also more, in blocks of 64 rows' pairs.
+//     one launch; of fp32 activations also up to 256, in blocks of 16 to 64 rows' pairs.
 // The host picks shape and K split by a time estimate fitted on this GPU (q4_gemm_plan.h), e.g.
 // 20 tiles for the 17408-row matrices: 55 x 4 = 220 workgroups at M = 512.
 // Several weights of a call go out as one launch where that is estimated to take less: they
@@ -303,9 +303,9 @@ static int gemm_activations(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t
 }
 
 // Targets first .. first + count - 1 of a call in one launch: the shape `variant`, each target with the
-// K split of its own plan.
+// K split of its own plan; `convert`: the call's activations have not been converted yet.
 static int gemm_targets(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t first, uint32_t count, const TargetPlan *plans,
-                        int variant, char *error, size_t error_capacity)
+                        int variant, bool convert, char *error, size_t error_capacity)
 {
     const Q4Device &shape = *a.targets[first].w;  // columns and kind are the same for all
     const bool bytes_kernel = plans[first].bytes;
@@ -317,7 +317,7 @@ static int gemm_targets(mi355q_context *ctx, const Q4LinearArgs &a, uint32_t fir
     GemmGroup group;
     memset(&group, 0, sizeof group);
     GemmParams &p = group.shared;
-    int status = gemm_activations(ctx, a, x_columns, first == 0, p, error, error_capacity);
+    int status = gemm_activations(ctx, a, x_columns, convert, p, error, error_capacity);
     if (status != MI355Q_OK) return status;
     const Variant &chosen = variants[variant];
     const uint32_t tpb = 4u * chosen.ntw + chosen.extra;
@@ -532,23 +532,26 @@ int q4_gemm_linears(mi355q_context *ctx, const Q4LinearArgs &a, char *error, siz
     TargetPlan plans[kMaxTargets];
     RowsPlan together;
     GroupPlan group;
-    if (plan_gemm(ctx, a, plans, group, together)) return q4_rows_linears(ctx, a, together, error, error_capacity);
     bool taken[kMaxTargets];
-    const uint32_t pairs = plan_pairs(ctx, a, plans, taken, together);
+    const uint32_t pairs = plan_pairs(ctx, a, taken, together);
     if (pairs == a.count) return q4_rows_linears(ctx, a, together, error, error_capacity);
-    if (pairs != 0u) {  // those targets by q4_rows_kernel, the others as a call of their own
-        Q4LinearArgs part[2] = {a, a};
-        part[0].count = part[1].count = 0;
+    Q4LinearArgs rest = a;
+    if (pairs != 0u) {  // those targets by q4_rows_kernel, the others behind them on the same converted activations
+        Q4LinearArgs part = a;
+        part.count = rest.count = 0;
         for (uint32_t t = 0; t < a.count; ++t) {
-            Q4LinearArgs &to = part[taken[t] ? 0 : 1];
+            Q4LinearArgs &to = taken[t] ? part : rest;
             to.targets[to.count++] = a.targets[t];
         }
-        status = q4_rows_linears(ctx, part[0], together, error, error_capacity);
-        return status == MI355Q_OK ? q4_gemm_linears(ctx, part[1], error, error_capacity) : status;
+        status = q4_rows_linears(ctx, part, together, error, error_capacity);
+        if (status != MI355Q_OK) return status;
     }
-    if (group.variant >= 0) return gemm_targets(ctx, a, 0, a.count, plans, group.variant, error, error_capacity);
-    for (uint32_t t = 0; t < a.count && status == MI355Q_OK; ++t)
-        status = gemm_targets(ctx, a, t, 1, plans, plans[t].variant, error, error_capacity);
+    if (plan_gemm(ctx, rest, plans, group, together)) return q4_rows_linears(ctx, rest, together, error, error_capacity);
+    const bool convert = pairs == 0u;
+    if (group.variant >= 0)
+        return gemm_targets(ctx, rest, 0, rest.count, plans, group.variant, convert, error, error_capacity);
+    for (uint32_t t = 0; t < rest.count && status == MI355Q_OK; ++t)
+        status = gemm_targets(ctx, rest, t, 1, plans, plans[t].variant, convert && t == 0u, error, error_capacity);
     return status;
 }
 

@@ -354,6 +354,19 @@ struct RowsPlan {
 constexpr double kRowsUnitUs[3][9] = {{0, 0, 0.327, 0.380, 0.389, 0.434, 0.483, 0, 0.733},
                                       {0, 0, 0.425, 0.506, 0.622, 0.647, 0.733, 0, 0.971},
                                       {0, 0, 0.782, 0.873, 0.991, 1.123, 1.186, 0, 1.382}};
+// A launch of T steps a block, without the conversion and the outputs.
+inline double rows_launch_us(uint32_t cus, uint32_t T, double outputs, const RowsPlan &plan)
+{
+    const uint32_t total = plan.blocks * T, units = plan.units, groups = (total + units - 1u) / units, rounds = (groups + cus - 1u) / cus;
+    const bool sharing = units % T != 0u && units < total;
+    const double mf = plan.mf, tiles = plan.tiles, filled = (double)groups / ((double)rounds * cus);
+    const double unit = std::max(kRowsUnitUs[plan.tiles / 8][plan.mf] * (1.0 + 0.0227 * mf * (filled - 0.75)), 0.051 * tiles * filled + 0.0483 * mf);
+    // ends of blocks in the longest run, and workgroups that share a block
+    const double ends = !sharing ? std::max(1u, units / T) : T % units == 0u ? 1.0 : (units - 2u) / T + 2u;
+    const double sharers = T % units == 0u ? T / units : (T + units - 1.0) / units;
+    const double us = 3.78 + rounds * (units * unit + ends * (plan.pair ? 0.0119 : 0.0237) * mf * tiles);
+    return sharing ? us + 3.21 + sharers * (0.0781 + 1.53e-6 * outputs) : us;
+}
 inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows, double others_us, RowsPlan &plan)
 {
     const Q4Device &first = *a.targets[0].w;
@@ -383,22 +396,13 @@ inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t
     const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
     double outputs = 0.0, best_cost = 1e30;
     for (uint32_t t = 0; t < a.count; ++t) outputs += (double)a.M * a.targets[t].w->N;
-    const double mf = plan.mf;
     RowsPlan best = plan;
     for (const int tiles : {4, 8, 16}) {
         if (!shape(tiles)) return false;
         const uint32_t total = plan.blocks * T;
         for (const uint32_t want : {plan.blocks, cus / 2u, cus}) {
             plan.units = (total + want - 1u) / want;
-            const uint32_t units = plan.units, groups = (total + units - 1u) / units, rounds = (groups + cus - 1u) / cus;
-            const bool sharing = units % T != 0u && units < total;
-            const double filled = (double)groups / ((double)rounds * cus);
-            const double unit = std::max(kRowsUnitUs[tiles / 8][plan.mf] * (1.0 + 0.0227 * mf * (filled - 0.75)), 0.051 * tiles * filled + 0.0483 * mf);
-            // ends of blocks in the longest run, and workgroups that share a block
-            const double ends = !sharing ? std::max(1u, units / T) : T % units == 0u ? 1.0 : (units - 2u) / T + 2u;
-            const double sharers = T % units == 0u ? T / units : (T + units - 1.0) / units;
-            double cost = 3.78 + rounds * (units * unit + ends * (plan.pair ? 0.0119 : 0.0237) * mf * tiles);
-            if (sharing) cost += 3.21 + sharers * (0.0781 + 1.53e-6 * outputs);
+            const double cost = rows_launch_us(cus, T, outputs, plan);
             if (cost < best_cost) {
                 best_cost = cost;
                 best = plan;
@@ -416,61 +420,70 @@ inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t
     return best_cost <= most * others_us;
 }
 
-// ---- more than 128 rows, fp32 activations: q4_rows_kernel on whole blocks of 64 rows or less -----------
+// ---- 65 to 256 rows of fp32: q4_rows_kernel on whole blocks of 16 to 64 rows' pairs ------------------------
 
-// A call of targets 0 .. count - 1, whole blocks dealt to workgroups as evenly as they come: microseconds, and the blocks'
-// width.  Fitted to 600 timings on this GPU (210 calls from 512 x 512 to 6144 x 1536 and three of 1536 x 1536, 70 to
-// 1500 rows; 7 % rms): the conversion, then for every block of a workgroup its steps and its outputs.
-inline double pairs_us(uint32_t cus, const Q4LinearArgs &a, const uint32_t *of, uint32_t count, RowsPlan &plan)
+// Weights of 3 to 14 steps, fp32 outputs.  The other kernels multiply value and remainder rows like rows of their own,
+// in blocks whose fill and stores nothing hides (us, those and this kernel: three of 1280 x 1280 at 150 rows 21.9 and
+// 14.0, 1280 x 1280 at 150 rows 15.5 and 11.6, 5120 x 1280 at 150 rows 17.0 and 15.1, 140 x 1280 at 203 rows 14.2 and 11.5).
+// A weight has the bits of its own call in company, so it takes this kernel whatever shares the call: by the rows and
+// columns of x, which the weights of a call have in common, and not by an estimate of its own call, which parted
+// calls in two launches with a conversion each (2688 + 128 x 1280 at 319 rows 22 -> 33 us).  Weights more than four times as wide
+// as x, which no other of its layer is, are left out, and a call that has both kinds is the one that is parted.
+// More rows or wider weights fill the chip with the other kernels' larger blocks: calls whose outputs were more than 512 times
+// the columns of x lost at times (28440 x 384 at 152 rows 20 -> 27, 5120 x 1280 at 1345 rows 55 -> 64).  Of more than 14 steps
+// the others split K into more sums than this kernel's two, whose error is smaller.
+constexpr uint32_t kPairsRows = 256, kPairsSteps[2] = {3, 14}, kPairsWide = 4;
+inline bool pairs_take(const mi355q_context *ctx, const Q4LinearArgs &a, const Q4Device &w)
 {
-    const uint32_t T = a.targets[0].w->T, block_rows = (a.M + (a.M + 63u) / 64u - 1u) / ((a.M + 63u) / 64u);
-    plan.pair = true;
-    plan.m_blocks = (a.M + 63u) / 64u;
-    plan.mf = 2 * (int)((block_rows + 15u) / 16u);
-    double best = 1e30, outputs = 0.0;
-    for (uint32_t i = 0; i < count; ++i) outputs += (double)a.M * a.targets[of[i]].w->N * dtype_bytes(a.y_dtype) * 1e-6;
-    RowsPlan at = plan;
-    for (const int tiles : {4, 8}) {  // (16 tiles of so many rows add a row's products up in another order)
-        at.tiles = tiles;
-        uint64_t blocks = 0;
-        for (uint32_t i = 0; i < count; ++i) blocks += (uint64_t)((a.targets[of[i]].w->NT + tiles - 1u) / tiles) * plan.m_blocks;
-        if (blocks * T >= (1ull << 31)) continue;
-        const uint32_t rounds = (uint32_t)((blocks + cus - 1u) / cus);
-        at.blocks = (uint32_t)blocks;
-        at.units = rounds * T;
-        const double mf = plan.mf, filled = (double)((blocks + rounds - 1u) / rounds) / cus;
-        const double alone = 0.1192 * mf + 0.0753 * tiles - 0.0044 * mf * tiles - 0.412;
-        const double share = (0.2807 * mf - 0.1142 * tiles + 0.0194 * mf * tiles - 1.64) * (0.649 + 0.351 * filled);
-        const double us = 6.75 + 1.777e-6 * a.M * 2.0 * a.targets[0].w->K + rounds * (T * std::max(alone, share) + 0.0317 * mf * tiles) +
-                          0.188 * outputs;
-        if (us < best) {
-            best = us;
-            plan = at;
-        }
-    }
-    return best;
+    if (a.x_dtype != MI355Q_F32 || a.M <= 64u || a.x_columns != 0u || w.K % kStepColumns != 0u || ctx->gemm_order >= 0) return false;
+    if (ctx->force_gemm[1] >= 1)  // 32-bit offsets into a block's rows, and steps in all
+        return ctx->force_gemm[0] >= 11 && ctx->force_gemm[0] <= 13 && (uint64_t)w.K * 256u < (1ull << 32) &&
+               (uint64_t)(w.NT + 3u) / 4u * w.T * ((a.M + 15u) / 16u) * kMaxTargets < (1ull << 31);
+    return a.y_dtype == MI355Q_F32 && a.residual_dtype == MI355Q_F32 && a.M <= kPairsRows && w.T >= kPairsSteps[0] &&
+           w.T <= kPairsSteps[1] && w.N <= kPairsWide * w.K;
 }
 
-// Which targets of the call it takes (their number): those whose own call is estimated to take 2 % less, so that a weight
-// has the bits of its own call in company too.  Outputs do not depend on the blocks' width.  Rows of a few steps have
-// the most to gain: the other kernels multiply value and remainder rows like rows of their own, in blocks whose
-// fill and stores nothing hides (us, those and this kernel: three of 1280 x 1280 at 150 rows 21.9 and 16.1, at 1500 rows 50.7 and 47.3;
-// 5120 x 1280 at 700 rows 36.2 and 29.5, 1280 x 1280 at 300 rows 17.3 and 16.9, at 100 rows 14.2 and 15.5).  With
-// more steps than about sixteen they have K splits for weights that do not fill the chip (1280 x 5120 at 300 rows 26 and 46).
-// Of 58 calls of three weights 10 % less time, of 155 of one 2 %.
-inline uint32_t plan_pairs(const mi355q_context *ctx, const Q4LinearArgs &a, const TargetPlan *plans, bool *taken, RowsPlan &plan)
+// The targets that it takes (their number) and the launch for them.  The block is chosen by the estimate above (0.2 % more time
+// than the best timed one over 800 calls).  Outputs do not depend on it: in these forms two waves share a tile's columns.
+inline uint32_t plan_pairs(const mi355q_context *ctx, const Q4LinearArgs &a, bool *taken, RowsPlan &plan)
 {
-    const Q4Device &first = *a.targets[0].w;
-    if (a.x_dtype != MI355Q_F32 || a.M <= 64u || a.x_columns != 0u || first.K % kStepColumns != 0u || ctx->force_gemm[1] >= 1 ||
-        ctx->gemm_order >= 0 || (uint64_t)128u * first.K * sizeof(_Float16) >= (1ull << 32))
-        return 0;
-    const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
-    uint32_t of[kMaxTargets], count = 0;
+    const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount, T = a.targets[0].w->T;
+    uint32_t count = 0;
     for (uint32_t t = 0; t < a.count; ++t) {
-        taken[t] = a.targets[t].w->N % 4u == 0u && pairs_us(cus, a, &t, 1, plan) <= 0.98 * plans[t].us;
-        if (taken[t]) of[count++] = t;
+        taken[t] = pairs_take(ctx, a, *a.targets[t].w);
+        if (taken[t]) ++count;
     }
-    if (count != 0u && pairs_us(cus, a, of, count, plan) >= 1e30) return 0;
+    if (count == 0u) return 0;
+    RowsPlan at;
+    at.pair = true;
+    auto shape = [&](int tiles, int mf) {
+        at.tiles = tiles;
+        at.mf = mf;
+        at.m_blocks = (a.M + 8u * mf - 1u) / (8u * mf);
+        at.blocks = 0;
+        for (uint32_t t = 0; t < a.count; ++t)
+            if (taken[t]) at.blocks += (a.targets[t].w->NT + tiles - 1u) / tiles * at.m_blocks;
+        at.units = (at.blocks + cus - 1u) / cus * T;
+        return mf * tiles <= 64 && (mf > 2 || tiles == 4);  // (else a wave takes whole columns)
+    };
+    if (ctx->force_gemm[1] >= 1) {
+        // option "q4_gemm": 11, 12, 13 = 4, 8, 16 tiles a block; s = 1 .. 4 for 16 to 64 rows, 5 .. 8 for two blocks a workgroup, ...
+        const int s = ctx->force_gemm[1] - 1;
+        if (!shape(4 << (ctx->force_gemm[0] - 11), 2 * (s % 4 + 1))) return 0;
+        at.units = std::min((uint32_t)s / 4u + 1u, at.blocks) * T;
+        plan = at;
+        return count;
+    }
+    double best = 1e30;
+    for (const int tiles : {4, 8, 16})
+        for (const int mf : {2, 4, 6, 8}) {
+            if (!shape(tiles, mf)) continue;
+            const double us = rows_launch_us(cus, T, 0.0, at);
+            if (us < best) {
+                best = us;
+                plan = at;
+            }
+        }
     return count;
 }
 

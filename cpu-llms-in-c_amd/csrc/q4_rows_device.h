@@ -437,8 +437,9 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
                     }
                 }
             }
-        } else if (p.y_dtype == MI355Q_F32 && p.wide_stores && (p.residual == nullptr || (p.residual_dtype == MI355Q_F32 && (uintptr_t)p.residual % 16u == 0u))) {
+        } else if (p.y_dtype == MI355Q_F32 && (p.residual == nullptr || p.residual_dtype == MI355Q_F32)) {
             // the loads of a tile's residuals are on their way together
+            const bool wide = p.wide_stores && (uintptr_t)p.residual % 16u == 0u;
             float scale[OF];
 #pragma unroll
             for (int f = 0; f < OF; ++f) {
@@ -451,21 +452,35 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
                 if (n >= p.N) continue;
                 floatx4 more[OF];
 #pragma unroll
-                for (int f = 0; f < OF; ++f) more[f] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                for (int f = 0; f < OF; ++f) more[f] = floatx4{-0.0f, -0.0f, -0.0f, -0.0f};  // (which adds nothing, also to -0)
                 if (p.residual != nullptr) {
 #pragma unroll
                     for (int f = 0; f < OF; ++f) {
                         const uint32_t m = m0 + 16u * f + r;
-                        more[f] = *(const floatx4 *)((const float *)p.residual + (p.residual_is_bias ? 0 : (size_t)(m < M ? m : M - 1u) * p.N) + n);
+                        const float *const from = (const float *)p.residual + (p.residual_is_bias ? 0 : (size_t)(m < M ? m : M - 1u) * p.N);
+                        if (wide) {
+                            more[f] = *(const floatx4 *)(from + n);
+                        } else {
+#pragma unroll
+                            for (uint32_t j = 0; j < 4u; ++j) more[f][j] = from[n + j < p.N ? n + j : p.N - 1u];
+                        }
                     }
                 }
 #pragma unroll
                 for (int f = 0; f < OF; ++f) {
                     const uint32_t m = m0 + 16u * f + r;
+                    float *const to = (float *)p.y + (size_t)m * p.N + n;
                     floatx4 value;
 #pragma unroll
                     for (int j = 0; j < 4; ++j) value[j] = acc[t][f][j] * scale[f] + more[f][j];
-                    if (m < M) *(floatx4 *)((float *)p.y + (size_t)m * p.N + n) = value;
+                    if (m >= M) continue;
+                    if (wide) {
+                        *(floatx4 *)to = value;
+                    } else {
+#pragma unroll
+                        for (uint32_t j = 0; j < 4u; ++j)
+                            if (n + j < p.N) to[j] = value[j];
+                    }
                 }
             }
         } else

@@ -122,7 +122,9 @@ int mi355q_context_info(mi355q_context *ctx, mi355q_device_info *info,
  *   "q4_gemm"   = "VARIANT,SPLITS"              forces the GEMM's kernel variant and K split; variants 11,
  *                                               12, 13 are blocks of 4, 8, 16 tiles of the kernel for
  *                                               17 to 128 rows, whose second number is 1 for whole
- *                                               blocks, s > 1 for 64 (s - 1) workgroups that share them
+ *                                               blocks, s > 1 for 64 (s - 1) workgroups that share
+ *                                               them; of fp32 x beyond 64 rows 1 .. 4 for blocks of
+ *                                               16 .. 64 rows, 5 .. 8 for two of them a workgroup, ...
  *   "trace"     = "1"                           prints every launch's decomposition to stderr
  *   "in_kernel_slices" = "0"                    K slices are added by a second kernel
  *   "w8a8"      = "1" .. "4"                    W8A8: the kernel of tiles, with so many per workgroup

@@ -1,6 +1,6 @@
 // The planner of the GEMM calls (csrc/q4_gemm_plan.h) on the host: its estimates of the pipelined kernel
 // against a schedule that hands out every workgroup, the choice for one weight, and what planning a call takes.
-//   gemm_plan            prints "schedule ok", "choices ok", "widths ok", "rows ok", "order ok" and, a line a call, its name and microseconds
+//   gemm_plan            prints "schedule ok", "choices ok", "widths ok", "rows ok", "pairs ok", "order ok" and, a line a call, its name and microseconds
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -197,6 +197,40 @@ static int check_rows(const mi355q_context *ctx)
     return 0;
 }
 
+// fp32 calls of 65 rows and more: the weights of a call take q4_rows_kernel together or not at all, up to four times the columns
+// of x, so that such a call is one launch; and the launch is not estimated to take longer than theirs, but for the estimates' own error.
+static int check_pairs(const mi355q_context *ctx)
+{
+    std::mt19937 random(3);
+    for (int round = 0; round < 6000; ++round) {
+        const uint32_t T = 1u + (uint32_t)(random() % 18u), K = T * kStepColumns, M = 65u + (uint32_t)(random() % (round % 2 ? 200u : 1500u));
+        std::vector<uint32_t> widths(1 + random() % kMaxTargets);
+        for (uint32_t &N : widths) N = round == 0 ? 128u : 1u + (uint32_t)(random() % (4u * K));
+        Call call(M, K, widths);
+        call.a.x_dtype = call.a.y_dtype = call.a.residual_dtype = MI355Q_F32;
+        TargetPlan plans[kMaxTargets];
+        GroupPlan group;
+        RowsPlan rows, other;
+        bool taken[kMaxTargets];
+        const uint32_t count = plan_pairs(ctx, call.a, taken, rows);
+        if (count != 0u && count != call.a.count) {
+            printf("%u of %u weights at %u rows of %u\n", count, call.a.count, M, K);
+            return 1;
+        }
+        if (count == 0u) continue;
+        plan_gemm(ctx, call.a, plans, group, other);
+        double outputs = 0.0;
+        for (const uint32_t N : widths) outputs += (double)M * N;
+        const double us = rows_launch_us(kCus, T, outputs, rows) + 0.107e-6 * outputs * 4.0 + 3.24 + 1.86e-6 * 2.0 * M * K * 2.0;
+        if (us > 1.1 * group.us) {
+            printf("%u weights at %u rows of %u: %.1f us, as one launch of the others %.1f\n", call.a.count, M, K, us, group.us);
+            return 1;
+        }
+    }
+    printf("pairs ok\n");
+    return 0;
+}
+
 // Weights that share a launch go out one by one under option "gemm_order", whose two orders are one weight's.
 static int check_order(mi355q_context *ctx)
 {
@@ -243,7 +277,7 @@ int main()
     if (ctx == nullptr) return 1;
     ctx->props.multiProcessorCount = (int)kCus;
     ctx->gemm_order = -1;
-    if (check_choices(ctx) != 0 || check_widths(ctx) != 0 || check_rows(ctx) != 0 || check_order(ctx) != 0) return 1;
+    if (check_choices(ctx) != 0 || check_widths(ctx) != 0 || check_rows(ctx) != 0 || check_pairs(ctx) != 0 || check_order(ctx) != 0) return 1;
     printf("q_k_v_32_rows %.2f\n", planning_us(ctx, 32, 5120, {6144, 1024, 1024}));
     printf("q_k_v_512_rows %.2f\n", planning_us(ctx, 512, 5120, {6144, 1024, 1024}));
     printf("gate_up_512_rows %.2f\n", planning_us(ctx, 512, 5120, {17408, 17408}));

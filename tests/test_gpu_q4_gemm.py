@@ -376,13 +376,14 @@ def test_rows_kernel_pairs_precision(engine, oracle, gpu, force, forced, parts, 
     assert error <= bound
 
 
-@pytest.mark.parametrize("K,widths,by_rows", [(1280, (1280, 1280, 1280), 3), (640, (2048, 516, 1002), 2), (1152, (3072,), 1)])
-@pytest.mark.parametrize("M", [65, 129, 150, 193, 450])
+@pytest.mark.parametrize("K,widths,by_rows", [(1280, (1280, 1280, 1280), 3), (640, (2048, 516, 1002), 3),
+                                              (640, (2048, 2564, 516, 2561), 2), (1152, (3072,), 1), (384, (1, 1536), 2)])
+@pytest.mark.parametrize("M", [65, 129, 150, 193, 256])
 def test_pairs_of_many_rows(engine, oracle, gpu, force, capfd, K, widths, by_rows, M):
-    """fp32 activations beyond 128 matrix rows by q4_rows_kernel: two to eight blocks of rows, the last with one row or full,
-    more blocks than compute units and fewer, weights it takes beside one it does not (a width that is no multiple of
-    4).  Each output has the bits of its weight's own call, agrees with another kernel up to the order of
-    the sums, and the first weight's with the oracle."""
+    """65 to 256 fp32 rows by q4_rows_kernel: two to sixteen blocks of rows, the last with one row or full, weights it
+    takes beside wider ones that it does not, which run behind them on the same converted activations.  Each output
+    has the bits of its weight's own call, agrees with another kernel up to the order of the sums, and the first
+    weight's with the oracle."""
     kind = engine.META_BF16_PLANES
     x = make_x(engine, 201, M, K)
     planes = [engine.synth_q4_affine(202 + i, 0.02, N, K, kind) for i, N in enumerate(widths)]
@@ -405,8 +406,8 @@ def test_pairs_of_many_rows(engine, oracle, gpu, force, capfd, K, widths, by_row
             gpu.sync()
             printed.append(capfd.readouterr().err)
             results.append([gpu.download(p, (M, N), np.float32) for p, N in zip(outputs, widths)])
-        if M == 150:  # (other numbers of rows are the estimates' choice)
-            assert printed[1].count("q4 rows M=150") == by_rows and printed[0].count("q4 rows M=150") == 1
+        line = f"q4 rows M={M}"
+        assert [p.count(line) for p in printed] == [1, by_rows, 0]
         for together, alone, other in zip(*results):
             assert np.array_equal(together, alone)
             # K products of one row, of values and of remainders, summed in another order
@@ -416,6 +417,61 @@ def test_pairs_of_many_rows(engine, oracle, gpu, force, capfd, K, widths, by_row
         assert q4_relative_error(np.asarray(results[1][0], np.float64), ref) <= 1e-3
     finally:
         for pointer in [x_ptr] + outputs + biases:
+            gpu.free(pointer)
+        for weight in weights:
+            weight.destroy()
+
+
+@pytest.mark.parametrize("forced,tiles,rows,blocks", [
+    ("11,1", 4, 16, 1), ("11,6", 4, 32, 2), ("11,11", 4, 48, 3), ("11,8", 4, 64, 2), ("12,2", 8, 32, 1), ("12,10", 8, 32, 3),
+    ("12,7", 8, 48, 2), ("12,12", 8, 64, 3), ("13,2", 16, 32, 1), ("13,6", 16, 32, 2), ("13,10", 16, 32, 3)])
+@pytest.mark.parametrize("y_dtype,residual_dtype,shift", [("F32", "F32", 0), ("F32", "F32", 1), ("F32", "F16", 0), ("F16", "F32", 0),
+                                                          ("BF16", "BF16", 1), ("F32", None, 0)])
+@pytest.mark.parametrize("K,M", [(384, 150), (1152, 257)])
+def test_blocks_of_pairs(engine, gpu, force, capfd, forced, tiles, rows, blocks, y_dtype, residual_dtype, shift, K, M):
+    """Every block of fp32 pairs beyond 64 rows, one to three a workgroup: runs that end inside a weight and in the next
+    one, more blocks than compute units and fewer, a last block of rows partly filled, tiles beyond the matrix, widths
+    with and without 16-byte pieces; residual rows of every type, outputs of every type, also one element off
+    their alignment.  The bits do not depend on the block."""
+    kind, widths = engine.META_BF16_PLANES, (1284, 330, 64, 1002)
+    x = make_x(engine, 231, M, K)
+    weights = [gpu.q4_prepare(*engine.synth_q4_affine(232 + i, 0.02, N, K, kind), N, K, kind) for i, N in enumerate(widths)]
+    cell = {"F32": np.float32, "F16": np.float16, "BF16": np.uint16}
+
+    def rows_of(seed, N, dtype):
+        values = engine.synth_normal_f32(seed, 1.0, M * N).reshape(M, N)
+        return bf16_bits(values) if dtype == "BF16" else values.astype(cell[dtype])
+
+    residuals = [None if residual_dtype is None else gpu.to_device(rows_of(240 + i, N, residual_dtype)) for i, N in enumerate(widths)]
+    x_ptr = gpu.to_device(x)
+    width = np.dtype(cell[y_dtype]).itemsize
+    outputs = [gpu.alloc(M * N * width + 64) for N in widths]
+    try:
+        results = []
+        for how in (forced, "11,4", "4,1"):
+            print(f"blocks of pairs K={K} M={M} y={y_dtype} residual={residual_dtype} shift={shift} forced={how}", flush=True)
+            force("q4_gemm", how)
+            force("trace", "1")
+            capfd.readouterr()
+            targets = [(w, y + shift * width, r) for w, y, r in zip(weights, outputs, residuals)]
+            gpu.q4_sequence(engine.make_calls([(targets, x_ptr, engine.F32, M, getattr(engine, y_dtype),
+                                                getattr(engine, residual_dtype or "F32"))]))
+            gpu.sync()
+            printed = capfd.readouterr().err
+            if how == forced:
+                assert f"{rows // 8} fragments of pairs x {16 * tiles} columns" in printed
+                assert f"{blocks * K // 128} steps each" in printed
+            results.append([gpu.download(y + shift * width, (M, N), cell[y_dtype]) for y, N in zip(outputs, widths)])
+        for here, same, other in zip(*results):
+            assert np.array_equal(here.view(np.uint16), same.view(np.uint16)) and np.any(here != 0)
+            if y_dtype == "BF16":
+                here, other = ((v.astype(np.uint32) << 16).view(np.float32) for v in (here, other))
+            here, other = here.astype(np.float64), other.astype(np.float64)
+            # K products of one row, of values and of remainders, summed in another order; two roundings to 11 or 8 bits
+            rounding = {"F32": 0.0, "F16": 2.0 ** -11, "BF16": 2.0 ** -8}[y_dtype]
+            assert np.max(np.abs(here - other)) <= 2 * (K * 2.0 ** -24 + rounding) * np.max(np.abs(other))
+    finally:
+        for pointer in [x_ptr] + outputs + [r for r in residuals if r is not None]:
             gpu.free(pointer)
         for weight in weights:
             weight.destroy()
