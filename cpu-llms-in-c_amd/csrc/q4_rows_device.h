@@ -14,7 +14,9 @@ namespace mi355q {
 // taken, and with both in every wave a unit took the sum of the two (80 rows x 256 columns: 0.77 us for the loads,
 // 1.07 for the arithmetic, 1.75 together; without any wait for the data 1.68).
 // The multiplying waves share a unit as KS parts of its columns by 4 / KS groups of NT tiles.  With KS = 2 its rows are
-// read from LDS twice instead of four times, and two waves exchange halves of their sums when the block is done.
+// read from LDS twice instead of four times, and two waves exchange halves of their sums when the block is done, at the
+// workgroup's barriers (a wait for the other wave alone, by polling a word in LDS: layers of 17 to 48 rows 0.7 % more time, of
+// 64 to 96 rows 1.2 %).
 template <int MF, int NT, int KS, bool PAIR>
 struct RowsShape {
     static constexpr int kTiles = 4 / KS * NT, kQuarters = 4 / KS;
@@ -28,16 +30,11 @@ struct RowsShape {
     // Four units of codes: with up to six, requests to HBM run further ahead of the multiplying waves than they are of use
     // (us, six and four units: two of 17408 x 5120 at 32 rows 32.7 and 31.5, at 67 rows 45 and 43.7; 5120 x 17408 at 67
     // rows 28.2 and 27.4), and three are too few (6144 + 1024 + 1024 x 5120 at 48 rows 15.4 and, three, 19.8).
-    static constexpr int kCodeFit = (160 - (KS == 2 && MF < 4 ? 1 : 0) - kExchange - kRowSlots * kRowLoads) / kCodeLoads, kCodeSlots = kCodeFit > 4 ? 4 : kCodeFit;
+    static constexpr int kCodeFit = (160 - kExchange - kRowSlots * kRowLoads) / kCodeLoads, kCodeSlots = kCodeFit > 4 ? 4 : kCodeFit;
     static constexpr int kRounds = KS == 1 ? 0 : (NT / 2 * kFragments + kExchange / 4 - 1) / (kExchange / 4);  // of the exchange
-    // The two waves of an exchange meet at the workgroup's barriers, which wait for the fetching waves too, or, up to 48
-    // rows, wait for each other alone: a barrier there cost 1.8 us of a short run (512 + 256 + 256 x 1088 at 32 rows 10.0 ->
-    // 8.5 us), while at 67 rows polling took more than the barriers (27B layer 107.2 and 109.4 us).
-    static constexpr bool kBarriers = KS == 2 && MF >= 4;
     static constexpr int kRowWaves = 2 * kRowLoads > 5 * kCodeLoads ? 3 : 2 * kCodeLoads > 3 * kRowLoads ? 1 : 2;
     static constexpr uint32_t kRowBytes = kRowLoads * 1024u, kCodeBytes = kCodeLoads * 1024u, kCodesAt = kRowSlots * kRowBytes;
-    static constexpr uint32_t kExchangeAt = kCodesAt + kCodeSlots * kCodeBytes, kWordsAt = kExchangeAt + kExchange * 1024u;
-    static constexpr uint32_t kLds = kWordsAt + (KS == 2 && MF < 4 ? 32u : 0u);
+    static constexpr uint32_t kExchangeAt = kCodesAt + kCodeSlots * kCodeBytes, kLds = kExchangeAt + kExchange * 1024u;
     static_assert(!PAIR || MF % 2 == 0, "value and remainder rows in fragments of their own");
     static_assert(kRowSlots >= 3 && kCodeSlots >= 3, "a unit ahead of the one that is read ahead, at least");
 };
@@ -142,7 +139,7 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
                 asm volatile("s_barrier" ::: "memory");
                 if (fetched < count) next(ring + slot);
                 slot = slot == (SLOTS - 1) * bytes ? 0u : slot + bytes;
-                if constexpr (S::kBarriers) {
+                if constexpr (KS == 2) {
                     if (--left != 0u) continue;
                     for (int j = 0; j < 2 * S::kRounds; ++j) asm volatile("s_barrier" ::: "memory");
                     left = T < count - 1u - i ? T : count - 1u - i;
@@ -304,8 +301,6 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
                      "s"(p.residual_dtype), "s"(p.residual_is_bias));
     };
     enter_block();
-    uint32_t exchanged = 0;  // rounds of it
-    if (KS == 2 && !S::kBarriers && threadIdx.x < 8u) ((uint32_t *)((char *)rows_lds + S::kWordsAt))[threadIdx.x] = 0u;
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     read_meta();
     read_codes(std::integral_constant<int, 0>());
@@ -363,30 +358,12 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
             constexpr int AT_ONCE = S::kExchange / 4;
             char *const mine = (char *)rows_lds + S::kExchangeAt + wave * (AT_ONCE * 1024u) + lane * 16u;
             const char *const theirs = (const char *)rows_lds + S::kExchangeAt + (wave ^ 1u) * (AT_ONCE * 1024u) + lane * 16u;
-            // Without barriers: LDS serves a wave's accesses in their order, so a word that counts rounds follows what it tells of;
-            // each wave writes its own two words, and both pass through the same rounds, so every wait ends.
-            volatile uint32_t *const words = (volatile uint32_t *)((char *)rows_lds + S::kWordsAt);
-            auto reached = [&](uint32_t word, uint32_t rounds_done) __attribute__((always_inline)) {
-                while (__builtin_amdgcn_readfirstlane(words[word]) - rounds_done > 0x7fffffffu) {
-                }
-                asm volatile("" ::: "memory");
-            };
             static_for<S::kRounds>([&](auto round_c) __attribute__((always_inline)) {
                 constexpr int from = AT_ONCE * decltype(round_c)::value, until = from + AT_ONCE < KEPT * OF ? from + AT_ONCE : KEPT * OF;
-                if constexpr (S::kBarriers)
-                    asm volatile("s_barrier" ::: "memory");  // the round before has been read
-                else
-                    reached(4u + (wave ^ 1u), exchanged);
+                asm volatile("s_barrier" ::: "memory");  // the round before has been read
 #pragma unroll
                 for (int e = from; e < until; ++e) *(floatx4 *)(mine + (e - from) * 1024) = acc[KEPT + e / OF][e % OF];
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                if constexpr (S::kBarriers) {
-                    asm volatile("s_barrier" ::: "memory");
-                } else {
-                    exchanged += 1u;
-                    words[wave] = exchanged;  // written
-                    reached(wave ^ 1u, exchanged);
-                }
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
                 for (int e = from; e < until; ++e) {
                     const floatx4 more = *(const floatx4 *)(theirs + (e - from) * 1024);
@@ -394,7 +371,6 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
                     for (int j = 0; j < 4; ++j) acc[e / OF][e % OF][j] += more[j];
                 }
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                if constexpr (!S::kBarriers) words[4u + wave] = exchanged;  // read
             });
         }
         const bool partial = begin != 0u || step != T;
