@@ -413,9 +413,12 @@ __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
                     }
                 }
             }
-        } else if (p.y_dtype == MI355Q_F32 && (p.residual == nullptr || p.residual_dtype == MI355Q_F32)) {
-            // the loads of a tile's residuals are on their way together
-            const bool wide = p.wide_stores && (uintptr_t)p.residual % 16u == 0u;
+        } else if (p.y_dtype == MI355Q_F32 && (p.residual == nullptr || p.residual_dtype == MI355Q_F32) &&
+                   (PAIR || (p.wide_stores && (uintptr_t)p.residual % 16u == 0u))) {
+            // The loads of a tile's residuals are on their way together.  Outputs without 16-byte pieces here, too, but of pairs
+            // only: with this code in the other forms the loop above came out 6 to 8 % slower (two of 13440 x 3840 at 35 rows
+            // 20.0 -> 21.9 us).
+            const bool wide = !PAIR || (p.wide_stores && (uintptr_t)p.residual % 16u == 0u);
             float scale[OF];
 #pragma unroll
             for (int f = 0; f < OF; ++f) {
