@@ -99,7 +99,7 @@ __device__ __forceinline__ void store_from_float(void *base, int dtype, size_t i
 }
 
 // Loads that write LDS directly (uniform base + 32-bit lane offset); lane l's bytes land at
-// lds_base + 16 l (4 l).  NT: use-once data.  m0 is named as clobbered so that the compiler
+// lds_base + 16 l.  NT: use-once data.  m0 is named as clobbered so that the compiler
 // carries no value of its own in it across the statement (it warns that m0 is reserved, which is
 // the point).
 #pragma clang diagnostic push
@@ -117,13 +117,6 @@ __device__ __forceinline__ void load_lds_x4(uint32_t lane_offset, const char *ba
                      :
                      : "v"(lane_offset), "s"(base), "s"(lds_base)
                      : "memory", "m0");
-}
-__device__ __forceinline__ void load_lds_x1(uint32_t lane_offset, const char *base, uint32_t lds_base)
-{
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
-                 :
-                 : "v"(lane_offset), "s"(base), "s"(lds_base)
-                 : "memory", "m0");
 }
 #pragma clang diagnostic pop
 
