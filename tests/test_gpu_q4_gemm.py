@@ -737,10 +737,12 @@ def test_targets_whose_plans_differ(engine, gpu, force, capfd, x_dtype, y_dtype,
         assert np.array_equal(one, by_itself) and np.array_equal(other, by_itself)
 
 
-def test_targets_in_one_launch_replayed(engine, gpu):
+@pytest.mark.parametrize("K", [3072, 1280])
+def test_targets_in_one_launch_replayed(engine, gpu, K):
     """Shared launches, their conversion and the sums behind their K splits from a recorded graph: every replay, with
-    eager calls of other sizes and new inputs between them, has the bits of the eager calls."""
-    kind, K = engine.META_BF16_PLANES, 3072
+    eager calls of other sizes and new inputs between them, has the bits of the eager calls.  At 1280 columns the fp32
+    call goes out by two kernels on one conversion."""
+    kind = engine.META_BF16_PLANES
     weights = [gpu.q4_prepare(*engine.synth_q4_affine(201 + i, 0.02, N, K, kind), N, K, kind) for i, N in enumerate((6144, 100, 1001))]
     shapes = [(300, engine.F16, np.float16), (150, engine.F32, np.float32)]
     x_ptrs = [gpu.alloc(M * K * 4) for M, _, _ in shapes]
