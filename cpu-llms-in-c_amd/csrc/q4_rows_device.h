@@ -1,8 +1,10 @@
 // Device code of the affine-Q4 linear for 17..128 rows of x: more rows than the streaming kernel
-// takes, too few to keep the matrix cores busy; and for more rows of fp32 activations by weights of short rows.  Bound by memory, by what a launch costs besides (the
-// second kernel behind shared blocks 4 to 6 us), and by power: with random operands a unit of 80 rows x 256 columns
-// takes 1.45 us, with zeros in x 1.35, with zeros in both 1.15, at which its loads and its arithmetic each take
-// 0.7 and 1.1 alone.
+// takes, too few to keep the matrix cores busy; and for 65..256 rows of fp32 activations by weights of short rows.
+// Bound by the multiplying waves' own chain of reads from LDS, dequantization and matrix instructions, one wave a SIMD (us,
+// two of 17408 x 5120 at 32 and 67 rows 32.2 and 44.4; without any load 32.2 and 44.2, without arithmetic 27.4 and
+// 38.3; with eight multiplying waves instead of four it took 5 % longer at 32 rows, 9 % at 48), by power (on another GPU 35.9 and 49.6;
+// with zeros in x 33.7 and 44.3, in x and the codes 32.0 and 41.5), and by what a launch costs besides (the second
+// kernel behind shared blocks 4 to 6 us).
 #pragma once
 #include "q4_gemm_device.h"
 
@@ -15,8 +17,8 @@ namespace mi355q {
 // 1.07 for the arithmetic, 1.75 together; without any wait for the data 1.68).
 // The multiplying waves share a unit as KS parts of its columns by 4 / KS groups of NT tiles.  With KS = 2 its rows are
 // read from LDS twice instead of four times, and two waves exchange halves of their sums when the block is done, at the
-// workgroup's barriers (a wait for the other wave alone, by polling a word in LDS: layers of 17 to 48 rows 0.7 % more time, of
-// 64 to 96 rows 1.2 %).
+// workgroup's barriers (a wait for the other wave alone, by polling a word in LDS: layers of 17 to 48 rows 0.9 % more time, of
+// 49 to 96 rows 1 to 1.6 %).
 template <int MF, int NT, int KS, bool PAIR>
 struct RowsShape {
     static constexpr int kTiles = 4 / KS * NT, kQuarters = 4 / KS;
