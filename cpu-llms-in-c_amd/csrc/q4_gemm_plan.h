@@ -346,27 +346,31 @@ struct RowsPlan {
 //
 // It is taken up to 1.05 times the other kernels' estimate for several weights of up to 96 matrix rows, 0.98 times of more
 // where they are large, and up to 0.89 times otherwise, 0.95 of 16-bit outputs of up to 64 rows: 0.1 to 0.7 % more time than
-// with the better of the two, above 96 rows 1 to 2 % (us from HBM and between large calls, this kernel and the others: 14336 x 5376 at 67 rows 24.3 and 30.7, 21.5 and
-// 29.4; 5120 x 6144 at 48 rows 15.4 and 16.0, 14.7 and 13.5; 17408 x 5120 at 112 rows 41 and 37; 6144 + 1024 + 1024 x 5120
-// at 67 rows 18.0 and 26.2, 17.9 and 23.0; two of 3584 x 1024 at 128 rows from the Infinity Cache 10.8 and 9.9, of 17408 x 5120 61.5 and 65.4
-// between large calls).
+// with the better of the two, above 96 rows 1 to 2 % (us from HBM and between large calls, this kernel and the others:
+// 14336 x 5376 at 67 rows 24.3 and 30.7, 21.5 and 29.4; 5120 x 6144 at 48 rows 15.4 and 16.0, 14.7 and 13.5; 17408 x 5120
+// at 112 rows 41 and 37; 6144 + 1024 + 1024 x 5120 at 67 rows 18.0 and 26.2, 17.9 and 23.0; two of 3584 x 1024 at 128 rows
+// from the Infinity Cache 10.8 and 9.9; two of 17408 x 5120 at 128 rows between large calls 61.5 and 65.4).
 // A unit, by tiles a block (4, 8, 16) and fragments:
 constexpr double kRowsUnitUs[3][9] = {{0, 0, 0.327, 0.380, 0.389, 0.434, 0.483, 0, 0.733},
                                       {0, 0, 0.425, 0.506, 0.622, 0.647, 0.733, 0, 0.971},
                                       {0, 0, 0.782, 0.873, 0.991, 1.123, 1.186, 0, 1.382}};
+
 // A launch of T steps a block, without the conversion and the outputs.
 inline double rows_launch_us(uint32_t cus, uint32_t T, double outputs, const RowsPlan &plan)
 {
-    const uint32_t total = plan.blocks * T, units = plan.units, groups = (total + units - 1u) / units, rounds = (groups + cus - 1u) / cus;
+    const uint32_t total = plan.blocks * T, units = plan.units, groups = (total + units - 1u) / units;
+    const uint32_t rounds = (groups + cus - 1u) / cus;
     const bool sharing = units % T != 0u && units < total;
     const double mf = plan.mf, tiles = plan.tiles, filled = (double)groups / ((double)rounds * cus);
-    const double unit = std::max(kRowsUnitUs[plan.tiles / 8][plan.mf] * (1.0 + 0.0227 * mf * (filled - 0.75)), 0.051 * tiles * filled + 0.0483 * mf);
+    const double unit = std::max(kRowsUnitUs[plan.tiles / 8][plan.mf] * (1.0 + 0.0227 * mf * (filled - 0.75)),
+                                 0.051 * tiles * filled + 0.0483 * mf);
     // ends of blocks in the longest run, and workgroups that share a block
     const double ends = !sharing ? std::max(1u, units / T) : T % units == 0u ? 1.0 : (units - 2u) / T + 2u;
     const double sharers = T % units == 0u ? T / units : (T + units - 1.0) / units;
     const double us = 3.78 + rounds * (units * unit + ends * (plan.pair ? 0.0119 : 0.0237) * mf * tiles);
     return sharing ? us + 3.21 + sharers * (0.0781 + 1.53e-6 * outputs) : us;
 }
+
 inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t rows, double others_us, RowsPlan &plan)
 {
     const Q4Device &first = *a.targets[0].w;
@@ -428,7 +432,7 @@ inline bool rows_plan(const mi355q_context *ctx, const Q4LinearArgs &a, uint32_t
 // A weight has the bits of its own call in company, so it takes this kernel whatever shares the call: by the rows and
 // columns of x, which the weights of a call have in common, and not by an estimate of its own call, which parted
 // calls in two launches with a conversion each (2688 + 128 x 1280 at 319 rows 22 -> 33 us).  Weights more than four times as wide
-// as x, which no other of its layer is, are left out, and a call that has both kinds is the one that is parted.
+// as x are left out (those of an encoder's or a decoder's layer are not as wide); a call that has both kinds is parted.
 // More rows or wider weights fill the chip with the other kernels' larger blocks: calls whose outputs were more than 512 times
 // the columns of x lost at times (28440 x 384 at 152 rows 20 -> 27, 5120 x 1280 at 1345 rows 55 -> 64).  Of more than 14 steps
 // the others split K into more sums than this kernel's two, whose error is smaller.

@@ -61,7 +61,7 @@ struct RowsShape {
 // PAIR: x is 2 M rows, value and rounding remainder of each of the M rows (of fp32 activations);
 // a block's value rows lie in the first half of its stage, their remainders in the second.  Each has accumulators of its
 // own, which are added when the block is done: in one accumulator a row's products were rounded twice as often (relative
-// error against 64 bits of 1.8 to 2.8e-7 where it is 1.3 to 2.0e-7 now, K of 1216 to 2112; 0.6 % of a call's time).
+// error against 64 bits of 2.4 to 3.0e-7 where it is 1.7 to 2.1e-7 now, K of 1216 to 2112; 0.7 % of a call's time).
 template <int MF, int NT, int KS, bool PAIR>
 __global__ void __launch_bounds__(512, 2) q4_rows_kernel(const GemmGroup group)
 {
