@@ -468,7 +468,7 @@ inline uint32_t plan_pairs(const mi355q_context *ctx, const Q4LinearArgs &a, boo
         for (uint32_t t = 0; t < a.count; ++t)
             if (taken[t]) at.blocks += (a.targets[t].w->NT + tiles - 1u) / tiles * at.m_blocks;
         at.units = (at.blocks + cus - 1u) / cus * T;
-        return mf * tiles <= 64 && (mf > 2 || tiles == 4);  // (else a wave takes whole columns)
+        return mf * tiles <= 64;  // (else a wave takes whole columns)
     };
     if (ctx->force_gemm[1] >= 1) {
         // option "q4_gemm": 11, 12, 13 = 4, 8, 16 tiles a block; s = 1 .. 4 for 16 to 64 rows, 5 .. 8 for two blocks a workgroup, ...

@@ -492,10 +492,10 @@ static hipError_t launch_rows_of(mi355q_context *ctx, int mf, bool pair, uint32_
     auto of = [&](auto mf_c, auto pair_c) {
         constexpr int MF = decltype(mf_c)::value;
         constexpr bool PAIR = decltype(pair_c)::value;
-        // whole columns to a wave: up to 48 rows by 8 and 16 tiles, whose reading from LDS is cheaper than an exchange (us,
-        // 5120 x 6144 at 32 rows 13.6 and 14.4, 512 + 256 + 256 x 1088 8.1 and 10.3), and 96 and 128 rows by 16 tiles, for the
-        // accumulators' sake
-        constexpr int SPLIT = (NT >= 4 && MF <= 3) || (NT == 8 && MF >= 6) ? 2 : 1;
+        // whole columns to a wave: up to 32 rows of 16-bit activations by 8 and 16 tiles, whose reading from LDS is cheaper than
+        // an exchange (layers of 17 to 32 rows 0.8 % less time, of 33 to 48 0.8 % more, fp32 calls of 9 to 16 as much and a
+        // larger error), and 96 and 128 rows by 16 tiles, for the accumulators' sake
+        constexpr int SPLIT = (NT >= 4 && MF == 2 && !PAIR) || (NT == 8 && MF >= 6) ? 2 : 1;
         typedef RowsShape<MF, NT / SPLIT, KS / SPLIT, PAIR> S;
         bool &raised = ctx->rows_lds_raised[MF - 1][PAIR][S::kTiles / 8];
         const auto kernel = q4_rows_kernel<MF, NT / SPLIT, KS / SPLIT, PAIR>;

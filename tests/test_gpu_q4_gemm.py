@@ -351,7 +351,7 @@ def test_rows_kernel_pairs(engine, oracle, gpu, force, forced, N, K, M):
     run_case(engine, oracle, gpu, N, K, M, engine.META_F16_INTERLEAVED, engine.F32, engine.F32)
 
 
-@pytest.mark.parametrize("forced,M,parts", [("11,1", 16, 2), ("12,1", 16, 1), ("13,1", 16, 1), ("11,1", 32, 2), ("12,1", 32, 2),
+@pytest.mark.parametrize("forced,M,parts", [("11,1", 16, 2), ("12,1", 16, 2), ("13,1", 16, 2), ("11,1", 32, 2), ("12,1", 32, 2),
                                             ("13,1", 32, 2), ("11,1", 48, 2), ("12,1", 64, 2), ("13,1", 64, 1)])
 @pytest.mark.parametrize("K", [1280, 5120])
 def test_rows_kernel_pairs_precision(engine, oracle, gpu, force, forced, parts, M, K):
@@ -423,7 +423,7 @@ def test_pairs_of_many_rows(engine, oracle, gpu, force, capfd, K, widths, by_row
 
 
 @pytest.mark.parametrize("forced,tiles,rows,blocks", [
-    ("11,1", 4, 16, 1), ("11,6", 4, 32, 2), ("11,11", 4, 48, 3), ("11,8", 4, 64, 2), ("12,2", 8, 32, 1), ("12,10", 8, 32, 3),
+    ("11,1", 4, 16, 1), ("12,9", 8, 16, 3), ("13,5", 16, 16, 2), ("11,6", 4, 32, 2), ("11,11", 4, 48, 3), ("11,8", 4, 64, 2), ("12,2", 8, 32, 1), ("12,10", 8, 32, 3),
     ("12,7", 8, 48, 2), ("12,12", 8, 64, 3), ("13,2", 16, 32, 1), ("13,6", 16, 32, 2), ("13,10", 16, 32, 3)])
 @pytest.mark.parametrize("y_dtype,residual_dtype,shift", [("F32", "F32", 0), ("F32", "F32", 1), ("F32", "F16", 0), ("F16", "F32", 0),
                                                           ("BF16", "BF16", 1), ("F32", None, 0)])
